@@ -1,0 +1,258 @@
+// The float32 matrix product for gfx950: out[M, N] (+)= x[M, K] . w[N, K]^T on v_mfma_f32_16x16x4_f32, whose
+// products and sums are float32 (the same precision as multiply-adds on the vector units, at four times the rate a
+// plain tile reached there). It carries every projection of the 32-bit path; operands of mixed types and rows that
+// are no multiple of four floats go to gemm_generic.
+//
+// A wave owns MT tiles of 16 rows of x and NT tiles of 16 rows of w over one range of K and walks it in blocks of 16 k,
+// 1 KB of a tile: one 16-byte load a lane, four lanes on the 64 bytes of a row. The matrix instruction wants rows side
+// by side in lanes instead; loaded so, a load costs the vector cache about 65 cycles and not 16, which held 64 x 64
+// tiles to half of what the matrix cores give. So a block passes through LDS, in a place of the wave's own: written as
+// loaded, read by lane l at row l % 16 and floats 4 (l / 16) .. + 3, the places of a row's four pieces exchanged by
+// row / 4 so that neither way meets a bank twice. Four instructions take one of the four floats each - which k an
+// instruction sums is a permutation that both operands share.
+// The WK waves of a workgroup share one tile and cut its range of K between them, without a barrier on the way; their
+// sums meet in LDS and are added in the order of the waves. Where tiles are too few for the chip, K is cut over
+// workgroups as well and planes of partial sums are left for the consumer, who adds them in order. No atomics: every
+// sum's order follows from the sizes.
+//
+// Few rows are bound by the stream of w (4 bytes a weight): U blocks a wave are asked for while it works on U others;
+// many rows are bound by the matrix cores (157 TFLOP/s). Measured over 12288 x 2048: 1 row 19.8 us (5.1 TB/s), 301 rows
+// 150 us (101 TFLOP/s), 1000 rows 443 us (114 TFLOP/s); straight from memory into the operand registers, without LDS, the
+// same took 24.4, 200 and 602 us. The products of a 28-layer model 2048 wide: a step of four tokens 1.7 ms, 37.1 on the
+// plain tile (gemm_generic); a prompt of 301 tokens 10.1 ms, 48.5 there. Against 64 bits a sum over 16 to 48 chains is
+// off by half of what one chain is.
+#include "common.h"
+
+#include <math.h>
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+template <bool STREAM>
+__device__ __forceinline__ f32x4_t gf_load(const float* p) {
+  if (STREAM) return __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(p));
+  return *reinterpret_cast<const f32x4_t*>(p);
+}
+
+template <int MT, int NT, int WK, int U>
+__global__ __launch_bounds__(WK* TIE_WAVE) void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                float* __restrict__ out, int M, int N, int K,
+                                                                int accumulate, int gated, int splits, int row_tiles) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr bool STREAM = MT == 1;       // w is read once: past the caches
+  constexpr int STAGED = U * (MT + NT), SUMS = MT * NT;      // pieces of 1 KB a wave holds in LDS on the way, at the end
+  __shared__ f32x4_t lds[WK][STAGED > SUMS ? STAGED : SUMS][TIE_WAVE];
+  // Workgroups go to the eight dies in turn. The row tiles of one piece of w follow each other on one die, so that w
+  // comes from memory once and from that die's cache afterwards.
+  const int turn = blockIdx.x / 8;
+  const int unit = turn / row_tiles * 8 + blockIdx.x % 8;
+  const int col_tiles = (N + 16 * NT - 1) / (16 * NT);
+  if (unit >= col_tiles * splits) return;
+  const int t0 = turn % row_tiles * (16 * MT);
+  const int n0 = unit / splits * (16 * NT);
+  const int split = unit % splits;
+
+  const int lane = threadIdx.x & (TIE_WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TIE_WAVE);
+  const int row_in = lane / 4, piece_in = (lane % 4) ^ (lane / 16);              // what this lane loads of a tile's block
+  const int from = 4 * (lane % 16) + ((lane / 16) ^ (lane % 16 / 4));            // whose loaded piece it multiplies
+  const int blocks = (K + 15) / 16;
+  const int per = (blocks + splits * WK - 1) / (splits * WK);
+  const int begin = min(blocks, (split * WK + wave) * per);
+  const int end = min(blocks, begin + per);
+
+  // Rows beyond the operands' last are that row again: their sums are not stored.
+  const float* wb = w + static_cast<size_t>(n0) * K;
+  const float* xb = x + static_cast<size_t>(t0) * K;
+  unsigned wo[NT], xo[MT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) wo[j] = static_cast<unsigned>(min(16 * j + row_in, N - 1 - n0)) * static_cast<unsigned>(K);
+#pragma unroll
+  for (int m = 0; m < MT; ++m) xo[m] = static_cast<unsigned>(min(16 * m + row_in, M - 1 - t0)) * static_cast<unsigned>(K);
+
+  f32x4_t acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[m][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  f32x4_t aw[U][NT], ax[U][MT];          // what has been asked for
+  auto ask = [&](int first) {            // blocks behind the range's end: its last one again
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const unsigned k = min(16 * min(first + u, end - 1) + 4 * piece_in, K - 4);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) aw[u][j] = gf_load<STREAM>(wb + (wo[j] + k));
+#pragma unroll
+      for (int m = 0; m < MT; ++m) ax[u][m] = gf_load<false>(xb + (xo[m] + k));
+    }
+  };
+  auto stage = [&]() {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) lds[wave][u * (MT + NT) + j][lane] = aw[u][j];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) lds[wave][u * (MT + NT) + NT + m][lane] = ax[u][m];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");     // the wave's own lanes only: nothing to wait for
+  };
+  auto multiply = [&](int u) {
+    f32x4_t bw[NT], bx[MT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) bw[j] = lds[wave][u * (MT + NT) + j][from];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) bx[m] = lds[wave][u * (MT + NT) + NT + m][from];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bw[j][i], bx[m][i], acc[m][j], 0, 0, 0);
+  };
+
+  // Whole batches of U whole blocks; the next batch's loads are in flight behind this one's instructions.
+  const int whole = max(0, min(end, K / 16) - begin) / U;
+  const int rest = begin + whole * U;
+  if (begin < end) ask(begin);
+  for (int b = 1; b <= whole; ++b) {
+    stage();
+    if (begin + b * U < end) ask(begin + b * U);
+#pragma unroll
+    for (int u = 0; u < U; ++u) multiply(u);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  if (rest < end) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (16 * (rest + u) + 4 * piece_in >= K) {       // a K that ends inside a block: nothing from behind its end
+#pragma unroll
+        for (int j = 0; j < NT; ++j) aw[u][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < MT; ++m) ax[u][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+    stage();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (rest + u < end) multiply(u);
+  }
+
+  // Lane l of a tile's sums: row l % 16 of x, rows 4 (l / 16) .. + 3 of w.
+  float* plane = out + static_cast<size_t>(split) * M * N;
+  auto store = [&](int m, int j, int at, f32x4_t v) {
+    const int t = t0 + 16 * m + at % 16;
+    const int n = n0 + 16 * j + at / 16 * 4;
+    if (t >= M || n >= N) return;
+    float* o = plane + static_cast<size_t>(t) * N + n;
+    if (N % 4 == 0) {
+      f32x4_t* o4 = reinterpret_cast<f32x4_t*>(o);
+      *o4 = accumulate ? *o4 + v : v;
+    } else {
+      for (int i = 0; i < 4 && n + i < N; ++i) o[i] = accumulate ? o[i] + v[i] : v[i];
+    }
+  };
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) lds[wave][m * NT + j][lane] = acc[m][j];      // over the wave's own blocks
+  __syncthreads();
+  for (int tile = wave; tile < MT * NT; tile += WK) {
+    f32x4_t v = lds[0][tile][lane];
+#pragma unroll
+    for (int k = 1; k < WK; ++k) v += lds[k][tile][lane];
+    if (!gated) {
+      store(tile / NT, tile % NT, lane, v);
+      continue;
+    }
+    // A tile of w is 8 rows of gates and the 8 rows of ups that go with them: lane l holds gates 4 (l / 16) .. + 3 up to
+    // lane 31, the ups of lane l - 32 from there on.
+    f32x4_t up;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) up[i] = __shfl_down(v[i], 32, TIE_WAVE);
+    const int t = t0 + 16 * (tile / NT) + lane % 16;
+    const int n = n0 + 16 * (tile % NT);
+    if (lane >= 32 || t >= M || n >= N) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = (gated == 1 ? v[i] / (1.0f + expf(-v[i])) : gelu_tanh_exact(v[i])) * up[i];
+    *reinterpret_cast<f32x4_t*>(out + static_cast<size_t>(t) * (N / 2) + n / 2 + lane / 16 * 4) = v;
+  }
+#endif
+}
+
+// The shapes a workgroup comes in: tiles of 16 rows of x and of w, waves along K. Blocks asked for at a time: enough for
+// 4 to 12 KB a wave in flight, which LDS still holds for two workgroups a compute unit.
+struct GfShape { int mt, nt, wk; };
+static const GfShape GF_SHAPES[] = {{1, 1, 8}, {1, 2, 8}, {2, 1, 8}, {2, 2, 8}, {3, 2, 4}, {2, 4, 4}, {3, 4, 4}, {4, 4, 4}};
+#define GF_COUNT static_cast<int>(sizeof(GF_SHAPES) / sizeof(GF_SHAPES[0]))
+#define GF_MAX_SPLITS 16
+
+struct GfPlan { int shape, splits; };
+
+// The cheapest (shape, ranges of K) by an estimate of the time in microseconds: workgroups run in rounds of one a compute
+// unit, a round takes the matrix instructions of its range at full rate and the vector cache's time for its operands;
+// then w once from memory and the planes' way out, and back in at their reader. The factors are a least-squares fit to
+// 5 600 timed products of 1 to 1000 rows over seven weights of 1024 x 1024 to 12288 x 2048 (13 % root mean square); the
+// choice lies 5 % above the best timed candidate on average, 30 % at worst.
+static GfPlan gf_plan(int M, int N, int K, int splits_fixed) {
+  GfPlan best = {0, splits_fixed > 0 ? splits_fixed : 1};
+  double best_time = 0.0;
+  for (int splits = 1; splits <= 8; splits *= 2) {
+    if (splits_fixed > 0) splits = splits_fixed;
+    else if (splits > 1 && K / splits < 256) break;      // shorter ranges are all beginning and end
+    for (int i = 0; i < GF_COUNT; ++i) {
+      const GfShape s = GF_SHAPES[i];
+      const double k = static_cast<double>(K) / splits;
+      const double workgroups = static_cast<double>((M + 16 * s.mt - 1) / (16 * s.mt)) * ((N + 16 * s.nt - 1) / (16 * s.nt)) * splits;
+      const double rounds = ceil(workgroups / 256.0);
+      const double multiply = k / 4 * s.mt * s.nt * 32 / 4 / 2400;            // 32 cycles an instruction, four SIMDs
+      const double load = (s.mt + s.nt) * 64.0 * k / 64 / 2400;              // 64 bytes a cycle
+      const double plane = static_cast<double>(M) * N * 4 / 6.67e6;
+      const double time = 2.8 + rounds * (0.88 * multiply + 1.32 * load + 0.31) + 0.58 * N * 4.0 * K / 6.67e6 +
+                          2.3 * splits * plane + 1.33 * (splits - 1) * plane;
+      if (best_time == 0.0 || time < best_time) {
+        best = {i, splits};
+        best_time = time;
+      }
+    }
+    if (splits_fixed > 0) break;
+  }
+  return best;
+}
+
+// Ranges of K the product is best cut into when its caller adds planes of partial sums.
+extern "C" int tie_gemm_f32_splits(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? gf_plan(M, N, K, 0).splits : 1; }
+
+// splits > 1: out is [splits][M][N] planes of partial sums. gated 1 or 2: w's rows are 8 gates and 8 ups in turn, out is
+// [M][N / 2] and receives silu(gate) * up or gelu_tanh(gate) * up. shape: 0 lets the plan choose, otherwise entry shape - 1.
+extern "C" int tie_gemm_f32(const float* x, const float* w, float* out, int accumulate, int gated, int M, int N, int K,
+                            int splits, int shape, hipStream_t stream) {
+  if (M <= 0 || N <= 0 || K < 4 || K % 4 != 0 || K > (1 << 24) || splits < 1 || splits > GF_MAX_SPLITS ||
+      (splits > 1 && accumulate) || shape < 0 || shape > GF_COUNT || gated < 0 || gated > 2 ||
+      (gated && (accumulate || splits > 1 || N % 16 != 0)))
+    return TIE_BAD_ARGUMENT;
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) % 16 != 0)
+    return TIE_BAD_ARGUMENT;
+  const int chosen = shape > 0 ? shape - 1 : gf_plan(M, N, K, splits).shape;
+  const GfShape s = GF_SHAPES[chosen];
+  const int row_tiles = (M + 16 * s.mt - 1) / (16 * s.mt);
+  const long units = static_cast<long>((N + 16 * s.nt - 1) / (16 * s.nt)) * splits;
+  const long grid = (units + 7) / 8 * 8 * row_tiles;
+  if (grid > 0x7fffffffL) return TIE_BAD_ARGUMENT;
+#define LAUNCH(MT, NT, WK, U)                                                                                    \
+  gemm_f32_kernel<MT, NT, WK, U><<<static_cast<unsigned>(grid), WK * TIE_WAVE, 0, stream>>>(                     \
+      x, w, out, M, N, K, accumulate, gated, splits, row_tiles)
+  switch (chosen) {
+    case 0: LAUNCH(1, 1, 8, 4); break;
+    case 1: LAUNCH(1, 2, 8, 2); break;
+    case 2: LAUNCH(2, 1, 8, 2); break;
+    case 3: LAUNCH(2, 2, 8, 2); break;
+    case 4: LAUNCH(3, 2, 4, 2); break;
+    case 5: LAUNCH(2, 4, 4, 2); break;
+    case 6: LAUNCH(3, 4, 4, 2); break;
+    case 7: LAUNCH(4, 4, 4, 1); break;
+    default: return TIE_BAD_ARGUMENT;
+  }
+#undef LAUNCH
+  return tie_launch_status();
+}

@@ -52,6 +52,7 @@ _SOURCES = {
     "elementwise": ("tie_elementwise", "elementwise.hip"),
     "gemm_generic": ("tie_gemm_generic", "gemm_generic.hip"),
     "attention_generic": ("tie_attention_generic", "attention_generic.hip"),
+    "gemm_f32": ("tie_gemm_f32", "gemm_f32.hip"),
     "skinny_gemm_bf16": ("tie_skinny_gemm_bf16", "skinny_gemm_bf16.hip"),
     "gemm_bf16": ("tie_gemm_bf16", "gemm_bf16.hip"),
     "sample_filtered": ("tie_sample_filtered", "sample_filtered.hip"),
@@ -136,6 +137,10 @@ _SIGNATURES = {
     "gemm_generic": {
         "tie_gemm_generic": [_c_void, _c_int, _c_void, _c_int, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int,
                              _c_void],
+    },
+    "gemm_f32": {
+        "tie_gemm_f32_splits": [_c_int, _c_int, _c_int],
+        "tie_gemm_f32": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
     },
     "attention_generic": {
         "tie_paged_attention_generic": [_c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_int, _c_void, _c_void,
@@ -692,6 +697,41 @@ def gemm_generic(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate
         _code(out, "matmul output"), int(accumulate), T, N, K, _stream())
 
 
+def gemm_f32_takes(x, w, out) -> bool:
+    """Whether ``gemm_f32`` takes these operands: float32 throughout, rows of whole 16-byte pieces."""
+    return x.dtype == torch.float32 and w.dtype == torch.float32 and out.dtype == torch.float32 and \
+        x.shape[1] % 4 == 0 and 4 <= x.shape[1] <= (1 << 24) and \
+        (x.data_ptr() | w.data_ptr() | out.data_ptr()) % 16 == 0
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_f32_splits(M: int, N: int, K: int) -> int:
+    """Ranges of K a float32 product is best cut into when its caller adds planes of partial sums."""
+    return int(_lib("gemm_f32").tie_gemm_f32_splits(M, N, K))
+
+
+def gemm_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool = False, splits: int = 1,
+             shape: int = 0, gated: int = 0) -> None:
+    """out (+)= x @ w.T for float32 operands on the float32 matrix instructions; K % 4 == 0 (``gemm_f32_takes``).
+
+    ``splits`` > 1: out is ``[splits, M, N]`` and receives one plane of partial sums per range of K. ``shape`` picks a
+    workgroup shape of csrc/gemm_f32.hip (1 to 8); 0 lets its plan choose. ``gated`` 1 + an activation's number: w is a
+    gate/up pair interleaved by ``interleave_gate_up`` and out ``[M, N / 2]`` receives act(gate) * up."""
+    _gpu(x, "matmul input")
+    _gpu(w, "matmul weight")
+    _gpu(out, "matmul output")
+    M, K = x.shape
+    N, K2 = w.shape
+    want = (M, N // 2) if gated else (splits, M, N) if splits > 1 else (M, N)
+    if K != K2 or tuple(out.shape) != want or (splits > 1 and accumulate) or (gated and (splits > 1 or accumulate or N % 16)):
+        raise InvalidArgument(f"matmul: input {list(x.shape)}, weight {list(w.shape)}, output {list(out.shape)}, {splits} "
+                              f"ranges of K, accumulate={accumulate}")
+    if not gemm_f32_takes(x, w, out):
+        raise InvalidArgument("gemm_f32 takes float32 operands on 16-byte addresses with K % 4 == 0")
+    _call(_lib("gemm_f32").tie_gemm_f32, "gemm_f32", x.data_ptr(), w.data_ptr(), out.data_ptr(), int(accumulate),
+          int(gated), M, N, K, int(splits), int(shape), _stream())
+
+
 class PackedWeight:
     """A bfloat16 ``[N, K]`` weight stored as ``[N/16][K/32]`` blocks of 1 KB in the matrix cores' operand order.
 
@@ -914,11 +954,13 @@ def decode_product_rows(M: int, w, gated: bool = False) -> bool:
 
 def linear_swiglu(x: torch.Tensor, w_interleaved: torch.Tensor, out: torch.Tensor,
                   row_scale: Optional[RowScale] = None, activation: str = "silu") -> None:
-    """out = act(x @ gate.T) * (x @ up.T) in one product over the interleaved weight; bfloat16 only.
+    """out = act(x @ gate.T) * (x @ up.T) in one product over the interleaved weight; bfloat16 or float32 operands.
     ``row_scale`` as in ``skinny_gemm_bf16`` (up to ``NORM_EPILOGUE_ROWS`` rows); ``activation`` "silu" or
     "gelu_tanh"."""
     gated = 1 + GATE_ACTIVATIONS[activation]
-    if decode_product_rows(x.shape[0], w_interleaved, gated=True):
+    if w_interleaved.dtype == torch.float32:
+        gemm_f32(x, w_interleaved, out, gated=gated)
+    elif decode_product_rows(x.shape[0], w_interleaved, gated=True):
         skinny_gemm_bf16(x, w_interleaved, out, gated=gated, row_scale=row_scale)
     elif row_scale is not None:
         raise InvalidArgument(f"{x.shape[0]} rows without their norm's factor: only the decode product applies it")
@@ -957,6 +999,8 @@ def linear(x: torch.Tensor, w, out: torch.Tensor, accumulate: bool = False, row_
     elif isinstance(w, PackedWeight):
         raise InvalidArgument(f"a packed weight is read by the bfloat16 products only: input {x.dtype}, output "
                               f"{out.dtype}, accumulate={accumulate}")
+    elif gemm_f32_takes(x, w, out):
+        gemm_f32(x, w, out, accumulate)
     else:
         gemm_generic(x, w, out, accumulate)
 

@@ -35,9 +35,11 @@ FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC", "-shared",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"]
 
 # Flags of single sources. The attention kernels rescale their output accumulators with ordinary
-# multiplications between matrix instructions: these then work on vector registers directly.
-SOURCE_FLAGS = {"attention_prefill_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
-                "attention_decode_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+# multiplications between matrix instructions: these then work on vector registers directly. The float32 product's
+# accumulators, up to 64 registers, are otherwise copied between the two register files at the ends of its loop.
+_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+SOURCE_FLAGS = {"attention_prefill_bf16.hip": _VGPR_FORM, "attention_decode_bf16.hip": _VGPR_FORM,
+                "gemm_f32.hip": _VGPR_FORM}
 
 _loaded: Dict[str, ctypes.CDLL] = {}
 _lock = threading.Lock()

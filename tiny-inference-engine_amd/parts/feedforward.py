@@ -59,6 +59,7 @@ import torch
 
 from .. import kernels
 from ..errors import InvalidArgument, UnsupportedError
+from ..weights.binder import BFLOAT16
 from .base import FeedForward, StepContext, TensorSpec, register_part
 from .linear import Linear
 
@@ -88,9 +89,9 @@ class SwiGLU(FeedForward):
     def load(self, fetch, mode, device) -> None:
         self.down.load(fetch)
         gate, up = fetch(self.gate_up.names[0], "matrix"), fetch(self.gate_up.names[1], "matrix")
-        # bfloat16 weights and widths in steps of 8: gate and up rows are interleaved so that one
+        # Weights in the activations' own type and widths in steps of 8: gate and up rows are interleaved so that one
         # product computes both and its epilogue applies silu(gate) * up before anything is stored.
-        self.fused = gate.dtype == torch.bfloat16 and up.dtype == torch.bfloat16 and \
+        self.fused = gate.dtype == up.dtype == (torch.bfloat16 if mode == BFLOAT16 else torch.float32) and \
             self.intermediate % 8 == 0 and self.hidden % 8 == 0
         if self.fused:
             self.gate_up.set_weight(kernels.interleave_gate_up(gate, up))
@@ -100,7 +101,7 @@ class SwiGLU(FeedForward):
     def forward(self, ctx: StepContext, h: torch.Tensor, residual: Optional[torch.Tensor]):
         T = h.shape[0]
         act = ctx.scratch("swiglu.act", (T, self.intermediate))
-        if self.fused and h.dtype == torch.bfloat16:
+        if self.fused and h.dtype == self.gate_up.weight.dtype:
             kernels.linear_swiglu(h, self.gate_up.weight, act, row_scale=Linear.row_scale_for(ctx, h, self.gate_up.weight),
                                   activation=self.activation)
         else:

@@ -158,10 +158,18 @@ class Linear:
 
         The decode product decides by the weight's shape alone up to 16 rows and by its plan for the number of rows
         above (up to 32 rows, or 64 where the tiled product is not the faster); the tiled product is cut along K
-        when its tiles alone would leave most of the GPU idle.
+        when its tiles alone would leave most of the GPU idle, and so is the float32 product.
         """
         M, K = x.shape
         w = self.weight
+        if x.dtype == torch.float32 and w.dtype == torch.float32 and K % 4 == 0 and (self.bias is None or bias_added):
+            splits = kernels.gemm_f32_splits(M, w.shape[0], K)
+            if splits > 1:
+                planes = ctx.scratch(name, (splits, M, w.shape[0]), torch.float32)
+                if kernels.gemm_f32_takes(x, w, planes):
+                    kernels.gemm_f32(x, w, planes, splits=splits)
+                    return planes
+            return None
         if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or K % 8 or (self.bias is not None and not bias_added):
             return None      # planes hold the product alone: a bias must have gone to the target already
         decode_product = kernels.decode_product_rows(M, w)
