@@ -1,11 +1,11 @@
 """The float32 kernels on the matrix cores against float64: every workgroup shape of the product at the edges of its
-tiles and of K."""
+tiles and of K, and the attention over all head sizes, groups, masks, caps, sinks, page types and shares."""
 
 import pytest
 import torch
 
 import plain_qwen3 as plain
-from test_gpu_kernels import close, rnd
+from test_gpu_kernels import attention_case, close, rnd
 
 pytestmark = pytest.mark.gpu
 F64 = torch.float64
@@ -73,8 +73,92 @@ def test_gemm_f32_keeps_a_bad_row_to_itself():
         assert torch.equal(out[keep[0]][:, keep[1]], good[keep[0]][:, keep[1]])
 
 
+def run(case, H, S, Dh, nsplit=1, **more):
+    from tie_amd import kernels
+
+    KVH = case["kc"].shape[1]
+    new = (case["query_start"][1:] - case["query_start"][:-1]).tolist()
+    q = case["q"]
+    out = torch.full_like(q, float("nan"))
+    part_o = torch.full((q.shape[0] * H * nsplit * Dh,), float("nan"), device="cuda")
+    part_ml = torch.full((q.shape[0] * H * nsplit * 2,), float("nan"), device="cuda")
+    kernels.attention_f32(q, case["kc"], case["vc"], out, case["query_start"], case["context_lens"], case["tables"],
+                          kernels.attention_f32_tiles(new, H // KVH), H, Dh ** -0.5, nsplit=nsplit,
+                          part_o=part_o if nsplit > 1 else None, part_ml=part_ml if nsplit > 1 else None, **more)
+    return out
+
+
+@pytest.mark.parametrize("nsplit", [1, 2, 16])
+@pytest.mark.parametrize("H,KVH,Dh,bs", [(4, 2, 16, 16), (6, 2, 32, 16), (3, 1, 48, 32), (4, 4, 64, 16), (5, 5, 80, 16),
+                                         (14, 2, 96, 64), (16, 1, 112, 16), (16, 8, 128, 16), (20, 1, 144, 16),
+                                         (40, 2, 192, 16), (2, 1, 256, 16)])
+def test_attention_f32_mixed_batch(H, KVH, Dh, bs, nsplit):
+    # a whole prompt, a portion that continues a cached prefix, single decoded tokens, a one-token prompt
+    case, S = attention_case(H, KVH, Dh, bs, lens_new=[13, 37, 1, 1, 1], lens_ctx=[13, 61, 40, 300, 1], seed=3)
+    close(run(case, H, S, Dh, nsplit), case["want"], 1e-5, f"attention H={H} KVH={KVH} Dh={Dh}, {nsplit} shares")
+
+
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_attention_f32_many_sequences(nsplit):
+    """More sequences than a wave has lanes, single tokens and portions mixed; then single tokens alone."""
+    new = [1 + (i * 7) % 5 for i in range(70)]
+    case, S = attention_case(4, 2, 32, 16, lens_new=new, lens_ctx=[n + (i * 13) % 90 for i, n in enumerate(new)], seed=4)
+    close(run(case, 4, S, 32, nsplit), case["want"], 1e-5, "seventy sequences")
+    case, S = attention_case(4, 2, 32, 16, lens_new=[1] * 70, lens_ctx=[1 + i for i in range(70)], seed=5)
+    close(run(case, 4, S, 32, nsplit), case["want"], 1e-5, "seventy single tokens")
+
+
+@pytest.mark.parametrize("nsplit", [1, 4])
+@pytest.mark.parametrize("window", [1, 5, 16, 17, 100])
+def test_attention_f32_window_edges(window, nsplit):
+    case, S = attention_case(4, 2, 16, 16, lens_new=[9, 1, 20], lens_ctx=[30, 141, 20], seed=7, window=window)
+    close(run(case, 4, S, 16, nsplit, window=window), case["want"], 1e-5, f"window {window}")
+
+
+@pytest.mark.parametrize("more", [{"chunk": 1}, {"chunk": 24}, {"softcap": 5.0}, {"sinks": True}, {"chunk": 24, "sinks": True},
+                                  {"window": 20, "softcap": 2.0, "sinks": True}])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("nsplit", [1, 5])
+def test_attention_f32_against_the_generic_kernel(more, dtype, nsplit):
+    """Chunks, caps, sinks and narrow pages: the same as the kernel that walks key by key, whose tests hold these."""
+    from tie_amd import kernels
+
+    H, KVH, Dh = 8, 2, 64
+    case, S = attention_case(H, KVH, Dh, 16, lens_new=[33, 1, 1, 50], lens_ctx=[33, 200, 7, 90], seed=9)
+    for name in ("kc", "vc"):
+        case[name] = torch.nan_to_num(case[name].clamp(-6e4, 6e4).to(dtype))
+    more = dict(more)
+    if more.get("sinks"):
+        more["sinks"] = rnd(H, seed=11).cuda()
+    want = torch.empty_like(case["q"])
+    kernels.paged_attention_generic(case["q"], case["kc"], case["vc"], want, case["query_start"], case["context_lens"],
+                                    case["tables"], case["seq_of_row"], H, Dh ** -0.5, **more)
+    # two float32 orders of the same sums of up to 200 terms
+    close(run(case, H, S, Dh, nsplit, **more), want.cpu().to(F64), 4e-6, f"{more} over {dtype}")
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_attention_f32_values_that_are_no_numbers(bad):
+    """A value that is no number reaches the rows that see its key, at every place of a tile, and no other row."""
+    from tie_amd import kernels
+
+    H, KVH, Dh, n = 4, 2, 32, 37
+    for key in (0, 3, 16, 21, 36):
+        case, S = attention_case(H, KVH, Dh, 16, lens_new=[n], lens_ctx=[n], seed=12)
+        clean = run(case, H, S, Dh)
+        page = int(case["tables"][0, key // 16])
+        case["vc"][page, 1, 5, key % 16] = bad
+        out = run(case, H, S, Dh).view(n, H, Dh)
+        want = clean.view(n, H, Dh).clone()
+        seen = ~torch.isfinite(out)
+        expect = torch.zeros_like(seen)
+        expect[key:, 2:, 5] = True                      # the heads of KV head 1, its sixth dimension, rows from the key on
+        assert torch.equal(seen, expect), f"key {key}"
+        close(out[~expect], want[~expect].cpu().to(F64), 2e-6, f"the other results, key {key}")
+
+
 def test_the_32_bit_path_takes_these_kernels():
-    """The dispatcher: operands the kernel takes go there (other results only by rounding), the others as before."""
+    """The dispatchers: operands the kernels take go there (other results only by rounding), the others as before."""
     from tie_amd import kernels
 
     x, w = rnd(5, 64, seed=1).cuda(), rnd(24, 64, seed=2).cuda()

@@ -53,6 +53,7 @@ _SOURCES = {
     "gemm_generic": ("tie_gemm_generic", "gemm_generic.hip"),
     "attention_generic": ("tie_attention_generic", "attention_generic.hip"),
     "gemm_f32": ("tie_gemm_f32", "gemm_f32.hip"),
+    "attention_f32": ("tie_attention_f32", "attention_f32.hip"),
     "skinny_gemm_bf16": ("tie_skinny_gemm_bf16", "skinny_gemm_bf16.hip"),
     "gemm_bf16": ("tie_gemm_bf16", "gemm_bf16.hip"),
     "sample_filtered": ("tie_sample_filtered", "sample_filtered.hip"),
@@ -141,6 +142,11 @@ _SIGNATURES = {
     "gemm_f32": {
         "tie_gemm_f32_splits": [_c_int, _c_int, _c_int],
         "tie_gemm_f32": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
+    },
+    "attention_f32": {
+        "tie_attention_f32": [_c_void, _c_void, _c_void, _c_int, _c_void, _c_void, _c_void, _c_void, _c_int, _c_int, _c_int,
+                              _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_int, _c_int, _c_void, _c_int,
+                              _c_void, _c_void, _c_void],
     },
     "attention_generic": {
         "tie_paged_attention_generic": [_c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_int, _c_void, _c_void,
@@ -1172,6 +1178,69 @@ def paged_attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
         float(softcap or 0.0), int(window or 0), int(chunk or 0), int(keep_first or 0), _ptr(sinks), _stream())
 
 
+def attention_f32_takes(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, out: torch.Tensor,
+                        keep_first: int = 0) -> bool:
+    """Whether ``attention_f32`` takes these operands: float32 queries, pages and head sizes in steps of 16."""
+    Dh, bs = k_cache.shape[3], k_cache.shape[2]
+    return q.dtype == torch.float32 and out.dtype == torch.float32 and Dh % 16 == 0 and 16 <= Dh <= 256 and \
+        bs % 16 == 0 and not keep_first and \
+        (q.data_ptr() | out.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0
+
+
+def attention_f32_tiles(new_tokens, group_size: int) -> int:
+    """Column tiles of a step: 16 columns of (query row, query head of a KV head) of one sequence each."""
+    rows = 16 // group_size if group_size <= 16 else 1
+    return sum(-(-n // rows) for n in new_tokens)
+
+
+def attention_f32_splits(tiles: int, num_kv_heads: int, group_size: int, max_context: int) -> int:
+    """Shares the keys of every column tile are cut into: more than one only where the tiles alone leave CUs idle."""
+    workgroups = tiles * num_kv_heads * -(-group_size // 16)
+    by_fill = 512 // max(1, workgroups)
+    by_length = -(-max_context // 16) // 16                 # at least sixteen tiles of 16 keys a share
+    return max(1, min(16, by_fill, by_length))
+
+
+def attention_f32(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, out: torch.Tensor,
+                  query_start: torch.Tensor, context_lens: torch.Tensor, block_tables: torch.Tensor, tiles: int,
+                  num_heads: int, scale: float, window: Optional[int] = None, softcap: Optional[float] = None,
+                  chunk: Optional[int] = None, sinks: Optional[torch.Tensor] = None, nsplit: int = 1,
+                  part_o: Optional[torch.Tensor] = None, part_ml: Optional[torch.Tensor] = None) -> None:
+    """What ``paged_attention_generic`` computes, on the float32 matrix instructions (``attention_f32_takes``).
+
+    ``tiles``: ``attention_f32_tiles`` of the step's sequences. ``nsplit`` > 1: every tile's keys are cut into that many
+    shares; ``part_o`` and ``part_ml`` hold their results until they are merged."""
+    for t, name in ((q, "queries"), (out, "attention output"), (k_cache, "k cache"), (v_cache, "v cache")):
+        _gpu(t, name)
+    NB, KVH, bs, Dh = k_cache.shape
+    _check_cache(k_cache, v_cache, KVH, bs, Dh)
+    T, H = q.shape[0], num_heads
+    if tuple(q.shape) != (T, H * Dh) or tuple(out.shape) != (T, H * Dh) or H % KVH:
+        raise InvalidArgument(f"attention: q {list(q.shape)} / out {list(out.shape)} do not fit {H} heads of {Dh} over "
+                              f"{KVH} kv heads")
+    if not attention_f32_takes(q, k_cache, v_cache, out):
+        raise InvalidArgument("attention_f32 takes float32 queries, head sizes up to 256 and pages in steps of 16")
+    S = context_lens.numel()
+    _i32(query_start, "query_start", S + 1)
+    _i32(context_lens, "context_lens")
+    _i32(block_tables, "block tables")
+    if block_tables.dim() != 2 or block_tables.shape[0] < S:
+        raise InvalidArgument(f"block tables {list(block_tables.shape)} do not cover {S} sequences")
+    if window and chunk:
+        raise InvalidArgument("attention takes a sliding window or causal chunks, not both")
+    if sinks is not None:
+        _f32(sinks, "attention sinks", (H,))
+    if nsplit > 1:
+        for t, n, name in ((part_o, T * H * nsplit * Dh, "partial outputs"), (part_ml, T * H * nsplit * 2, "partial sums")):
+            if t is None or _f32(t, name).numel() < n:
+                raise InvalidArgument(f"attention: {name} of {nsplit} shares need {n} floats")
+    _call(_lib("attention_f32").tie_attention_f32, "attention_f32", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+          _cache_code(k_cache, q, "k cache"), out.data_ptr(), query_start.data_ptr(), context_lens.data_ptr(),
+          block_tables.data_ptr(), int(tiles), T, S, H, KVH, Dh, bs, block_tables.shape[1], float(scale),
+          float(softcap or 0.0), int(window or 0), int(chunk or 0), _ptr(sinks), int(nsplit), _ptr(part_o), _ptr(part_ml),
+          _stream())
+
+
 _argmax_workspace = {}
 
 
@@ -1746,6 +1815,20 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                                    step.block_tables, items, num_heads, scale, window, nsplit, part_o, part_ml,
                                    merge_rows if nsplit > 1 else None, softcap=softcap, chunk=chunk, sinks=sinks,
                                    keep_first=keep_first)
+        return
+    if scratch is not None and num_heads % KVH == 0 and attention_f32_takes(q, k_cache, v_cache, out, keep_first):
+        G, T = num_heads // KVH, q.shape[0]
+        key = ("attention_f32_tiles", G)
+        tiles = batch.memo.get(key)
+        if tiles is None:
+            tiles = batch.memo[key] = attention_f32_tiles(batch.host_new_tokens, G)
+        nsplit = attention_f32_splits(tiles, KVH, G, min(batch.plan_context, reach or batch.plan_context))
+        part_o = part_ml = None
+        if nsplit > 1:
+            part_o = scratch("attention.split_o", (T * num_heads * nsplit * Dh,), torch.float32)
+            part_ml = scratch("attention.split_ml", (T * num_heads * nsplit * 2,), torch.float32)
+        attention_f32(q, k_cache, v_cache, out, batch.query_start, batch.context_lens, step.block_tables, tiles, num_heads,
+                      scale, window, softcap, chunk, sinks, nsplit, part_o, part_ml)
         return
     paged_attention_generic(q, k_cache, v_cache, out, batch.query_start, batch.context_lens, step.block_tables,
                             batch.seq_of_row, num_heads, scale, window, softcap, chunk, sinks, keep_first)

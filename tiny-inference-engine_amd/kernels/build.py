@@ -39,7 +39,7 @@ FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC", "-shared",
 # accumulators, up to 64 registers, are otherwise copied between the two register files at the ends of its loop.
 _VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 SOURCE_FLAGS = {"attention_prefill_bf16.hip": _VGPR_FORM, "attention_decode_bf16.hip": _VGPR_FORM,
-                "gemm_f32.hip": _VGPR_FORM}
+                "attention_f32.hip": _VGPR_FORM, "gemm_f32.hip": _VGPR_FORM}
 
 _loaded: Dict[str, ctypes.CDLL] = {}
 _lock = threading.Lock()
