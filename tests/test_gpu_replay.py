@@ -299,6 +299,36 @@ def test_layers_of_one_shape_run_from_one_layers_launch_list(tmp_path, dtype, us
             assert torch.equal(row, got[False][rid][position]), f"request {rid}, position {position}"
 
 
+@pytest.mark.parametrize("layers", [4, 7])
+def test_a_product_left_pending_carries_over_between_launch_lists(tmp_path, layers):
+    """In steps of a few rows a layer leaves its last product to the next one's first norm, over a stream wide enough
+    for that. The layers run from the third one's launches must take the weight of the layer before them, and the
+    head's norm that of the last layer: the bits of a run in which every layer runs its own code."""
+    from conftest import TINY_B
+    from tie_amd import kernels
+    from tie_amd.engine.replay import TraceReplayer
+    from tie_amd.weights.random_init import write_random_model
+
+    cfg = dict(TINY_B, num_hidden_layers=layers, hidden_size=4096, intermediate_size=128)
+    assert kernels.norm_epilogue_rows(4096, 128) >= 4
+    folder = tmp_path / "wide"
+    write_random_model(folder, cfg, seed=32, dtype="bfloat16", device="cuda:0")
+    requests = th.make_requests(cfg["vocab_size"], [2, 4, 9], seed=9)
+    for use_graphs in (False, True):
+        got = {}
+        for replay in (True, False):
+            rep = TraceReplayer.from_folder(folder, "bfloat16", 256, use_graphs=use_graphs)
+            rep.model.replay_layers = replay
+            got[replay] = {}
+            for plan in (th.whole(requests), th.portions(requests, (3, 1, 2, 4))):
+                for key, rows in th.collect(rep, plan).items():
+                    got[replay][key, len(got[replay])] = rows
+            assert (rep.model.layers_replayed > 0) == replay
+        assert list(got[True]) == list(got[False])
+        for key, rows in got[True].items():
+            assert all(torch.equal(rows[p], got[False][key][p]) for p in rows), f"request {key}"
+
+
 @pytest.mark.parametrize("name", ["A", "B"])
 def test_a_corrupted_page_is_caught(folders, name):
     """The bound the bfloat16 checks use must not be so wide that a wrong page of the cache passes under it. A

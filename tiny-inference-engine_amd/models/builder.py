@@ -20,6 +20,7 @@ from ..errors import InvalidArgument
 from .. import kernels
 from ..parts import base as parts_base
 from ..parts.base import Part, StepContext, TensorSpec, build_part
+from ..parts.linear import Linear
 from ..weights.binder import BFLOAT16, check_tensors, normalize_mode, place_tensor
 from ..weights.loader import ModelFiles, load_model_folder
 from ..weights.safetensors_io import StoredTensor
@@ -71,6 +72,26 @@ def _walk_parts(obj, tensors, classes, seen, scalars=None, path="") -> None:
             _walk_parts(getattr(obj, name), tensors, classes, seen, scalars, f"{path}.{name}")
     elif scalars is not None:
         scalars.append((path, ("object", type(obj).__qualname__, id(obj))))     # unknown: alike only if the very same
+
+
+def _projections(obj, found, seen) -> list:
+    """The ``Linear`` objects of an object tree of parts, in a fixed order: layers of one shape list theirs alike."""
+    if isinstance(obj, Linear):
+        if id(obj) not in seen:
+            seen.add(id(obj))
+            found.append(obj)
+    elif isinstance(obj, Part):
+        if id(obj) not in seen:
+            seen.add(id(obj))
+            for name in sorted(vars(obj)):
+                _projections(getattr(obj, name), found, seen)
+    elif isinstance(obj, (list, tuple)):
+        for value in obj:
+            _projections(value, found, seen)
+    elif isinstance(obj, dict):
+        for name in sorted(obj, key=str):
+            _projections(obj[name], found, seen)
+    return found
 
 
 def _constants(scalars, tensor_names) -> tuple:
@@ -236,14 +257,16 @@ class Model:
             start = end
 
     def _entry_tensors(self, ctx: StepContext, index: int, cache) -> list:
-        """(address, bytes) of everything entry ``index`` owns on the device: its layer's tensors and its cache."""
+        """(address, bytes) of everything the launches of entry ``index`` may point to that is not the step's: its
+        layer's tensors and its cache, and the tensors of the layer before it, whose last product its first norm
+        launches in steps of a few rows (``StepContext.defer_product``)."""
         tensors = list(self._layer_tensors[index])
         for binding in (cache if isinstance(cache, tuple) else (cache,)):
             for name in ("k_cache", "v_cache", "state"):
                 t = getattr(binding, name, None)
                 if isinstance(t, torch.Tensor):
                     tensors.append((t.data_ptr(), t.numel() * t.element_size()))
-        return tensors
+        return tensors + self._layer_tensors[index - 1]
 
     @staticmethod
     def _launch_list(noted_a, noted_b, tensors_a, tensors_b) -> Optional[List[_Launch]]:
@@ -282,6 +305,10 @@ class Model:
         (the first may differ: it settles what the entry before it left), the launches of the second and third
         are noted and compared, and the others run from that list with their own addresses, which takes a
         fraction of the host time; small models' steps of many short kernels wait for the host otherwise.
+
+        In steps of a few rows a layer may leave its last product pending in the step context. The next layer's list
+        begins with that product, over the weight of the layer before, and behind the last of the layers the context
+        is told that it is now this layer's product that is pending.
         """
         def run(index):
             cache = ctx.cache_of(index)
@@ -300,6 +327,11 @@ class Model:
             noted.append(record)
             tensors.append(self._entry_tensors(ctx, index, cache))
         launches = self._launch_list(noted[0], noted[1], tensors[0], tensors[1])
+        pending, place = ctx.pending_linear, None
+        if pending is not None:
+            place = next((i for i, l in enumerate(self._projections_of(start + 2)) if l is pending), None)
+            if place is None:              # a product of no part of the layer: nothing to put in its place
+                launches = None
         for index in range(start + 3, end):
             if launches is None:
                 run(index)
@@ -314,6 +346,11 @@ class Model:
                 else:
                     kernels.replay_call(launch.fn, launch.what, launch.args)
             self.layers_replayed += 1
+        if launches is not None and place is not None:
+            ctx.pending_linear = self._projections_of(end - 1)[place]
+
+    def _projections_of(self, index: int) -> list:
+        return _projections(self.layers[self.spec.order[index].layer].parts(), [], set())
 
     # ------------------------------------------------------------------ step
     def forward(self, ctx: StepContext) -> Optional[torch.Tensor]:
@@ -321,11 +358,7 @@ class Model:
         batch = ctx.batch
         x = self.embedding.forward(ctx, batch.tokens)
         index, entries = 0, len(self.spec.order)
-        # Layers run from another's launch list only where a layer's launches are its own: in steps of a few rows a
-        # sub-layer's last product may stay pending in the step context for the next layer's norm to launch, and a
-        # replayed launch list would not carry that over.
-        replay = self.replay_layers and self.layer_hook is None and not (
-            kernels.NORMS_IN_PRODUCTS and batch.num_tokens <= kernels.NORM_EPILOGUE_ROWS)
+        replay = self.replay_layers and self.layer_hook is None
         while index < entries:
             alike_to = self._alike.get(index) if replay else None
             if alike_to is not None:

@@ -227,6 +227,17 @@ class StepContext:
             return linear, x
         return None
 
+    @property
+    def pending_linear(self):
+        """The projection whose product is pending, or None. Setting it puts the same projection of another layer in its
+        place: the target and the rows are the step's, the weight is that layer's (``models.builder``)."""
+        return None if self._pending is None else self._pending[1]
+
+    @pending_linear.setter
+    def pending_linear(self, linear) -> None:
+        target, _, x = self._pending
+        self._pending = (target, linear, x)
+
     # A block's last pass over the residual may be left for the block behind it, which merges it into its own first
     # pass (take_late with the same key); whoever needs the residual before that calls settle(), which runs it.
     def leave_late(self, key, run, payload) -> None:
