@@ -460,6 +460,33 @@ def test_gemm_bf16_loaded_straight_into_lds(M, N, K, tile):
             close(gated, g / (1 + torch.exp(-g)) * u, 8e-3, "gated product")
 
 
+@pytest.mark.parametrize("M,N", [(1, 64), (130, 208), (257, 400)])
+@pytest.mark.parametrize("slices", [3, 4, 5, 6, 7, 11, 12, 13, 32])
+def test_tiles_that_stage_two_slices_at_a_time(M, N, slices):
+    """Every number of slices of 32 along K, even and odd, in one range and in ranges: the sums of the tiles whose ring
+    holds pairs of slices are those of the 256 x 256 tile, whose ring holds single ones, bit for bit; over rows and over
+    packed blocks."""
+    from tie_amd import kernels
+
+    K = 32 * slices
+    x = rnd(M, K, seed=39, dtype=torch.bfloat16).cuda()
+    w = rnd(N, K, seed=40, scale=0.1, dtype=torch.bfloat16).cuda()
+    x[0, K - 1] = float("inf")                       # what lies behind a row or a range must not reach a sum
+    packed = kernels.pack_weight(w)
+    for splits in (1, 2, 3):
+        if slices - -(-slices // splits) * (splits - 1) < 3:
+            continue
+        shape = (M, N) if splits == 1 else (splits, M, N)
+        want = torch.full(shape, float("nan"), device="cuda")
+        kernels.gemm_bf16(x, w, want, tile=4, splits=splits)
+        assert bool(torch.isfinite(want[..., 1:, :]).all())
+        for tile in (5, 6, 7, 8, 9, 10, 11):
+            for weight in (w, packed):
+                out = torch.full(shape, 7.0, device="cuda")
+                kernels.gemm_bf16(x, weight, out, tile=tile, splits=splits)
+                assert torch.equal(torch.nan_to_num(out, nan=1e30), torch.nan_to_num(want, nan=1e30)), (tile, splits)
+
+
 @pytest.mark.parametrize("N,K", [(16, 96), (48, 128), (208, 4096), (1024, 352)])
 def test_packed_weight_feeds_both_products_the_same_numbers(N, K):
     """The blocked weight layout changes where bytes lie, not one sum: results equal the row-major ones bit for bit."""

@@ -302,7 +302,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
   constexpr int PA = BM / 64;                   // wave instructions that stage x's rows (16 rows each, 4 waves)
   constexpr int PB = BN / 64;                   // wave instructions that stage w's rows likewise
   static_assert(BM == 256 || BM == 128 || BM == 64, "rows of a tile");
-  constexpr int BUF = (BM + BN) * BK;           // elements of one stage
+  constexpr int G = GdShape<BM, BN>::GROUP;     // slices that x's rows are staged by
   extern __shared__ bf16_t lds[];
 
   const int total = tiles_m * tiles_n;
@@ -329,16 +329,16 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
 
   // One wave instruction fills 16 rows of 64 bytes: pass p of wave v covers rows 64 p + 16 v + lane / 4.
   // Rows beyond the matrix are clamped to its last one (their products are never stored).
-  const int lr = gd_stage_row(lane, wave);
-  const int lchunk = gd_stage_chunk(lane, lr);
+  const int ar = gd_stage_row<G>(lane, wave), br = gd_stage_row<1>(lane, wave);
+  const int a_chunk = gd_stage_chunk<G>(lane, ar), b_chunk = gd_stage_chunk<1>(lane, br);
   const unsigned row_bytes = static_cast<unsigned>(K) * 2;
   const int kblocks = K / BK;
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<bf16_t*>(x_all + static_cast<size_t>(row0) * K + static_cast<size_t>(k_begin) * BK), 0,
       static_cast<int>(min(BM, M - row0) * row_bytes - k_begin * BK * 2), GD_RSRC_FLAGS);
-  unsigned a_off[PA], b_off[PB];
+  unsigned a_off[PA * G], b_off[PB];
 #pragma unroll
-  for (int p = 0; p < PA; ++p) a_off[p] = min(lr + p * 64, M - 1 - row0) * row_bytes + lchunk * 16;
+  for (int p = 0; p < PA * G; ++p) a_off[p] = min(ar + p * (64 / G), M - 1 - row0) * row_bytes + a_chunk * 16;
   // w: rows like x's, or (PW) the packed layout, where the 16 rows x 32 k that one wave instruction
   // stages are one block of 1 KB: block (tile, k-block) at ((tile * kblocks) + k-block) * 1 KB.
   const int tile0 = col0 / 16, last_tile = (N - 1) / 16;
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
   unsigned b_tile_off[PB];   // PW: wave-uniform byte offset of this wave's block row
 #pragma unroll
   for (int p = 0; p < PB; ++p) {
-    b_off[p] = PW ? lane * 16 : min(lr + p * 64, N - 1 - col0) * row_bytes + lchunk * 16;
+    b_off[p] = PW ? lane * 16 : min(br + p * 64, N - 1 - col0) * row_bytes + b_chunk * 16;
     b_tile_off[p] = PW ? static_cast<unsigned>(min(p * 4 + wave, last_tile - tile0)) * kblocks * 1024 : 0;
   }
 
@@ -415,7 +415,7 @@ static int launch_gemm_dma(const void* x, const void* w, void* out, int epi, int
   const int k_slices = K / GD_BK;
   const int per_split = (k_slices + splits - 1) / splits;
   if (k_slices - per_split * (splits - 1) < 3) return TIE_BAD_ARGUMENT;   // the last range would be too short
-  const size_t shared = sizeof(bf16_t) * GD_STAGES * (BM + BN) * GD_BK;
+  const size_t shared = GdShape<BM, BN>::LDS_BYTES;
   const dim3 grid(tiles_m * tiles_n, splits);
 #define LAUNCH(EPI)                                                                                          \
   {                                                                                                          \
@@ -449,17 +449,19 @@ static bool gemm_dma_takes(const void* x, const void* w, const void* out, int N,
 // Which tile, and how many ranges of K (planes of partial sums that the caller adds), a product takes when
 // left to choose.
 //
-// Up to 64 rows over packed weights: a score (below); 65 to 128 rows: few_rows_us. Above that, for shapes the
-// straight-to-LDS tiles take: the cheapest of (tile, ranges) by an estimate of the time, whose constants were chosen
-// on sweeps over the projections of four shapes (widths 2048, 3072, 4096 and 5120) at 160 to 2048 rows, every
-// candidate timed with the kernel that consumes its planes, so that the choice lies as close to the best candidate
-// as it can (2.2 % above it on average, 3.6 % with the constants fitted to times of three shapes before):
-//   * a compute unit holds one workgroup (two of the 128 x 128 tile), so the workgroups run in rounds of
-//     256; a round that is nearly empty lasts as long as a full one, which is what a rule by thresholds
+// Up to 64 rows over packed weights: a score (below). Above that, for shapes the straight-to-LDS tiles take: the cheapest
+// of (tile, ranges) by an estimate of the time:
+//   * a compute unit holds one workgroup (three of the 64 x 128 tile), so the workgroups run in rounds of 256; a round
+//     that is nearly empty lasts as long as a full one, which is what a rule by thresholds
 //     gets wrong (768 rows of 256 x 128 tiles over 6144 columns and two ranges: 288 workgroups, two rounds);
-//   * a round is a few microseconds of start and end plus its slices of 32 along K at the tile's own pace;
+//   * a round is a few microseconds of start and end plus its slices of 32 along K at the tile's own pace, both more where
+//     it fills every compute unit;
 //   * every plane is written once here and read once by its consumer.
-// Without the straight-to-LDS tiles (odd K or N) the older tiles and their rule stand.
+// The constants are a least-squares fit, tile by tile, to sweeps over eight packed projections (2048 x 2048 to
+// 24576 x 4096, every tile, 1 to 8 ranges) at 200 to 2048 rows, and to those at 96 and 128 rows, where the weights come
+// from memory by few workgroups; 6 to 14 % root mean square. The choice lies 0.7 % above the best forced (tile, ranges)
+// on average and 16 % at most, on the best at 96 and 128 rows. Rows of fewer than 65 over row-major weights and odd K or N
+// stay with the older tiles and their rule.
 struct GemmPlan { int tile, splits; };
 
 static int legacy_splits(int M, int N, int K) {
@@ -476,69 +478,37 @@ static int legacy_splits(int M, int N, int K) {
   return 1;
 }
 
-struct DmaTile { int id, bm, bn; float start_us, full_us, slice_us; int per_cu; };
-// start_us: a round's start and end; full_us: what a round costs more when it fills every compute unit (measured
-// for the 256 x 256 and 256 x 192 tiles, whatever the length of K: 256 workgroups of the first start about 11 us
-// later than 192);
-// slice_us: one slice of 32 along K with the compute unit to itself.
-static const DmaTile kDmaTiles[] = {{4, 256, 256, 8.8f, 7.9f, 0.67f, 1}, {10, 256, 192, 5.f, 5.4f, 0.55f, 1},
-                                    {5, 256, 128, 6.25f, 0.f, 0.53f, 1}, {6, 128, 256, 6.25f, 1.f, 0.50f, 1},
-                                    {7, 128, 128, 3.24f, 1.f, 0.324f, 2}};
+// start_us: a round's start and end; slice_us: one slice of 32 along K while most compute units are idle. From half a round
+// of workgroups to a full one both grow, by full_us and by the factor 1 + press: the units share the L2 and the clock.
+// per_cu workgroups on one compute unit each take `shared` times as long.
+struct DmaTile { int id, bm, bn; float start_us, full_us, slice_us, press; int per_cu; float shared; };
+static const DmaTile kDmaTiles[] = {
+    {4, 256, 256, 8.57f, 7.37f, 0.629f, 0.17f, 1, 1.f}, {10, 256, 192, 6.14f, 2.53f, 0.580f, 0.15f, 1, 1.f},
+    {5, 256, 128, 6.91f, 0.00f, 0.367f, 0.32f, 1, 1.f}, {6, 128, 256, 6.20f, 0.91f, 0.400f, 0.18f, 1, 1.f},
+    {11, 128, 192, 5.10f, 0.0f, 0.327f, 0.12f, 1, 1.f}, {7, 128, 128, 3.48f, 0.91f, 0.250f, 0.14f, 1, 1.f}};
+static const DmaTile kFewRowsTiles[] = {
+    {6, 128, 256, 6.11f, 3.12f, 0.440f, 0.20f, 1, 1.f}, {7, 128, 128, 3.91f, 0.68f, 0.276f, 0.43f, 1, 1.f},
+    {8, 64, 256, 3.62f, 0.87f, 0.373f, 0.27f, 1, 1.f}, {9, 64, 128, 3.19f, 4.31f, 0.248f, 0.23f, 3, 2.06f}};
 
-static float estimated_us(const DmaTile& t, int M, int N, int K, int ranges) {
+static float estimated_us(const DmaTile& t, int M, int N, int K, int ranges, float plane_us_per_mb) {
   const long wgs = static_cast<long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * ranges;
   const int k_slices = K / GD_BK;
   const int slices = (k_slices + ranges - 1) / ranges;
   const long slots = 256L * t.per_cu;
-  const float pace = t.slice_us * (t.per_cu > 1 && wgs > 256 ? 1.94f : 1.0f);   // two workgroups share the matrix cores
+  const float pace = t.slice_us * (t.per_cu > 1 && wgs > 256 ? t.shared : 1.0f);
   auto round_us = [&](float fill) {
-    const float crowded = fminf(fmaxf((fill - 0.75f) * 4.0f, 0.f), 1.f);
-    return t.start_us + t.full_us * crowded + slices * pace;
+    const float crowded = fminf(fmaxf((fill - 0.5f) * 2.0f, 0.f), 1.f);
+    return t.start_us + t.full_us * crowded + slices * pace * (1.0f + t.press * crowded);
   };
   float us = static_cast<float>(wgs / slots) * round_us(1.0f);
   if (wgs % slots) us += round_us(static_cast<float>(wgs % slots) / slots);
   const float plane_mb = static_cast<float>(M) * N * 4e-6f;
-  return ranges > 1 ? us + ranges * plane_mb * 0.2f : us;   // planes written here, read by the consumer: MB / (TB/s) = us
-}
-
-// 65 to 128 rows: a workgroup's pace is set by the bytes it loads a slice of 32 along K, its rows of x and its
-// columns of w (about 40 GB/s a compute unit), and all of them together by the weights' bytes (5.5 TB/s);
-// workgroups run in rounds of 256. Fitted to sweeps over the projections of the 1.7B, 8B and 32B shapes at 80,
-// 96 and 128 rows: 8B gate/up at 128 rows 61 us on 128 x 128 tiles (192 workgroups) against 82 on 128 x 256 (96).
-struct FewRowsTile { int id, bm, bn; };
-static const FewRowsTile kFewRowsTiles[] = {{6, 128, 256}, {7, 128, 128}, {8, 64, 256}, {9, 64, 128}};
-
-static float few_rows_us(const FewRowsTile& t, int M, int N, int K, int ranges) {
-  const long wgs = static_cast<long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * ranges;
-  const int k_slices = K / GD_BK;
-  const int slices = (k_slices + ranges - 1) / ranges;
-  const float per_slice = static_cast<float>(t.bm + t.bn) * (GD_BK * 2) / 40000.f;
-  float us = static_cast<float>((wgs + 255) / 256) * (4.f + slices * per_slice);
-  us = fmaxf(us, static_cast<float>(N) * K * 2e-6f / 5.5f);
-  if (ranges > 1) us += ranges * static_cast<float>(M) * N * 4e-6f * (1.0f / 6.0f + 1.0f / 5.0f);
-  return us;
+  return ranges > 1 ? us + ranges * plane_mb * plane_us_per_mb : us;   // planes written here, read by the consumer
 }
 
 // splits: 0 = free to choose (the caller adds planes), else the number of ranges the caller has fixed (1: none).
 static GemmPlan gemm_plan(int M, int N, int K, bool straight_to_lds, int splits, bool packed) {
   const bool may_split = splits == 0;
-  if (straight_to_lds && packed && M > 64 && M <= 128) {
-    // 65 to 128 rows over packed weights: the weights are read once by few workgroups, so what counts is that
-    // one round of workgroups fills the compute units. The cheapest of (tile, ranges) by few_rows_us.
-    GemmPlan best = {7, may_split ? 1 : splits};
-    float best_us = 0.f;
-    for (int r = may_split ? 1 : splits; r <= (may_split ? 8 : splits); r *= 2) {
-      if (may_split && r > 1 && K / r < 512) break;
-      for (const FewRowsTile& t : kFewRowsTiles) {
-        const float us = few_rows_us(t, M, N, K, r);
-        if (best_us == 0.f || us < best_us * 0.98f) {       // ties go to fewer planes, then to the larger tile
-          best = {t.id, r};
-          best_us = us;
-        }
-      }
-    }
-    return best;
-  }
   if (straight_to_lds && packed && M <= 64) {
     // Up to 64 rows over packed weights: tiles of 64 rows, one workgroup a compute unit, the weights read once. The
     // cheapest (tile, ranges) by a score of three factors: what the 64 rows of x cost beside a tile's columns
@@ -567,20 +537,24 @@ static GemmPlan gemm_plan(int M, int N, int K, bool straight_to_lds, int splits,
     }
     return best;
   }
-  if (straight_to_lds && M > 128) {
+  if (straight_to_lds && (M > 128 || (packed && M > 64))) {
     GemmPlan best = {4, may_split ? 1 : splits};
     float best_us = 0.f;
     const int k_slices = K / GD_BK;
+    auto offer = [&](const DmaTile& t, int r) {
+      const float us = estimated_us(t, M, N, K, r, M <= 128 ? 0.24f : 0.32f);
+      if (best_us == 0.f || us < best_us * 0.98f) {         // ties go to fewer planes, then to the larger tile
+        best = {t.id, r};
+        best_us = us;
+      }
+    };
     for (int r = may_split ? 1 : splits; r <= (may_split ? 8 : splits); r *= 2) {
       const int per = (k_slices + r - 1) / r;
       if (may_split && r > 1 && (K / r < 512 || k_slices - per * (r - 1) < 3)) break;
-      for (const DmaTile& t : kDmaTiles) {
-        const float us = estimated_us(t, M, N, K, r);
-        if (best_us == 0.f || us < best_us * 0.98f) {       // ties go to fewer planes, then to the larger tile
-          best = {t.id, r};
-          best_us = us;
-        }
-      }
+      if (M <= 128)
+        for (const DmaTile& t : kFewRowsTiles) offer(t, r);
+      else
+        for (const DmaTile& t : kDmaTiles) offer(t, r);
     }
     return best;
   }
@@ -610,7 +584,8 @@ extern "C" int tie_gemm_bf16_splits(int M, int N, int K, int packed) {
 // The tile a product left to choose runs on (the numbers of tie_gemm_bf16's `tile`), with `splits` ranges of K
 // fixed by the caller (1: none) or 0 for the plan's own number; for tests and sweeps.
 extern "C" int tie_gemm_bf16_tile(int M, int N, int K, int packed, int splits) {
-  return gemm_plan(M, N, K, straight_to_lds_shape(N, K), splits, packed != 0).tile;
+  const int tile = gemm_plan(M, N, K, straight_to_lds_shape(N, K), splits, packed != 0).tile;
+  return tile == 11 ? 6 : tile;        // 128 x 192 goes by the number of 128 x 256, whose narrower form it is
 }
 
 // out_dtype: TIE_F32 or TIE_BF16; accumulate adds into a float32 output; gated (bfloat16 output of N / 2
@@ -633,13 +608,13 @@ extern "C" int tie_gemm_bf16(const void* x, const void* w, void* out, int out_dt
   if (splits > 1 && (accumulate || gated || out_dtype != TIE_F32)) return TIE_BAD_ARGUMENT;
   const int epi = gated ? (gated == 2 ? 4 : 3) : (accumulate ? 2 : (out_dtype == TIE_F32 ? 0 : 1));
   const bool straight = gemm_dma_takes(x, w, out, N, K, splits);
-  if (packed && (N % 16 != 0 || !straight || (tile != 0 && (tile < 4 || tile > 10)))) return TIE_BAD_ARGUMENT;
+  if (packed && (N % 16 != 0 || !straight || (tile != 0 && (tile < 4 || tile > 11)))) return TIE_BAD_ARGUMENT;
   if (tile == 0) {
     tile = gemm_plan(M, N, K, straight, splits, packed != 0).tile;
   } else if (tile < 4 && splits > 1) {
     tile = 1;
   }
-  if (tile >= 4 && tile <= 10) {
+  if (tile >= 4 && tile <= 11) {
     if (!straight) return TIE_BAD_ARGUMENT;
 #define DMA(BM, BN)                                                                            \
   return packed ? launch_gemm_dma<BM, BN, true>(x, w, out, epi, M, N, K, splits, stream)       \
@@ -651,7 +626,8 @@ extern "C" int tie_gemm_bf16(const void* x, const void* w, void* out, int out_dt
       case 7: DMA(128, 128);
       case 8: DMA(64, 256);
       case 9: DMA(64, 128);
-      default: DMA(256, 192);
+      case 10: DMA(256, 192);
+      default: DMA(128, 192);
     }
 #undef DMA
   }

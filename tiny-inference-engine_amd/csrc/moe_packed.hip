@@ -115,7 +115,7 @@ __global__ __launch_bounds__(256) void moe_packed_many_rows_kernel(const bf16_t*
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr bool GATED = MODE == 1 || MODE == 3 || MODE == 4;
   constexpr bool GATHER = MODE != 0;
-  constexpr int TN = BN / 64, TM = BM / 64;
+  constexpr int TN = BN / 64, TM = BM / 64, G = GdShape<BM, BN>::GROUP;
   extern __shared__ bf16_t lds[];
   const int total = *rw.num_tiles * tiles_n;
   const int per_xcd = (total + 7) / 8;
@@ -128,15 +128,15 @@ __global__ __launch_bounds__(256) void moe_packed_many_rows_kernel(const bf16_t*
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int fr = lane & 31, fk = lane >> 5;
-  const int lr = gd_stage_row(lane, wave), lchunk = gd_stage_chunk(lane, lr);
+  const int lr = gd_stage_row<G>(lane, wave), lchunk = gd_stage_chunk<G>(lane, lr);
   const unsigned row_bytes = static_cast<unsigned>(K) * 2;
   const int kblocks = K / 32;
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<bf16_t*>(x), 0, static_cast<int>(x_rows * row_bytes), GD_RSRC_FLAGS);
-  unsigned a_off[BM / 64], b_off[BN / 64], b_tile_off[BN / 64];
+  unsigned a_off[BM * G / 64], b_off[BN / 64], b_tile_off[BN / 64];
 #pragma unroll
-  for (int p = 0; p < BM / 64; ++p) {
-    const int place = place0 + min(lr + p * 64, rows - 1);     // rows beyond the tile's end: computed, never stored
+  for (int p = 0; p < BM * G / 64; ++p) {
+    const int place = place0 + min(lr + p * (64 / G), rows - 1);     // rows beyond the tile's end: computed, never stored
     const int src = GATHER ? rw.slot_at[place] / rw.top : place;
     a_off[p] = static_cast<unsigned>(src) * row_bytes + lchunk * 16;
   }
@@ -202,7 +202,7 @@ template <int BM, int BN, int MODE>
 static int launch_many_rows(const void* x, const void* w, void* out, const MoeRows& rw, int max_tiles, int x_rows, int N,
                             int K, GateParams gp, hipStream_t stream) {
   const int tiles_n = (N + BN - 1) / BN;
-  const size_t shared = GD_LDS_BYTES(BM, BN);
+  const size_t shared = GdShape<BM, BN>::LDS_BYTES;
   static bool raised = false;
   if (!raised) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_packed_many_rows_kernel<BM, BN, MODE>),

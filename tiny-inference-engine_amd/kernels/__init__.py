@@ -912,7 +912,7 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: b
     """out (+)= x @ w.T for bfloat16 operands on the matrix cores, any number of rows; K % 8 == 0.
 
     ``tile`` picks the workgroup tile (1 = 128x128, 2 = 256x256, 3 = 256x128; 4 = 256x256, 5 = 256x128, 6 = 128x256,
-    7 = 128x128, 8 = 64x256, 9 = 64x128 and 10 = 256x192 with operand slices loaded straight into LDS, which need
+    7 = 128x128, 8 = 64x256, 9 = 64x128, 10 = 256x192 and 11 = 128x192 with operand slices loaded straight into LDS, which need
     K % 32 == 0 and N % 4 == 0; 0 lets the kernel choose);
     ``gated`` and ``splits`` as in ``skinny_gemm_bf16`` (planes of partial sums, ``[splits, M, N]`` float32).
     """
