@@ -980,6 +980,44 @@ def test_prefill_items_cover_the_rows_the_kernel_takes_per_item():
         assert [first for _, first in items] == [0, rows, 2 * rows], f"group of {group}"
 
 
+@pytest.mark.parametrize("H,KVH,Dh,bs", [(16, 1, 256, 16), (4, 2, 256, 64), (8, 2, 128, 16), (3, 1, 32, 16)])
+@pytest.mark.parametrize("nsplit,window", [(1, None), (2, None), (1, 33)])
+def test_attention_prefill_bf16_scores_that_climb_and_fall(H, KVH, Dh, bs, nsplit, window):
+    """Scores whose running maximum rises by little and by much from tile to tile, or falls: the reference of a row's
+    probabilities follows it only in steps. Rows around the edges of tiles of 32 keys and of 64."""
+    lens_new, lens_ctx = [31, 32, 33, 64, 65, 100], [31, 64, 161, 320, 65, 1000]
+    case, S = attention_case(H, KVH, Dh, bs, lens_new=lens_new, lens_ctx=lens_ctx, seed=37, dtype=torch.bfloat16,
+                             window=window)
+    scale = Dh ** -0.5
+    q, want, start = case["q"].cpu().float(), [], 0
+    for s, (new, ctx) in enumerate(zip(lens_new, lens_ctx)):
+        pages = case["tables"][s, :math.ceil(ctx / bs)].long().cpu()
+        k = case["kc"].cpu()[pages].transpose(1, 2).reshape(-1, KVH, Dh)[:ctx].float()
+        v = case["vc"].cpu()[pages].permute(0, 3, 1, 2).reshape(-1, KVH, Dh)[:ctx].float()
+        # a direction of its own for the climb: scores of 12 sqrt(position / 32) upwards, downwards, or in a saw
+        height = {0: 1.0, 1: -1.0}.get(s % 3, 0.0) * 12.0 * (torch.arange(ctx) / 32.0).sqrt()
+        if s % 3 == 2:
+            height = (torch.arange(ctx) % 96) * 0.5
+        k[:, :, 0] = (height / 4.0)[:, None].to(torch.bfloat16).float()
+        q[start:start + new].view(new, H, Dh)[:, :, 0] = float(torch.tensor(4.0 / scale).to(torch.bfloat16))
+        kc = case["kc"].cpu()
+        for j, page in enumerate(pages.tolist()):
+            rows = slice(j * bs, min(ctx, (j + 1) * bs))
+            kc[page, :, :rows.stop - rows.start] = k[rows].transpose(0, 1).to(torch.bfloat16)
+        case["kc"] = kc.cuda()
+        score = torch.einsum("rhd,khd->hrk", q[start:start + new].view(new, H, Dh),
+                             k.repeat_interleave(H // KVH, 1)).double() * scale
+        at, key = torch.arange(ctx - new, ctx)[:, None], torch.arange(ctx)[None]
+        seen = (key <= at) & (key > at - (window or ctx + 1))
+        p = torch.softmax(score.masked_fill(~seen, -math.inf), -1)
+        want.append(torch.einsum("hrk,khd->rhd", p, v.repeat_interleave(H // KVH, 1).double()).reshape(new, H * Dh))
+        start += new
+    case["q"] = q.to(torch.bfloat16).cuda()
+    out = run_prefill(case, H, KVH, lens_new, window=window, nsplit=nsplit, staging=2)
+    # probabilities and outputs are rounded to bfloat16 (2^-9 of values up to about 4 in size)
+    close(out, torch.cat(want).float(), 1e-2, f"prefill attention, climbing scores, H={H} KVH={KVH} Dh={Dh} splits={nsplit}")
+
+
 @pytest.mark.parametrize("where", ["first", "page_edge", "tile_edge", "tile_edge_64", "far", "last"])
 def test_attention_prefill_bf16_finds_one_far_key(where):
     spike = {"first": lambda ctx: 0, "page_edge": lambda ctx: 16 * 3 - 1, "tile_edge": lambda ctx: 32 * 7,

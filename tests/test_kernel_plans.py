@@ -49,6 +49,9 @@ def test_key_shares_never_exceed_what_the_merge_takes():
                 for context in contexts:
                     n = kernels.prefill_splits(items, kv_heads, group, context, 64 * items)
                     assert 1 <= n <= kernels.MAX_KEY_SPLITS, (items, kv_heads, group, context, n)
+    # one workgroup on each CU: a second beside it for long contexts that are read, and only for those
+    assert [kernels.prefill_splits(32, 8, 2, context, 2048) for context in (1024, 2047, 2048, 16000)] == [1, 1, 2, 2]
+    assert kernels.prefill_splits(32, 8, 2, 16000, 2048, 512) == 1 and kernels.prefill_splits(33, 8, 2, 16000, 2112) == 1
 
 
 def test_sizes_no_kernel_takes_are_refused_when_the_model_is_built():

@@ -449,17 +449,17 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 //
 // The kernel above copies a tile through registers: per tile a thread looks up eight pages, forms eight
 // addresses, loads eight pieces and writes them to LDS, and that arithmetic is a third of its vector
-// instructions. Here a block of 16 keys lies in one page, and wave w stages block w of every tile (64 keys =
-// four blocks): it reads the block's page number with a scalar load, makes the block's keys and values a
-// buffer each, and issues DH / 32 + DH / 32 load instructions whose per-lane offsets never change; no vector
+// instructions. Here a block of 16 keys lies in one page, and wave w stages block w of every tile of 64 keys
+// (of a tile of 32, a half of block w / 2): it reads the block's page number with a scalar load, makes the block's
+// keys and values a buffer each, and issues load instructions whose per-lane offsets never change; no vector
 // arithmetic, no staging registers, no LDS write instructions. One instruction fills 1 KB of consecutive
 // LDS (lane l's 16 bytes at byte 16 l), so the layout is made by choosing what each lane fetches:
 //
-//   keys    [64 rows][DH], unpadded. Row r of a block of 16 holds key pi(r) of the block, pi swapping the
+//   keys    [KD rows][DH], unpadded. Row r of a block of 16 holds key pi(r) of the block, pi swapping the
 //           second and third group of four (0-3, 8-11, 4-7, 12-15): the score product then leaves a lane the
 //           probabilities of 8 consecutive keys, which is the order of the values. 16-byte chunk c of a row
 //           sits at chunk c ^ swizzle(row), which spreads the 16 rows that 16 lanes read over the banks.
-//   values  [4 blocks][DH rows][16 keys], as they lie in a page; the halves of 8 keys of row d swap when
+//   values  [KD / 16 blocks][DH rows][16 keys], as they lie in a page; the halves of 8 keys of row d swap when
 //           (d / 8) is odd, for the banks.
 //
 // The next tile's loads are issued before the current tile's arithmetic and land in the other buffer;
@@ -468,10 +468,18 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 // what lies outside a row's range is masked by position, as above.
 constexpr bool DMA_HEAD_DIM = DH == 32 || DH == 64 || DH == 128 || DH == 256;
 constexpr int KC = DH / 8;                                      // 16-byte chunks of a key row
-constexpr int DMA_LOADS = DH / 32 > 0 ? DH / 32 : 1;            // load instructions a wave issues per tile for keys; as many for values
+// Keys of a tile. Heads of 256 take 32: two buffers of 64 keys would be 128 KB, one workgroup on a compute unit, and
+// the scores of 64 keys beside 128 accumulators and 64 registers of queries do not fit a wave's 256 registers (33 were
+// spilled, and a reload waits for the loads in flight). A prompt of 2048 over one KV head of 256: 16 query heads
+// 204 us with tiles of 64, 106 with 32; 32 query heads 357 and 115. Heads of 128 stay at 64: 51 us, 63 with 32.
+constexpr int KD = DH == 256 ? 32 : 64;
+constexpr int KU = KD / 32;                                     // 32-key score tiles of a tile
+constexpr int KB = KD / 16;                                     // blocks of 16 keys
+constexpr int BLOCK_WAVES = 4 / KB;                             // waves that share the loads of a block
+constexpr int DMA_LOADS = DH >= 32 ? DH / 32 / BLOCK_WAVES : 1; // load instructions a wave issues per tile for keys; as many for values
 constexpr int K_SWZ_SHIFT = KC >= 16 ? 0 : (KC == 8 ? 1 : 2);   // rows that share 256 bytes: 1, 2 or 4
 constexpr int K_SWZ_MASK = (KC < 16 ? KC : 16) - 1;
-constexpr int DMA_TILE = 2 * KT * DH;                           // bf16 elements of one buffer: keys, then values
+constexpr int DMA_TILE = 2 * KD * DH;                           // bf16 elements of one buffer: keys, then values
 typedef __attribute__((address_space(3))) void ap_lds_void_t;
 // Fourth word of a raw buffer descriptor on gfx9-family GPUs: 32-bit float data format, destination
 // selects x, y, z, w; no swizzle, no stride.
@@ -483,7 +491,7 @@ __device__ __forceinline__ int key_of_row16(int r) {
   return ((g == 1 ? 2 : (g == 2 ? 1 : g)) << 2) | (r & 3);
 }
 
-// One tile of 64 keys for a wave's 32 rows, from the LDS layout above. A function of its own with pointers that
+// One tile of KD keys for a wave's 32 rows, from the LDS layout above. A function of its own with pointers that
 // are promised not to alias: the compiler, which otherwise makes every LDS read wait for all loads into LDS
 // that are in flight (here: the next tile's), then leaves the waiting to the kernel's own wait and barrier.
 template <bool CAPPED>
@@ -491,10 +499,10 @@ __device__ __forceinline__ void attend_tile_from_lds(const bf16_t* __restrict__ 
                                                      const Frag (&qf)[KS], floatx16 (&acc)[DT], float& m, float& l,
                                                      const int (&k_frag)[KS], int v_frag, int base, int pos, int lo,
                                                      int hi, bool whole, float scale_log2e, float cap) {
-  floatx16 sc[2];
+  floatx16 sc[KU];
   const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
+  for (int u = 0; u < KU; ++u) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       Frag a;
@@ -505,7 +513,7 @@ __device__ __forceinline__ void attend_tile_from_lds(const bf16_t* __restrict__ 
   if constexpr (CAPPED) {     // capped scores: cap * tanh(s / cap), still in the units of the unscaled product
     const float inv_cap = 1.f / cap;
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < KU; ++u)
 #pragma unroll
       for (int v = 0; v < 16; ++v) sc[u][v] = cap * tanh_fast(sc[u][v] * inv_cap);
   }
@@ -513,7 +521,7 @@ __device__ __forceinline__ void attend_tile_from_lds(const bf16_t* __restrict__ 
   // block of 16 hold its keys in the order 0-3, 8-11, 4-7, 12-15).
   if (!whole) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < KU; ++u)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int kp = base + u * 32 + 16 * (v / 8) + hi * 8 + (v % 8);
@@ -522,17 +530,21 @@ __device__ __forceinline__ void attend_tile_from_lds(const bf16_t* __restrict__ 
   }
   float tile_max = -INFINITY;
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int u = 0; u < KU; ++u)
 #pragma unroll
     for (int v = 0; v < 16; ++v) tile_max = fmaxf(tile_max, sc[u][v]);
   tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, TIE_WAVE));
-  const float m_new = fmaxf(m, tile_max);
+  // A row's reference m follows its running maximum only once that is 2^8 above it: the probabilities stay below 2^8,
+  // where bfloat16 and the float32 sums are as precise as below 1, and the accumulators are seldom rescaled (with 32 rows
+  // to a wave some row's maximum rises in most tiles of a short prompt). Decided for each row by itself, so that no row's
+  // result depends on its neighbours. Prompts of 2048: heads of 128 51.2 -> 48.8 us, of 256 106 -> 93.
+  const float m_new = (tile_max - m) * scale_log2e > 8.f ? tile_max : m;   // m = -inf: the first keys a row sees
   const float neg_mc = (m_new == -INFINITY) ? 0.f : -m_new * scale_log2e;
   const float corr = __builtin_amdgcn_exp2f(fmaf(m, scale_log2e, neg_mc));   // m = -inf: 0
-  Frag pf[4];
+  Frag pf[KB];
   float psum = 0.f;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < KB; ++j)
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
       const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[j / 2][(j % 2) * 8 + e], scale_log2e, neg_mc));   // masked: 0
@@ -553,7 +565,7 @@ __device__ __forceinline__ void attend_tile_from_lds(const bf16_t* __restrict__ 
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < KB; ++j) {
       Frag a;
       a.u4 = *reinterpret_cast<const uint4*>(v_lds + j * 16 * DH + dt * 32 * 16 + v_frag);
       acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, pf[j].v, acc[dt], 0, 0, 0);
@@ -621,7 +633,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     for (int v = 0; v < 16; ++v) acc[dt][v] = 0.f;
   float m = -INFINITY, l = 0.f;
 
-  int tile_begin = wg_first / KT, tile_end = wg_last / KT;       // inclusive
+  int tile_begin = wg_first / KD, tile_end = wg_last / KD;       // inclusive
   if (nsplit > 1) {
     const int per = (tile_end - tile_begin + nsplit) / nsplit;   // ceil(count / nsplit)
     tile_begin += split * per;
@@ -630,13 +642,14 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   const bool empty = tile_begin > tile_end;
 
   // What each lane fetches with load n of a block, as byte offsets into the block's keys and values.
+  const int block = wave / BLOCK_WAVES, load0 = wave % BLOCK_WAVES * DMA_LOADS;
   unsigned k_voff[DMA_LOADS], v_voff[DMA_LOADS];
 #pragma unroll
   for (int n = 0; n < DMA_LOADS; ++n) {
-    const int chunk = n * 64 + lane;                       // LDS chunk within the block's 16 rows
+    const int chunk = (load0 + n) * 64 + lane;             // LDS chunk within the block's 16 rows
     const int r16 = chunk / KC, c_lds = chunk % KC;
     k_voff[n] = static_cast<unsigned>(key_of_row16(r16) * DH * 2 + ((c_lds ^ key_swizzle(r16)) * 16));
-    const int slot = n * 64 + lane;                        // LDS slot within the block's DH rows of two halves
+    const int slot = (load0 + n) * 64 + lane;              // LDS slot within the block's DH rows of two halves
     const int d = slot >> 1, half = (slot & 1) ^ ((d >> 3) & 1);
     v_voff[n] = static_cast<unsigned>((d * block_size + half * 8) * 2);
   }
@@ -645,18 +658,18 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   const size_t head_elems = static_cast<size_t>(kvh) * block_size * DH;
   // The page of block `wave` of tile `tile` (a scalar load), looked up one tile before the block is loaded
   // so that no load waits for it.
-  auto page_of_block = [&](int tile) { return table[min(max(tile * KT + wave * 16, first16), last16) >> block_shift]; };
+  auto page_of_block = [&](int tile) { return table[min(max(tile * KD + block * 16, first16), last16) >> block_shift]; };
   // Block `wave` of tile `tile`, which lies in `page`, into buffer `buf`.
   auto issue = [&](int tile, int buf, int page) {
-    const int p16 = min(max(tile * KT + wave * 16, first16), last16);
+    const int p16 = min(max(tile * KD + block * 16, first16), last16);
     const int off = p16 & (block_size - 1);
     const bf16_t* kb = k_cache + static_cast<size_t>(page) * page_elems + head_elems + static_cast<size_t>(off) * DH;
     const bf16_t* vb = v_cache + static_cast<size_t>(page) * page_elems + head_elems + off;
     const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(kb), 0, 16 * DH * 2, AP_RSRC_FLAGS);
     const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<bf16_t*>(vb), 0, (DH * block_size - off) * 2, AP_RSRC_FLAGS);
-    bf16_t* kdst = lds + buf * DMA_TILE + wave * 16 * DH;
-    bf16_t* vdst = lds + buf * DMA_TILE + KT * DH + wave * 16 * DH;
+    bf16_t* kdst = lds + buf * DMA_TILE + block * 16 * DH + load0 * 512;
+    bf16_t* vdst = lds + buf * DMA_TILE + KD * DH + block * 16 * DH + load0 * 512;
 #pragma unroll
     for (int n = 0; n < DMA_LOADS; ++n)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rsrc, (ap_lds_void_t*)(kdst + n * 512), 16, k_voff[n], 0, 0, 0);
@@ -682,15 +695,15 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   for (int tile = tile_begin; tile <= tile_end; ++tile) {
     const int buf = (tile - tile_begin) & 1;
     const bf16_t* k_lds = lds + buf * DMA_TILE;
-    const bf16_t* v_lds = k_lds + KT * DH;
+    const bf16_t* v_lds = k_lds + KD * DH;
     if (tile < tile_end) {
       issue(tile + 1, buf ^ 1, next_page);           // that buffer was last read before the barrier below
       if (tile + 1 < tile_end) next_page = page_of_block(tile + 2);
     }
 
-    const int base = tile * KT;
+    const int base = tile * KD;
     if (wave_active && base <= wave_last) {
-      const bool whole = base + KT - 1 <= wave_min_pos && base >= first_visible_key(wave_last, window) &&
+      const bool whole = base + KD - 1 <= wave_min_pos && base >= first_visible_key(wave_last, window) &&
                          wave_row0 + 32 <= n_new;
       attend_tile_from_lds<CAPPED>(k_lds, v_lds, qf, acc, m, l, k_frag, v_frag, base, pos, lo, hi, whole, scale_log2e, cap);
     }
@@ -763,7 +776,9 @@ static int launch_prefill_dma(const dim3 grid, hipStream_t stream, const bf16_t*
                               float* part_o, float* part_ml, const float* sinks) {
   const int block_shift = __builtin_ctz(block_size);
   const long planes = static_cast<long>(grid.y) * grid.z;
-  const int flip_from = (nsplit == 1 && planes >= 2 && planes * grid.x <= 2L * compute_units())
+  // Both halves of one resident round, as above; shares of the keys are long and short as their items are (16 heads of
+  // 256 over one KV head, prompt of 2048, two shares: 95 -> 84 us).
+  const int flip_from = (planes >= 2 && planes * grid.x <= 2L * compute_units())
                             ? static_cast<int>(planes / 2) : 0x7fffffff;
   constexpr size_t lds_bytes = 2 * static_cast<size_t>(DMA_TILE) * sizeof(bf16_t);
   static bool configured = false;
