@@ -15,9 +15,10 @@
 // 128-byte lines. With one slice a row is half a line, for which the vector cache takes as long: the product then stood
 // at 11 TB/s from the L2, which gives loads of whole lines 33, however many stages were in flight. Measured, four stages
 // of one slice against three of two: 512 rows over 4096 x 12288 on 256 x 128 66.1 -> 58.6 us, 2048 rows over
-// 4096 x 4096 on 128 x 256 74.7 -> 64.1, 128 rows over 24576 x 4096 on 128 x 128 58.0 -> 47.4. Tiles of 256 x 256 and
-// 256 x 192 have no room for that (two stages of two slices lose 10 to 15 %); tiles of 64 x 128 are better off with
-// three workgroups a compute unit (10 to 20 %).
+// 4096 x 4096 on 128 x 256 74.7 -> 64.1, 128 rows over 24576 x 4096 on 128 x 128 58.0 -> 47.4, 2048 rows over
+// 4096 x 12288 on 256 x 128 231 -> 185; experts of 768 x 2048, 256 rows each, on 128 x 256 86.5 -> 78.7 and 63.4 -> 59.8.
+// Tiles of 256 x 256 and 256 x 192 have no room for that (two stages of two slices lose 10 to 15 %); tiles of 64 x 128
+// are better off with three workgroups a compute unit (10 to 20 %).
 //
 // A staged row of x is G x 64 bytes, unpadded; its 16-byte chunks are exchanged by the row's number (gd_swizzle), which
 // spreads the 32 rows a fragment read touches over the banks. Rows beyond M or N are clamped to the
@@ -41,7 +42,7 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 // Stages of the ring and slices of a group, by the tile (above).
 template <int BM, int BN>
 struct GdShape {
-  static constexpr bool PAIRS = BM * BN >= 128 * 128 && (BM + BN) * 3 * 2 * GD_BK * 2 <= 120 * 1024;
+  static constexpr bool PAIRS = BM * BN >= 128 * 128 && (BM + BN) * 3 * 2 * GD_BK * 2 <= 150 * 1024;
   static constexpr int GROUP = PAIRS ? 2 : 1;
   static constexpr int STAGES = PAIRS ? 3 : 4;
   static constexpr int LDS_BYTES = STAGES * GROUP * (BM + BN) * GD_BK * 2;

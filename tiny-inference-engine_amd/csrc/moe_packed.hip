@@ -190,12 +190,14 @@ __global__ __launch_bounds__(256) void moe_packed_many_rows_kernel(const bf16_t*
 }
 
 // Rows of a row tile by the average number of rows an expert gets (sweeps over 32 experts of 768 x 2048 and 64 of
-// 1536 x 4096, 1 to 2048 tokens, four experts each): 256 only where the wider tile still leaves more than one round of
-// workgroups for the compute units. inner: an expert's inner size.
+// 1536 x 4096, 1 to 4096 tokens, four experts each): 256 only where the wider tile still leaves more than one round of
+// workgroups for the compute units. Both products of 64 experts of 1536 x 4096 in tiles of 128 x 256 and of 256 x 256:
+// 128 rows an expert 617 and 653 us, 256 rows 963 and 881; of 32 experts of 768 x 2048: 256 rows 139 and 181, 512 rows
+// 245 and 214. inner: an expert's inner size.
 extern "C" int tie_moe_packed_tile_rows(int slots, int real, int inner) {
   if (slots < 12L * real) return 16;
   if (slots < 48L * real) return 64;
-  return slots >= 96L * real && static_cast<long>(real) * inner >= 128L * 384 ? 256 : 128;
+  return slots >= 384L * real || (slots >= 192L * real && static_cast<long>(real) * inner >= 128L * 384) ? 256 : 128;
 }
 
 template <int BM, int BN, int MODE>
