@@ -332,19 +332,22 @@ __global__ __launch_bounds__(WAVES* TIE_WAVE) void skinny_gemm_kernel(const bf16
 // weight block of 1 KB needs MT blocks of x, and a compute unit serves a load instruction of a wave in about 65
 // cycles whether it comes from HBM or from L2, so at 64 rows (7 loads for 3 KB of weights) the weights stream
 // at 3.6 TB/s. Here the WAVES waves of a workgroup walk the SAME range of K, each over its own RT weight
-// tiles, and share x: a chunk of U k-blocks of all rows goes from global memory straight into LDS (buffer
-// loads with the lds flag; one instruction brings one 16-row block of 32 k, lane l's 16 bytes - row l % 16,
-// k-chunk l / 16 - to byte 16 l, which is the order the matrix core takes its A operand) and all waves read
-// their fragments from there. Weights still go from memory straight into registers, non-temporally. x then
-// costs MT / (WAVES x RT) of the weights' load instructions.
+// tiles, and share x: a chunk of U = 4 k-blocks of all rows goes from global memory straight into LDS (buffer
+// loads with the lds flag) and all waves read their fragments from there. Weights still go from memory straight into
+// registers, non-temporally. x then costs MT / (WAVES x RT) of the weights' load instructions.
+//
+// One instruction brings four rows of a chunk, 256 consecutive bytes each, in the rows' own order but for the pieces of
+// 16 bytes, which are exchanged by the row's number (rows_swizzle) so that the 16 rows of a fragment lie on different
+// banks. Brought in the order of the matrix core's operand instead (16 rows' 64 bytes, neighbouring lanes on different
+// rows), an instruction kept the vector cache four times as long: at 64 rows 12288 x 2048 gated 16.9 -> 14.5 us,
+// 24576 x 4096 gated 44.4 -> 40.4, 6144 x 4096 in two ranges 16.2 -> 14.0.
 //
 // Both streams run DEPTH chunks ahead of the arithmetic, through a ring of DEPTH + 1 LDS buffers and register
 // sets, and a step waits only until the NEXT chunk has landed (loads complete in the order they were asked
 // for, so that is when at most the loads of the DEPTH - 1 chunks after it are outstanding): the queue of
 // loads never runs empty. (Waiting for everything at each chunk's barrier, as a first version did, left a wave
-// idle for a memory latency a chunk: gate/up of the 8B shape at 64 rows 54 us, now 42.) What bounds it now is
-// x itself: every workgroup reads all of it, 512 KB beside its 785 KB of weights on that shape, and a compute
-// unit takes about 38 GB/s.
+// idle for a memory latency a chunk: gate/up of the 8B shape at 64 rows 54 us, now 40.) What bounds it now is
+// x itself: every workgroup reads all of it, 512 KB beside its 785 KB of weights on that shape.
 //
 // The sums are the very ones of the kernel above: a plane's range of K is walked in the same four parts
 // of per_wave k-blocks, each summed by the matrix core in k order, and the parts are added in their order
@@ -353,6 +356,10 @@ __global__ __launch_bounds__(WAVES* TIE_WAVE) void skinny_gemm_kernel(const bf16
 // The matrix instructions of one chunk: x from LDS, the weights from registers. A function of its own with
 // restrict pointers, so that the compiler knows these LDS reads from the loads into LDS that are in flight
 // (otherwise it waits for all of them before the first read).
+// 16-byte pieces of a row of a chunk lie exchanged by the row's number, over the LDS banks.
+template <int U>
+__device__ __forceinline__ int rows_swizzle(int row) { return row & (4 * U - 1); }
+
 template <int MT, int RT, int U, bool FULL>
 __device__ __forceinline__ void rows_chunk(const bf16_t* __restrict__ xc, const bf16x8_t (&wr)[RT][U],
                                            floatx4 (&acc)[MT][RT], int kb0, int kb_hi, int lane) {
@@ -361,7 +368,8 @@ __device__ __forceinline__ void rows_chunk(const bf16_t* __restrict__ xc, const 
     if (FULL || kb0 + u < kb_hi) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        const sk_u32x4_t av = *reinterpret_cast<const sk_u32x4_t*>(xc + (u * MT + mt) * 512 + lane * 8);
+        const sk_u32x4_t av = *reinterpret_cast<const sk_u32x4_t*>(
+            xc + (mt * 16 + (lane & 15)) * (U * 32) + (((u * 4 + (lane >> 4)) ^ rows_swizzle<U>(lane & 15)) * 8));
         const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(&av);
 #pragma unroll
         for (int t = 0; t < RT; ++t) acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, wr[t][u], acc[mt][t], 0, 0, 0);
@@ -406,13 +414,13 @@ __global__ __launch_bounds__(WAVES* TIE_WAVE) void skinny_rows_kernel(const bf16
   // x as a buffer: rows beyond M lie beyond its end and read as zeros.
   const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<bf16_t*>(x), 0, static_cast<int>(static_cast<size_t>(M) * K * 2), SK_RSRC_FLAGS);
-  const unsigned lane_off = (static_cast<unsigned>(lane & 15) * K + (lane >> 4) * 8) * 2;   // bytes, within a 16-row block
-  const unsigned tile_rows = 16u * K * 2;
+  static_assert(U == 4, "an instruction brings four rows of a chunk");
+  const unsigned row_bytes = static_cast<unsigned>(K) * 2;
 
   // Chunk c: k-blocks kb_lo + c U and the U - 1 after it. Its loads, into set S of the ring: every wave issues
-  // the same number of them whatever the chunk (the waits count instructions): the blocks (u, mt) of x are dealt
-  // to the waves in turn, a wave with one block fewer loads one of the others' again, and k-blocks beyond the
-  // range are the range's last again (their products are not formed).
+  // the same number of them whatever the chunk (the waits count instructions): the blocks of four rows of x are dealt
+  // to the waves in turn, a wave with one block fewer loads one of the others' again, and what lies beyond the
+  // range is the range's last again (its products are not formed).
   bf16x8_t wr[NS][RT][U];
   auto issue = [&](auto set, int chunk) {
     constexpr int S = decltype(set)::value;
@@ -420,9 +428,10 @@ __global__ __launch_bounds__(WAVES* TIE_WAVE) void skinny_rows_kernel(const bf16
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       const int b = (i * WAVES + wave) % (U * MT);
-      const int u = b / MT, mt = b % MT;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, (sk_lds_void_t*)(&xs[S][(u * MT + mt) * 512]), 16,
-                                               lane_off + mt * tile_rows, min(kb0 + u, kb_hi - 1) * 64, 0, 0);
+      const int row = b * 4 + (lane >> 4);
+      const int piece = min(kb0 * 4 + ((lane & 15) ^ rows_swizzle<U>(row & 15)), kb_hi * 4 - 1);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, (sk_lds_void_t*)(&xs[S][b * 512]), 16,
+                                               row * row_bytes + piece * 16, 0, 0, 0);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
