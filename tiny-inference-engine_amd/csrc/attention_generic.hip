@@ -1,7 +1,7 @@
 // Paged causal attention with float32 arithmetic for any head size, block size,
 // head grouping and window: one workgroup per (query row, query head), used for
-// prompt portions and decoded tokens alike. It is the true 32-bit path and the
-// fallback for shapes the MFMA kernels refuse.
+// prompt portions and decoded tokens alike: the fallback for shapes the
+// matrix-core kernels refuse.
 //
 // Query row t of sequence s sits at position pos = ctx[s] - n_new[s] + (t - qs[s])
 // and reads keys start..pos through the sequence's block table, where start = 0,

@@ -599,7 +599,7 @@ extern "C" int tie_gemm_bf16_tile(int M, int N, int K, int packed, int splits) {
 //       6 = 128x256, 7 = 128x128, 8 = 64x256, 9 = 64x128 likewise, for fewer rows; 10 = 256x192 likewise, for
 //       widths that 256 columns a tile leave with a round of workgroups that does not fill the compute units.
 // packed: w is stored in blocks of 16 rows x 32 k, 1 KB each, in the matrix cores' operand order (as the
-//       decode product reads it); N % 16 == 0, and only tiles 4 and 5 read it.
+//       decode product reads it); N % 16 == 0, and only the tiles that load straight into LDS read it.
 extern "C" int tie_gemm_bf16(const void* x, const void* w, void* out, int out_dtype, int accumulate, int gated, int M,
                              int N, int K, int tile, int splits, int packed, hipStream_t stream) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || splits < 1) return TIE_BAD_ARGUMENT;

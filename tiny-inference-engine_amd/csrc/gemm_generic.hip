@@ -1,7 +1,7 @@
 // The plain matrix product for gfx950: out[T, N] (+)= x[T, K] . w[N, K]^T with
 // float32 multiply-adds on the vector units, for any sizes and any mix of
-// float32 / bfloat16 operands. It is the true 32-bit path of every projection
-// and the fallback for shapes the MFMA kernels refuse. Each output element is
+// float32 / bfloat16 operands: the fallback for operands of mixed types and for
+// shapes the matrix-core kernels refuse. Each output element is
 // summed over k in ascending order by one thread, so a row's result does not
 // depend on how many other rows the call holds.
 // Reference contraction: src/backend/cpu/cpu_backend.cpp:93-139 (x @ w^T, weights [out, in]).
