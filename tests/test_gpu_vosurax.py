@@ -548,6 +548,27 @@ def test_layers_of_one_shape_run_from_one_launch_list(folders, name, entries):
             assert all(torch.equal(got[0][rid][p], got[1][rid][p]) for p in range(len(toks)))
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("layers", [6, 7])
+def test_norms_behind_two_mixers_keep_their_layers_weights(tmp_path, layers, dtype):
+    """Layers of one shape without feed-forwards: what a layer leaves for the next one's first pass reads that layer's own
+    norms, in steps of few rows and of many, the last layer's as well: the bits of a run of every layer's own code."""
+    from tie_amd.engine.replay import TraceReplayer
+
+    config = dict(CONFIGS["D"], layers=[dict(CONFIGS["D"]["layers"][0], mlp=None)] * layers)
+    folder = write_model(tmp_path / "m", config, 23, dtype)
+    requests = th.make_requests(config["vocab"], [5, 40], seed=24)
+    want = reference(folder, config, requests)
+    for rid, tokens in requests.items():
+        got = []
+        for replay in (True, False):
+            rep = TraceReplayer.from_folder(folder, dtype, 256, block_size=16)
+            rep.model.replay_layers = replay
+            got.append(th.collect(rep, th.whole({rid: tokens})))
+        check(got[0], {rid: want[rid]}, TOLERANCE[dtype], f"{layers} layers, {len(tokens)} rows")
+        assert all(torch.equal(got[0][rid][p], got[1][rid][p]) for p in range(len(tokens)))
+
+
 def test_a_fault_of_one_position_or_one_term_would_show(folders):
     """The engine agrees with the plain model, and the plain model with one mechanism slightly off does not agree
     with the engine by a wide margin."""

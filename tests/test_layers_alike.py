@@ -4,6 +4,8 @@ cache plane of their own (or all read one), must run their own code."""
 
 import dataclasses
 
+import pytest
+
 from conftest import TINY_B
 
 import tie_amd  # noqa: F401  (registers the architecture and the parts)
@@ -59,3 +61,91 @@ def test_entries_that_share_some_cache_planes_are_not_alike():
     assert alike(dataclasses.replace(spec, order=shared)) == {0: 4}
     one_plane = own[:4] + tuple(LayerCall(l, 3) for l in range(4, 8))
     assert alike(dataclasses.replace(spec, order=one_plane)) == {0: 4, 4: 8}
+
+
+def launches_of_steps(monkeypatch, config, dtype, tensors, rows):
+    """What steps of ``rows`` tokens launch with layers run from a launch list and with every layer running its own code,
+    as ``(kernel, arguments)``: the model's host code with the launches themselves left out."""
+    import torch
+
+    from tie_amd import kernels
+    from tie_amd.cache.manager import CacheManager
+    from tie_amd.engine.batch import StepEntry
+    from tie_amd.engine.runner import ModelRunner
+    from tie_amd.models.builder import load_model_from_tensors
+
+    log, got, replayed = [], [], 0
+
+    def call(fn, what, *args):
+        if kernels._recording is not None:
+            kernels._recording.append((fn, args, what))
+        log.append((what, args))
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda self: True), raising=False)
+    monkeypatch.setattr(kernels, "_call", call)
+    monkeypatch.setattr(kernels, "replay_call", lambda fn, what, args: log.append((what, tuple(args))))
+    monkeypatch.setattr(kernels, "_stream", lambda: 0)
+    model = load_model_from_tensors(config, tensors, dtype, "cpu")
+    cache = CacheManager(model.cache_plan, block_size=16, num_blocks=32, dtype=dtype, device=torch.device("cpu"))
+    runner = ModelRunner(model, cache)
+    request = cache.new_request()
+    assert cache.reserve(request, rows)
+    for replay in (False, True, False):            # the first settles the scratch memory
+        model.replay_layers, model.layers_replayed = replay, 0
+        log.clear()
+        runner.step([StepEntry(request, 0, list(range(rows)), [rows - 1])])
+        got.append(list(log))
+        replayed = max(replayed, model.layers_replayed)
+    # A step's work lists are new tensors: only addresses of weights, of scratch memory and of the cache are compared.
+    kept = [tensor for tensors in model._layer_tensors.values() for tensor in tensors]
+    kept += [(t.data_ptr(), t.numel() * t.element_size()) for t in runner.workspace._buffers.values()]
+    kept += [(t.data_ptr(), t.numel() * t.element_size()) for t in (*cache.kv.values(), *cache.state.values())]
+
+    def comparable(args):
+        return tuple(a if not isinstance(a, int) or a < 1 << 32 or any(0 <= a - at < size for at, size in kept)
+                     else "the step's" for a in args)
+
+    return [[(what, comparable(args)) for what, args in log] for log in got[1:]] + [model, replayed]
+
+
+def norms_behind_two_mixers(layers):
+    from vosurax_fixtures import _parallel
+
+    return {"architecture": "Vosurax", "vocab": 64, "width": 48, "norm": {"eps": 1e-5},
+            "layers": [{**_parallel((4, 2, 16, 32, 0.3, 40), (2, 40, 72, 5.0)), "mlp": None} for _ in range(layers)]}
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("rows", [5, 40])
+@pytest.mark.parametrize("layers", [6, 7])
+def test_a_pass_left_for_the_next_layer_keeps_its_own_layers_weights(monkeypatch, layers, rows, dtype):
+    """A layer without a feed-forward leaves the norms behind its two mixers to the next layer's first pass: every pass
+    reads the weights of the layer that left it, the last one's behind the last layer."""
+    from vosurax_fixtures import make_tensors
+
+    config = norms_behind_two_mixers(layers)
+    listed, own, model, replayed = launches_of_steps(monkeypatch, config, dtype, make_tensors(config, 3, dtype), rows)
+    assert model._alike == {0: layers}
+    assert [args[4] for what, args in listed if what == "add_normed_results"] == \
+        [layer.mixer.norm_weights[0].data_ptr() for layer in model.layers]
+    assert listed == own
+
+
+@pytest.mark.parametrize("rows", [3, 40])
+@pytest.mark.parametrize("width", [64, 4096])
+def test_a_launch_list_launches_what_every_layers_own_code_does(monkeypatch, width, rows):
+    """In a step of a few rows every sub-layer leaves its last product to the next norm: over the weight of the layer it
+    ends, which for a layer's first norm is the layer before."""
+    import torch
+
+    from tie_amd.models import expected_tensors_for_config
+    from tie_amd.weights.random_init import random_tensors
+
+    config = dict(TINY_B, num_hidden_layers=7, hidden_size=width, intermediate_size=128)
+    specs = [s for s in expected_tensors_for_config(config) if not s.optional]
+    tensors = dict(random_tensors(specs, 5, torch.bfloat16, device="cpu"))
+    listed, own, model, replayed = launches_of_steps(monkeypatch, config, "bfloat16", tensors, rows)
+    assert replayed == 4
+    assert listed == own
+    pending = sum(what == "skinny_gemm_bf16_norm" and args[15] is not None for what, args in own)   # a next norm's weight
+    assert pending == (13 if rows == 3 else 0)

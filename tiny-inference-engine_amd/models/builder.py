@@ -153,6 +153,7 @@ class Model:
         self.layers_replayed = 0                      # entries of the run order run from another's launch list
         self._alike: Dict[int, int] = {}              # first entry of a run of layers alike -> one past its last
         self._layer_tensors: Dict[int, list] = {}     # entry -> (address, bytes) of its layer's device tensors
+        self._layer_projections: Dict[int, list] = {}     # entry -> its layer's Linear objects, in one order
 
     # --------------------------------------------------------------- tensors
     def _all_parts(self):
@@ -213,13 +214,14 @@ class Model:
         the same places, the same kind of cache binding; each entry a layer of its own, and each with a cache plane
         of its own or all reading one.
         """
-        self._alike, self._layer_tensors = {}, {}
+        self._alike, self._layer_tensors, self._layer_projections = {}, {}, {}
         signatures = []
         for index, call in enumerate(self.spec.order):
             tensors, classes, scalars = [], [], []
             layer_parts = self.layers[call.layer].parts()
             _walk_parts(layer_parts, tensors, classes, set(), scalars)
             self._layer_tensors[index] = [(address, size) for address, size, _, _ in tensors]
+            self._layer_projections[index] = _projections(layer_parts, [], set())
             entry = self.cache_plan.calls[index]
             binding = None if entry is None else tuple((e.group, e.writes) for e in entry) \
                 if isinstance(entry, tuple) else (entry.group, entry.writes)
@@ -256,17 +258,29 @@ class Model:
                 self._alike[start] = end
             start = end
 
-    def _entry_tensors(self, ctx: StepContext, index: int, cache) -> list:
+    def _entry_tensors(self, ctx: StepContext, index: int, cache, place: Optional[int]) -> list:
         """(address, bytes) of everything the launches of entry ``index`` may point to that is not the step's: its
-        layer's tensors and its cache, and the tensors of the layer before it, whose last product its first norm
-        launches in steps of a few rows (``StepContext.defer_product``)."""
+        layer's tensors and its cache. ``place``: the layer before left its projection of that place pending
+        (``_pending_place``), and this layer's first launch reads that weight."""
         tensors = list(self._layer_tensors[index])
         for binding in (cache if isinstance(cache, tuple) else (cache,)):
             for name in ("k_cache", "v_cache", "state"):
                 t = getattr(binding, name, None)
                 if isinstance(t, torch.Tensor):
                     tensors.append((t.data_ptr(), t.numel() * t.element_size()))
-        return tensors + self._layer_tensors[index - 1]
+        if place is not None:
+            weight = self._layer_projections[index - 1][place].weight
+            weight = weight.blocks if isinstance(weight, kernels.PackedWeight) else weight
+            tensors.append((weight.data_ptr(), weight.numel() * weight.element_size()))
+        return tensors
+
+    def _pending_place(self, ctx: StepContext, index: int) -> Optional[int]:
+        """Which of the projections of entry ``index``'s layer has its product pending in the step context: its place
+        among them, the same for every layer of the shape; None where nothing is pending, -1 for a product of another
+        object, which no other layer's can stand in for."""
+        if ctx.pending_linear is None:
+            return None
+        return next((i for i, l in enumerate(self._layer_projections[index]) if l is ctx.pending_linear), -1)
 
     @staticmethod
     def _launch_list(noted_a, noted_b, tensors_a, tensors_b) -> Optional[List[_Launch]]:
@@ -308,7 +322,10 @@ class Model:
 
         In steps of a few rows a layer may leave its last product pending in the step context. The next layer's list
         begins with that product, over the weight of the layer before, and behind the last of the layers the context
-        is told that it is now this layer's product that is pending.
+        is told that it is now this layer's product that is pending. That weight is all a list may take from the layer
+        before: a pass left for the next layer (``StepContext.leave_late``) that reads other tensors of its own layer (the
+        norms behind two mixers) makes two layers' launches differ in an address of neither's, and every layer runs its
+        own code.
         """
         def run(index):
             cache = ctx.cache_of(index)
@@ -317,6 +334,8 @@ class Model:
             return cache
 
         run(start)
+        place = self._pending_place(ctx, start)
+        carried = place is None or place >= 0
         noted, tensors = [], []
         for index in (start + 1, start + 2):
             record = kernels.start_recording()
@@ -325,18 +344,14 @@ class Model:
             finally:
                 kernels.stop_recording()
             noted.append(record)
-            tensors.append(self._entry_tensors(ctx, index, cache))
-        launches = self._launch_list(noted[0], noted[1], tensors[0], tensors[1])
-        pending, place = ctx.pending_linear, None
-        if pending is not None:
-            place = next((i for i, l in enumerate(self._projections_of(start + 2)) if l is pending), None)
-            if place is None:              # a product of no part of the layer: nothing to put in its place
-                launches = None
+            tensors.append(self._entry_tensors(ctx, index, cache, place if carried else None))
+            carried = carried and self._pending_place(ctx, index) == place
+        launches = self._launch_list(noted[0], noted[1], tensors[0], tensors[1]) if carried else None
         for index in range(start + 3, end):
             if launches is None:
                 run(index)
                 continue
-            own = self._entry_tensors(ctx, index, ctx.cache_of(index))
+            own = self._entry_tensors(ctx, index, ctx.cache_of(index), place)
             for launch in launches:
                 if launch.patches:
                     args = list(launch.args)
@@ -347,10 +362,7 @@ class Model:
                     kernels.replay_call(launch.fn, launch.what, launch.args)
             self.layers_replayed += 1
         if launches is not None and place is not None:
-            ctx.pending_linear = self._projections_of(end - 1)[place]
-
-    def _projections_of(self, index: int) -> list:
-        return _projections(self.layers[self.spec.order[index].layer].parts(), [], set())
+            ctx.pending_linear = self._layer_projections[end - 1][place]
 
     # ------------------------------------------------------------------ step
     def forward(self, ctx: StepContext) -> Optional[torch.Tensor]:
