@@ -471,7 +471,7 @@ constexpr int KC = DH / 8;                                      // 16-byte chunk
 // Keys of a tile. Heads of 256 take 32: two buffers of 64 keys would be 128 KB, one workgroup on a compute unit, and
 // the scores of 64 keys beside 128 accumulators and 64 registers of queries do not fit a wave's 256 registers (33 were
 // spilled, and a reload waits for the loads in flight). A prompt of 2048 over one KV head of 256: 16 query heads
-// 204 us with tiles of 64, 106 with 32; 32 query heads 357 and 115. Heads of 128 stay at 64: 51 us, 63 with 32.
+// 224 us with tiles of 64, 103 with 32; 32 query heads 360 and 115. Heads of 128 stay at 64: 51 us, 63 with 32.
 constexpr int KD = DH == 256 ? 32 : 64;
 constexpr int KU = KD / 32;                                     // 32-key score tiles of a tile
 constexpr int KB = KD / 16;                                     // blocks of 16 keys
@@ -534,11 +534,10 @@ __device__ __forceinline__ void attend_tile_from_lds(const bf16_t* __restrict__ 
 #pragma unroll
     for (int v = 0; v < 16; ++v) tile_max = fmaxf(tile_max, sc[u][v]);
   tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, TIE_WAVE));
-  // A row's reference m follows its running maximum only once that is 2^8 above it: the probabilities stay below 2^8,
-  // where bfloat16 and the float32 sums are as precise as below 1, and the accumulators are seldom rescaled (with 32 rows
-  // to a wave some row's maximum rises in most tiles of a short prompt). Decided for each row by itself, so that no row's
-  // result depends on its neighbours. Prompts of 2048: heads of 128 51.2 -> 48.8 us, of 256 106 -> 93.
-  const float m_new = (tile_max - m) * scale_log2e > 8.f ? tile_max : m;   // m = -inf: the first keys a row sees
+  // The reference is the running maximum itself: the largest probability, rounded to bfloat16 for the product but not for
+  // the sum psum, is then exactly 1. (A reference that follows in steps of 2^8 spares most rescales of the accumulators,
+  // 2 to 13 us of a prompt of 2048, and leaves 1.7 times the error for scores of deviation 2, 3.3 times at 8.)
+  const float m_new = fmaxf(m, tile_max);
   const float neg_mc = (m_new == -INFINITY) ? 0.f : -m_new * scale_log2e;
   const float corr = __builtin_amdgcn_exp2f(fmaf(m, scale_log2e, neg_mc));   // m = -inf: 0
   Frag pf[KB];

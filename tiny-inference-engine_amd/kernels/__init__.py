@@ -1719,8 +1719,11 @@ def prefill_splits(num_items: int, num_kv_heads: int, group_size: int, max_conte
     """Shares the keys of every prefill item are cut into: more than one only where the items alone leave CUs idle.
 
     One workgroup on each of the 256 CUs is such a step too where contexts are long: two shares put a second
-    beside it and even out short and long rows. 2048 rows, 16 query heads over 8 KV heads of 128: 52 us whole and 49
-    in two shares, after 14000 earlier positions 343 and 270; a context of 1024 is better whole (28 us, 35), and so are rows that reach no further.
+    beside it and even out short and long rows. 2048 rows, 16 query heads over 8 KV heads of 128: 55 us whole and 50
+    in two shares, after 14000 earlier positions 332 and 276; over one KV head of 256 103 and 83; a context of 1024 is
+    better whole (29 us, 36), and so are rows that reach no further. Above 256 workgroups nothing is cut: with 288 three
+    shares take 180 us for 223 behind 6000 earlier positions and 64 for 59 in a prompt, with 384 up to four shares gain
+    6 % or lose 6 %, with 504 two lose 9 to 28 %.
     """
     passes = -(-group_size // min(group_size, 4))
     workgroups = num_items * num_kv_heads * passes
