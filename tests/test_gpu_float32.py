@@ -157,6 +157,28 @@ def test_attention_f32_values_that_are_no_numbers(bad):
         close(out[~expect], want[~expect].cpu().to(F64), 2e-6, f"the other results, key {key}")
 
 
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_attention_f32_scores_of_minus_infinity(nsplit):
+    """A key whose score is -inf weighs nothing beside any other, also where it is all a tile shows a row, or all that one
+    wave of a workgroup or one share holds: the same as the kernel that walks key by key."""
+    from tie_amd import kernels
+
+    H, KVH, Dh, n = 4, 2, 32, 140
+    for keys in ((0,), (16,), (31, 32), (48, 49, 50), tuple(range(64, 80)), tuple(range(1, 140))):
+        case, S = attention_case(H, KVH, Dh, 16, lens_new=[n], lens_ctx=[n], seed=13)
+        case["q"].view(n, H, Dh)[:, :, 2].abs_().add_(0.1)
+        for key in keys:
+            case["kc"][int(case["tables"][0, key // 16]), :, key % 16, 2] = -float("inf")
+        want = torch.empty_like(case["q"])
+        kernels.paged_attention_generic(case["q"], case["kc"], case["vc"], want, case["query_start"], case["context_lens"],
+                                        case["tables"], case["seq_of_row"], H, Dh ** -0.5)
+        out = run(case, H, S, Dh, nsplit)
+        there = torch.isfinite(want)
+        assert bool(there[1:].all()) and bool(there[0].all()) == (0 not in keys)     # row 0 sees key 0 alone
+        assert torch.equal(torch.isfinite(out), there), f"keys {keys}"
+        close(out[there], want[there].cpu().to(F64), 4e-6, f"keys {keys}")
+
+
 def test_the_32_bit_path_takes_these_kernels():
     """The dispatchers: operands the kernels take go there (other results only by rounding), the others as before."""
     from tie_amd import kernels

@@ -171,7 +171,7 @@ __global__ __launch_bounds__(W* TIE_WAVE) void attention_f32_kernel(
     float own = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[i] = partly && (key0 + i < start || key0 + i > pos) ? 0.f : expf(p[i] - m);
+      p[i] = p[i] == -INFINITY ? 0.f : expf(p[i] - m);      // hidden, or a score of -inf: no weight, also where m is -inf
       own += p[i];
     }
     l += own;
