@@ -107,7 +107,7 @@ def test_cache_pages_are_sized_by_the_cache_dtype():
         CacheManager(plan, block_size=4, num_blocks=8, dtype="int8")
 
 
-TILE_ROWS_COLS = {4: (256, 256), 5: (256, 128), 6: (128, 256), 7: (128, 128), 10: (256, 192)}
+TILE_ROWS_COLS = {4: (256, 256), 5: (256, 128), 6: (128, 256), 7: (128, 128), 10: (256, 192), 11: (128, 192)}
 
 
 def test_the_tiled_product_plans_by_rounds_of_workgroups():

@@ -585,8 +585,7 @@ extern "C" int tie_gemm_bf16_splits(int M, int N, int K, int packed) {
 // The tile a product left to choose runs on (the numbers of tie_gemm_bf16's `tile`), with `splits` ranges of K
 // fixed by the caller (1: none) or 0 for the plan's own number; for tests and sweeps.
 extern "C" int tie_gemm_bf16_tile(int M, int N, int K, int packed, int splits) {
-  const int tile = gemm_plan(M, N, K, straight_to_lds_shape(N, K), splits, packed != 0).tile;
-  return tile == 11 ? 6 : tile;        // 128 x 192 goes by the number of 128 x 256, whose narrower form it is
+  return gemm_plan(M, N, K, straight_to_lds_shape(N, K), splits, packed != 0).tile;
 }
 
 // out_dtype: TIE_F32 or TIE_BF16; accumulate adds into a float32 output; gated (bfloat16 output of N / 2
