@@ -457,11 +457,15 @@ static bool gemm_dma_takes(const void* x, const void* w, const void* out, int N,
 //   * a round is a few microseconds of start and end plus its slices of 32 along K at the tile's own pace, both more where
 //     it fills every compute unit;
 //   * every plane is written once here and read once by its consumer.
-// The constants are a least-squares fit, tile by tile, to sweeps over eight packed projections (2048 x 2048 to
-// 24576 x 4096, every tile, 1 to 8 ranges) at 200 to 2048 rows, and to those at 96 and 128 rows, where the weights come
-// from memory by few workgroups; 6 to 14 % root mean square. The choice lies 0.7 % above the best forced (tile, ranges)
-// on average and 16 % at most, on the best at 96 and 128 rows. Rows of fewer than 65 over row-major weights and odd K or N
-// stay with the older tiles and their rule.
+// start, full, slice and press are a least-squares fit, tile by tile, to sweeps over eight packed projections (2048 x 2048
+// to 24576 x 4096, every tile, 1 to 8 ranges) at 200 to 2048 rows, and to those at 96 and 128 rows, where the weights come
+// from memory by few workgroups; lead and scatter were then chosen, above 128 rows, on the projections of eight layer
+// shapes 1024 to 8192 wide at ten row counts, full tiles and not, and 22 weights of random sizes (768 to 40000 rows, K 768
+// to 20000) at random row counts, every candidate timed with its consumer and the weights from memory. The choice lies
+// 0.9 % above the best forced (tile, ranges) there, 1.1 % over 22 random weights held out, 10 % at worst but for K above
+// 8000 over fewer than 2000 rows of w (35 %); without the two it lay 1.9 and 1.3 % above and took 98 us where 81 do
+// (576 rows over 4096 x 12288). 65 to 128 rows: 0.4 % above the best over the eight shapes, 0.9 % over the random weights,
+// 15 % at worst. Rows of fewer than 65 over row-major weights and odd K or N stay with the older tiles and their rule.
 struct GemmPlan { int tile, splits; };
 
 static int legacy_splits(int M, int N, int K) {
@@ -480,22 +484,31 @@ static int legacy_splits(int M, int N, int K) {
 
 // start_us: a round's start and end; slice_us: one slice of 32 along K while most compute units are idle. From half a round
 // of workgroups to a full one both grow, by full_us and by the factor 1 + press: the units share the L2 and the clock.
+// lead: what a slice gains as the last row tile empties: its workgroups run ahead and bring w into the L2 for the others
+// (576 rows over 4096 x 12288 in two ranges of 256 x 256 take 117 us, 512 take 146). scatter: what it loses where the tiles
+// are no multiple of eight, so that the row tiles of one piece of w do not follow each other on one die.
 // per_cu workgroups on one compute unit each take `shared` times as long.
-struct DmaTile { int id, bm, bn; float start_us, full_us, slice_us, press; int per_cu; float shared; };
-static const DmaTile kDmaTiles[] = {
-    {4, 256, 256, 8.57f, 7.37f, 0.629f, 0.17f, 1, 1.f}, {10, 256, 192, 6.14f, 2.53f, 0.580f, 0.15f, 1, 1.f},
-    {5, 256, 128, 6.91f, 0.00f, 0.367f, 0.32f, 1, 1.f}, {6, 128, 256, 6.20f, 0.91f, 0.400f, 0.18f, 1, 1.f},
-    {11, 128, 192, 5.10f, 0.0f, 0.327f, 0.12f, 1, 1.f}, {7, 128, 128, 3.48f, 0.91f, 0.250f, 0.14f, 1, 1.f}};
-static const DmaTile kFewRowsTiles[] = {
-    {6, 128, 256, 6.11f, 3.12f, 0.440f, 0.20f, 1, 1.f}, {7, 128, 128, 3.91f, 0.68f, 0.276f, 0.43f, 1, 1.f},
-    {8, 64, 256, 3.62f, 0.87f, 0.373f, 0.27f, 1, 1.f}, {9, 64, 128, 3.19f, 4.31f, 0.248f, 0.23f, 3, 2.06f}};
+struct DmaTile { int id, bm, bn; float start_us, full_us, slice_us, press, lead, scatter; int per_cu; float shared; };
+static const DmaTile kDmaTiles[] = {{4, 256, 256, 8.57f, 7.37f, 0.629f, 0.17f, 0.17f, 0.18f, 1, 1.f},
+                                    {10, 256, 192, 6.14f, 2.53f, 0.580f, 0.15f, 0.18f, 0.f, 1, 1.f},
+                                    {5, 256, 128, 6.91f, 0.f, 0.367f, 0.32f, 0.11f, 0.11f, 1, 1.f},
+                                    {6, 128, 256, 6.20f, 0.91f, 0.400f, 0.18f, 0.10f, 0.16f, 1, 1.f},
+                                    {11, 128, 192, 5.10f, 0.f, 0.327f, 0.12f, 0.f, 0.12f, 1, 1.f},
+                                    {7, 128, 128, 3.48f, 0.91f, 0.250f, 0.14f, 0.12f, 0.19f, 1, 1.f}};
+static const DmaTile kFewRowsTiles[] = {{6, 128, 256, 6.11f, 3.12f, 0.440f, 0.20f, 0.f, 0.f, 1, 1.f},
+                                        {7, 128, 128, 3.91f, 0.68f, 0.276f, 0.43f, 0.f, 0.f, 1, 1.f},
+                                        {8, 64, 256, 3.62f, 0.87f, 0.373f, 0.27f, 0.f, 0.f, 1, 1.f},
+                                        {9, 64, 128, 3.19f, 4.31f, 0.248f, 0.23f, 0.f, 0.f, 3, 2.06f}};
 
 static float estimated_us(const DmaTile& t, int M, int N, int K, int ranges, float plane_us_per_mb) {
-  const long wgs = static_cast<long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * ranges;
+  const int row_tiles = (M + t.bm - 1) / t.bm;
+  const long tiles = static_cast<long>(row_tiles) * ((N + t.bn - 1) / t.bn), wgs = tiles * ranges;
   const int k_slices = K / GD_BK;
   const int slices = (k_slices + ranges - 1) / ranges;
   const long slots = 256L * t.per_cu;
-  const float pace = t.slice_us * (t.per_cu > 1 && wgs > 256 ? t.shared : 1.0f);
+  const float empty = 1.0f - static_cast<float>(M - (row_tiles - 1) * t.bm) / t.bm;       // share of the last row tile
+  const float pace = t.slice_us * (t.per_cu > 1 && wgs > 256 ? t.shared : 1.0f) * (1.0f - t.lead * empty) *
+                     (tiles % 8 != 0 && row_tiles > 1 ? 1.0f + t.scatter : 1.0f);
   auto round_us = [&](float fill) {
     const float crowded = fminf(fmaxf((fill - 0.5f) * 2.0f, 0.f), 1.f);
     return t.start_us + t.full_us * crowded + slices * pace * (1.0f + t.press * crowded);
