@@ -375,14 +375,15 @@ def test_skinny_gemm_bf16_at_the_widths_of_other_model_sizes(M, N, K, gated):
         assert torch.equal(again, planes), f"tiles {rt}, batch {u}: the sums depend on the launch's shape"
 
 
-@pytest.mark.parametrize("M,N,K", [(33, 65536, 1024), (64, 65552, 1024), (40, 65552, 1056), (64, 65520, 1024)])
+@pytest.mark.parametrize("M,N,K", [(33, 65536, 3072), (64, 65552, 3072), (40, 65552, 3104), (64, 65520, 3072),
+                                   (33, 65536, 1024), (64, 65552, 2560)])
 def test_products_of_33_to_64_rows_around_the_width_of_a_vocabulary(M, N, K):
     from tie_amd import kernels
 
     x = rnd(M, K, seed=43, dtype=torch.bfloat16).cuda()
     w = rnd(N, K, seed=44, scale=0.05, dtype=torch.bfloat16).cuda()
     packed = kernels.pack_weight(w)
-    assert kernels.decode_product_rows(M, packed) == (N >= 65536 and K % 512 == 0)
+    assert kernels.decode_product_rows(M, packed) == (N >= 65536 and K >= 3072 and K % 512 == 0)
     out = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
     kernels.linear(x, packed, out)
     close(out, plain.linear(x.cpu(), w.cpu()), 1e-5, f"vocabulary product {M}x{N}x{K}")

@@ -581,11 +581,13 @@ static GemmPlan gemm_plan(int M, int N, int K, bool straight_to_lds, int splits,
 static bool straight_to_lds_shape(int N, int K) { return K % GD_BK == 0 && N % 4 == 0 && K <= (1 << 22) && K >= 3 * GD_BK; }
 
 // Whether a product of 33 to 64 rows runs faster here than on the decode product: over packed weights whose
-// shape the tiles that load straight into LDS take, unless it is gated and not very wide, or a vocabulary wide (64 rows
-// over 151936 x 4096: 273 us here, 254 there where K is in whole chunks of its four parts; measured).
+// shape the tiles that load straight into LDS take, unless it is gated and not very wide, or a vocabulary wide with K in
+// whole chunks of the decode product's four parts and long enough. 64 rows, here and there: 151936 x 4096 279 and 256 us,
+// 200064 x 8192 684 and 614, 65536 x 3072 78.5 and 77.9; over seven widths from 65536 to 262144 and K from 3072 to 8192 there is
+// 0.86 to 1.03 of here. Shorter rows are too short for its parts: 65536 x 1024 30.0 and 39.8, 98304 x 2048 90 and 98.
 extern "C" int tie_gemm_bf16_wins_few_rows(int M, int N, int K, int packed, int gated) {
   if (M <= 32 || M > 64 || !packed || !straight_to_lds_shape(N, K) || N % 16 != 0 || K < 1024) return 0;
-  return gated ? N >= 32768 : N < 65536 || K % 512 != 0;
+  return gated ? N >= 32768 : N < 65536 || K < 3072 || K % 512 != 0;
 }
 
 // Ranges of K that a product of M rows over w[N, K] is best cut into when its caller adds planes of
