@@ -164,6 +164,20 @@ def test_the_tiled_product_plans_for_a_last_row_tile_that_is_nearly_empty():
     assert kernels.gemm_tile(576, 19456, 2560, True, 1) == 4
 
 
+def test_experts_take_wide_row_tiles_where_these_still_fill_the_gpu():
+    """(experts, inner size): rows of a tile at 40, 100, 200, 400 and 600 rows an expert. Many or wide experts take 256
+    from 192 on, smaller sets from 480 (16 experts of 512 at 384 rows: 41 us in tiles of 128, 56 in tiles of 256)."""
+    import torch
+    from tie_amd import kernels
+
+    for real, inner, want in ((64, 1536, [64, 128, 256, 256, 256]),
+                              (32, 768, [64, 128, 128, 128, 256]), (16, 512, [64, 128, 128, 128, 256]),
+                              (64, 256, [64, 128, 128, 128, 128]), (192, 256, [64, 128, 256, 256, 256])):
+        got = [kernels.moe_tile_rows(torch.bfloat16, torch.bfloat16, 1024, inner, n * real, real, packed=True)
+               for n in (40, 100, 200, 400, 600)]
+        assert got == want, (real, inner)
+
+
 def test_the_prefill_attention_kernel_refuses_caches_it_cannot_address():
     """Its addresses are 32-bit counts of 8 bytes, a page's number times the page's size by a 24-bit multiply."""
     import torch
