@@ -130,7 +130,8 @@ def main(argv=None) -> int:
                 if M > 16:
                     tiles_tried = ((8, "64 x 256"), (9, "64 x 128")) if M <= 64 else \
                         ((6, "128 x 256"), (7, "128 x 128"), (8, "64 x 256"), (9, "64 x 128")) if M <= 128 else \
-                        ((4, "256 x 256"), (10, "256 x 192"), (5, "256 x 128"), (6, "128 x 256"), (7, "128 x 128"))
+                        ((4, "256 x 256"), (10, "256 x 192"), (5, "256 x 128"), (6, "128 x 256"), (11, "128 x 192"),
+                         (7, "128 x 128"))
                     for tile, shape in tiles_tried:
                         def tiled(i, tile=tile, s=s):
                             if gated:
