@@ -611,7 +611,8 @@ extern "C" int tie_gemm_bf16_tile(int M, int N, int K, int packed, int splits) {
 //       3 = 256x128 (eight waves of 64x64), 4 = 256x256 and 5 = 256x128 loaded straight into LDS (four
 //       waves of 128x128 or 128x64; K % 32 == 0, N % 4 == 0, 16-byte aligned operands, else refused),
 //       6 = 128x256, 7 = 128x128, 8 = 64x256, 9 = 64x128 likewise, for fewer rows; 10 = 256x192 likewise, for
-//       widths that 256 columns a tile leave with a round of workgroups that does not fill the compute units.
+//       widths that 256 columns a tile leave with a round of workgroups that does not fill the compute units;
+//       11 = 128x192 likewise.
 // packed: w is stored in blocks of 16 rows x 32 k, 1 KB each, in the matrix cores' operand order (as the
 //       decode product reads it); N % 16 == 0, and only the tiles that load straight into LDS read it.
 extern "C" int tie_gemm_bf16(const void* x, const void* w, void* out, int out_dtype, int accumulate, int gated, int M,

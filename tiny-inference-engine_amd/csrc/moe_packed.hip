@@ -191,8 +191,8 @@ __global__ __launch_bounds__(256) void moe_packed_many_rows_kernel(const bf16_t*
 
 // Rows of a row tile by the average number of rows an expert gets (sweeps over seventeen sets of 8 to 128 experts of
 // 256 to 4096 x 1024 to 4096, 96 to 1000 rows an expert, unevenly spread, both products): 256 only where the wider tile
-// still leaves more than one round of workgroups for the compute units, for smaller sets only where most experts fill two
-// of them, and never over an inner size of a few slices. Tiles of 128 x 256 and of 256 x 256: 64 experts of 1536 x 4096,
+// still leaves more than one round of workgroups for the compute units; for smaller sets only where most experts fill two
+// of them and the inner size is more than a few slices. Tiles of 128 x 256 and of 256 x 256: 64 experts of 1536 x 4096,
 // 128 rows an expert 617 and 653 us, 256 rows 963 and 881; 32 of 768 x 2048, 384 rows 190 and 200, 512 rows 245 and 214;
 // 16 of 512 x 1024, 384 rows 41 and 56, 512 rows 64 and 55; 64 of 256 x 1024, 512 rows 120 and 129. inner: an expert's
 // inner size.

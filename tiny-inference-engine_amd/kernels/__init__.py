@@ -2148,8 +2148,8 @@ class ExpertRows:
 
 def moe_tile_rows(x_dtype: torch.dtype, w_dtype: torch.dtype, hidden: int, intermediate: int, slots: int,
                   real: int, packed: bool = False) -> int:
-    """Rows of a row tile of the experts' products, which also says which kernels run them: 16, 64 or 128 (by the rows an
-    expert gets on average) for the matrix-core kernels, which take bfloat16 rows and weights whose inner sizes
+    """Rows of a row tile of the experts' products, which also says which kernels run them: 16, 64, 128 or, over packed
+    weights, 256 (by the rows an expert gets on average) for the matrix-core kernels, which take bfloat16 rows and weights whose inner sizes
     are multiples of 8; the float32 kernels' tile otherwise."""
     if packed:                 # weights of ``pack_experts``
         return int(_lib("moe_packed").tie_moe_packed_tile_rows(slots, real, intermediate))
