@@ -476,13 +476,16 @@ def test_gemm_bf16_loaded_straight_into_lds(M, N, K, tile):
 
 @pytest.mark.parametrize("tile", [4, 10])
 @pytest.mark.parametrize("slices,splits", [(95, 1), (96, 1), (97, 1), (193, 2)])
-def test_tiles_whose_rows_begin_a_slice_apart(tile, slices, splits):
-    """From 96 slices of a range on, row tile i begins with slice i and goes round: the sums of another order. A sum of K
-    bfloat16 products lies within sqrt(K) * 6e-8 of the exact one, relative to the root of the summed squares."""
+def test_a_row_keeps_its_bits_wherever_it_lies(tile, slices, splits):
+    """Tiles of 256 rows over short and long ranges: the order of a sum is that of k, whichever row tile holds the row, so
+    equal rows give equal bits, and tiles of 128 rows the same ones. A sum of K bfloat16 products lies within
+    sqrt(K) * 6e-8 of the exact one, relative to the root of the summed squares."""
     from tie_amd import kernels
 
     M, N, K = 700, 208, 32 * slices
     x = rnd(M, K, seed=61, dtype=torch.bfloat16).cuda()
+    x[256:512] = x[:256]
+    x[512:] = x[:M - 512]
     w = rnd(N, K, seed=62, scale=0.1, dtype=torch.bfloat16).cuda()
     want = x.double() @ w.double().T
     bound = want.abs().max() * 6e-8 * K ** 0.5
@@ -491,10 +494,11 @@ def test_tiles_whose_rows_begin_a_slice_apart(tile, slices, splits):
         kernels.gemm_bf16(x, weight, out, tile=tile, splits=splits)
         got = out.double() if splits == 1 else out.double().sum(0)
         assert bool(((got - want).abs() <= bound).all()), (tile, slices, float((got - want).abs().max() / bound))
-        if slices < 96:
-            same = torch.empty_like(out)
-            kernels.gemm_bf16(x, weight, same, tile=7, splits=splits)
-            assert torch.equal(out, same)
+        planes = out.view(splits, M, N)
+        assert torch.equal(planes[:, 256:512], planes[:, :256]) and torch.equal(planes[:, 512:], planes[:, :M - 512])
+        same = torch.empty_like(out)
+        kernels.gemm_bf16(x, weight, same, tile=7, splits=splits)
+        assert torch.equal(out, same)
 
 
 @pytest.mark.parametrize("M,N", [(1, 64), (130, 208), (257, 400)])

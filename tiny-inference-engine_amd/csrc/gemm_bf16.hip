@@ -356,9 +356,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
   }
 
   floatx16 acc[TM][TN];
-  constexpr bool SKEW = BM == 256 && G == 1;
-  gemm_dma_tile<BM, BN, PW, SKEW>(lds, a_rsrc, a_off, b_rsrc, b_off, b_tile_off, k_tiles, acc,
-                                 SKEW && k_tiles >= 96 ? tile_m % k_tiles : 0);
+  gemm_dma_tile<BM, BN, PW>(lds, a_rsrc, a_off, b_rsrc, b_off, b_tile_off, k_tiles, acc);
 
   const bool gated_n = EPI == 3 || EPI == 4;
 #pragma unroll

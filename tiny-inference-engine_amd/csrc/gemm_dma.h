@@ -66,19 +66,11 @@ __device__ __forceinline__ int gd_stage_chunk(int lane, int row) { return (lane 
 // PW, lane * 16 with `b_tile_off` the byte offset of block row 4 p + wave. A lane ends with, in acc[i][j], row
 // wm BM / 2 + 32 i + lane % 32 and in word 4 g + v column wn BN / 2 + 32 j + 8 g + 4 (lane / 32) + v, wm = wave / 2 and
 // wn = wave % 2.
-//
-// SKEW (groups of one slice): the tile's sums begin with slice `first` of its range and go round. Workgroups of one piece of
-// w that start a slice apart, row tile by row tile, no longer all wait for the same lines from memory: each finds in the L2
-// what the ones ahead of it have brought, and brings one slice for the others. Without, and with (one slice a row tile; two
-// or three are alike, a quarter of the range and more loses): 2048 rows over 24576 x 4096 350 and 332 us, over 4096 x 12288
-// in two ranges 169 and 164, 3000 rows over 4096 x 4096 104 and 94; ranges of 96 slices 97 to 98 % of the time, of 64 slices
-// 98 to 102 %, which therefore stay as they lie. Tiles that stage two slices, whose lines come whole, gain nothing or lose
-// (512 rows over 12288 x 2048 33.0 and 34.9).
-template <int BM, int BN, bool PW, bool SKEW = false>
+template <int BM, int BN, bool PW>
 __device__ __forceinline__ void gemm_dma_tile(bf16_t* lds, const __amdgpu_buffer_rsrc_t a_rsrc,
                                               const unsigned (&a_off)[BM * GdShape<BM, BN>::GROUP / 64], const __amdgpu_buffer_rsrc_t b_rsrc,
                                               const unsigned (&b_off)[BN / 64], const unsigned (&b_tile_off)[BN / 64],
-                                              int k_tiles, floatx16 (&acc)[BM / 64][BN / 64], int first = 0) {
+                                              int k_tiles, floatx16 (&acc)[BM / 64][BN / 64]) {
   constexpr int G = GdShape<BM, BN>::GROUP, STAGES = GdShape<BM, BN>::STAGES;
   constexpr int BK = GD_BK;
   constexpr int TN = BN / 64;                   // 32-column MFMA tiles of a wave
@@ -97,21 +89,19 @@ __device__ __forceinline__ void gemm_dma_tile(bf16_t* lds, const __amdgpu_buffer
   const int fk = lane >> 5;
 
   const int steps = (k_tiles + G - 1) / G;      // groups of G slices; a last one may lack some
-  static_assert(!SKEW || G == 1, "a range goes round in whole groups");
-  auto place = [&](int t) { return SKEW ? (t + first < k_tiles ? t + first : t + first - k_tiles) : t; };      // in memory
   auto stage = [&](int s) { return lds + s * BUF; };          // group t lies in stage t % STAGES
   auto issue_x = [&](int t, int s) {           // of a group that lacks slices: what follows in memory, unused
     bf16_t* buf = stage(s);
 #pragma unroll
     for (int p = 0; p < PA * G; ++p)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_void_t*)(buf + (p * 64 + wave * 16) * BK), 16, a_off[p],
-                                               place(t) * G * BK * 2, 0, 0);
+                                               t * G * BK * 2, 0, 0);
   };
   auto issue_w = [&](int t, int s) {
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       bf16_t* buf = stage(s) + G * BM * BK + g * BN * BK;
-      const int kt = G == 1 ? place(t) : min(t * G + g, k_tiles - 1);      // a slice that is not there: the last one again, unused
+      const int kt = G == 1 ? t : min(t * G + g, k_tiles - 1);      // a slice that is not there: the last one again, unused
 #pragma unroll
       for (int p = 0; p < PB; ++p)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, (lds_void_t*)(buf + (p * 64 + wave * 16) * BK), 16,
