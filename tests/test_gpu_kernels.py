@@ -1154,6 +1154,32 @@ def test_attention_prefill_bf16_loses_what_rounding_its_probabilities_loses(H, K
     assert mine <= 1.25 * online, f"error {mine:.3e}, {online:.3e} with the running maximum as the reference"
 
 
+@pytest.mark.parametrize("H,KVH,Dh", [(4, 1, 128), (2, 2, 64), (3, 1, 32)])
+def test_attention_prefill_bf16_sums_probabilities_in_the_order_of_the_keys(H, KVH, Dh):
+    """One tile of 64 keys, the first of probability 1 and the others of 2^-24. Half of a row's keys (0 to 7, 16 to 23 and
+    so on) are summed behind the first, one by one, and each is rounded away; the other half sum to 2^-19 exactly. Sums
+    of a part of the first half beside it would leave up to 2^-19 more."""
+    from tie_amd import kernels
+
+    n, ctx, bs, nsplit = 33, 64, 16, 2
+    case, S = attention_case(H, KVH, Dh, bs, lens_new=[n], lens_ctx=[ctx], seed=43, dtype=torch.bfloat16)
+    q, kc = torch.zeros(n, H, Dh, dtype=torch.bfloat16), torch.zeros_like(case["kc"]).cpu()
+    q[:, :, 0] = 1.0
+    kc[..., 0] = -24.0
+    kc[int(case["tables"][0, 0]), :, 0, 0] = 0.0
+    scale = float(np.float32(1 / np.log2(np.e)))                    # a score is an exponent of 2
+    assert np.float32(scale) * np.float32(np.log2(np.e)) == 1
+    out = torch.empty_like(case["q"])
+    part_o = torch.full((n, H, nsplit, Dh), float("nan"), device="cuda")
+    part_ml = torch.full((n, H, nsplit, 2), float("nan"), device="cuda")
+    items = torch.tensor(kernels.prefill_items([n], H // KVH), dtype=torch.int32).cuda()
+    kernels.attention_prefill_bf16(q.view(n, H * Dh).cuda(), kc.cuda(), case["vc"], out, case["query_start"],
+                                   case["context_lens"], case["tables"], items, H, scale, staging=2, nsplit=nsplit,
+                                   merge_rows=i32(list(range(n))), part_o=part_o, part_ml=part_ml)
+    last = part_ml[-1].cpu()                                         # the row that sees all keys; one tile: share 0 alone
+    assert torch.equal(last[:, 0], torch.tensor([0.0, 1.0 + 2.0 ** -19]).expand(H, 2)), last[0, 0].tolist()
+
+
 @pytest.mark.parametrize("where", ["first", "page_edge", "tile_edge", "tile_edge_64", "far", "last"])
 def test_attention_prefill_bf16_finds_one_far_key(where):
     spike = {"first": lambda ctx: 0, "page_edge": lambda ctx: 16 * 3 - 1, "tile_edge": lambda ctx: 32 * 7,

@@ -549,7 +549,7 @@ __device__ __forceinline__ void attend_tile_from_lds(const bf16_t* __restrict__ 
   }
   if constexpr (NEXT) __builtin_amdgcn_sched_barrier(0);
   if constexpr (NEXT) score_tile_from_lds(k_next, qf, next, k_frag);
-  // Four chains: a maximum or a sum that waits for the one before it costs a wave twice its own time.
+  // Four chains: a maximum that waits for the one before it costs a wave twice its own time.
   float part[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
@@ -565,18 +565,18 @@ __device__ __forceinline__ void attend_tile_from_lds(const bf16_t* __restrict__ 
   const float neg_mc = (m_new == -INFINITY) ? 0.f : -m_new * scale_log2e;
   const float corr = __builtin_amdgcn_exp2f(fmaf(m, scale_log2e, neg_mc));   // m = -inf: 0
   Frag pf[KB];
-  float psum[4] = {0.f, 0.f, 0.f, 0.f};
+  float psum = 0.f;          // in the order of a lane's keys
 #pragma unroll
   for (int j = 0; j < KB; ++j)
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
       const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[j / 2][(j % 2) * 8 + e], scale_log2e, neg_mc));   // masked: 0
       const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[j / 2][(j % 2) * 8 + e + 1], scale_log2e, neg_mc));
-      psum[e % 4] += p0;
-      psum[e % 4 + 1] += p1;
+      psum += p0;
+      psum += p1;
       pf[j].w[e / 2] = pack2(p0, p1);
     }
-  l = l * corr + ((psum[0] + psum[1]) + (psum[2] + psum[3]));
+  l = l * corr + psum;
   if constexpr (NEXT) {
     // a matrix instruction and a fragment, then five vector instructions: what its 32 cycles cover
     __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
