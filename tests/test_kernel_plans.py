@@ -165,8 +165,8 @@ def test_the_tiled_product_plans_for_a_last_row_tile_that_is_nearly_empty():
 
 
 def test_float32_products_of_many_rows_take_pieces():
-    """(rows, w): the shape and the ranges of K. Float32 instructions up to about 100 rows, bfloat16 pieces above (the
-    fastest of all forced ones, or within 3 %); K beyond a descriptor's reach stays on the former."""
+    """(rows, w): float32 instructions up to 32 rows over every w and to about 130 over 2048 x 2048, bfloat16 pieces above, from
+    fewer rows the larger w is; K beyond a descriptor's reach stays on the former."""
     from tie_amd import kernels
 
     for M, N, K, pieces in ((4, 2048, 2048, False), (64, 4096, 2048, False), (48, 2048, 6144, False), (200, 4096, 2048, True),
@@ -176,6 +176,25 @@ def test_float32_products_of_many_rows_take_pieces():
         assert (kernels.gemm_f32_shape(M, N, K, splits) > 8) == pieces, (M, N, K)
         assert splits in (1, 2, 4, 8)
     assert kernels.gemm_f32_shape(301, 12288, 2048) == 10 and kernels.gemm_f32_shape(48, 12288, 2048) <= 8
+
+
+def test_float32_products_run_on_what_was_fastest():
+    """Up to 32 rows no weight takes pieces, in however many ranges of K. (rows, w): the choices within a tenth of the fastest
+    one that was timed."""
+    from tie_amd import kernels
+
+    weights = ((512, 3072), (1024, 1024), (2048, 2048), (4096, 2048), (2048, 6144), (2560, 9728), (6144, 4096), (12288, 2048),
+               (12288, 4096), (24576, 4096), (32000, 2048), (32000, 6144), (151936, 2048))
+    for M in (1, 2, 3, 4, 5, 8, 16, 17, 24, 32):
+        for N, K in weights:
+            for splits in (kernels.gemm_f32_splits(M, N, K), 1, 2, 8):
+                assert kernels.gemm_f32_shape(M, N, K, splits) <= 8, (M, N, K, splits)
+    for M, N, K, good in ((5, 2048, 2048, {(2, 8), (1, 4), (1, 2)}), (16, 2048, 2048, {(2, 8), (1, 4), (1, 2), (2, 4)}),
+                          (16, 151936, 2048, {(2, 1), (2, 2)}), (8, 151936, 2048, {(1, 1), (2, 1), (2, 2)}),
+                          (24, 12288, 4096, {(6, 4), (4, 2), (4, 4), (6, 8), (6, 1)}), (128, 4096, 2048, {(8, 2)}),
+                          (64, 6144, 4096, {(12, 4), (9, 8), (10, 8)}), (200, 4096, 2048, {(9, 4), (10, 4), (12, 2)})):
+        splits = kernels.gemm_f32_splits(M, N, K)
+        assert (kernels.gemm_f32_shape(M, N, K, splits), splits) in good, (M, N, K, kernels.gemm_f32_shape(M, N, K, splits), splits)
 
 
 def test_experts_take_wide_row_tiles_where_these_still_fill_the_gpu():
