@@ -197,6 +197,17 @@ def test_float32_products_run_on_what_was_fastest():
         assert (kernels.gemm_f32_shape(M, N, K, splits), splits) in good, (M, N, K, kernels.gemm_f32_shape(M, N, K, splits), splits)
 
 
+def test_float32_products_of_one_and_two_rows_run_on_multiply_adds():
+    """Over w of 1024 rows and more; three and four rows were no faster there over any w but one of nineteen, and up to a
+    sixth slower."""
+    from tie_amd import kernels
+
+    for N, K in ((2048, 2048), (4096, 4096), (12288, 2048), (19456, 2560), (12288, 4096), (151936, 2048), (5120, 640)):
+        for M in (1, 2, 3, 4, 5):
+            assert (kernels.gemm_f32_shape(M, N, K, 1) < 0) == (M <= 2), (M, N, K)
+    assert kernels.gemm_f32_shape(1, 512, 3072, 1) > 0
+
+
 def test_experts_take_wide_row_tiles_where_these_still_fill_the_gpu():
     """(experts, inner size): rows of a tile at 40, 100, 200, 400 and 600 rows an expert. Many or wide experts take 256
     from 192 on, smaller sets from 480 (16 experts of 512 at 384 rows: 41 us in tiles of 128, 56 in tiles of 256)."""

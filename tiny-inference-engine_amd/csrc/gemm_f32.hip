@@ -1,9 +1,9 @@
 // The float32 matrix product for gfx950: out[M, N] (+)= x[M, K] . w[N, K]^T on v_mfma_f32_16x16x4_f32, whose
 // products and sums are float32 (the same precision as multiply-adds on the vector units, at four times the rate a
 // plain tile reached there). It carries the projections of the 32-bit path over few rows, gemm_f32_pieces those over many,
-// gemm_f32_rows those of one to four (gemm_f32_plan.h chooses); operands of mixed types and rows that are no multiple of four floats go to gemm_generic,
-// routed experts to moe_gemm_generic. Shape and ranges follow from the
-// step's sizes: a row's sums in steps of other sizes agree to rounding, not bit for bit as the plain tile's do.
+// gemm_f32_rows those of one and two (gemm_f32_plan.h chooses); operands of mixed types and rows that are no multiple of
+// four floats go to gemm_generic, routed experts to moe_gemm_generic. Shape and ranges follow from the step's sizes: a
+// row's sums in steps of other sizes agree to rounding, not bit for bit as the plain tile's do.
 //
 // A wave owns MT tiles of 16 rows of x and NT tiles of 16 rows of w over one range of K and walks it in blocks of 32 k,
 // 2 KB of a tile: two 16-byte loads a lane, eight lanes on the 128 bytes of a row, one whole line. The matrix instruction
