@@ -208,6 +208,22 @@ def test_float32_products_of_one_and_two_rows_run_on_multiply_adds():
     assert kernels.gemm_f32_shape(1, 512, 3072, 1) > 0
 
 
+def test_float32_products_on_pieces_sum_in_enough_chains():
+    """A product on pieces (shapes 9 to 12: one or two groups of waves along K, times the ranges of K) in fewer than two chains
+    is further off than the float32 instructions', which have four at least (2.3e-7 and 1.7e-7 of a sum of 2048 numbers of
+    one sign)."""
+    from tie_amd import kernels
+
+    seen = 0
+    for N, K in ((512, 3072), (2048, 2048), (4096, 2048), (2048, 6144), (12288, 2048), (24576, 4096), (2560, 9728), (4096, 1000)):
+        for M in (33, 64, 100, 128, 200, 256, 301, 512, 700, 1000, 2000):
+            for splits in (kernels.gemm_f32_splits(M, N, K), 1, 2):
+                shape = kernels.gemm_f32_shape(M, N, K, splits)
+                seen += shape > 8
+                assert shape <= 8 or (1, 2, 1, 2)[shape - 9] * splits >= 2, (M, N, K, splits, shape)
+    assert seen > 100
+
+
 def test_experts_take_wide_row_tiles_where_these_still_fill_the_gpu():
     """(experts, inner size): rows of a tile at 40, 100, 200, 400 and 600 rows an expert. Many or wide experts take 256
     from 192 on, smaller sets from 480 (16 experts of 512 at 384 rows: 41 us in tiles of 128, 56 in tiles of 256)."""

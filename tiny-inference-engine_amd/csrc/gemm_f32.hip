@@ -207,7 +207,9 @@ extern "C" int tie_gemm_f32_splits(int M, int N, int K) { return M > 0 && N > 0 
 // The shape a product with so many ranges of K takes: 1 to 8 for tie_gemm_f32, 8 + 1 to 8 + 4 for tie_gemm_f32_pieces,
 // -1 to -3 for tie_gemm_f32_rows.
 extern "C" int tie_gemm_f32_shape(int M, int N, int K, int splits) {
-  return M > 0 && N > 0 && K > 0 && splits > 0 ? gf_plan(M, N, K, splits).shape + 1 : 1;
+  if (M <= 0 || N <= 0 || K <= 0 || splits <= 0) return 1;
+  const GfPlan plan = gf_plan(M, N, K, 0);
+  return (plan.splits == splits ? plan : gf_plan(M, N, K, splits)).shape + 1;
 }
 
 // splits > 1: out is [splits][M][N] planes of partial sums. gated 1 or 2: w's rows are 8 gates and 8 ups in turn, out is
