@@ -164,6 +164,43 @@ def test_the_tiled_product_plans_for_a_last_row_tile_that_is_nearly_empty():
     assert kernels.gemm_tile(576, 19456, 2560, True, 1) == 4
 
 
+def test_single_rows_beside_portions_share_their_keys_by_their_own_launch(monkeypatch):
+    """32 sequences of 8 KV heads, a wave to a whole sequence where they run alone. In one launch with a portion (heads of 128)
+    they are cut in two, unless a window leaves them less than two shares of 128 keys; heads of 256 have a launch of their own,
+    and its plan, in the same step."""
+    import torch
+
+    from tie_amd import kernels
+
+    shares = []
+    monkeypatch.setattr(kernels, "attention_mixed_bf16", lambda *a, **k: shares.append(("mixed", k["single_nsplit"])))
+    monkeypatch.setattr(kernels, "attention_decode_bf16", lambda *a, **k: shares.append(("decode", a[11])))
+    monkeypatch.setattr(kernels, "attention_prefill_bf16", lambda *a, **k: None)
+    S, KVH, bs = 32, 8, 16
+
+    class Step:
+        block_tables = torch.zeros(S + 1, 256, dtype=torch.int32)
+
+    def scratch(name, shape, dtype):
+        return torch.empty(0)
+
+    for order in ((128, 256), (256, 128)):
+        class Batch:
+            all_decode, num_seqs, plan_context, memo = False, S + 1, 4096, {}
+            host_new_tokens, host_context_lens = [64] + [1] * S, [64] + [4000] * S
+            query_start = context_lens = seq_of_row = None
+
+        shares.clear()
+        for Dh in order:
+            for window in (None, 128):
+                H = KVH * 2
+                q = torch.empty(S + 64, H * Dh, dtype=torch.bfloat16)
+                cache = torch.empty(1, KVH, bs, Dh, dtype=torch.bfloat16)
+                kernels.paged_attention(q, cache, cache.transpose(2, 3), torch.empty_like(q), Step, Batch, H, Dh ** -0.5, window, scratch)
+        want = {128: [("mixed", 2), ("mixed", 1)], 256: [("decode", 1), ("decode", 1)]}
+        assert shares == want[order[0]] + want[order[1]], (order, shares)
+
+
 def test_float32_products_of_many_rows_take_pieces():
     """(rows, w): float32 instructions up to 32 rows over every w and to about 130 over 2048 x 2048, bfloat16 pieces above, from
     fewer rows the larger w is; K beyond a descriptor's reach stays on the former."""

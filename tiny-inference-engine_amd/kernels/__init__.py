@@ -1888,13 +1888,14 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         # Both kinds of rows in one launch, where its kernel takes them.
         together = bool(num_single) and items is not None and not keep_first and attention_mixed_takes(Dh, bs)
         if num_single:
-            shares_key = ("single_row_shares", KVH, reach)
+            shares_key = ("single_row_shares", KVH, reach, together)
             planned = batch.memo.get(shares_key)
             if planned is None:                # this step runs eagerly: the shares' length goes to the device by itself
                 lens = [c for c, n in zip(batch.host_context_lens, batch.host_new_tokens) if n == 1]
                 nsplit, length = decode_share_plan(lens, KVH, batch.plan_context, bs, reach)
                 if together and not length:
-                    nsplit = max(nsplit, min(-(-MIXED_WAVES // (num_single * KVH)), batch.plan_context // 128, MAX_KEY_SPLITS))
+                    keys = min(batch.plan_context, reach or batch.plan_context)
+                    nsplit = max(nsplit, min(-(-MIXED_WAVES // (num_single * KVH)), keys // 128, MAX_KEY_SPLITS))
                 planned = batch.memo[shares_key] = (
                     nsplit, torch.tensor([length], dtype=torch.int32).to(q.device) if length else None)
             nsplit, share_tiles = planned
