@@ -164,6 +164,20 @@ def test_the_tiled_product_plans_for_a_last_row_tile_that_is_nearly_empty():
     assert kernels.gemm_tile(576, 19456, 2560, True, 1) == 4
 
 
+def test_the_common_launch_takes_what_its_library_says(monkeypatch):
+    """Heads of 32, 64 and 128 over pages of 16, 32, ... positions; what the kernel's library answers is the rule."""
+    from tie_amd import kernels
+
+    for Dh in (16, 32, 48, 64, 96, 128, 256, 20):
+        for bs in (4, 8, 12, 16, 32, 48, 64):
+            assert kernels.attention_mixed_takes(Dh, bs) == (Dh in (32, 64, 128) and bs in (16, 32, 64)), (Dh, bs)
+    asked = []
+    monkeypatch.setattr(kernels, "_lib", lambda key, Dh=0: type("L", (), {"tie_attention_mixed_takes": staticmethod(lambda bs: asked.append((Dh, bs)) or 0)}))
+    kernels.attention_mixed_takes.cache_clear()
+    assert not kernels.attention_mixed_takes(128, 16) and asked == [(128, 16)]
+    kernels.attention_mixed_takes.cache_clear()
+
+
 def test_single_rows_beside_portions_share_their_keys_by_their_own_launch(monkeypatch):
     """32 sequences of 8 KV heads, a wave to a whole sequence where they run alone. In one launch with a portion (heads of 128)
     they are cut in two, unless a window leaves them less than two shares of 128 keys; heads of 256 have a launch of their own,

@@ -1749,9 +1749,10 @@ def attention_prefill_bf16(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
         _ptr(_sinks(sinks, num_heads, window, chunk)), int(keep_first or 0), _stream())
 
 
+@functools.lru_cache(maxsize=64)
 def attention_mixed_takes(head_dim: int, block_size: int) -> bool:
     """Whether portions and single rows of a step over pages of this size run as one launch (``attention_mixed_bf16``)."""
-    return head_dim in (32, 64, 128) and prefill_loads_straight(head_dim, block_size)
+    return head_dim in MFMA_HEAD_DIMS and bool(_lib("attention_prefill_bf16", head_dim).tie_attention_mixed_takes(block_size))
 
 
 def attention_mixed_bf16(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, out: torch.Tensor,
