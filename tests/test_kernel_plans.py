@@ -241,7 +241,8 @@ def test_float32_products_run_on_what_was_fastest():
             for splits in (kernels.gemm_f32_splits(M, N, K), 1, 2, 8):
                 assert kernels.gemm_f32_shape(M, N, K, splits) <= 8, (M, N, K, splits)
     for M, N, K, good in ((5, 2048, 2048, {(2, 8), (1, 4), (1, 2)}), (16, 2048, 2048, {(2, 8), (1, 4), (1, 2), (2, 4)}),
-                          (16, 151936, 2048, {(2, 1), (2, 2)}), (8, 151936, 2048, {(1, 1), (2, 1), (2, 2)}),
+                          (16, 151936, 2048, {(2, 1), (2, 2)}), (8, 151936, 2048, {(1, 1), (2, 2)}),
+                          (3, 151936, 2048, {(1, 1)}), (4, 151936, 2048, {(1, 1), (2, 2)}), (5, 32000, 2048, {(1, 1), (2, 2)}),
                           (24, 12288, 4096, {(6, 4), (4, 2), (4, 4), (6, 8), (6, 1)}), (128, 4096, 2048, {(8, 2)}),
                           (64, 6144, 4096, {(12, 4), (9, 8), (10, 8)}), (200, 4096, 2048, {(9, 4), (10, 4), (12, 2)})):
         splits = kernels.gemm_f32_splits(M, N, K)
