@@ -749,9 +749,9 @@ __device__ __forceinline__ void attention_prefill_dma_group(
     // While a tile's softmax runs, the matrix cores make the scores of the tile behind it: its keys have landed already,
     // and those of the tile behind that go where this one's keys lay. Values stay one tile ahead. One after the other, a
     // wave's matrix instructions (1024 cycles a tile) and its vector ones (about 900) add up, and two waves a SIMD made up
-    // for it only in part. Without and with, heads of 128: 2048 rows of 32 heads over 8 62.0 and 57.7 us, behind 8192
-    // earlier positions 350 and 317, 4096 rows 226 and 194; 512 rows of 16 heads behind 15872, with the merge, 93.6 and
-    // 87.1. The scores of the last tile's successor are made of whatever lies there and dropped. What bounds it now: every
+    // for it only in part. Without and with, heads of 128: 2048 rows of 32 heads over 8 59 and 56 us, behind 8192
+    // earlier positions 331 and 319, 4096 rows 214 and 195; 512 rows of 16 heads behind 15872, with the merge, 91 and
+    // 90. The scores of the last tile's successor are made of whatever lies there and dropped. What bounds it now: every
     // wave reads all of a tile from LDS, 2048 cycles for eight waves, as many as their matrix instructions take.
     if (!empty && wave_active && tile_begin * KD <= wave_last) score_tile_from_lds(lds, qf, scores[0], k_frag);
     meet();

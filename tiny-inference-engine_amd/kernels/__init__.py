@@ -740,9 +740,11 @@ def gemm_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bo
     """out (+)= x @ w.T for float32 operands; K % 4 == 0 (``gemm_f32_takes``).
 
     ``splits`` > 1: out is ``[splits, M, N]`` and receives one plane of partial sums per range of K. ``shape`` picks a
-    workgroup shape of csrc/gemm_f32.hip (1 to 8, on float32 instructions) or csrc/gemm_f32_pieces.hip (9 to 12, on
-    bfloat16 pieces whose sum is the number) or csrc/gemm_f32_rows.hip (-1 to -3: up to 4 rows, one plane); 0 lets the plan choose. ``gated`` 1 + an activation's number: w is a
-    gate/up pair interleaved by ``interleave_gate_up`` and out ``[M, N / 2]`` receives act(gate) * up."""
+    workgroup shape of csrc/gemm_f32.hip (1 to 8, on float32 instructions), of csrc/gemm_f32_pieces.hip (9 to 12, on
+    three bfloat16 pieces of every number, whose sum is the number whatever its size; of the nine products of pieces the
+    three smallest, below 2^-24 of the whole together, are left out) or of csrc/gemm_f32_rows.hip (-1 to -3: up to 4 rows,
+    one plane); 0 lets the plan choose. ``gated`` 1 + an activation's number: w is a gate/up pair interleaved by
+    ``interleave_gate_up`` and out ``[M, N / 2]`` receives act(gate) * up."""
     _gpu(x, "matmul input")
     _gpu(w, "matmul weight")
     _gpu(out, "matmul output")
@@ -1402,9 +1404,13 @@ def sample_rows_filtered(logits: torch.Tensor, inv_temperature: torch.Tensor, un
           top_k.data_ptr(), top_p.data_ptr(), _ptr(rows), count, out.data_ptr(), R, V, _stream())
 
 
-# Up to this many workgroups of single decoded rows run in the prefill attention kernel beside a step's prompt
-# portions rather than in a launch (and a merge) of the decode kernel of their own; a row costs a 32-row tile
-# there, so many of them are better off in the decode kernel, which takes a group's heads as its columns.
+# Up to this many workgroups of single decoded rows run as items of the prefill attention kernel beside a step's prompt
+# portions rather than as waves of the decode kernel. A row costs a 32-row tile there, where the decode kernel takes a
+# group's heads as its columns, but no launch and no merge of its own. The number was found where the decode kernel's waves
+# need both, as they still do for heads and pages that attention_mixed_bf16 does not take. Where it does, waves of their own
+# would cost neither: 1 to 15 rows beside portions of 64 to 1000, 8 KV heads of 128, a whole step of 28 layers of 16 heads as
+# items 2606 to 5285 us and as waves 2.4 % more to 4.9 % less, of 36 layers of 32 heads 1.2 % more to 12 % less (8 rows of
+# 4000 keys beside 500: 11672 and 10251 us; 15 of 200 beside 1000: 16509 and 16715). The line stands where it was.
 SINGLE_ROWS_RIDE_ALONG = 128
 # Waves of single rows beside portions in one launch: theirs hold two tiles of keys, so a wave to a whole sequence, which the
 # rule for steps of single rows alone takes at 256 (sequence, KV head) pairs, keeps too little on its way (32 sequences of
