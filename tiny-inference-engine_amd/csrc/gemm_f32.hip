@@ -1,7 +1,7 @@
 // The float32 matrix product for gfx950: out[M, N] (+)= x[M, K] . w[N, K]^T on v_mfma_f32_16x16x4_f32, whose
 // products and sums are float32 (the same precision as multiply-adds on the vector units, at four times the rate a
 // plain tile reached there). It carries the projections of the 32-bit path over few rows, gemm_f32_pieces those over many,
-// gemm_f32_rows those of one and two (gemm_f32_plan.h chooses); operands of mixed types and rows that are no multiple of
+// gemm_f32_rows those of one to four (gemm_f32_plan.h chooses); operands of mixed types and rows that are no multiple of
 // four floats go to gemm_generic, routed experts to moe_gemm_generic. Shape and ranges follow from the step's sizes: a
 // row's sums in steps of other sizes agree to rounding, not bit for bit as the plain tile's do.
 //

@@ -1,5 +1,4 @@
-// The float32 product for one and two rows (up to four if asked for), gfx950: out[M, N] (+)= x[M, K] . w[N, K]^T on ordinary
-// multiply-adds. So few rows are bound by the stream of w, 4 bytes a weight, and here nothing stands in its way: a load is
+// The float32 product for one to four rows, gfx950: out[M, N] (+)= x[M, K] . w[N, K]^T on ordinary multiply-adds. So few rows are bound by the stream of w, 4 bytes a weight, and here nothing stands in its way: a load is
 // 1 KB of one row of w, w goes from memory to the registers that multiply it, without LDS, and x is read for the rows there
 // are, where the matrix instructions (gemm_f32.hip) take 16.
 //
@@ -11,8 +10,8 @@
 // half to two thirds of what the matrix instructions' longer chains are.
 //
 // Measured, one row and four, with the best of the float32 matrix instructions beside it: a gated 12288 x 2048 18.6 us and
-// 19.1 (20.3 and 18.9), 151936 x 2048 175 (7.1 TB/s) and 186 (183 and 180), 4096 x 4096 13.5 and 13.9 (13.7 and 12.9), so
-// three and four rows are left to those. Three and four chunks a batch gained nothing over a wave's 2 to 10
+// 19.1 (20.3 and 18.9), 151936 x 2048 175 (7.1 TB/s) and 186 (183 and 180), 4096 x 4096 13.5 and 13.9 (13.7 and 12.9).
+// Three and four chunks a batch gained nothing over a wave's 2 to 10
 // (registers, and waves, against it); at eight rows x outweighs w (23.5 us, 19.7). Built and slower: the RMS norms' work in
 // this kernel's ends, as the bfloat16 decode product does it (four rows, a step of 28 layers: 2189 -> 2317 us, though
 // 55 norm kernels of 3.3 us go: the stream read behind the sums and the sums of squares ahead of them cost more).
