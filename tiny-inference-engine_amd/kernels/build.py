@@ -32,7 +32,8 @@ CSRC = pathlib.Path(__file__).resolve().parent.parent / "csrc"
 ARCH = "gfx950"
 # Packed float32 instructions are switched off for all device code.
 FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC", "-shared",
-         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"]
+         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument",
+         "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
 # Flags of single sources. The attention kernels rescale their output accumulators with ordinary
 # multiplications between matrix instructions: these then work on vector registers directly. The float32 product's
