@@ -691,6 +691,54 @@ def test_attention_decode_that_prepares_its_own_queries(H, KVH, Dh, bs, planes, 
     assert torch.equal(kc3, kc1) and torch.equal(vc3, vc1)
 
 
+@pytest.mark.parametrize("nsplit,share_tiles,planes,bs,window,write_kv",
+                         [(1, 0, 1, 16, None, True), (1, 0, 8, 16, 300, True), (2, 0, 3, 16, None, True), (3, 0, 5, 32, None, True),
+                          (4, 0, 8, 16, 300, True), (8, 40, 2, 16, None, True), (70, 0, 4, 16, None, True),
+                          (5, 0, 4, 16, None, False), (1, 0, 2, 32, None, False)])
+def test_attention_decode_with_the_newest_token_as_a_share_of_its_own(nsplit, share_tiles, planes, bs, window, write_kv):
+    """A prepared step cut into shares gives the newest token one of its own; alone (one share) a wave takes it behind its
+    tiles. Any number of planes, page tables longer than the 256 entries a wave keeps of them (8300 and 4200 keys in pages
+    of 16), shares without keys, and a cache that holds the token already, against the q/k kernel and the decode
+    attention that looks its pages up per lane."""
+    from tie_amd import kernels
+
+    H, KVH, Dh = 8, 2, 128
+    lens = [1, 33, 4096, 4200, 8300]
+    case, S = attention_case(H, KVH, Dh, bs, lens_new=[1] * len(lens), lens_ctx=lens, seed=47, dtype=torch.bfloat16,
+                             window=window)
+    width = (H + 2 * KVH) * Dh
+    qkv = (rnd(planes, S, width, seed=48) / planes).cuda()
+    weight = (1 + 0.1 * rnd(Dh, seed=49)).cuda()
+    inv_freq = torch.from_numpy(plain.rope_inv_freq(1e4, Dh)).float().cuda()
+    positions = i32([c - 1 for c in lens])
+    tables = case["tables"]
+    slots = i32([int(tables[s, (c - 1) // bs]) * bs + (c - 1) % bs for s, c in enumerate(lens)])
+    angles = torch.empty(S, Dh, device="cuda")
+    kernels.rope_angles(positions, inv_freq, angles)
+
+    class Batch:
+        all_decode, num_seqs, plan_context = True, S, max(lens)
+        query_start, context_lens = case["query_start"], case["context_lens"]
+
+    class Step:
+        block_tables = tables
+        key_shares = (nsplit, i32([share_tiles]) if share_tiles else None)
+
+    kc1, vc1 = case["kc"].clone(), case["vc"].clone()
+    q = torch.empty(S, H * Dh, dtype=torch.bfloat16, device="cuda")
+    kernels.qk_norm_rope_kv_write(qkv[0], q, weight, weight, 1e-5, inv_freq, positions, slots, kc1, vc1, H, KVH, Dh, bs,
+                                  planes=planes, plane_stride=S * width, angles=angles)
+    apart = torch.full_like(q, float("nan"))
+    kernels.attention_decode_bf16(q, kc1, vc1, apart, case["query_start"], case["context_lens"], tables, S, H, Dh ** -0.5,
+                                  window, 1, depth=1)
+    kc2, vc2 = (case["kc"].clone(), case["vc"].clone()) if write_kv else (kc1.clone(), vc1.clone())
+    fused = torch.full_like(q, float("nan"))
+    kernels.paged_attention_prepared(qkv, weight, weight, 1e-5, angles, write_kv, kc2, vc2, fused, Step, Batch, H, Dh ** -0.5,
+                                     window, lambda name, shape, dtype: torch.full(shape, float("nan"), dtype=dtype, device="cuda"))
+    assert torch.equal(kc2, kc1) and torch.equal(vc2, vc1), "the newest keys or values differ"
+    close(fused, apart, 1e-2, f"{nsplit} shares, {planes} planes")     # probabilities in bfloat16, summed in other orders
+
+
 @pytest.mark.parametrize("H,KVH,Dh,bs", [(6, 2, 32, 16), (5, 5, 80, 16), (8, 2, 128, 16), (2, 1, 256, 32), (4, 4, 112, 64)])
 @pytest.mark.parametrize("nsplit,window", [(1, None), (2, None), (5, None), (1, 100), (3, 77)])
 def test_attention_decode_bf16_with_tiles_in_flight(H, KVH, Dh, bs, nsplit, window):

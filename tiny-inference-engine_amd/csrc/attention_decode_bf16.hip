@@ -190,19 +190,39 @@ __global__ __launch_bounds__(TIE_WAVE) void attention_decode_kernel(
               sinks);
 }
 
-// One wave a workgroup; shares are the fastest part of its number.
-template <int DEPTH, bool PREPARE, bool CAPPED, bool KEEPS = false>
+// One wave a workgroup; shares are the fastest part of its number. Newest tokens that are shares of their own come
+// behind all others (places from num_seqs on), as they are short: between the others they would shift which compute
+// units carry one wave more (8 sequences of 8 KV heads and 4090 keys, 512 long waves and 64 short ones: 4 % of a step).
+template <int DEPTH, DecodePrepare PREPARE, bool CAPPED, bool KEEPS = false>
 __global__ __launch_bounds__(TIE_WAVE) void attention_decode_ring_kernel(
-    const bf16_t* __restrict__ q, bf16_t* k_cache, bf16_t* v_cache,
-    bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
     const int* __restrict__ query_start, const int* __restrict__ context_lens,
-    const int* __restrict__ block_tables, const int* __restrict__ seq_ids, int H, int KVH, int block_size,
-    int block_shift, int max_blocks, float scale_log2e, float cap, int window, int nsplit,
-    const float* __restrict__ sinks, const int* __restrict__ share_tiles,
-    QkSource src, int keep) {
+    const int* __restrict__ block_tables, const int* __restrict__ seq_ids, int max_blocks, int num_seqs, int window, int nsplit,
+    int H, int KVH,
+    const bf16_t* __restrict__ q, bf16_t* k_cache, bf16_t* v_cache,
+    bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, int block_size,
+    int block_shift, float scale_log2e, float cap,
+    const float* __restrict__ sinks, const int* __restrict__ share_tiles, QkSource src, int keep) {
+  constexpr bool PREPARES = PREPARE != PREPARE_NOTHING;
+  __shared__ int table_lds[TABLE_AHEAD];
+  __shared__ __attribute__((aligned(16))) bf16_t q_lds[PREPARES ? 16 * DH : 8], newest_lds[PREPARES ? 2 * DH : 8];
+  const int lane = threadIdx.x;
+  if constexpr (PREPARE == PREPARE_SHARES) {
+    if (static_cast<int>(blockIdx.z) >= num_seqs) {
+      const int units = gridDim.y;
+      const int at = ((static_cast<int>(blockIdx.z) - num_seqs) * units + static_cast<int>(blockIdx.y)) *
+                         static_cast<int>(gridDim.x) + static_cast<int>(blockIdx.x);
+      if (at < units * num_seqs)
+        attention_decode_newest<CAPPED>(lane, at % units, at / units, k_cache, v_cache, part_o, part_ml, query_start,
+                                        context_lens, block_tables, seq_ids, H, KVH, block_size, block_shift, max_blocks,
+                                        scale_log2e, cap, nsplit, src, q_lds, newest_lds);
+      return;
+    }
+  }
   attention_decode_ring_wave<DEPTH, PREPARE, CAPPED, KEEPS>(
-      static_cast<int>(threadIdx.x), static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x),
-      static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z), q, k_cache, v_cache, out, part_o, part_ml, query_start, context_lens, block_tables, seq_ids, H, KVH, block_size, block_shift, max_blocks, scale_log2e, cap, window, nsplit, sinks, share_tiles, src, keep);
+      lane, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), static_cast<int>(blockIdx.y),
+      static_cast<int>(blockIdx.z), q, k_cache, v_cache, out, part_o, part_ml, query_start, context_lens, block_tables, seq_ids,
+      H, KVH, block_size, block_shift, max_blocks, scale_log2e, cap, window, nsplit, sinks, share_tiles, src, keep, table_lds,
+      q_lds, newest_lds);
 }
 
 #include "attention_merge.h"
@@ -220,7 +240,7 @@ static int launch_decode(const bf16_t* q, const QkSource* src, bf16_t* k_cache, 
   // kept first positions go beside a window, with uncapped scores and queries that come ready
   if (keep < 0 || (keep > 0 && (window <= 0 || softcap > 0.f || src != nullptr))) return TIE_BAD_ARGUMENT;
   const int column_groups = KVH > 0 ? (H / KVH + 15) / 16 : 1;    // waves of up to 16 query heads a KV head
-  if (num_seqs <= 0 || num_seqs > 65535 || H <= 0 || KVH <= 0 || KVH * column_groups > 65535 || H % KVH != 0 ||
+  if (num_seqs <= 0 || num_seqs > 65535 || (src != nullptr && num_seqs > 32767) || H <= 0 || KVH <= 0 || KVH * column_groups > 65535 || H % KVH != 0 ||
       (src != nullptr && H / KVH > 16) ||
       block_size < 4 || (block_size & (block_size - 1)) != 0 || max_blocks <= 0 || nsplit <= 0 ||
       nsplit > MERGE_MAX_SPLITS || depth < 0 || depth > 4 || (depth > 1 && block_size < 16) ||
@@ -233,28 +253,33 @@ static int launch_decode(const bf16_t* q, const QkSource* src, bf16_t* k_cache, 
   if (src != nullptr && (depth < 2 || !PREPARE_HEAD_DIM)) return TIE_BAD_ARGUMENT;
   if (share_tiles != nullptr && (depth < 2 || nsplit == 1)) return TIE_BAD_ARGUMENT;   // the ring kernel's, with a merge
   const dim3 grid(nsplit, KVH * column_groups, num_seqs);
+  // A prepared step whose newest tokens are shares of their own: the grid holds the other shares, then those.
+  const bool newest_alone = src != nullptr && src->write_kv && nsplit > 1;
+  const int tile_shares = newest_alone ? nsplit - 1 : nsplit;      // the ring kernel's `shares`
+  const dim3 prepared_grid(tile_shares, KVH * column_groups, num_seqs + (newest_alone ? (num_seqs + tile_shares - 1) / tile_shares : 0));
   const int block_shift = __builtin_ctz(block_size);
   const float scale_log2e = scale * 1.44269504088896340736f;
   const float cap = softcap > 0.f ? softcap / scale : 0.f;   // softcap * tanh(scale s / softcap) = scale * cap tanh(s / cap)
+#define RING_ARGS query_start, context_lens, block_tables, seq_ids, max_blocks, num_seqs, window, nsplit, H, KVH, q, k_cache, \
+                  v_cache, out, part_o, part_ml, block_size, block_shift, scale_log2e, cap, sinks, share_tiles
+  // Capped scores are an instantiation of their own: the uncapped kernels carry none of it.
+#define LAUNCH_RING(DEPTH)                                                                                               \
+  {                                                                                                                      \
+    if (keep > 0) {                                                                                                      \
+      attention_decode_ring_kernel<DEPTH, PREPARE_NOTHING, false, true><<<grid, TIE_WAVE, 0, stream>>>(RING_ARGS, QkSource{}, keep); \
+    } else if (src == nullptr && cap > 0.f) {                                                                            \
+      attention_decode_ring_kernel<DEPTH, PREPARE_NOTHING, true><<<grid, TIE_WAVE, 0, stream>>>(RING_ARGS, QkSource{}, 0); \
+    } else if (src == nullptr) {                                                                                         \
+      attention_decode_ring_kernel<DEPTH, PREPARE_NOTHING, false><<<grid, TIE_WAVE, 0, stream>>>(RING_ARGS, QkSource{}, 0); \
+    } else if constexpr (PREPARE_HEAD_DIM) {                                                                             \
+      if (nsplit > 1)                                                                                                    \
+        attention_decode_ring_kernel<DEPTH, PREPARE_SHARES, false><<<prepared_grid, TIE_WAVE, 0, stream>>>(RING_ARGS, *src, 0); \
+      else                                                                                                               \
+        attention_decode_ring_kernel<DEPTH, PREPARE_WHOLE, false><<<grid, TIE_WAVE, 0, stream>>>(RING_ARGS, *src, 0);    \
+    }                                                                                                                    \
+  }
 #define ARGS out, part_o, part_ml, query_start, context_lens, block_tables, seq_ids, H, KVH, block_size, block_shift, \
              max_blocks, scale_log2e, cap, window, nsplit, sinks
-  // Capped scores are an instantiation of their own: the uncapped kernels carry none of it.
-#define LAUNCH_RING(DEPTH)                                                                                   \
-  {                                                                                                          \
-    if (keep > 0) {                                                                                          \
-      attention_decode_ring_kernel<DEPTH, false, false, true><<<grid, TIE_WAVE, 0, stream>>>(                \
-          q, k_cache, v_cache, ARGS, share_tiles, QkSource{}, keep);                                         \
-    } else if (src == nullptr && cap > 0.f) {                                                                \
-      attention_decode_ring_kernel<DEPTH, false, true><<<grid, TIE_WAVE, 0, stream>>>(                       \
-          q, k_cache, v_cache, ARGS, share_tiles, QkSource{}, 0);                                            \
-    } else if (src == nullptr) {                                                                             \
-      attention_decode_ring_kernel<DEPTH, false, false><<<grid, TIE_WAVE, 0, stream>>>(                      \
-          q, k_cache, v_cache, ARGS, share_tiles, QkSource{}, 0);                                            \
-    } else if constexpr (PREPARE_HEAD_DIM) {                                                                 \
-      attention_decode_ring_kernel<DEPTH, true, false><<<grid, TIE_WAVE, 0, stream>>>(q, k_cache, v_cache,   \
-                                                                                      ARGS, share_tiles, *src, 0); \
-    }                                                                                                        \
-  }
 #define LAUNCH_PLAIN(WIDE)                                                                                   \
   {                                                                                                          \
     if (keep > 0)                                                                                            \
@@ -270,6 +295,7 @@ static int launch_decode(const bf16_t* q, const QkSource* src, bf16_t* k_cache, 
   else LAUNCH_PLAIN(false)
 #undef LAUNCH_PLAIN
 #undef LAUNCH_RING
+#undef RING_ARGS
 #undef ARGS
   int status = tie_launch_status();
   if (status != TIE_OK || nsplit == 1) return status;
@@ -315,7 +341,8 @@ extern "C" int tie_attention_decode_bf16_with(const void* q, const void* k_cache
 // projection's output: qkv is float32 [planes][rows][in_row] (plane p at qkv + p * plane_stride; a row holds H
 // query heads, KVH key heads, KVH value heads), summed over the planes by the kernel; q_weight / k_weight (or
 // null) the per-head RMS norm weights with eps; angles [rows][head_dim] the step's table of cos and sin.
-// write_kv = 0 where the cache is another layer's and holds the token already. Pages of 16 positions or more
+// write_kv = 0 where the cache is another layer's and holds the token already. Where it is written and nsplit > 1, the
+// newest token is a share of its own, the last: the cached keys are cut into nsplit - 1. Pages of 16 positions or more
 // and head sizes 32, 64, 128, 256; refused otherwise (tie_attention_decode_prepares tells).
 extern "C" int tie_attention_decode_prepares(int block_size) { return PREPARE_HEAD_DIM && block_size >= 16 ? 1 : 0; }
 

@@ -13,7 +13,11 @@
 //   rows given (prefill: results kept per row of the step)      slot rows[y], output row rows[y];
 //   otherwise  (decode: results kept per sequence of the launch) slot y, output row
 //                                                                query_start[seq_ids ? seq_ids[y] : y].
-__global__ void attention_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+// The first AHEAD splits' accumulators are asked for together with the maxima and sums, so that one trip to memory
+// brings all (33 splits of 32 heads: 2.9 -> 1.8 us from the first instruction to the last; the accumulators behind
+// the weights, eight at a time, were two trips more). A workgroup has one thread a dimension, or more threads.
+template <int AHEAD>
+__global__ __launch_bounds__(256) void attention_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                        bf16_t* __restrict__ out, const int* __restrict__ rows,
                                        const int* __restrict__ query_start, const int* __restrict__ seq_ids,
                                        int H, int nsplit, const float* __restrict__ sinks) {
@@ -27,6 +31,14 @@ __global__ void attention_merge_kernel(const float* __restrict__ part_o, const f
   const int i = threadIdx.x;
   const float mi = i < nsplit ? part_ml[(slot0 + i) * 2] : -INFINITY;
   const float li = i < nsplit ? part_ml[(slot0 + i) * 2 + 1] : 0.f;
+  const float* po = part_o + slot0 * DH + min(i, DH - 1);
+  float ahead[AHEAD];
+#pragma unroll
+  for (int k0 = 0; k0 < AHEAD; k0 += 8)
+    if (k0 < nsplit) {
+#pragma unroll
+      for (int k = k0; k < k0 + 8; ++k) ahead[k] = po[static_cast<size_t>(min(k, nsplit - 1)) * DH];
+    }
   const float sink_e = sinks != nullptr ? sinks[h] * TIE_LOG2E : -INFINITY;
   const float m = fmaxf(block_max(mi, scratch), sink_e);
   const float wi = (mi == -INFINITY) ? 0.f : exp2f(mi - m);
@@ -38,17 +50,18 @@ __global__ void attention_merge_kernel(const float* __restrict__ part_o, const f
   float L = 0.f;
   for (int k = 0; k < nsplit; ++k) L += weighted_sum[k];   // ascending order, the same in every thread
   if (sinks != nullptr) L += exp2f(sink_e - m);
-  for (int d = threadIdx.x; d < DH; d += blockDim.x) {
-    float o = 0.f;
+  // Every accumulator is asked for whatever its weight (they are in flight together); a split without weight is empty
+  // and may have written nothing, so what came back for it is not used.
+  float o = 0.f;
+#pragma unroll
+  for (int k = 0; k < AHEAD; ++k)
+    if (k < nsplit) o += (weight[k] != 0.f ? ahead[k] : 0.f) * weight[k];
 #pragma unroll 8
-    for (int k = 0; k < nsplit; ++k) {
-      // every load is asked for whatever the weight (they are in flight together); a split without weight is
-      // empty and may have written nothing, so what came back for it is not used
-      const float p = part_o[(slot0 + k) * DH + d];
-      o += (weight[k] != 0.f ? p : 0.f) * weight[k];
-    }
-    out[(static_cast<size_t>(t) * H + h) * DH + d] = float_to_bf16(o / L);
+  for (int k = AHEAD; k < nsplit; ++k) {
+    const float p = po[static_cast<size_t>(k) * DH];
+    o += (weight[k] != 0.f ? p : 0.f) * weight[k];
   }
+  if (i < DH) out[(static_cast<size_t>(t) * H + h) * DH + i] = float_to_bf16(o / L);
 }
 
 // Threads of a merge workgroup: enough for one thread per split and per dimension, at most 256.
@@ -136,7 +149,11 @@ static inline void launch_attention_merge(const float* part_o, const float* part
     attention_merge_wave_kernel<<<(pairs + MERGE_WAVES - 1) / MERGE_WAVES, MERGE_WAVES * TIE_WAVE, 0, stream>>>(
         part_o, part_ml, out, rows, query_start, seq_ids, H, nsplit, pairs, sinks);
   } else {
-    attention_merge_kernel<<<dim3(H, count), attention_merge_threads(nsplit), 0, stream>>>(
-        part_o, part_ml, out, rows, query_start, seq_ids, H, nsplit, sinks);
+    const dim3 grid(H, count);
+    const int threads = attention_merge_threads(nsplit);
+    if (nsplit <= 16)
+      attention_merge_kernel<16><<<grid, threads, 0, stream>>>(part_o, part_ml, out, rows, query_start, seq_ids, H, nsplit, sinks);
+    else
+      attention_merge_kernel<72><<<grid, threads, 0, stream>>>(part_o, part_ml, out, rows, query_start, seq_ids, H, nsplit, sinks);
   }
 }

@@ -881,11 +881,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const int at = static_cast<int>(blockIdx.x) * single.waves + wave;
     const int pair = at / single.nsplit;
     if (pair >= units * single.sequences) return;
-    attention_decode_ring_wave<MIXED_DEPTH, false, CAPPED>(
+    attention_decode_ring_wave<MIXED_DEPTH, PREPARE_NOTHING, CAPPED>(
         static_cast<int>(threadIdx.x) % TIE_WAVE, at - pair * single.nsplit, single.nsplit, pair % units, pair / units, q,
         const_cast<bf16_t*>(k_cache), const_cast<bf16_t*>(v_cache), out, single.part_o, single.part_ml, query_start,
         context_lens, block_tables, single.seq_ids, H, KVH, block_size, block_shift, max_blocks, scale_log2e, cap, window,
-        single.nsplit, sinks, single.share_tiles, QkSource{}, 0);
+        single.nsplit, sinks, single.share_tiles, QkSource{}, 0, reinterpret_cast<int*>(smem) + wave * TABLE_AHEAD);
     return;
   }
   const int at = static_cast<int>(blockIdx.x) - decode_groups;

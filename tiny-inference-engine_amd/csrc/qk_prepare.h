@@ -73,28 +73,41 @@ __device__ __forceinline__ qk_f4_t load4_planes(const TX* p, size_t plane_stride
 }
 
 // RMS norm of one head: lane i of the head's LPH lanes holds elements 4 i .. 4 i + 3 (a) and the four they pair
-// with in the second half (b); the sums of squares meet by shuffles inside the head's lanes. All LPH lanes of
-// a head call this together. Formula: src/backend/cpu/cpu_backend.cpp:141-159 over one head (src/model/qwen3.cpp:222-223).
+// with in the second half (b), wa and wb the norm's weights of those; the sums of squares meet by shuffles inside the
+// head's lanes. All LPH lanes of a head call this together. Formula: src/backend/cpu/cpu_backend.cpp:141-159 over one
+// head (src/model/qwen3.cpp:222-223).
 template <int LPH>
-__device__ __forceinline__ void qk_head_norm(qk_f4_t& a, qk_f4_t& b, const float* __restrict__ w, float eps, int p0) {
-  constexpr int Dh = LPH * 8, half = LPH * 4;
-  float ss = (a[0] * a[0] + b[0] * b[0]) + (a[1] * a[1] + b[1] * b[1]) + (a[2] * a[2] + b[2] * b[2]) +
-             (a[3] * a[3] + b[3] * b[3]);
+__device__ __forceinline__ void qk_head_norm_by(qk_f4_t& a, qk_f4_t& b, qk_f4_t wa, qk_f4_t wb, float eps) {
+  constexpr int Dh = LPH * 8;
+  float ss = fmaf(a[0], a[0], b[0] * b[0]);
+#pragma unroll
+  for (int e = 1; e < 4; ++e) ss += fmaf(a[e], a[e], b[e] * b[e]);
 #pragma unroll
   for (int off = LPH / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, TIE_WAVE);
   const float inv = 1.0f / sqrtf(ss / static_cast<float>(Dh) + eps);
-  a = (a * inv) * load4(w + p0);
-  b = (b * inv) * load4(w + half + p0);
+  a = (a * inv) * wa;
+  b = (b * inv) * wb;
 }
 
-// Rotation of the pairs (i, i + head_dim / 2) by the angles of one token: row = cos of the head_dim / 2 angles,
-// then their sines. Formula: src/backend/cpu/cpu_backend.cpp:161-193, src/backend/rope.h:9-13.
+template <int LPH>
+__device__ __forceinline__ void qk_head_norm(qk_f4_t& a, qk_f4_t& b, const float* __restrict__ w, float eps, int p0) {
+  qk_head_norm_by<LPH>(a, b, load4(w + p0), load4(w + LPH * 4 + p0), eps);
+}
+
+// Rotation of the pairs (i, i + head_dim / 2) by the angles of one token: their cosines cs and sines sn.
+// Formula: src/backend/cpu/cpu_backend.cpp:161-193, src/backend/rope.h:9-13. Which product is rounded and which goes
+// into the sum whole is said here (and for the squares above): left to the compiler, it differed from kernel to kernel.
+__device__ __forceinline__ void qk_rotate_by(qk_f4_t a, qk_f4_t b, qk_f4_t cs, qk_f4_t sn, qk_f4_t& o1, qk_f4_t& o2) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    o1[e] = fmaf(a[e], cs[e], -(b[e] * sn[e]));
+    o2[e] = fmaf(b[e], cs[e], a[e] * sn[e]);
+  }
+}
+
+// The same by a token's row of the table: cos of the head_dim / 2 angles, then their sines.
 template <int LPH>
 __device__ __forceinline__ void qk_rotate_by_table(qk_f4_t a, qk_f4_t b, const float* __restrict__ row, int p0,
                                                    qk_f4_t& o1, qk_f4_t& o2) {
-  constexpr int half = LPH * 4;
-  const qk_f4_t cs = load4(row + p0);
-  const qk_f4_t sn = load4(row + half + p0);
-  o1 = a * cs - b * sn;
-  o2 = b * cs + a * sn;
+  qk_rotate_by(a, b, load4(row + p0), load4(row + LPH * 4 + p0), o1, o2);
 }

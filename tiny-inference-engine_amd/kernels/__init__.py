@@ -1657,6 +1657,8 @@ def paged_attention_prepared(planes: torch.Tensor, q_weight: Optional[torch.Tens
     nsplit, share_tiles = step_key_shares(step, S, KVH, batch.plan_context, bs)
     part_o = part_ml = None
     if nsplit > 1:
+        if write_kv:       # the newest token is a share of its own
+            nsplit = min(nsplit + 1, MAX_KEY_SPLITS)
         part_o = scratch("attention.split_o", (S * H * nsplit * Dh,), torch.float32)
         part_ml = scratch("attention.split_ml", (S * H * nsplit * 2,), torch.float32)
     _call(_lib("attention_decode_bf16", Dh).tie_attention_decode_prepared_bf16, "attention_decode_prepared_bf16",
