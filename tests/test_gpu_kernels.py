@@ -207,6 +207,42 @@ def test_qk_norm_rope_rotates_part_of_a_head_and_neighbouring_pairs(H, KVH, Dh, 
             close(kc[slot // bs, :, slot % bs], k_want[t], 2e-6, f"k of token {t}, rotary_dim {rotary_dim}, {pairing}")
 
 
+@pytest.mark.parametrize("planes", [2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("T,mix,biased,cache", [(5, None, False, torch.bfloat16), (5, "blend", True, torch.bfloat16),
+                                                (35, "keep", True, torch.bfloat16), (35, "blend", False, torch.bfloat16),
+                                                (5, "blend", True, torch.float32)])
+def test_qk_norm_rope_sums_any_number_of_planes(planes, T, mix, biased, cache):
+    """The planes of a cut projection, asked for all at once in counts of 1, 2, 4 or 8 and beyond them one by one, against
+    their sum handed over in one piece: the same bits in queries, caches and kept values, with and without a bias and
+    values blended across layers, with the values of 35 rows (four groups of eight tokens and a rest) stored apart."""
+    from tie_amd import kernels
+
+    H, KVH, Dh, bs, eps = 4, 2, 128, 16, 1e-5
+    width = (H + 2 * KVH) * Dh
+    parts = rnd(planes, T, width, seed=61).cuda()
+    whole = parts[0].clone()
+    for s in range(1, planes):
+        whole += parts[s]
+    qw, kw = (1 + 0.1 * rnd(Dh, seed=62)).cuda(), (1 + 0.1 * rnd(Dh, seed=63)).cuda()
+    bias = rnd(width, seed=64).cuda() if biased else None
+    lam = torch.tensor([0.3], device="cuda")
+    table = torch.empty(T, Dh, device="cuda")
+    inv_freq = torch.from_numpy(plain.rope_inv_freq(1e4, Dh)).cuda()
+    kernels.rope_angles(i32(range(T)), inv_freq, table)
+    results = []
+    for rows, count in ((parts[0], planes), (whole, 1)):
+        first = rnd(T, KVH * Dh, seed=65).cuda()
+        kc = torch.zeros(T // bs + 2, KVH, bs, Dh, device="cuda", dtype=cache)
+        vc = torch.zeros(T // bs + 2, KVH, Dh, bs, device="cuda", dtype=cache)
+        q = torch.empty(T, H * Dh, device="cuda", dtype=cache)
+        kernels.qk_norm_rope_kv_write(rows, q, qw, kw, eps, inv_freq, i32(range(T)), i32(range(3, T + 3)), kc, vc, H, KVH, Dh, bs,
+                                      planes=count, plane_stride=T * width, angles=table, bias=bias,
+                                      value_mix=None if mix is None else (mix, first) if mix == "keep" else (mix, first, lam))
+        results.append((q, kc, vc, first))
+    for name, a, b in zip(("queries", "keys", "values", "kept values"), *results):
+        assert torch.equal(a, b), f"{name} differ, {planes} planes"
+
+
 def attention_case(H, KVH, Dh, bs, lens_new, lens_ctx, seed, dtype=torch.float32, window=None, spike=None):
     """Builds a batch of sequences with scattered, unordered block tables; returns kernel inputs and the plain result."""
     rng = np.random.RandomState(seed)

@@ -465,14 +465,16 @@ struct ValueMix {
   int width;
 };
 
+// (1 - lambda) v + lambda first, the second product rounded, in every kernel.
+__device__ __forceinline__ float blend_value(float lam, float v, float first) { return fmaf(1.0f - lam, v, lam * first); }
+
 __device__ __forceinline__ float mix_value(const ValueMix& vm, float v, size_t t, int KVH, int h, int d) {
   if (vm.mode == 0 || d >= vm.width) return v;
   const size_t index = (t * KVH + h) * vm.width + d;
   if (vm.mode == 1) {
     vm.first[index] = v;
   } else {
-    const float lam = *vm.lambda;
-    v = (1.0f - lam) * v + lam * vm.first[index];
+    v = blend_value(*vm.lambda, v, vm.first[index]);
   }
   return v;
 }
@@ -595,7 +597,54 @@ __global__ void qk_norm_rope_kv_write_kernel(const TX* qkv, TQ* q_out, const flo
 #define VROWS_THREADS 256
 #define VROWS_TOKENS 8
 
-template <typename TX, typename TC>
+// N elements of the projection, each the sum of its planes: all asked for before the first is added (sums made one
+// after the other, behind a test of the number of planes, were a trip to memory each: 64 rows of an 8B layer 8.4 us,
+// now 5.6). PLANES: 1, 2, 4 or 8, at least as many as there are up to eight; one beyond the last is the last again and
+// not added. Planes are added in order.
+template <int N, int PLANES, typename TX>
+struct PlanedElements {
+  float part[N][PLANES];
+  const TX* at[N];
+  __device__ __forceinline__ void ask(int i, const TX* p, size_t plane_stride, int planes) {
+    at[i] = p;
+#pragma unroll
+    for (int s = 0; s < PLANES; ++s)
+      part[i][s] = load_as_float(p + static_cast<size_t>(PLANES == 1 ? 0 : min(s, planes - 1)) * plane_stride);
+  }
+  __device__ __forceinline__ float sum(int i, size_t plane_stride, int planes) const {
+    float v = part[i][0];
+#pragma unroll
+    for (int s = 1; s < PLANES; ++s) v = s < planes ? v + part[i][s] : v;
+    if (PLANES == 8)
+      for (int s = 8; s < planes; ++s) v += load_as_float(at[i] + static_cast<size_t>(s) * plane_stride);
+    return v;
+  }
+};
+
+// The same for N runs of four elements.
+template <int N, int PLANES, typename TX>
+struct PlanedFours {
+  qk_f4_t part[N][PLANES];
+  const TX* at[N];
+  __device__ __forceinline__ void ask(int i, const TX* p, size_t plane_stride, int planes) {
+    at[i] = p;
+#pragma unroll
+    for (int s = 0; s < PLANES; ++s)
+      part[i][s] = load4(p + static_cast<size_t>(PLANES == 1 ? 0 : min(s, planes - 1)) * plane_stride);
+  }
+  __device__ __forceinline__ qk_f4_t sum(int i, size_t plane_stride, int planes) const {
+    qk_f4_t v = part[i][0];
+#pragma unroll
+    for (int s = 1; s < PLANES; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = s < planes ? v[e] + part[i][s][e] : v[e];
+    if (PLANES == 8)
+      for (int s = 8; s < planes; ++s) v += load4(at[i] + static_cast<size_t>(s) * plane_stride);
+    return v;
+  }
+};
+
+template <typename TX, typename TC, int PLANES>
 __device__ __forceinline__ void v_write_rows(const TX* __restrict__ qkv, const int* __restrict__ slots,
                                              TC* __restrict__ v_cache, int T, int KVH, int Dh, int block_size,
                                              int in_row, int v_offset, size_t plane_stride, int planes, int head,
@@ -614,13 +663,25 @@ __device__ __forceinline__ void v_write_rows(const TX* __restrict__ qkv, const i
   for (int i = 1; i < VROWS_TOKENS; ++i) together = together && slot[i] == slot[0] + i;
   for (int d = Dh >= VROWS_THREADS ? threadIdx.x : threadIdx.x % Dh; d < Dh; d += VROWS_THREADS) {
     const TX* in = qkv + static_cast<size_t>(t0) * in_row + v_offset + static_cast<size_t>(head) * Dh + d;
+    PlanedElements<VROWS_TOKENS, PLANES, TX> sums;
+#pragma unroll
+    for (int i = 0; i < VROWS_TOKENS; ++i) sums.ask(i, in + static_cast<size_t>(min(i, n - 1)) * in_row, plane_stride, planes);
+    const float b = bias_at(bias, static_cast<size_t>(v_offset) + static_cast<size_t>(head) * Dh + d);
+    const size_t kept = (static_cast<size_t>(t0) * KVH + head) * vm.width + d, kept_stride = static_cast<size_t>(KVH) * vm.width;
+    const bool mixed = d < vm.width;
+    float first[VROWS_TOKENS], lam = 0.f;
+    if (vm.mode == 2) {
+      lam = *vm.lambda;
+#pragma unroll
+      for (int i = 0; i < VROWS_TOKENS; ++i) first[i] = mixed ? vm.first[kept + min(i, n - 1) * kept_stride] : 0.f;
+    }
     float v[VROWS_TOKENS];
 #pragma unroll
-    for (int i = 0; i < VROWS_TOKENS; ++i)
-      v[i] = i < n ? mix_value(vm, load_planes(in + static_cast<size_t>(i) * in_row, plane_stride, planes) +
-                                       bias_at(bias, static_cast<size_t>(v_offset) + static_cast<size_t>(head) * Dh + d),
-                               t0 + i, KVH, head, d)
-                   : 0.f;
+    for (int i = 0; i < VROWS_TOKENS; ++i) {
+      v[i] = sums.sum(i, plane_stride, planes) + b;
+      if (vm.mode == 1 && mixed && i < n) vm.first[kept + i * kept_stride] = v[i];
+      if (vm.mode == 2 && mixed) v[i] = blend_value(lam, v[i], first[i]);
+    }
     if (together) {
       TC* dst = v_cache + (static_cast<size_t>(slot[0] / block_size) * KVH + head) * Dh * block_size +
                 static_cast<size_t>(d) * block_size + slot[0] % block_size;
@@ -644,7 +705,7 @@ __device__ __forceinline__ void v_write_rows(const TX* __restrict__ qkv, const i
 // The sums of squares meet by shuffles inside the lanes of a head. Whole heads rotated as halves only.
 #define QK4_THREADS 256
 
-template <typename TX, typename TQ, typename TC, int LPH>   // LPH: lanes per head = head_dim / 8
+template <typename TX, typename TQ, typename TC, int LPH, int PLANES>   // LPH: lanes per head = head_dim / 8
 __global__ __launch_bounds__(QK4_THREADS) void qk_norm_rope_kv_write4_kernel(
     const TX* qkv, TQ* q_out, const float* __restrict__ q_w, const float* __restrict__ k_w, float eps,
     const float* __restrict__ inv_freq, const float* __restrict__ angles, const int* __restrict__ positions,
@@ -658,7 +719,7 @@ __global__ __launch_bounds__(QK4_THREADS) void qk_norm_rope_kv_write4_kernel(
   if (static_cast<int>(blockIdx.x) >= qk_blocks) {
     if constexpr (sizeof(TC) == 2) {
       const int b = blockIdx.x - qk_blocks;
-      v_write_rows<TX, TC>(qkv, slots, v_cache, tokens, KVH, Dh, block_size, in_row, v_col, plane_stride, planes,
+      v_write_rows<TX, TC, PLANES>(qkv, slots, v_cache, tokens, KVH, Dh, block_size, in_row, v_col, plane_stride, planes,
                            b % KVH, b / KVH, vm, bias);
     }
     return;
@@ -679,17 +740,46 @@ __global__ __launch_bounds__(QK4_THREADS) void qk_norm_rope_kv_write4_kernel(
     const int sub = threadIdx.x % LPH;
     in = qkv + static_cast<size_t>(t) * in_row + v_col + static_cast<size_t>(slot_index - H - KVH) * Dh;
     const size_t c0 = static_cast<size_t>(v_col) + static_cast<size_t>(slot_index - H - KVH) * Dh;
+    PlanedElements<8, PLANES, TX> sums;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sums.ask(i, in + sub + LPH * i, plane_stride, planes);
+    const size_t kept = (static_cast<size_t>(t) * KVH + (slot_index - H - KVH)) * vm.width;
+    float bv[8], first[8], lam = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) bv[i] = bias_at(bias, c0 + sub + LPH * i);
+    if (vm.mode == 2) {
+      lam = *vm.lambda;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) first[i] = sub + LPH * i < vm.width ? vm.first[kept + sub + LPH * i] : 0.f;
+    }
     float v[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      v[i] = mix_value(vm, load_planes(in + sub + LPH * i, plane_stride, planes) + bias_at(bias, c0 + sub + LPH * i), t,
-                       KVH, slot_index - H - KVH, sub + LPH * i);
+    for (int i = 0; i < 8; ++i) {
+      const bool mixed = sub + LPH * i < vm.width;
+      v[i] = sums.sum(i, plane_stride, planes) + bv[i];
+      if (vm.mode == 1 && mixed) vm.first[kept + sub + LPH * i] = v[i];
+      if (vm.mode == 2 && mixed) v[i] = blend_value(lam, v[i], first[i]);
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) store_from_float(dst + static_cast<size_t>(sub + LPH * i) * block_size, v[i]);
     return;
   }
-  qk_f4_t a = load4_planes(in + p0, plane_stride, planes);
-  qk_f4_t b = load4_planes(in + half + p0, plane_stride, planes);
+  // Everything that is read is asked for before the first of it is used.
+  PlanedFours<2, PLANES, TX> sums;
+  sums.ask(0, in + p0, plane_stride, planes);
+  sums.ask(1, in + half + p0, plane_stride, planes);
+  const float* w = is_q ? q_w : k_w;
+  const bool by_table = angles != nullptr;
+  qk_f4_t wa, wb, cs, sn;
+  if (w != nullptr) {
+    wa = load4(w + p0);
+    wb = load4(w + half + p0);
+  }
+  if (by_table) {
+    cs = load4(angles + static_cast<size_t>(t) * Dh + p0);
+    sn = load4(angles + static_cast<size_t>(t) * Dh + half + p0);
+  }
+  qk_f4_t a = sums.sum(0, plane_stride, planes), b = sums.sum(1, plane_stride, planes);
   if (bias != nullptr) {
     const float* bh = bias + static_cast<size_t>(slot_index) * Dh;
 #pragma unroll
@@ -699,11 +789,10 @@ __global__ __launch_bounds__(QK4_THREADS) void qk_norm_rope_kv_write4_kernel(
     }
   }
 
-  const float* w = is_q ? q_w : k_w;
-  if (w != nullptr) qk_head_norm<LPH>(a, b, w, eps, p0);
+  if (w != nullptr) qk_head_norm_by<LPH>(a, b, wa, wb, eps);
   qk_f4_t o1 = a, o2 = b;
-  if (angles != nullptr) {
-    qk_rotate_by_table<LPH>(a, b, angles + static_cast<size_t>(t) * Dh, p0, o1, o2);
+  if (by_table) {
+    qk_rotate_by(a, b, cs, sn, o1, o2);
   } else if (inv_freq != nullptr) {
     const float pos = static_cast<float>(positions[t]);
 #pragma unroll
@@ -807,17 +896,24 @@ extern "C" int tie_qk_norm_rope_kv_write(const void* qkv, int in_dtype, void* q_
     if (blocks > 0x7fffffffL) return TIE_BAD_ARGUMENT;
     const dim3 grid4(static_cast<unsigned>(blocks));
 #define LAUNCH4_L(TX, TQ, TC, LPH)                                                                            \
-  qk_norm_rope_kv_write4_kernel<TX, TQ, TC, LPH><<<grid4, QK4_THREADS, 0, stream>>>(                          \
+  {                                                                                                           \
+    if (planes == 1) LAUNCH4_P(TX, TQ, TC, LPH, 1);                                                           \
+    else if (planes == 2) LAUNCH4_P(TX, TQ, TC, LPH, 2);                                                      \
+    else if (planes <= 4) LAUNCH4_P(TX, TQ, TC, LPH, 4);                                                      \
+    else LAUNCH4_P(TX, TQ, TC, LPH, 8);                                                                       \
+  }
+#define LAUNCH4_P(TX, TQ, TC, LPH, PLANES)                                                                    \
+  qk_norm_rope_kv_write4_kernel<TX, TQ, TC, LPH, PLANES><<<grid4, QK4_THREADS, 0, stream>>>(                  \
       static_cast<const TX*>(qkv), static_cast<TQ*>(q_out), q_w, k_w, eps, inv_freq, angles, positions, slots, \
       static_cast<TC*>(k_cache), static_cast<TC*>(v_cache), static_cast<TQ*>(k_dense), H, KVH, block_size,   \
       in_row, q_row, k_row, static_cast<size_t>(plane_stride), planes, heads_here, T, blocks_a_token, v_col, vm, bias)
 #define LAUNCH4(TX, TQ, TC)                         \
   {                                                 \
-    if (lph == 4) LAUNCH4_L(TX, TQ, TC, 4);         \
-    else if (lph == 8) LAUNCH4_L(TX, TQ, TC, 8);    \
-    else if (lph == 16) LAUNCH4_L(TX, TQ, TC, 16);  \
-    else if (lph == 32) LAUNCH4_L(TX, TQ, TC, 32);  \
-    else LAUNCH4_L(TX, TQ, TC, 64);                 \
+    if (lph == 4) LAUNCH4_L(TX, TQ, TC, 4)          \
+    else if (lph == 8) LAUNCH4_L(TX, TQ, TC, 8)     \
+    else if (lph == 16) LAUNCH4_L(TX, TQ, TC, 16)   \
+    else if (lph == 32) LAUNCH4_L(TX, TQ, TC, 32)   \
+    else LAUNCH4_L(TX, TQ, TC, 64)                  \
   }
     if (in_dtype == TIE_F32 && q_dtype == TIE_F32 && cache_dtype == TIE_F32) LAUNCH4(float, float, float)
     else if (in_dtype == TIE_F32 && q_dtype == TIE_BF16 && cache_dtype == TIE_BF16) LAUNCH4(float, bf16_t, bf16_t)
@@ -827,6 +923,7 @@ extern "C" int tie_qk_norm_rope_kv_write(const void* qkv, int in_dtype, void* q_
     else return TIE_BAD_ARGUMENT;
 #undef LAUNCH4
 #undef LAUNCH4_L
+#undef LAUNCH4_P
     return tie_launch_status();
   }
   const dim3 grid(heads, T);

@@ -53,25 +53,6 @@ __device__ __forceinline__ void store4<f16_t>(f16_t* p, qk_f4_t v) {
   *reinterpret_cast<qk_h4_t*>(p) = __builtin_convertvector(v, qk_h4_t);
 }
 
-template <typename TX>
-__device__ __forceinline__ qk_f4_t load4_planes(const TX* p, size_t plane_stride, int planes) {
-  if (planes == 2) return load4(p) + load4(p + plane_stride);
-  if (planes == 4 || planes == 8) {
-    qk_f4_t part[8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-      part[s] = s < planes ? load4(p + static_cast<size_t>(s) * plane_stride) : qk_f4_t{0.f, 0.f, 0.f, 0.f};
-    qk_f4_t v = part[0];
-#pragma unroll
-    for (int s = 1; s < 8; ++s)
-      if (s < planes) v += part[s];
-    return v;
-  }
-  qk_f4_t v = load4(p);
-  for (int s = 1; s < planes; ++s) v += load4(p + static_cast<size_t>(s) * plane_stride);
-  return v;
-}
-
 // RMS norm of one head: lane i of the head's LPH lanes holds elements 4 i .. 4 i + 3 (a) and the four they pair
 // with in the second half (b), wa and wb the norm's weights of those; the sums of squares meet by shuffles inside the
 // head's lanes. All LPH lanes of a head call this together. Formula: src/backend/cpu/cpu_backend.cpp:141-159 over one
@@ -89,11 +70,6 @@ __device__ __forceinline__ void qk_head_norm_by(qk_f4_t& a, qk_f4_t& b, qk_f4_t 
   b = (b * inv) * wb;
 }
 
-template <int LPH>
-__device__ __forceinline__ void qk_head_norm(qk_f4_t& a, qk_f4_t& b, const float* __restrict__ w, float eps, int p0) {
-  qk_head_norm_by<LPH>(a, b, load4(w + p0), load4(w + LPH * 4 + p0), eps);
-}
-
 // Rotation of the pairs (i, i + head_dim / 2) by the angles of one token: their cosines cs and sines sn.
 // Formula: src/backend/cpu/cpu_backend.cpp:161-193, src/backend/rope.h:9-13. Which product is rounded and which goes
 // into the sum whole is said here (and for the squares above): left to the compiler, it differed from kernel to kernel.
@@ -103,11 +79,4 @@ __device__ __forceinline__ void qk_rotate_by(qk_f4_t a, qk_f4_t b, qk_f4_t cs, q
     o1[e] = fmaf(a[e], cs[e], -(b[e] * sn[e]));
     o2[e] = fmaf(b[e], cs[e], a[e] * sn[e]);
   }
-}
-
-// The same by a token's row of the table: cos of the head_dim / 2 angles, then their sines.
-template <int LPH>
-__device__ __forceinline__ void qk_rotate_by_table(qk_f4_t a, qk_f4_t b, const float* __restrict__ row, int p0,
-                                                   qk_f4_t& o1, qk_f4_t& o2) {
-  qk_rotate_by(a, b, load4(row + p0), load4(row + LPH * 4 + p0), o1, o2);
 }
