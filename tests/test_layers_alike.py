@@ -149,3 +149,50 @@ def test_a_launch_list_launches_what_every_layers_own_code_does(monkeypatch, wid
     assert listed == own
     pending = sum(what == "skinny_gemm_bf16_norm" and args[15] is not None for what, args in own)   # a next norm's weight
     assert pending == (13 if rows == 3 else 0)
+
+
+def test_a_launch_list_as_words(monkeypatch):
+    """What one native call runs for several layers: pointers and whole numbers (negative ones too), a float's bits, None
+    as a null pointer, and every layer's own addresses where they belong; a refused launch is reported by its name."""
+    import ctypes
+    import struct
+
+    import numpy as np
+
+    from tie_amd import kernels
+    from tie_amd.errors import InvalidArgument
+
+    norm = kernels._lib("elementwise").tie_rms_norm
+    first = (norm, "rms_norm", (1000, 0, 2000, 1e-6, 3000, 1, None, 4, 256, 7), ((0, 1, 16), (4, 0, 0)))
+    second = (norm, "second norm", (1000, 0, 2000, -0.5, 3000, 1, None, -4, 256, 7), ())
+    assert kernels.LaunchList.takes([first, second])
+    assert not kernels.LaunchList.takes([first, (kernels._order_streams, "order_streams", (None, None), ())])
+    ran = {}
+
+    class Recorder:
+        @staticmethod
+        def tie_run_launch_list(entries, first_word, count, words, words_a_layer, layers, failed):
+            ran["words"] = np.ctypeslib.as_array(ctypes.cast(words, ctypes.POINTER(ctypes.c_uint64)), (layers, words_a_layer)).copy()
+            return 0
+
+    listed = kernels.LaunchList([first, second])
+    real = kernels._lib
+    monkeypatch.setattr(kernels, "_lib", lambda key, *a: Recorder if key == "launch_list" else real(key, *a))
+    listed.run([[50, 60], [2 ** 40, 2 ** 41]])
+    eps, half = (struct.unpack("<I", struct.pack("<f", v))[0] for v in (1e-6, -0.5))
+    rest = [1000, 0, 2000, half, 3000, 1, 0, 2 ** 64 - 4, 256, 7]
+    assert ran["words"].tolist() == [[76, 0, 2000, eps, 50, 1, 0, 4, 256, 7] + rest,
+                                     [2 ** 41 + 16, 0, 2000, eps, 2 ** 40, 1, 0, 4, 256, 7] + rest]
+    monkeypatch.setattr(kernels, "_lib", real)
+    with pytest.raises(InvalidArgument, match="second norm"):       # refused before anything is launched
+        kernels.LaunchList([second]).run([[0, 0]])
+
+
+def test_lists_go_to_the_device_together():
+    import torch
+
+    from tie_amd import kernels
+
+    a, none, b = kernels.upload_ints("cpu", [3, 1, 2], [], [7])
+    assert none is None and a.dtype == b.dtype == torch.int32 and a.tolist() == [3, 1, 2] and b.tolist() == [7]
+    assert kernels.upload_ints("cpu", [], []) == [None, None]

@@ -328,6 +328,17 @@ class CacheManager:
         nb, kvh, bs, dh = tensor.shape[2:]
         return tensor[plane, 0], tensor[plane, 1].view(nb, kvh, dh, bs)
 
+    def plane_places(self, group: int, plane: int) -> "list":
+        """``(address, bytes)`` of what ``kv_planes`` (keys, values) or ``state_plane`` returns, without making views."""
+        tensor = self.kv.get(group)
+        if tensor is None:
+            tensor = self.state[group]
+            size = tensor.stride(0) * tensor.element_size()
+            return [(tensor.data_ptr() + plane * size, size)]
+        size = tensor.stride(1) * tensor.element_size()
+        at = tensor.data_ptr() + plane * 2 * size
+        return [(at, size), (at + size, size)]
+
     def state_plane(self, group: int, plane: int) -> torch.Tensor:
         """The states of one plane: ``[max_state_slots, *shape]``."""
         return self.state[group][plane]

@@ -375,3 +375,9 @@ extern "C" int tie_attention_decode_bf16(const void* q, const void* k_cache, con
                                         block_tables, seq_ids, num_seqs, H, KVH, block_size, max_blocks, scale, softcap,
                                         window, nsplit, nullptr, 0, 0, nullptr, stream);
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_attention_decode_bf16)
+TIE_LIST_ENTRY(tie_attention_decode_prepared_bf16)
+TIE_LIST_ENTRY(tie_attention_decode_bf16_with)
+TIE_LIST_ENTRY(tie_attention_decode_bf16_keeping)

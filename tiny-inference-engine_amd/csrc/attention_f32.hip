@@ -342,3 +342,6 @@ extern "C" int tie_attention_f32(const float* q, const void* k_cache, const void
   attention_f32_merge_kernel<<<dim3(H, T), TIE_WAVE, 0, stream>>>(part_o, part_ml, out, H, Dh, nsplit, sinks);
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_attention_f32)

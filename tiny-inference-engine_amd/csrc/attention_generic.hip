@@ -153,3 +153,6 @@ extern "C" int tie_paged_attention_generic(const void* q, int q_dtype, const voi
 #undef LAUNCH
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_paged_attention_generic)

@@ -1177,3 +1177,9 @@ extern "C" int tie_attention_mixed_bf16(const void* q, const void* k_cache, cons
   }
   return status;
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_attention_prefill_bf16)
+TIE_LIST_ENTRY(tie_attention_prefill_bf16_with)
+TIE_LIST_ENTRY(tie_attention_prefill_bf16_keeping)
+TIE_LIST_ENTRY(tie_attention_mixed_bf16)

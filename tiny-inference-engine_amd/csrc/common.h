@@ -5,6 +5,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+#include <utility>
+
 // Element type codes of the C interface.
 #define TIE_F32 0
 #define TIE_BF16 1
@@ -137,6 +140,37 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
   for (int w = 1; w < waves; ++w) total = fmaxf(total, scratch[w]);
   return total;
 }
+
+// A launch as data: TIE_LIST_ENTRY(f) defines f_list, which calls the C function f with its arguments from an array of
+// 64-bit words (pointers and whole numbers as they are, a float's bits in the lower half), so that launch_list.hip runs
+// a layer's launches one after the other without a call from Python for each.
+template <typename A>
+static inline A tie_argument(uint64_t word) {
+  if constexpr (std::is_pointer<A>::value) {
+    return reinterpret_cast<A>(word);
+  } else if constexpr (std::is_same<A, float>::value) {
+    const uint32_t bits = static_cast<uint32_t>(word);
+    float value;
+    __builtin_memcpy(&value, &bits, sizeof(value));
+    return value;
+  } else {
+    static_assert(std::is_integral<A>::value, "pointers, floats and whole numbers");
+    return static_cast<A>(word);
+  }
+}
+
+template <typename... A, size_t... I>
+static inline int tie_call_words(int (*f)(A...), const uint64_t* words, std::index_sequence<I...>) {
+  return f(tie_argument<A>(words[I])...);
+}
+
+template <typename... A>
+static inline int tie_call_words(int (*f)(A...), const uint64_t* words) {
+  return tie_call_words(f, words, std::index_sequence_for<A...>{});
+}
+
+#define TIE_LIST_ENTRY(f) \
+  extern "C" int f##_list(const uint64_t* words) { return tie_call_words(&f, words); }
 
 static inline int tie_launch_status() {
   hipError_t e = hipGetLastError();

@@ -466,3 +466,6 @@ extern "C" int tie_delta_chunks(const float* tok, int row, float* out, int out_r
   delta_chunk_outputs_kernel<<<grid, DC_THREADS, 0, stream>>>(g, out, out_row);
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_delta_chunks)

@@ -824,3 +824,11 @@ extern "C" int tie_grouped_gated_rms_norm(const float* o, int o_row, const float
     return TIE_BAD_ARGUMENT;
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_conv_qkv)
+TIE_LIST_ENTRY(tie_conv_state_update)
+TIE_LIST_ENTRY(tie_delta_prepare)
+TIE_LIST_ENTRY(tie_gated_delta_scan)
+TIE_LIST_ENTRY(tie_gated_delta_scan_chunked)
+TIE_LIST_ENTRY(tie_grouped_gated_rms_norm)

@@ -1557,3 +1557,17 @@ extern "C" int tie_sample(const float* logits, const float* row_max, const float
                                                                     other_uniform, take_other, drew_none, rows, out, V);
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_poly_norm)
+TIE_LIST_ENTRY(tie_scale_softcap)
+TIE_LIST_ENTRY(tie_rms_norm)
+TIE_LIST_ENTRY(tie_swiglu)
+TIE_LIST_ENTRY(tie_cast)
+TIE_LIST_ENTRY(tie_scale_rows)
+TIE_LIST_ENTRY(tie_add_bias)
+TIE_LIST_ENTRY(tie_rope_angles)
+TIE_LIST_ENTRY(tie_qk_norm_rope_kv_write)
+TIE_LIST_ENTRY(tie_norm_add_norm)
+TIE_LIST_ENTRY(tie_gelu)
+TIE_LIST_ENTRY(tie_add_partials_rms_norm)

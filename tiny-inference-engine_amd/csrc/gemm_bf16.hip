@@ -651,3 +651,6 @@ extern "C" int tie_gemm_bf16(const void* x, const void* w, void* out, int out_dt
   if (tile == 3) return launch_gemm<256, 128, 64, 4, 2>(x, w, out, epi, M, N, K, splits, stream);
   return launch_gemm<128, 128, 64, 2, 2>(x, w, out, epi, M, N, K, splits, stream);
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_gemm_bf16)

@@ -254,3 +254,6 @@ extern "C" int tie_gemm_f32(const float* x, const float* w, float* out, int accu
 #undef LAUNCH
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_gemm_f32)

@@ -152,3 +152,6 @@ extern "C" int tie_gemm_f32_rows(const float* x, const float* w, float* out, int
 #undef LAUNCH
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_gemm_f32_rows)

@@ -96,3 +96,6 @@ extern "C" int tie_gemm_generic(const void* x, int x_dtype, const void* w, int w
 #undef LAUNCH
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_gemm_generic)

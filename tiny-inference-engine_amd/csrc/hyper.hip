@@ -377,3 +377,7 @@ extern "C" int tie_hyper_connection(float* streams, long stream_stride, int S, i
     return TIE_BAD_ARGUMENT;
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_layer_norm)
+TIE_LIST_ENTRY(tie_hyper_connection)

@@ -322,3 +322,8 @@ extern "C" int tie_head_linear(const void* x, int x_dtype, int x_row, int x_head
 #undef HL
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_rms_norm_columns)
+TIE_LIST_ENTRY(tie_latent_prepare)
+TIE_LIST_ENTRY(tie_head_linear)

@@ -919,3 +919,8 @@ extern "C" int tie_rotate_heads(float* rows, int row, int q_col, int k_col, cons
   rotate_heads_kernel<<<dim3((pairs + 255) / 256, T), 256, 0, stream>>>(rows, row, q_col, k_col, angles, rot, heads, d);
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_matrix_state_walk)
+TIE_LIST_ENTRY(tie_matrix_state_chunks)
+TIE_LIST_ENTRY(tie_rotate_heads)

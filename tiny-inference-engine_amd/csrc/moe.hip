@@ -819,3 +819,11 @@ extern "C" int tie_moe_combine(const float* parts, const int* where, const float
     return TIE_BAD_ARGUMENT;
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_moe_route)
+TIE_LIST_ENTRY(tie_moe_route_align)
+TIE_LIST_ENTRY(tie_moe_align)
+TIE_LIST_ENTRY(tie_moe_gemm_generic)
+TIE_LIST_ENTRY(tie_moe_gemm_bf16)
+TIE_LIST_ENTRY(tie_moe_combine)

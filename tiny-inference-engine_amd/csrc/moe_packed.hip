@@ -264,3 +264,6 @@ extern "C" int tie_moe_gemm_packed(const void* x, int x_rows, const void* w, voi
 #undef MANY
   return TIE_BAD_ARGUMENT;
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_moe_gemm_packed)

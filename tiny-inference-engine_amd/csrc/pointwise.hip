@@ -140,3 +140,8 @@ extern "C" int tie_gate_rows(void* rows, int dtype, const float* gate, int gate_
 #undef GATE
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_dynamic_tanh)
+TIE_LIST_ENTRY(tie_gate_rows)
+TIE_LIST_ENTRY(tie_token_gate)

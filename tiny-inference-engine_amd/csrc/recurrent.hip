@@ -153,3 +153,7 @@ extern "C" int tie_min_gru_scan(const float* proj, int row, void* out, int out_d
 #undef LAUNCH_PASS
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_gated_rms_norm)
+TIE_LIST_ENTRY(tie_min_gru_scan)

@@ -342,3 +342,7 @@ extern "C" int tie_add_normed_results(float* x, const float* a, long a_stride, i
   else return TIE_BAD_ARGUMENT;
   return tie_launch_status();
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_add_results)
+TIE_LIST_ENTRY(tie_add_normed_results)

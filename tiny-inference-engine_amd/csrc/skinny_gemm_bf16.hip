@@ -837,3 +837,8 @@ extern "C" int tie_skinny_gemm_bf16_norm(const void* x, const void* w, void* out
   const SkNorm norm = {scale_squares, scale_tiles, scale_n, scale_eps, next_w, static_cast<bf16_t*>(next_x), squares};
   return launch_skinny(x, w, out, out_dtype, accumulate, gated, M, N, K, splits, packed, rt, u, waves, norm, stream);
 }
+
+// What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_skinny_gemm_bf16_with)
+TIE_LIST_ENTRY(tie_skinny_gemm_bf16)
+TIE_LIST_ENTRY(tie_skinny_gemm_bf16_norm)

@@ -11,8 +11,10 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import struct
 from typing import Dict, Optional
 
+import numpy as np
 import torch
 
 from ..errors import InvalidArgument, KernelUnavailable
@@ -70,6 +72,7 @@ _SOURCES = {
     "latent": ("tie_latent", "latent.hip"),
     "pointwise": ("tie_pointwise", "pointwise.hip"),
     "residual": ("tie_residual", "residual.hip"),
+    "launch_list": ("tie_launch_list", "launch_list.hip"),
 }
 # libraries compiled once per head size: key -> (file stem prefix, source)
 _PER_HEAD_DIM = {
@@ -82,6 +85,9 @@ MAX_HEAD_DIM = 512        # the largest head size any attention kernel takes (th
 MAX_STEP_TOKENS = 65535   # rows of one step: a grid dimension of the row-wise kernels
 
 _SIGNATURES = {
+    "launch_list": {
+        "tie_run_launch_list": [_c_void, _c_void, _c_int, _c_void, _c_int, _c_int, ctypes.POINTER(_c_int)],
+    },
     "machine_peaks": {
         "tie_stream_read": [_c_void, ctypes.c_longlong, _c_int, _c_void, _c_void, _c_void],
         "tie_mfma_rate": [_c_int, _c_int, _c_void, _c_void, _c_void],
@@ -310,6 +316,8 @@ def _lib(key: str, head_dim: int = 0):
             f = getattr(lib, fn)
             f.argtypes = argtypes
             f.restype = _c_int
+            entry = getattr(lib, fn + "_list", None)           # the same function over an array of words
+            f.list_entry = None if entry is None else ctypes.cast(entry, _c_void).value
         _libs[cache_key] = lib
     return lib
 
@@ -364,6 +372,49 @@ def order_streams(waiting: torch.cuda.Stream, first: torch.cuda.Stream) -> None:
 def replay_call(fn, what: str, args) -> None:
     """A noted launch again, with the arguments given (see ``models.builder``: layers of one shape)."""
     _check(fn(*args), what)
+
+
+class LaunchList:
+    """Noted launches as arrays that one native call runs for any number of layers (csrc/launch_list.hip): about 2.5 us a
+    launch where a call from Python takes 4 to 7. ``launches``: ``(fn, what, args, patches)``, a patch being ``(argument,
+    tensor, offset)``: the argument is the layer's address of that tensor, plus the offset."""
+
+    def __init__(self, launches):
+        self.names = [what for _, what, _, _ in launches]
+        words, first, position, slot, offset = [], [], [], [], []
+        for fn, _, args, patches in launches:
+            position += [len(words) + p for p, _, _ in patches]
+            slot += [s for _, s, _ in patches]
+            offset += [o for _, _, o in patches]
+            first.append(len(words))
+            words += [_float_word(a) if t is _c_float else (a or 0) & 0xFFFFFFFFFFFFFFFF for t, a in zip(fn.argtypes, args)]
+        self.entries = np.array([fn.list_entry for fn, _, _, _ in launches], dtype=np.uint64)
+        self.first = np.array(first, dtype=np.int32)
+        self.words = np.array(words, dtype=np.uint64)
+        self.position, self.slot = np.array(position, dtype=np.int64), np.array(slot, dtype=np.int64)
+        self.offset = np.array(offset, dtype=np.uint64)
+
+    @staticmethod
+    def takes(launches) -> bool:
+        """Whether every one of these is a launch that has a list entry, with arguments that fit its words."""
+        return all(getattr(fn, "list_entry", None) and len(args) == len(fn.argtypes) and
+                   all(a is None or isinstance(a, (int, float) if t is _c_float else int) for t, a in zip(fn.argtypes, args))
+                   for fn, _, args, _ in launches)
+
+    def run(self, addresses) -> None:
+        """``addresses``: a row a layer, its tensors' addresses."""
+        words = np.repeat(self.words[None], len(addresses), axis=0)
+        if len(self.position):
+            words[:, self.position] = np.asarray(addresses, dtype=np.uint64)[:, self.slot] + self.offset
+        failed = _c_int(0)
+        status = _lib("launch_list").tie_run_launch_list(
+            self.entries.ctypes.data, self.first.ctypes.data, len(self.names), words.ctypes.data, words.shape[1], len(words),
+            ctypes.byref(failed))
+        _check(status, self.names[failed.value])
+
+
+def _float_word(value: float) -> int:
+    return struct.unpack("<I", struct.pack("<f", value))[0]
 
 
 def _check(status: int, what: str) -> None:
@@ -423,6 +474,27 @@ def _cache_code(cache: torch.Tensor, beside: torch.Tensor, name: str) -> int:
     if code == F16 and beside.dtype != torch.float32:
         raise InvalidArgument(f"a float16 {name} goes with float32 queries, not {beside.dtype}")
     return code
+
+
+def upload_ints(device, *lists) -> list:
+    """int32 tensors of these lists on the device (None for an empty one), by one copy that the host does not wait for.
+
+    From pageable memory the host waits for the copy, which is behind everything queued so far: a step with a prompt
+    portion so stood still once or three times in its first layer, and the GPU with it until the host had launched the
+    next kernels (a prompt of 23 tokens on the 1.7B shape 1750 us, now 1450)."""
+    device = torch.device(device)
+    values = np.array([i for l in lists for i in l], dtype=np.int32)
+    if device.type == "cuda":
+        host = torch.empty(len(values), dtype=torch.int32, pin_memory=True)     # given back when the copy has run
+        host.numpy()[:] = values
+        there = host.to(device, non_blocking=True)
+    else:
+        there = torch.from_numpy(values).to(device)
+    out, at = [], 0
+    for l in lists:
+        out.append(there[at:at + len(l)] if l else None)
+        at += len(l)
+    return out
 
 
 def _i32(t: torch.Tensor, name: str, numel: Optional[int] = None) -> torch.Tensor:
@@ -1888,10 +1960,9 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             for n in new:
                 starts.append(starts[-1] + n)
             merge_rows = [starts[s] + r for s in sorted({it[0] for it in items}) for r in range(new[s])]
+            flat, rows, ids = upload_ints(q.device, [i for it in items for i in it], merge_rows, single)
             work = batch.memo[key] = (
-                torch.tensor(single, dtype=torch.int32).to(q.device) if single else None, len(single),
-                torch.tensor(items, dtype=torch.int32).to(q.device) if items else None, len(items),
-                torch.tensor(merge_rows, dtype=torch.int32).to(q.device) if items else None,
+                ids, len(single), None if flat is None else flat.view(-1, 2), len(items), rows,
                 max((batch.host_context_lens[it[0]] for it in items), default=0))
         seq_ids, num_single, items, num_items, merge_rows, items_context = work
         # Both kinds of rows in one launch, where its kernel takes them.
@@ -1905,8 +1976,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                 if together and not length:
                     keys = min(batch.plan_context, reach or batch.plan_context)
                     nsplit = max(nsplit, min(-(-MIXED_WAVES // (num_single * KVH)), keys // 128, MAX_KEY_SPLITS))
-                planned = batch.memo[shares_key] = (
-                    nsplit, torch.tensor([length], dtype=torch.int32).to(q.device) if length else None)
+                planned = batch.memo[shares_key] = (nsplit, upload_ints(q.device, [length] if length else [])[0])
             nsplit, share_tiles = planned
             part_o = part_ml = None
             if nsplit > 1:
@@ -1996,9 +2066,8 @@ def scan_chunks(batch, device, rows: int = SCAN_CHUNK_ROWS, force: bool = False)
             first.append(len(items))
         if len(items) > MAX_STEP_TOKENS:
             return None
-        memo = batch.memo[key] = ScanChunks(torch.tensor(items, dtype=torch.int32).to(device),
-                                            torch.tensor(first, dtype=torch.int32).to(device), len(items),
-                                            max(b - a for _, a, b in items))
+        flat, starts = upload_ints(device, [i for item in items for i in item], first)
+        memo = batch.memo[key] = ScanChunks(flat.view(-1, 3), starts, len(items), max(b - a for _, a, b in items))
     return memo
 
 

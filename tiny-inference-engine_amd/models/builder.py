@@ -263,6 +263,9 @@ class Model:
         layer's tensors and its cache. ``place``: the layer before left its projection of that place pending
         (``_pending_place``), and this layer's first launch reads that weight."""
         tensors = list(self._layer_tensors[index])
+        if isinstance(cache, list):          # places alone (StepContext.cache_places)
+            tensors += cache
+            cache = None
         for binding in (cache if isinstance(cache, tuple) else (cache,)):
             for name in ("k_cache", "v_cache", "state"):
                 t = getattr(binding, name, None)
@@ -347,6 +350,16 @@ class Model:
             tensors.append(self._entry_tensors(ctx, index, cache, place if carried else None))
             carried = carried and self._pending_place(ctx, index) == place
         launches = self._launch_list(noted[0], noted[1], tensors[0], tensors[1]) if carried else None
+        if launches is not None and torch.device(ctx.device).type == "cuda":
+            listed = [(launch.fn, launch.what, launch.args, launch.patches) for launch in launches]
+            if kernels.LaunchList.takes(listed):
+                kernels.LaunchList(listed).run(
+                    [[address for address, _ in self._entry_tensors(ctx, index, ctx.cache_places(index), place)]
+                     for index in range(start + 3, end)])
+                self.layers_replayed += end - start - 3
+                if place is not None:
+                    ctx.pending_linear = self._layer_projections[end - 1][place]
+                return
         for index in range(start + 3, end):
             if launches is None:
                 run(index)

@@ -320,6 +320,15 @@ class StepContext:
             return tuple(self._bind(e) for e in entry)
         return self._bind(entry)
 
+    def cache_places(self, call_index: int) -> list:
+        """``(address, bytes)`` of the tensors that ``cache_of`` binds for that entry, in its order: keys and values, or
+        states, a need after the other."""
+        entry = self.cache_plan.calls[call_index]
+        if entry is None:
+            return []
+        return [place for e in (entry if isinstance(entry, tuple) else (entry,))
+                for place in self.cache_manager.plane_places(e.group, e.plane)]
+
     def _bind(self, entry):
         from ..cache.spec import PagedKV
 
