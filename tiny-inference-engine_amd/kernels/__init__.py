@@ -1548,6 +1548,7 @@ BALANCED_SHARES_GRID = 8
 # shorter pays (16 sequences of 8 KV heads, 100 to 4000 keys, 4 shares each: 37.7 us a layer, shares of one
 # length 36.8 to 44.8; one sequence of 32 k keys beside 23 of 1 k: 176 -> 74).
 BALANCED_SHARES_MAX_EQUAL = 3
+TILES_A_WALK = 174       # tiles of 32 keys that a step's waves bring at 4.75 TB/s while one of them walks a tile in 0.6 us
 
 
 def decode_share_plan(context_lens, num_kv_heads: int, plan_context: int, block_size: int = 16,
@@ -1566,7 +1567,11 @@ def decode_share_plan(context_lens, num_kv_heads: int, plan_context: int, block_
     grow) is empty (those steps: 68, 62, 43 and 52 us; 64 sequences, 2 of them long: 94 -> 53). Taken only if the
     longest share gets half as long, a quarter where a sequence's own shares are more than three: between that
     and equal the merge and the empty shares cost what the balance gains (56 sequences, a quarter long: 94 -> 109
-    us at two thirds; two of 16 k beside six of 2 k: 56 -> 57 at a third).
+    us at two thirds; two of 16 k beside six of 2 k: 56 -> 57 at a third). And only where the longest share is what the
+    step waits for: a wave walks a tile in 0.6 us, in which all together bring ``TILES_A_WALK`` tiles from memory, so a
+    longest share below that part of all tiles ends with the others, and empty shares and the merge are for nothing (64
+    sequences of 94 to 1500 keys 44.2 us as they are and 46 in shares of 17 tiles, of 31 to 500 18.1 and 22; 56, a quarter
+    4000 and the others 800, 69.5 and 71; but 32 of 62 to 1000 21.3 and 20.9, 32, a quarter 4096 beside 1400, 82 and 57).
     """
     S = len(context_lens)
     equal = decode_splits(S, num_kv_heads, plan_context, block_size)
@@ -1592,6 +1597,8 @@ def decode_share_plan(context_lens, num_kv_heads: int, plan_context: int, block_
         else:
             lo = mid + 1
     before = -(-longest // equal)
+    if before * TILES_A_WALK <= num_kv_heads * sum(tiles):
+        return equal, 0
     if (2 * lo > before) if equal <= BALANCED_SHARES_MAX_EQUAL else (4 * lo >= before):
         return equal, 0
     grid = BALANCED_SHARES_GRID
