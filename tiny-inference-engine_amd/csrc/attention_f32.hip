@@ -87,6 +87,10 @@ __global__ __launch_bounds__(W* TIE_WAVE) void attention_f32_kernel(
   }
   s = __builtin_amdgcn_readfirstlane(s);
   first_row = __builtin_amdgcn_readfirstlane(first_row);
+  const int* table = block_tables + static_cast<size_t>(s) * max_blocks;
+  // The table's first entries come with the lengths, so that the first tile of a short context is not asked for a trip
+  // to memory later.
+  const int table_ahead = table[min(lane, max_blocks - 1)];
   const int start_row = query_start[s];
   const int n_new = query_start[s + 1] - start_row;
   const int cached = context_lens[s] - n_new;                // row i sits at position cached + i
@@ -97,7 +101,6 @@ __global__ __launch_bounds__(W* TIE_WAVE) void attention_f32_kernel(
   const int my_head = kvh * group + 16 * head_tile + (valid ? r % heads : 0);
   const int pos = cached + my_row;
   const int start = first_visible_key(pos, window, chunk);
-  const int* table = block_tables + static_cast<size_t>(s) * max_blocks;
 
   // Key tiles of 16 this workgroup's share holds, wave by wave in turn.
   const int tile_lo = first_visible_key(cached + first_row, window, chunk) / 16;
@@ -120,20 +123,18 @@ __global__ __launch_bounds__(W* TIE_WAVE) void attention_f32_kernel(
 
   f32x4_t kf[DT], vf[DT];
   const unsigned key_at = r * DH + 4 * c, value_at = r * block_size + 4 * c;      // this lane's place in a tile
-  auto ask_keys = [&](int tile) {
-    const int page = table[tile * 16 / block_size];
+  auto page_of = [&](int tile) { return table[tile * 16 / block_size]; };
+  auto ask_keys = [&](int tile, int page) {
     const TC* p = k_cache + ((static_cast<size_t>(page) * KVH + kvh) * block_size + tile * 16 % block_size) * DH;
 #pragma unroll
     for (int j = 0; j < DT; ++j) kf[j] = af_load4(p + (key_at + 16 * j));
   };
-  auto values_of = [&](int tile) {
-    const int page = table[tile * 16 / block_size];
-    return v_cache + (static_cast<size_t>(page) * KVH + kvh) * DH * block_size + tile * 16 % block_size;
-  };
-  int tile = lo + wave;
-  if (tile < hi) ask_keys(tile);
-  for (; tile < hi; tile += W) {
-    const TC* vp = values_of(tile);
+  // A tile of page `page`. With NEXT the keys of this wave's tile behind it, of page `next_page`, are asked for as soon as
+  // this one's are read. Two instantiations and not a condition: behind one the compiler does not know how many loads
+  // are younger than the values it waits for, and waits for the next keys too.
+  auto step = [&](int tile, int page, int next_page, auto has_next) {
+    constexpr bool NEXT = decltype(has_next)::value;
+    const TC* vp = v_cache + (static_cast<size_t>(page) * KVH + kvh) * DH * block_size + tile * 16 % block_size;
 #pragma unroll
     for (int j = 0; j < DT; ++j) vf[j] = af_load4(vp + 16 * j * block_size + value_at);
     f32x4_t sc = {0.f, 0.f, 0.f, 0.f};
@@ -145,7 +146,7 @@ __global__ __launch_bounds__(W* TIE_WAVE) void attention_f32_kernel(
         if (i % 2 == 0) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], qf[j][i], sc, 0, 0, 0);
         else sc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], qf[j][i], sc2, 0, 0, 0);
       }
-    if (tile + W < hi) ask_keys(tile + W);
+    if constexpr (NEXT) ask_keys(tile + W, next_page);
     const int key0 = tile * 16 + 4 * c;
     const bool partly = tile * 16 < full_from || tile * 16 + 15 > full_to;      // some column does not see some key
     float p[4];
@@ -211,6 +212,19 @@ __global__ __launch_bounds__(W* TIE_WAVE) void attention_f32_kernel(
         }
       }
     }
+  };
+  int tile = lo + wave;
+  if (tile < hi) {
+    const int entry = tile * 16 / block_size;
+    int page = entry < TIE_WAVE ? __builtin_amdgcn_readlane(table_ahead, entry) : table[entry];
+    ask_keys(tile, page);
+    while (tile + W < hi) {
+      const int next_page = page_of(tile + W);
+      step(tile, page, next_page, std::true_type{});
+      page = next_page;
+      tile += W;
+    }
+    step(tile, page, 0, std::false_type{});
   }
   l += __shfl_xor(l, 16, TIE_WAVE);
   l += __shfl_xor(l, 32, TIE_WAVE);
@@ -263,7 +277,10 @@ __global__ __launch_bounds__(W* TIE_WAVE) void attention_f32_kernel(
 #endif
 }
 
-// One wave a (row, head): its shares' maxima and sums first, then four dimensions a lane, in the order of the shares.
+// One wave a (row, head): its shares' maxima and sums, four dimensions a lane, in the order of the shares. The first
+// AHEAD shares' accumulators are asked for together with the maxima and sums: one trip to memory (four rows of 16 heads
+// in 5 shares: 3.9 us with a trip a share).
+template <int AHEAD>
 __global__ __launch_bounds__(TIE_WAVE) void attention_f32_merge_kernel(const float* __restrict__ part_o,
                                                                        const float* __restrict__ part_ml,
                                                                        float* __restrict__ out, int H, int Dh, int nsplit,
@@ -273,20 +290,23 @@ __global__ __launch_bounds__(TIE_WAVE) void attention_f32_merge_kernel(const flo
   const float* ml = part_ml + where * nsplit * 2;
   const float mine = lane < nsplit ? ml[2 * lane] : -INFINITY;
   const float sum = lane < nsplit ? ml[2 * lane + 1] : 0.f;
+  const int d = 4 * lane;                       // head sizes up to 256
+  const float* po = part_o + where * nsplit * Dh + (d < Dh ? d : 0);
+  f32x4_t ahead[AHEAD];
+#pragma unroll
+  for (int k = 0; k < AHEAD; ++k) ahead[k] = af_load4(po + min(k, nsplit - 1) * Dh);
   const float sink = sinks != nullptr ? sinks[blockIdx.x] : -INFINITY;
   const float m = fmaxf(wave_max(mine), sink);
   const float weight = af_weight(mine, m);
   float l = af_weight(sink, m);
   for (int k = 0; k < nsplit; ++k) l += __shfl(weight, k, TIE_WAVE) * __shfl(sum, k, TIE_WAVE);
-  for (int d0 = 0; d0 < Dh; d0 += 4 * TIE_WAVE) {
-    const int d = d0 + 4 * lane;
-    f32x4_t o = {0.f, 0.f, 0.f, 0.f};
-    for (int k = 0; k < nsplit; ++k) {
-      const float f = __shfl(weight, k, TIE_WAVE);
-      if (d < Dh) o += af_load4(part_o + (where * nsplit + k) * Dh + d) * f;
-    }
-    if (d < Dh) *reinterpret_cast<f32x4_t*>(out + where * Dh + d) = o / l;
-  }
+  f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < AHEAD; ++k)
+    if (k < nsplit) o += ahead[k] * __shfl(weight, k, TIE_WAVE);
+#pragma unroll 8
+  for (int k = AHEAD; k < nsplit; ++k) o += af_load4(po + k * Dh) * __shfl(weight, k, TIE_WAVE);
+  if (d < Dh) *reinterpret_cast<f32x4_t*>(out + where * Dh + d) = o / l;
 }
 
 // Column tiles: one a sequence in steps of single tokens, otherwise counted by the caller, who knows the sequences'
@@ -339,7 +359,10 @@ extern "C" int tie_attention_f32(const float* q, const void* k_cache, const void
 #undef LAUNCH
   int status = tie_launch_status();
   if (status != TIE_OK || nsplit == 1) return status;
-  attention_f32_merge_kernel<<<dim3(H, T), TIE_WAVE, 0, stream>>>(part_o, part_ml, out, H, Dh, nsplit, sinks);
+  const dim3 pairs(H, T);
+  if (nsplit <= 4) attention_f32_merge_kernel<4><<<pairs, TIE_WAVE, 0, stream>>>(part_o, part_ml, out, H, Dh, nsplit, sinks);
+  else if (nsplit <= 8) attention_f32_merge_kernel<8><<<pairs, TIE_WAVE, 0, stream>>>(part_o, part_ml, out, H, Dh, nsplit, sinks);
+  else attention_f32_merge_kernel<24><<<pairs, TIE_WAVE, 0, stream>>>(part_o, part_ml, out, H, Dh, nsplit, sinks);
   return tie_launch_status();
 }
 
