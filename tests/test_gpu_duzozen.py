@@ -96,6 +96,34 @@ def test_the_routers_choice(E, groups, keep, top):
     assert ids.cpu().tolist() == chosen.tolist()
 
 
+@pytest.mark.parametrize("E,groups,keep,top,group_top", [(36, 4, 2, 4, 1), (64, 8, 4, 4, 1), (64, 64, 5, 5, 2), (12, 2, 1, 6, 2),
+                                                         (63, 9, 2, 14, 2), (40, 5, 2, 9, 3), (66, 6, 2, 4, 1)])
+@pytest.mark.parametrize("silenced", [False, True])
+def test_the_routers_choice_among_groups_with_ties(E, groups, keep, top, group_top, silenced):
+    """Groups of up to 64 experts are ranked across a wave's lanes; more experts, groups scored by three and choices that
+    are -inf go one by one. Coarse logits make ties, in groups and in experts: the lower index goes first."""
+    from tie_amd import kernels
+
+    T, size = 33, E // groups
+    logits = (rnd(T, E, seed=E + top, scale=2.0) * 2).round() / 2
+    correction = (rnd(E, seed=8) * 0.01).round() * 0.01
+    if silenced:
+        correction[::size * 2] = -math.inf          # one expert of every other group
+    ids, w = torch.empty(T, top, dtype=torch.int32, device="cuda"), torch.empty(T, top, device="cuda")
+    kernels.moe_route(logits.cuda(), correction.cuda(), groups, keep, top, ids, w, scoring="sigmoid", group_top=group_top)
+    kernels_score = 1.0 / (1.0 + torch.exp(-logits.cuda())).cpu()      # equal logits stay equal, different ones apart
+    choice = kernels_score + correction
+    for t in range(T):
+        c = choice[t].tolist()
+        best = [sorted(c[g * size:(g + 1) * size], reverse=True)[:group_top] for g in range(groups)]
+        kept = sorted(range(groups), key=lambda g: (-round(sum(best[g]), 5), g))[:keep]
+        open_to = sorted((e for e in range(E) if e // size in kept), key=lambda e: (-round(c[e], 5), e))[:top]
+        if any(c[e] == -math.inf for e in open_to):
+            continue                                  # fewer experts than are to be chosen
+        assert ids[t].tolist() == open_to, t
+        close(w[t], kernels_score[t, open_to], 1e-6, "weights")
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T,real,identity,top,K,F_", [(1, 4, 0, 2, 32, 16), (7, 6, 2, 3, 64, 24), (150, 5, 3, 2, 96, 48),
                                                      (33, 3, 1, 4, 40, 20), (300, 12, 4, 4, 128, 64), (500, 3, 0, 2, 72, 136),

@@ -70,15 +70,20 @@ __device__ __forceinline__ void wave_order() {
 
 // One row by one wave without groups and with up to 64 PER experts: lane l holds the experts l, l + 64, ..., counts how
 // many stand before each of its own (ties to the lower index), and writes those that `top` or fewer stand before.
-template <int PER>
+// GROUPED (up to 64 experts, an expert a lane; a group's score the sum of its one or two best): a lane finds its group's
+// score among its group's lanes and counts the groups before its own; the experts of other than the `keep` best groups
+// stand behind all others. 8 rows of 36 experts in 4 groups, with the sort behind it: 10.7 us one choice after the other
+// through LDS, 6.6 so. Everything that is read is asked for first.
+template <int PER, bool GROUPED = false>
 __device__ void route_row_ranked(const RouteParams& p, size_t t, int lane, int* ids_lds) {
   const float* z = p.logits + t * p.row;
   const int E = p.E, top = p.top, slots = top + p.shared;
-  float score[PER], choice[PER];
+  float score[PER], choice[PER], corrected[PER];
   float m = -INFINITY;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int e = lane + i * TIE_WAVE;
+    corrected[i] = e < E && p.correction != nullptr ? p.correction[e] : 0.f;
     score[i] = e < E ? z[e] + (p.bias != nullptr ? p.bias[e] : 0.f) : -INFINITY;
     m = fmaxf(m, score[i]);
   }
@@ -101,8 +106,25 @@ __device__ void route_row_ranked(const RouteParams& p, size_t t, int lane, int* 
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int e = lane + i * TIE_WAVE;
-    choice[i] = e < E ? score[i] + (p.correction != nullptr ? p.correction[e] : 0.f) : -INFINITY;
+    choice[i] = e < E ? score[i] + corrected[i] : -INFINITY;
     before[i] = 0;
+  }
+  if constexpr (GROUPED) {
+    static_assert(PER == 1, "an expert a lane");
+    const int size = E / p.groups, g = min(lane / size, p.groups - 1);
+    float best = -INFINITY, second = -INFINITY;
+    for (int j = 0; j < size; ++j) {
+      const float v = __shfl(choice[0], g * size + j, TIE_WAVE);
+      second = fmaxf(second, fminf(best, v));
+      best = fmaxf(best, v);
+    }
+    const float total = p.group_top > 1 && size > 1 ? best + second : best;
+    int groups_before = 0;
+    for (int h = 0; h < p.groups; ++h) {
+      const float v = __shfl(total, h * size, TIE_WAVE);
+      groups_before += (v > total || (v == total && h < g)) ? 1 : 0;
+    }
+    if (groups_before >= p.keep) choice[0] = -INFINITY;
   }
 #pragma unroll
   for (int ib = 0; ib < PER; ++ib) {
@@ -151,6 +173,17 @@ __device__ void route_row(const RouteParams& p, float* lds, size_t t, int lane, 
     else if (p.E <= 2 * TIE_WAVE) route_row_ranked<2>(p, t, lane, ids_lds);
     else route_row_ranked<4>(p, t, lane, ids_lds);
     return;
+  }
+  // With groups: where the kept ones hold enough experts, and no choice is infinite (a -inf would stand among those of the
+  // other groups; a sigmoid's or softmax's score is finite, and a correction that is not is the general way's).
+  if (p.E <= TIE_WAVE && p.shared <= TIE_WAVE && p.scoring != SCORE_LOGIT && p.group_top <= 2 &&
+      p.keep * (p.E / p.groups) >= p.top) {
+    const float own = lane < p.E ? p.logits[t * p.row + lane] + (p.bias != nullptr ? p.bias[lane] : 0.f) +
+                                       (p.correction != nullptr ? p.correction[lane] : 0.f) : 0.f;
+    if (!__any(!(fabsf(own) < INFINITY))) {
+      route_row_ranked<1, true>(p, t, lane, ids_lds);
+      return;
+    }
   }
   const float *logits = p.logits, *bias = p.bias, *correction = p.correction;
   const int row = p.row, E = p.E, groups = p.groups, keep = p.keep, top = p.top, scoring = p.scoring;
