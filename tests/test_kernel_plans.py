@@ -52,6 +52,14 @@ def test_key_shares_never_exceed_what_the_merge_takes():
     # one workgroup on each CU: a second beside it for long contexts that are read, and only for those
     assert [kernels.prefill_splits(32, 8, 2, context, 2048) for context in (1024, 2047, 2048, 16000)] == [1, 1, 2, 2]
     assert kernels.prefill_splits(32, 8, 2, 16000, 2048, 512) == 1 and kernels.prefill_splits(33, 8, 2, 16000, 2112) == 1
+    # beside waves of single rows: never more shares than alone, few workgroups as alone, 64 and more cut for 256 places
+    for items in (1, 4, 8, 16, 40):
+        for context in (64, 500, 1181, 2000, 16000):
+            alone = kernels.prefill_splits(items, 8, 2, context, 64 * items)
+            beside = kernels.prefill_splits(items, 8, 2, context, 64 * items, beside_waves=True)
+            assert 1 <= beside <= alone and (items >= 8 or beside == alone) and (beside == 1 or items * 8 * beside <= 256 or items < 8)
+    assert [kernels.prefill_splits(n, 8, 2, c, 64 * n, beside_waves=True) for n, c in ((8, 1181), (8, 2000), (16, 1000), (8, 500))] \
+        == [2, 4, 2, 2]
 
 
 def test_sizes_no_kernel_takes_are_refused_when_the_model_is_built():

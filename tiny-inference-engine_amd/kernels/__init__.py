@@ -1900,7 +1900,7 @@ def attention_mixed_bf16(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
 
 
 def prefill_splits(num_items: int, num_kv_heads: int, group_size: int, max_context: int, num_rows: int,
-                   reach: Optional[int] = None) -> int:
+                   reach: Optional[int] = None, beside_waves: bool = False) -> int:
     """Shares the keys of every prefill item are cut into: more than one only where the items alone leave CUs idle.
 
     One workgroup on each of the 256 CUs is such a step too where contexts are long: two shares put a second
@@ -1909,13 +1909,22 @@ def prefill_splits(num_items: int, num_kv_heads: int, group_size: int, max_conte
     better whole (29 us, 36), and so are rows that reach no further. Above 256 workgroups nothing is cut: with 288 three
     shares take 180 us for 223 behind 6000 earlier positions and 64 for 59 in a prompt, with 384 up to four shares gain
     6 % or lose 6 %, with 504 two lose 9 to 28 %.
+
+    ``beside_waves``: the launch carries waves of single rows too, which hold a part of the chip and set the launch's time;
+    64 workgroups and more are then cut for 256 places, in shares of about eight tiles (two at least), which is less to
+    write and to merge (31 sequences of up to 1900 keys beside 481 rows behind 700, 16 heads over 8: 4 shares 49 us a layer
+    with the merge, 2 shares 40; beside 1000 rows 4 shares 3 to 7 us more than 2; beside 500 behind 1500 8 shares 2 to 6 us
+    more than 4). With fewer workgroups the portion's chain of tiles is the longer one and is cut as if it were alone.
     """
     passes = -(-group_size // min(group_size, 4))
     workgroups = num_items * num_kv_heads * passes
     if workgroups > 256 or (workgroups == 256 and min(max_context, reach or max_context) < 2048) or num_rows > 65535:
         return 1
     by_fill = 512 // max(1, workgroups)
-    by_length = max(1, -(-max_context // 64) // 4)          # at least four 64-key tiles a share
+    tiles = -(-max_context // 64)
+    by_length = max(1, tiles // 4)          # at least four 64-key tiles a share
+    if beside_waves and workgroups >= 64:
+        by_fill, by_length = 256 // workgroups, min(by_length, max(2, (tiles + 4) // 8))
     return max(1, min(8, by_fill, by_length))
 
 
@@ -2006,7 +2015,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             rows = q.shape[0]
             # by the longest context among the portions themselves: a single row of 32 k keys beside them says nothing
             # about how many tiles a portion's share would hold
-            nsplit = prefill_splits(num_items, KVH, G, items_context, rows, reach)
+            nsplit = prefill_splits(num_items, KVH, G, items_context, rows, reach, together)
             part_o = part_ml = None
             if nsplit > 1:
                 part_o = scratch("attention.prefill_split_o", (rows * num_heads * nsplit * Dh,), torch.float32)
