@@ -207,6 +207,32 @@ def test_qk_norm_rope_rotates_part_of_a_head_and_neighbouring_pairs(H, KVH, Dh, 
             close(kc[slot // bs, :, slot % bs], k_want[t], 2e-6, f"k of token {t}, rotary_dim {rotary_dim}, {pairing}")
 
 
+@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("N,K", [(16, 1024), (2048, 2048), (1040, 3072), (2048, 6144), (512, 5120), (2032, 8192)])
+def test_the_end_of_a_sub_layer_in_workgroups_of_half_a_tile(M, N, K):
+    """Up to eight rows over few columns: 8 columns a workgroup, 32 parts of K; the stream, the next norm's rows and the sums
+    of squares, and the product that applies their factor, against the plain formula. Every batch of k-blocks (1 to 4)."""
+    from tie_amd import kernels
+
+    x, w = rnd(M, K, seed=71).bfloat16(), (rnd(N, K, seed=72) * K ** -0.5).bfloat16()
+    stream, norm_w = rnd(M, N, seed=73), 1 + 0.2 * rnd(N, seed=74)
+    weight = kernels.pack_weight(w.cuda())
+    assert kernels.norm_square_columns(M, weight) == 8 and kernels.norm_square_columns(9, weight) == 16
+    got = stream.clone().cuda()
+    rows = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    squares = torch.full((M, N // 8), float("nan"), device="cuda")
+    kernels.skinny_gemm_bf16(x.cuda(), weight, got, accumulate=True, next_norm=(norm_w.cuda(), rows, squares))
+    want = stream.to(F64) + x.to(F64) @ w.to(F64).T
+    close(got, want, 2e-6, "stream")                      # K float32 sums of bfloat16 products
+    close(rows, want * norm_w, 5e-3, "the next norm's rows")          # bfloat16
+    close(squares, (got.cpu().to(F64) ** 2).view(M, -1, 8).sum(2), 1e-6, "sums of squares")
+    after = (rnd(96, N, seed=75) * N ** -0.5).bfloat16()
+    if N % 32 == 0:
+        out = torch.empty(M, 96, device="cuda")
+        kernels.skinny_gemm_bf16(rows, kernels.pack_weight(after.cuda()), out, row_scale=kernels.RowScale(squares, N, 1e-6))
+        close(out, plain.rms_norm(want, norm_w, 1e-6) @ after.to(F64).T, 5e-3, "the product behind the norm")
+
+
 @pytest.mark.parametrize("planes", [2, 3, 4, 5, 8, 9])
 @pytest.mark.parametrize("T,mix,biased,cache", [(5, None, False, torch.bfloat16), (5, "blend", True, torch.bfloat16),
                                                 (35, "keep", True, torch.bfloat16), (35, "blend", False, torch.bfloat16),

@@ -327,6 +327,89 @@ __global__ __launch_bounds__(WAVES* TIE_WAVE) void skinny_gemm_kernel(const bf16
   }
 }
 
+// ------------------------------------------------------------------ ends of sub-layers over few columns, up to 8 rows
+// A compute unit takes 38 GB/s of cold memory whatever it asks for, and a product of 128 tiles that is not cut along K
+// leaves half of the 256 idle. Here a workgroup owns 8 of a tile's 16 columns and its sixteen waves, each in two halves of
+// lanes, 32 parts of K: lanes 0 .. 7 of a group of 16 hold the eight rows of w (and of x) over one part, lanes 8 .. 15 the
+// same rows over the next, so that one matrix instruction forms both parts' sums in the two 8 x 8 blocks of its diagonal
+// (the other two blocks are products of different parts of K and dropped). A load still brings whole lines: 8 rows of a
+// packed block are 128 consecutive bytes a chunk of k. In chains of a layer's products at 2048 columns: O (K 2048) 4.5 ->
+// 3.9 us, down (K 6144) 9.0 -> 6.9 at one row, 5.1 -> 4.4 and 11.1 -> 8.5 at eight. The parts and halves are added in
+// their order. Sums of squares are left per 8 columns: squares[m][n / 8].
+#define SK_HALF_WAVES 16
+#define SK_HALF_ROWS 8
+
+// U: k-blocks of either half in one batch of loads; steps: k-blocks of a part, a multiple of U.
+template <int U>
+__global__ __launch_bounds__(SK_HALF_WAVES* TIE_WAVE) void skinny_half_tile_kernel(const bf16_t* __restrict__ x,
+                                                                                   const bf16_t* __restrict__ w,
+                                                                                   float* __restrict__ out, int M, int N, int K,
+                                                                                   int steps, SkNorm norm) {
+  __shared__ float red[SK_HALF_WAVES][256];
+  const int lane = threadIdx.x & (TIE_WAVE - 1);
+  const int wave = threadIdx.x / TIE_WAVE;
+  const int row = lane & 7, half = (lane >> 3) & 1, g = lane >> 4;
+  const int n0 = blockIdx.x * 8;
+  // The elements thread e < 64 ends up with: row e / 8, column e % 8. Asked for before the weights (see above).
+  const int m_end = (threadIdx.x & 63) >> 3, n_end = n0 + (threadIdx.x & 7);
+  const bool ends = threadIdx.x < 64 && m_end < M;
+  float stream_now = 0.f, next_weight = 0.f;
+  if (threadIdx.x < 64) {        // one wave; its lanes beyond M read row 0
+    stream_now = out[static_cast<size_t>(ends ? m_end : 0) * N + n_end];
+    next_weight = norm.next_w[n_end];
+  }
+  const int kb = (2 * wave + half) * steps;
+  const bf16_t* wp = w + (static_cast<size_t>(n0 / 16) * (K / 32) + kb) * 512 + (g * 16 + (n0 & 8) + row) * 8;
+  const bool there = row < M;
+  const bf16_t* xp = x + static_cast<size_t>(there ? row : 0) * K + kb * 32 + g * 8;
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  auto load = [&](bf16x8_t (&b)[U], bf16x8_t (&a)[U], int at) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      b[u] = load_weight_frag<true>(wp + static_cast<size_t>(at + u) * 512);
+      const bf16x8_t piece = load_frag(xp + (at + u) * 32);
+      a[u] = there ? piece : zero_frag();
+    }
+  };
+  auto multiply = [&](const bf16x8_t (&b)[U], const bf16x8_t (&a)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u], acc, 0, 0, 0);
+  };
+  bf16x8_t b[U], a[U];
+  load(b, a, 0);
+  for (int at = U; at < steps; at += U) {
+    bf16x8_t nb[U], na[U];
+    load(nb, na, at);
+    multiply(b, a);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      b[u] = nb[u];
+      a[u] = na[u];
+    }
+  }
+  multiply(b, a);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) red[wave][(g * 4 + v) * 16 + (lane & 15)] = acc[v];
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  float sum = 0.f;
+#pragma unroll
+  for (int wv = 0; wv < SK_HALF_WAVES; ++wv) {
+    sum += red[wv][m_end * 16 + (threadIdx.x & 7)];
+    sum += red[wv][(8 + m_end) * 16 + 8 + (threadIdx.x & 7)];
+  }
+  const float now = stream_now + sum;
+  if (ends) {
+    out[static_cast<size_t>(m_end) * N + n_end] = now;
+    norm.next_x[static_cast<size_t>(m_end) * N + n_end] = float_to_bf16(now * next_weight);
+  }
+  float sq = now * now;
+  sq += __shfl_xor(sq, 1, TIE_WAVE);
+  sq += __shfl_xor(sq, 2, TIE_WAVE);
+  sq += __shfl_xor(sq, 4, TIE_WAVE);
+  if (ends && (threadIdx.x & 7) == 0) norm.squares[static_cast<size_t>(m_end) * (N / 8) + blockIdx.x] = sq;
+}
+
 // ------------------------------------------------------------------ 17 to 64 rows: x through LDS
 // With more than one 16-row tile of x the kernel above spends most of its load instructions on x: every
 // weight block of 1 KB needs MT blocks of x, and a compute unit serves a load instruction of a wave in about 65
@@ -670,6 +753,12 @@ extern "C" int tie_skinny_norm_epilogue_rows(int N, int K) {
   return 0;
 }
 
+// Whether such a product of M rows runs in workgroups of half a tile (tie_skinny_gemm_bf16_norm_halves): up to eight rows,
+// where half tiles leave every compute unit at most one workgroup, K in steps of 1024.
+extern "C" int tie_skinny_norm_halves(int M, int N, int K) {
+  return M >= 1 && M <= SK_HALF_ROWS && N % 16 == 0 && N / 8 <= compute_units() && K > 0 && K % 1024 == 0 ? 1 : 0;
+}
+
 // gated: w holds blocks of 16 rows = 8 gate rows then 8 up rows of the same 8 outputs; out has N / 2 columns
 // and receives silu(gate) * up (gated == 1) or gelu_tanh(gate) * up (gated == 2).
 // splits > 1: out is float32 [splits, M, N], plane s holding the sums over the s-th range of K.
@@ -838,7 +927,29 @@ extern "C" int tie_skinny_gemm_bf16_norm(const void* x, const void* w, void* out
   return launch_skinny(x, w, out, out_dtype, accumulate, gated, M, N, K, splits, packed, rt, u, waves, norm, stream);
 }
 
+// The end of a sub-layer in workgroups of half a tile, where tie_skinny_norm_halves says so: packed w, out += sums in
+// place, next_x = bf16(out * next_w), squares[M][N / 8] = sums of out^2 per 8 columns.
+extern "C" int tie_skinny_gemm_bf16_norm_halves(const void* x, const void* w, float* out, int M, int N, int K,
+                                                const float* next_w, void* next_x, float* squares, hipStream_t stream) {
+  if (!tie_skinny_norm_halves(M, N, K) || x == nullptr || w == nullptr || out == nullptr || next_w == nullptr ||
+      next_x == nullptr || squares == nullptr ||
+      (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 != 0)
+    return TIE_BAD_ARGUMENT;
+  const SkNorm norm = {nullptr, 0, 1.f, 0.f, next_w, static_cast<bf16_t*>(next_x), squares};
+  const int steps = K / 1024;               // k-blocks of each of the 32 parts
+#define LAUNCH_HALF(U)                                                                  \
+  skinny_half_tile_kernel<U><<<N / 8, SK_HALF_WAVES * TIE_WAVE, 0, stream>>>(           \
+      static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), out, M, N, K, steps, norm)
+  if (steps % 4 == 0) LAUNCH_HALF(4);
+  else if (steps % 3 == 0) LAUNCH_HALF(3);
+  else if (steps % 2 == 0) LAUNCH_HALF(2);
+  else LAUNCH_HALF(1);
+#undef LAUNCH_HALF
+  return tie_launch_status();
+}
+
 // What a launch list may hold (common.h).
+TIE_LIST_ENTRY(tie_skinny_gemm_bf16_norm_halves)
 TIE_LIST_ENTRY(tie_skinny_gemm_bf16_with)
 TIE_LIST_ENTRY(tie_skinny_gemm_bf16)
 TIE_LIST_ENTRY(tie_skinny_gemm_bf16_norm)

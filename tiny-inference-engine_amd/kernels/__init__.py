@@ -237,6 +237,9 @@ _SIGNATURES = {
         "tie_skinny_gemm_bf16": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                  _c_int, _c_void],
         "tie_skinny_norm_epilogue_rows": [_c_int, _c_int],
+        "tie_skinny_norm_halves": [_c_int, _c_int, _c_int],
+        "tie_skinny_gemm_bf16_norm_halves": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void,
+                                             _c_void],
         "tie_skinny_gemm_bf16_norm": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                       _c_int, _c_void, _c_int, _c_float, _c_float, _c_void, _c_void, _c_void, _c_int,
                                       _c_int, _c_int, _c_void],
@@ -958,7 +961,8 @@ def skinny_gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumu
     a gated product); ``next_norm = (weight [N], next_x bfloat16 [M, N], squares float32 [M, N / 16])`` with
     ``accumulate`` and one plane: out is the residual stream, and beside ``out += x @ w.T`` the epilogue leaves
     ``next_x = bfloat16(out * weight)`` and the sums of ``out ** 2`` per 16-column tile for the norm that follows
-    (a ``RowScale`` for whoever multiplies ``next_x``).
+    (a ``RowScale`` for whoever multiplies ``next_x``). Where ``norm_square_columns`` says 8, squares of that width,
+    ``[M, N / 8]``, have the product run in workgroups of 8 columns.
     """
     if splits > 1:
         if out.dim() != 3 or out.shape[0] != splits or out.dtype != torch.float32 or accumulate or gated:
@@ -989,13 +993,19 @@ def skinny_gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumu
     if next_norm is not None:
         next_w, next_x, squares_out = next_norm
         _f32(next_w, "the next norm's weight", (N,))
-        _f32(squares_out, "sums of squares", (M, N // 16))
+        halves = row_scale is None and not (tiles or loads or waves) and norm_square_columns(M, w) == 8 and \
+            tuple(squares_out.shape) == (M, N // 8)
+        _f32(squares_out, "sums of squares", (M, N // 8) if halves else (M, N // 16))
         _gpu(next_x, "the next norm's rows")
         if splits != 1 or gated or not accumulate or out.dtype != torch.float32 or N % 16 or \
                 next_x.dtype != torch.bfloat16 or tuple(next_x.shape) != (M, N) or not next_x.is_contiguous() or \
                 not squares_out.is_contiguous():
             raise InvalidArgument("a product that prepares the next norm adds to a float32 stream in one plane, is not "
                                   f"gated, and leaves bfloat16 rows [{M}, {N}] (N in steps of 16)")
+        if halves:
+            _call(_lib("skinny_gemm_bf16").tie_skinny_gemm_bf16_norm_halves, "skinny_gemm_bf16_norm", x.data_ptr(), w.data_ptr(),
+                  out.data_ptr(), M, N, K, next_w.data_ptr(), next_x.data_ptr(), squares_out.data_ptr(), _stream())
+            return
     _call(_lib("skinny_gemm_bf16").tie_skinny_gemm_bf16_norm, "skinny_gemm_bf16_norm",
         x.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out, "matmul output"), int(accumulate), int(gated), M, N, K,
         int(splits), int(isinstance(w, PackedWeight)), _ptr(squares_in), tiles_in, n_in, eps_in, _ptr(next_w),
@@ -1085,6 +1095,17 @@ def norm_epilogue_rows(N: int, K: int) -> int:
     with the next norm's work in its epilogue (``skinny_gemm_bf16(next_norm=...)``) rather than as planes that a
     norm kernel adds; 0 where it never is. Never above ``NORM_EPILOGUE_ROWS``."""
     return min(NORM_EPILOGUE_ROWS, int(_lib("skinny_gemm_bf16").tie_skinny_norm_epilogue_rows(N, K)))
+
+
+@functools.lru_cache(maxsize=None)
+def _norm_halves(M: int, N: int, K: int) -> bool:
+    return bool(_lib("skinny_gemm_bf16").tie_skinny_norm_halves(M, N, K))
+
+
+def norm_square_columns(M: int, w) -> int:
+    """Columns that a sum of squares covers where a product of M rows over ``w`` is best run with the next norm's work in
+    its epilogue: 8 where workgroups of half a tile fill the compute units better (``tie_skinny_norm_halves``), else 16."""
+    return 8 if isinstance(w, PackedWeight) and _norm_halves(M, *w.shape) else 16
 
 
 def applies_row_scale(x: torch.Tensor, w) -> bool:

@@ -69,7 +69,8 @@ class RMSNorm(Norm):
             pending = ctx.take_pending_product(x)
             if pending is not None:
                 linear, rows_in = pending
-                squares = ctx.scratch(out_name + ".squares", (count, self.dim // 16), torch.float32)
+                columns = kernels.norm_square_columns(count, linear.weight)
+                squares = ctx.scratch(out_name + ".squares", (count, self.dim // columns), torch.float32)
                 linear.add_to_and_prepare_norm(rows_in, x, self.weight, out, squares)
                 ctx.set_row_scale(out, kernels.RowScale(squares, self.dim, self.eps))
                 return out
