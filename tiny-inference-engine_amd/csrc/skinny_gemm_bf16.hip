@@ -193,43 +193,73 @@ __global__ __launch_bounds__(WAVES* TIE_WAVE) void skinny_gemm_kernel(const bf16
   // Main loop: batches of U blocks. The loads of the next batch are issued before the matrix instructions
   // of the current one, so 2 U blocks of every tile are in flight per wave: a workgroup's share of a narrow
   // weight is a few dozen KB, and it is the bytes in flight, not the instruction rate, that its time hangs on.
+  // Two register sets take turns (a copy from one to the other would wait for its loads), and lanes beyond the
+  // rows read row 0 (loads under a lane's condition would make the compiler wait for all that are in flight; a
+  // row of x reaches its own row of the sums only, and theirs are dropped at the store). 16 rows over 12288 x 2048
+  // gated 12.2 -> 11.4 us, over 4096 x 4096 9.2 -> 8.8, 24 rows 11.3 -> 10.9; others 0 to 3 %. Not in wide workgroups,
+  // which read as much of x as of w: what those lanes bring costs more than the waiting there (12 rows over
+  // 4096 x 12288 22.3 us, and 23.2 with either or both).
   const int batches = (min(kb_end, K / 32) - kb_begin) / U;
   if (batches > 0) {
-    bf16x8_t b[RT][U], a[MT][U];
-    auto load_batch = [&](bf16x8_t (&bb)[RT][U], bf16x8_t (&aa)[MT][U], int at) {
+    bf16x8_t b[2][RT][U], a[2][MT][U];
+    auto load_batch = [&](auto set, int at) {
+      constexpr int S = decltype(set)::value;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int k = (at + u) * 32 + g * 8;
 #pragma unroll
-        for (int t = 0; t < RT; ++t) bb[t][u] = load_weight_frag<PACKED>(wp[t] + static_cast<size_t>(at + u) * KB_STRIDE);
+        for (int t = 0; t < RT; ++t) b[S][t][u] = load_weight_frag<PACKED>(wp[t] + static_cast<size_t>(at + u) * KB_STRIDE);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) aa[mt][u] = xvalid[mt] ? load_frag(xp[mt] + k) : zero_frag();
+        for (int mt = 0; mt < MT; ++mt)
+          a[S][mt][u] = WAVES == SK_WAVES || xvalid[mt] ? load_frag(xp[mt] + k) : zero_frag();
       }
+      if constexpr (WAVES == SK_WAVES) __builtin_amdgcn_sched_barrier(0);      // asked for here, not where they are used
     };
-    auto multiply = [&](const bf16x8_t (&bb)[RT][U], const bf16x8_t (&aa)[MT][U]) {
+    auto multiply = [&](auto set) {
+      constexpr int S = decltype(set)::value;
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int t = 0; t < RT; ++t)
-            acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aa[mt][u], bb[t][u], acc[mt][t], 0, 0, 0);
+            acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[S][mt][u], b[S][t][u], acc[mt][t], 0, 0, 0);
     };
-    load_batch(b, a, kb);
-    for (int i = 1; i < batches; ++i) {
-      bf16x8_t nb[RT][U], na[MT][U];
-      load_batch(nb, na, kb + U);
-      multiply(b, a);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-#pragma unroll
-        for (int t = 0; t < RT; ++t) b[t][u] = nb[t][u];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) a[mt][u] = na[mt][u];
+    constexpr std::integral_constant<int, 0> first{};
+    constexpr std::integral_constant<int, 1> second{};
+    load_batch(first, kb);
+    int i = 1;
+    if constexpr (WAVES == SK_WAVES) {
+      for (; i + 1 < batches; i += 2) {
+        load_batch(second, kb + U);
+        multiply(first);
+        load_batch(first, kb + 2 * U);
+        multiply(second);
+        kb += 2 * U;
       }
-      kb += U;
+      if (i < batches) {
+        load_batch(second, kb + U);
+        multiply(first);
+        multiply(second);
+        kb += U;
+      } else {
+        multiply(first);
+      }
+    } else {
+      for (; i < batches; ++i) {
+        load_batch(second, kb + U);
+        multiply(first);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+          for (int t = 0; t < RT; ++t) b[0][t][u] = b[1][t][u];
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) a[0][mt][u] = a[1][mt][u];
+        }
+        kb += U;
+      }
+      multiply(first);
     }
-    multiply(b, a);
     kb += U;
   }
   // Remainder, one block at a time; the last block may be partly beyond K.
@@ -360,34 +390,40 @@ __global__ __launch_bounds__(SK_HALF_WAVES* TIE_WAVE) void skinny_half_tile_kern
   }
   const int kb = (2 * wave + half) * steps;
   const bf16_t* wp = w + (static_cast<size_t>(n0 / 16) * (K / 32) + kb) * 512 + (g * 16 + (n0 & 8) + row) * 8;
-  const bool there = row < M;
-  const bf16_t* xp = x + static_cast<size_t>(there ? row : 0) * K + kb * 32 + g * 8;
+  const bf16_t* xp = x + static_cast<size_t>(row < M ? row : 0) * K + kb * 32 + g * 8;   // (beyond M: row 0, not stored)
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-  auto load = [&](bf16x8_t (&b)[U], bf16x8_t (&a)[U], int at) {
+  bf16x8_t b[2][U], a[2][U];          // two batches take turns
+  auto load = [&](auto set, int at) {
+    constexpr int S = decltype(set)::value;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      b[u] = load_weight_frag<true>(wp + static_cast<size_t>(at + u) * 512);
-      const bf16x8_t piece = load_frag(xp + (at + u) * 32);
-      a[u] = there ? piece : zero_frag();
+      b[S][u] = load_weight_frag<true>(wp + static_cast<size_t>(at + u) * 512);
+      a[S][u] = load_frag(xp + (at + u) * 32);
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  auto multiply = [&](const bf16x8_t (&b)[U], const bf16x8_t (&a)[U]) {
+  auto multiply = [&](auto set) {
+    constexpr int S = decltype(set)::value;
 #pragma unroll
-    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u], acc, 0, 0, 0);
+    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[S][u], b[S][u], acc, 0, 0, 0);
   };
-  bf16x8_t b[U], a[U];
-  load(b, a, 0);
-  for (int at = U; at < steps; at += U) {
-    bf16x8_t nb[U], na[U];
-    load(nb, na, at);
-    multiply(b, a);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      b[u] = nb[u];
-      a[u] = na[u];
-    }
+  constexpr std::integral_constant<int, 0> first{};
+  constexpr std::integral_constant<int, 1> second{};
+  load(first, 0);
+  int at = U;
+  for (; at + U < steps; at += 2 * U) {
+    load(second, at);
+    multiply(first);
+    load(first, at + U);
+    multiply(second);
   }
-  multiply(b, a);
+  if (at < steps) {
+    load(second, at);
+    multiply(first);
+    multiply(second);
+  } else {
+    multiply(first);
+  }
 #pragma unroll
   for (int v = 0; v < 4; ++v) red[wave][(g * 4 + v) * 16 + (lane & 15)] = acc[v];
   __syncthreads();
