@@ -229,6 +229,30 @@ def test_experts_over_packed_weights(T, E, top, F_, K, kind, tile):
     close(out, want, 2e-2, f"packed experts in tiles of {tile}")
 
 
+@pytest.mark.parametrize("blocks", [3, 4, 5, 8, 9, 12, 15, 16, 21, 24, 25, 28, 29, 32, 33, 37, 45, 53, 64, 70])
+def test_packed_experts_of_few_rows_take_every_batch_of_blocks(blocks):
+    """Four waves take every fourth block of 32 k, 8, 6, 4, 2 or 1 at once: every first batch and what can follow it."""
+    from tie_amd import kernels
+
+    bf, K, N, T, E = torch.bfloat16, 32 * blocks, 112, 5, 3
+    h, w_in, gate = rnd(T, K, seed=1).to(bf), rnd(E, N, K, seed=2, scale=0.1).to(bf), rnd(E, N, K, seed=4, scale=0.1).to(bf)
+    ids = torch.tensor([[0], [2], [0], [2], [0]], dtype=torch.int32)
+    get = scratch_memory()
+    rows = kernels.moe_align(ids.cuda(), E, 16, get)
+    place = rows.where.cpu().view(-1).long()
+    e = ids.view(-1).long()
+    act = get("act", (T, N), bf)
+    packed = kernels.pack_weight(kernels.interleave_gate_up(gate.reshape(E * N, K), w_in.reshape(E * N, K)).cuda())
+    kernels.moe_gate_up(h.cuda(), None, packed, rows, act)
+    a, b = (torch.einsum("tk,tnk->tn", h.to(F64), m[e].to(F64)) for m in (gate, w_in))
+    close(act.cpu()[place], torch.nn.functional.silu(a) * b, 1e-2, "gate and up")     # stored in bfloat16: 2^-9 of each
+    parts = get("parts", (T, N))
+    by_place = torch.empty_like(h)
+    by_place[place] = h
+    kernels.moe_down(by_place.cuda(), kernels.pack_weight(w_in.reshape(E * N, K).cuda()), rows, parts)
+    close(parts.cpu()[place], b, 6e-6, "down")                # exact products, float32 sums of K <= 2240
+
+
 @pytest.mark.parametrize("activation", ["silu", "sigmoid"])
 def test_the_gated_norm_of_the_heads_outputs(activation):
     from tie_amd import kernels

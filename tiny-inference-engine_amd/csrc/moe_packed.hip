@@ -7,7 +7,12 @@
 //
 // Row tiles of 16 (few rows an expert: decode steps): a workgroup takes one row tile and NT block rows; its four waves
 // take every fourth k-block each and add their sums through LDS in wave order. A weight load of a wave is one block, 1 KB
-// of consecutive memory, and DEPTH k-blocks are asked for before the first is used.
+// of consecutive memory, and DEPTH k-blocks are asked for before the first is used. What bounds it at few rows is the chain
+// of lookups in front of the stream of weights (tile, end of the expert's places, slot, x's row): the tile is read
+// together with the count of tiles, and the first weights are asked for before the slot is waited for. Gate and up, down
+// of 32 experts of 768 x 2048, 4 a row: 1 row 7.9 and 4.8 us -> 6.5 and 4.4, 8 rows 26.8 and 13.4 -> 25.7 and 12.2, 32
+// rows 37.4 and 19.5 -> 33.6 and 18.8. Weights before x's rows, all in registers of their own: mixed, the compiler gave
+// them 40 registers in turn and waited in between. Six blocks at once: an inner size of 768 in one trip.
 // Row tiles of 64, 128 or 256 (many rows an expert): the dense product's tile (gemm_dma.h), x's rows gathered by slot on
 // their way into LDS. Which tiles exist is known on the device only; the grid covers the most there can be, and the
 // workgroups that have one are numbered so that each of the 8 XCDs works on a contiguous run of tiles (an expert's row
@@ -31,16 +36,25 @@ __global__ __launch_bounds__(256) void moe_packed_few_rows_kernel(const bf16_t* 
   constexpr bool GATED = MODE == 1 || MODE == 3 || MODE == 4;
   constexpr bool GATHER = MODE != 0;
   const int tile = blockIdx.x;
-  if (tile >= *rw.num_tiles) return;                         // the whole workgroup leaves
+  // The tile comes with the count of tiles, not behind it: the grid covers the table, whose places behind the count hold
+  // nothing that is used.
+  const int tiles = *rw.num_tiles;
+  const int e = rw.tiles[2 * tile], place0 = rw.tiles[2 * tile + 1];
+  asm volatile("" ::"s"(e), "s"(place0));                    // else the compiler moves their loads behind the branch
+  if (tile >= tiles) return;                                 // the whole workgroup leaves
   __shared__ floatx4_t sums[NT][4][TIE_WAVE];
   const int lane = threadIdx.x & (TIE_WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TIE_WAVE);
   const int r16 = lane & 15, quad = lane >> 4;
-  const int e = rw.tiles[2 * tile], place0 = rw.tiles[2 * tile + 1];
   const int rows = min(16, rw.offsets[e + 1] - place0);
   const int place = place0 + (r16 < rows ? r16 : 0);         // rows beyond the tile's end: computed, never stored
-  const size_t src = GATHER ? static_cast<size_t>(rw.slot_at[place] / rw.top) : static_cast<size_t>(place);
-  const bf16_t* xr = x + src * K + quad * 8;
+  const int slot = GATHER ? rw.slot_at[place] : 0;
+  const bf16_t* xr = x;
+  float slot_weight = 1.f;
+  auto look_up = [&]() {                                     // waits for the slot
+    if constexpr (MODE == 4) slot_weight = gp.slot_weights[slot];
+    xr = x + static_cast<size_t>(GATHER ? slot / rw.top : place) * K + quad * 8;
+  };
   const int kblocks = K / 32, block_rows = N / 16;
   const int b0 = blockIdx.y * NT;
   const bf16_t* wr[NT];
@@ -51,15 +65,18 @@ __global__ __launch_bounds__(256) void moe_packed_few_rows_kernel(const bf16_t* 
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) acc[nt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
   int kb = wave;
-  auto blocks = [&](auto depth) {                            // DEPTH of this wave's k-blocks, every load before the first use
+  auto blocks = [&](auto depth, auto first) {                // DEPTH of this wave's k-blocks, every load before the first use
     constexpr int DEPTH = decltype(depth)::value;
     uint4 xf[DEPTH], wf[NT][DEPTH];
 #pragma unroll
-    for (int i = 0; i < DEPTH; ++i) {
-      xf[i] = *reinterpret_cast<const uint4*>(xr + (kb + 4 * i) * 32);
+    for (int i = 0; i < DEPTH; ++i)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) wf[nt][i] = *reinterpret_cast<const uint4*>(wr[nt] + static_cast<size_t>(kb + 4 * i) * 512);
-    }
+    __builtin_amdgcn_sched_barrier(0);                       // the weights are on their way before the slot is waited for
+    if constexpr (decltype(first)::value) look_up();
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) xf[i] = *reinterpret_cast<const uint4*>(xr + (kb + 4 * i) * 32);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i)
 #pragma unroll
@@ -68,10 +85,25 @@ __global__ __launch_bounds__(256) void moe_packed_few_rows_kernel(const bf16_t* 
                                                           *reinterpret_cast<const bf16x8_t*>(&xf[i]), acc[nt], 0, 0, 0);
     kb += 4 * DEPTH;
   };
-  while (kb + 28 < kblocks) blocks(std::integral_constant<int, 8>{});
-  if (kb + 12 < kblocks) blocks(std::integral_constant<int, 4>{});
-  if (kb + 4 < kblocks) blocks(std::integral_constant<int, 2>{});
-  if (kb < kblocks) blocks(std::integral_constant<int, 1>{});
+  constexpr std::true_type first{};
+  constexpr std::false_type later{};
+  if (kb + 28 < kblocks) {
+    blocks(std::integral_constant<int, 8>{}, first);
+    while (kb + 28 < kblocks) blocks(std::integral_constant<int, 8>{}, later);
+  } else if (kb + 20 < kblocks) {
+    blocks(std::integral_constant<int, 6>{}, first);
+  } else if (kb + 12 < kblocks) {
+    blocks(std::integral_constant<int, 4>{}, first);
+  } else if (kb + 4 < kblocks) {
+    blocks(std::integral_constant<int, 2>{}, first);
+  } else {
+    if (kb < kblocks) blocks(std::integral_constant<int, 1>{}, first);
+    else look_up();
+  }
+  if (kb + 20 < kblocks) blocks(std::integral_constant<int, 6>{}, later);
+  if (kb + 12 < kblocks) blocks(std::integral_constant<int, 4>{}, later);
+  if (kb + 4 < kblocks) blocks(std::integral_constant<int, 2>{}, later);
+  if (kb < kblocks) blocks(std::integral_constant<int, 1>{}, later);
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) sums[nt][wave][lane] = acc[nt];
   __syncthreads();
@@ -81,7 +113,7 @@ __global__ __launch_bounds__(256) void moe_packed_few_rows_kernel(const bf16_t* 
     floatx4_t v = sums[nt][0][lane];
 #pragma unroll
     for (int p = 1; p < 4; ++p) v += sums[nt][p][lane];
-    if constexpr (MODE == 4) v *= gp.slot_weights[rw.slot_at[place]];
+    if constexpr (MODE == 4) v *= slot_weight;
     if constexpr (GATED) {
       float u[4];
 #pragma unroll
