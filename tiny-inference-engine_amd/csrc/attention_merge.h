@@ -14,8 +14,9 @@
 //   otherwise  (decode: results kept per sequence of the launch) slot y, output row
 //                                                                query_start[seq_ids ? seq_ids[y] : y].
 // The first AHEAD splits' accumulators are asked for together with the maxima and sums, so that one trip to memory
-// brings all (33 splits of 32 heads: 2.9 -> 1.8 us from the first instruction to the last; the accumulators behind
-// the weights, eight at a time, were two trips more). A workgroup has one thread a dimension, or more threads.
+// brings all; behind the weights, eight at a time, they were two trips more. The weights come out of LDS eight at a time
+// as well: one by one, each waited for, 33 splits of 32 heads took 1 us longer a launch (36 launches of a step, 3036 and
+// 3000 us). A workgroup has one thread a dimension, or more threads.
 template <int AHEAD>
 __global__ __launch_bounds__(256) void attention_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                        bf16_t* __restrict__ out, const int* __restrict__ rows,
@@ -42,20 +43,31 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const float* __res
   const float sink_e = sinks != nullptr ? sinks[h] * TIE_LOG2E : -INFINITY;
   const float m = fmaxf(block_max(mi, scratch), sink_e);
   const float wi = (mi == -INFINITY) ? 0.f : exp2f(mi - m);
-  if (i < nsplit) {
-    weight[i] = wi;
-    weighted_sum[i] = wi * li;
-  }
+  weight[i] = wi;                                          // no weight behind the last split
+  weighted_sum[i] = i < nsplit ? wi * li : 0.f;
   __syncthreads();
+  // Eight at a time, so that their reads from LDS are not waited for one by one: what is behind the last split adds zero.
   float L = 0.f;
-  for (int k = 0; k < nsplit; ++k) L += weighted_sum[k];   // ascending order, the same in every thread
+  for (int k0 = 0; k0 < nsplit; k0 += 8) {                 // ascending order, the same in every thread
+    float part[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) part[k] = weighted_sum[k0 + k];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) L += part[k];
+  }
   if (sinks != nullptr) L += exp2f(sink_e - m);
   // Every accumulator is asked for whatever its weight (they are in flight together); a split without weight is empty
   // and may have written nothing, so what came back for it is not used.
   float o = 0.f;
 #pragma unroll
-  for (int k = 0; k < AHEAD; ++k)
-    if (k < nsplit) o += (weight[k] != 0.f ? ahead[k] : 0.f) * weight[k];
+  for (int k0 = 0; k0 < AHEAD; k0 += 8)
+    if (k0 < nsplit) {
+      float w[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) w[k] = weight[k0 + k];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) o += (w[k] != 0.f ? ahead[k0 + k] : 0.f) * w[k];
+    }
 #pragma unroll 8
   for (int k = AHEAD; k < nsplit; ++k) {
     const float p = po[static_cast<size_t>(k) * DH];
