@@ -177,6 +177,37 @@ def test_experts_over_rows_sorted_on_the_device(dtype, T, real, identity, top, K
     close(x, x_want, tolerance, "experts, normed into the stream")
 
 
+# A row's values in groups of 8 (4 above 4096 wide) planes or parts: fewer, a whole group, one more, a third group.
+@pytest.mark.parametrize("n", [5, 1024, 1029, 2050, 4095, 4100, 8192])
+@pytest.mark.parametrize("terms", [1, 3, 4, 5, 8, 9, 17])
+@pytest.mark.parametrize("kind", ["planes", "parts", "parts of bfloat16 rows, unweighted"])
+def test_a_result_of_many_terms_normed_into_the_stream(n, terms, kind):
+    from tie_amd import kernels
+
+    T = 3
+    w_post, w_next = 1 + 0.2 * rnd(n, seed=1), 1 + 0.2 * rnd(n, seed=2)
+    x = rnd(T, n, seed=3)
+    if kind == "planes":
+        y = rnd(terms, T, n, seed=4)
+        want = y.to(F64).sum(0)
+        y = y.cuda()
+    else:
+        parts, self_rows = rnd(T * terms, n, seed=5), rnd(T, n, seed=6).to(torch.float32 if kind == "parts" else torch.bfloat16)
+        where = torch.arange(T * terms, dtype=torch.int32).flip(0).view(T, terms).contiguous()
+        where[1, terms // 2] = where[2, 0] = -1
+        parts[0] = float("nan")                                      # the place of row 2's last term, which is nobody's
+        where[2, terms - 1] = -1
+        weights = torch.rand(T, terms) if kind == "parts" else torch.ones(T, terms)
+        taken = torch.where(where[..., None] >= 0, parts[where.clamp(min=0).long()].to(F64), self_rows[:, None].to(F64))
+        want = (weights.to(F64)[..., None] * taken).sum(1)
+        y = kernels.RoutedParts(parts.cuda(), where.cuda(), weights.cuda() if kind == "parts" else None, self_rows.cuda())
+    got, out = x.cuda(), torch.full((T, n), float("nan"), device="cuda")
+    kernels.norm_add_norm(y, w_post.cuda(), 1e-5, got, w_next.cuda(), 1e-6, out)
+    x_want = x.to(F64) + plain.rms_norm(want, w_post, 1e-5)
+    close(got, x_want, 3e-6, "the stream")                           # float32 sums of 17 terms and n squares
+    close(out, plain.rms_norm(x_want, w_next, 1e-6), 3e-6, "the next norm")
+
+
 def attention_case(H, G, D, bs, lens_new, lens_ctx, seed, dtype, window, softcap, scale, spike=None):
     """Sequences in scattered pages; returns what the kernels take and the plain result for the new rows."""
     g = torch.Generator().manual_seed(seed)

@@ -71,7 +71,9 @@ __global__ void rms_norm_kernel(const TX* __restrict__ x, const float* __restric
 // Float32 rows of up to four float4 a thread (n % 4 == 0) stay in registers between the sum of
 // squares and the scaling. With COUNT > 0 the row first receives COUNT planes of partial sums
 // (x[r] += p_0[r] + p_1[r] + ..., written back): see the section on partial sums below. All loads
-// of a thread are issued before the first use; the kernel is bound by latency, not by bytes.
+// of a thread are issued before the first use; the kernel is bound by latency, not by bytes. A lane behind the row's end
+// asks for its last float4 again and counts nothing: with the loads behind that condition the compiler waited for all
+// that was asked for in their middle.
 template <typename TO, int COUNT, int V>
 __global__ void rms_norm_row_kernel(float* __restrict__ x, const float* __restrict__ partials, size_t plane_stride,
                                     const float* __restrict__ w, float eps, TO* __restrict__ out,
@@ -82,15 +84,14 @@ __global__ void rms_norm_row_kernel(float* __restrict__ x, const float* __restri
   float4 v[V], p[COUNT > 0 ? COUNT : 1][V], wv[V];
 #pragma unroll
   for (int j = 0; j < V; ++j) {
-    const int i = (threadIdx.x + j * blockDim.x) * 4;
-    const bool in = i < n;
-    v[j] = in ? *reinterpret_cast<const float4*>(x + row + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-    wv[j] = in ? *reinterpret_cast<const float4*>(w + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const int i = min(static_cast<int>(threadIdx.x + j * blockDim.x) * 4, n - 4);
+    v[j] = *reinterpret_cast<const float4*>(x + row + i);
+    wv[j] = *reinterpret_cast<const float4*>(w + i);
 #pragma unroll
     for (int s = 0; s < COUNT; ++s)
-      p[s][j] = in ? *reinterpret_cast<const float4*>(partials + static_cast<size_t>(s) * plane_stride + row + i)
-                   : make_float4(0.f, 0.f, 0.f, 0.f);
+      p[s][j] = *reinterpret_cast<const float4*>(partials + static_cast<size_t>(s) * plane_stride + row + i);
   }
+  __builtin_amdgcn_sched_barrier(0);
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < V; ++j) {
@@ -103,6 +104,7 @@ __global__ void rms_norm_row_kernel(float* __restrict__ x, const float* __restri
     }
     const int i = (threadIdx.x + j * blockDim.x) * 4;
     if (COUNT > 0 && i < n) *reinterpret_cast<float4*>(x + row + i) = v[j];
+    if (i >= n) v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
     ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
   }
   ss = block_sum(ss, scratch);
@@ -1008,34 +1010,85 @@ __global__ void norm_add_norm_kernel(const float* __restrict__ y, size_t plane_s
 }
 
 // The same with a thread's V values of the row in registers from the first load to the last store (n <= V x
-// threads): everything a thread reads - the result's planes or parts, the stream, both norm weights - is asked
-// for before the first sum, so the kernel waits for memory once. Steps of a few rows are bound by exactly that.
+// threads): the stream, both norm weights and up to G of the result's planes or parts are asked for before the first
+// sum, so the kernel waits for memory once, and once more for where the parts are. Steps of a few rows are bound by
+// exactly that. No load is behind a condition that lanes or the number of planes decide (one beyond the row's end or the
+// last plane is the last again): the compiler waited for each of those before it asked for the next.
 template <typename TO, int V>
 __global__ void norm_add_norm_row_kernel(const float* __restrict__ y, size_t plane_stride, int count, RoutedParts rp,
                                          const float* __restrict__ w_post, float eps_post, float* __restrict__ x,
                                          const float* __restrict__ w_next, float eps_next, TO* __restrict__ out,
                                          int n) {
+  constexpr int G = V == 8 ? 4 : 8;
   __shared__ float scratch[16];
   const size_t r = blockIdx.x;
   const size_t row = r * n;
-  float yv[V], xv[V], wp[V], wn[V];
+  float yv[V], xv[V], wp[V], wn[V], part[G][V];
+  int at[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) at[j] = min(static_cast<int>(threadIdx.x + j * blockDim.x), n - 1);
+  const float* next = w_next != nullptr ? w_next : w_post;
 #pragma unroll
   for (int j = 0; j < V; ++j) {
-    const int i = threadIdx.x + j * blockDim.x;
-    yv[j] = xv[j] = wp[j] = wn[j] = 0.f;
-    if (i < n) {
-      xv[j] = x[row + i];
-      wp[j] = w_post[i];
-      if (w_next != nullptr) wn[j] = w_next[i];
-      if (rp.parts != nullptr) {
-        yv[j] = routed_value(rp, r, i, n);
-      } else {
-        float v = y[row + i];
-        for (int s = 1; s < count; ++s) v += y[static_cast<size_t>(s) * plane_stride + row + i];
-        yv[j] = v;
+    xv[j] = x[row + at[j]];
+    wp[j] = w_post[at[j]];
+    wn[j] = next[at[j]];
+    yv[j] = 0.f;
+  }
+  if (rp.parts != nullptr) {
+    const bool self_f32 = rp.self_dtype == TIE_F32;
+    const float* weights = rp.weights != nullptr ? rp.weights : reinterpret_cast<const float*>(rp.where);
+    for (int k0 = 0; k0 < rp.top; k0 += G) {
+      int where[G];
+      float weight[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const size_t k = r * rp.top + min(k0 + g, rp.top - 1);
+        where[g] = rp.where[k];
+        weight[g] = weights[k];
       }
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int j = 0; j < V; ++j) part[g][j] = rp.parts[static_cast<size_t>(max(where[g], 0)) * n + at[j]];
+      uint32_t self[V];                      // as stored
+      if (self_f32) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) self[j] = static_cast<const uint32_t*>(rp.self)[row + at[j]];
+      } else {
+#pragma unroll
+        for (int j = 0; j < V; ++j) self[j] = static_cast<const bf16_t*>(rp.self)[row + at[j]];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        if (k0 + g < rp.top) {
+#pragma unroll
+          for (int j = 0; j < V; ++j) {
+            const float own = __uint_as_float(self_f32 ? self[j] : self[j] << 16);
+            yv[j] = fmaf(rp.weights != nullptr ? weight[g] : 1.f, where[g] >= 0 ? part[g][j] : own, yv[j]);
+          }
+        }
+    }
+  } else {
+    for (int s0 = 0; s0 < count; s0 += G) {
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int j = 0; j < V; ++j)
+          part[g][j] = y[static_cast<size_t>(min(s0 + g, count - 1)) * plane_stride + row + at[j]];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        if (s0 + g < count) {
+#pragma unroll
+          for (int j = 0; j < V; ++j) yv[j] = s0 + g == 0 ? part[g][j] : yv[j] + part[g][j];
+        }
     }
   }
+#pragma unroll
+  for (int j = 0; j < V; ++j)
+    if (static_cast<int>(threadIdx.x + j * blockDim.x) >= n) yv[j] = 0.f;
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < V; ++j) ss += yv[j] * yv[j];

@@ -363,8 +363,8 @@ __global__ __launch_bounds__(WAVES* TIE_WAVE) void skinny_gemm_kernel(const bf16
 // lanes, 32 parts of K: lanes 0 .. 7 of a group of 16 hold the eight rows of w (and of x) over one part, lanes 8 .. 15 the
 // same rows over the next, so that one matrix instruction forms both parts' sums in the two 8 x 8 blocks of its diagonal
 // (the other two blocks are products of different parts of K and dropped). A load still brings whole lines: 8 rows of a
-// packed block are 128 consecutive bytes a chunk of k. In chains of a layer's products at 2048 columns: O (K 2048) 4.5 ->
-// 3.9 us, down (K 6144) 9.0 -> 6.9 at one row, 5.1 -> 4.4 and 11.1 -> 8.5 at eight. The parts and halves are added in
+// packed block are 128 consecutive bytes a chunk of k. In chains of a layer's products at 2048 columns: O (K 2048) 4.4 ->
+// 4.0 us, down (K 6144) 9.0 -> 6.5 at one row, 5.0 -> 4.6 and 11.1 -> 8.7 at eight. The parts and halves are added in
 // their order. Sums of squares are left per 8 columns: squares[m][n / 8].
 #define SK_HALF_WAVES 16
 #define SK_HALF_ROWS 8

@@ -378,8 +378,8 @@ def replay_call(fn, what: str, args) -> None:
 
 
 class LaunchList:
-    """Noted launches as arrays that one native call runs for any number of layers (csrc/launch_list.hip): about 2.5 us a
-    launch where a call from Python takes 4 to 7. ``launches``: ``(fn, what, args, patches)``, a patch being ``(argument,
+    """Noted launches as arrays that one native call runs for any number of layers (csrc/launch_list.hip): about 3.0 us a
+    launch where a call from Python takes 4.2. ``launches``: ``(fn, what, args, patches)``, a patch being ``(argument,
     tensor, offset)``: the argument is the layer's address of that tensor, plus the offset."""
 
     def __init__(self, launches):
