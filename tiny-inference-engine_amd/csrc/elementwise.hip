@@ -601,7 +601,7 @@ __global__ void qk_norm_rope_kv_write_kernel(const TX* qkv, TQ* q_out, const flo
 
 // N elements of the projection, each the sum of its planes: all asked for before the first is added (sums made one
 // after the other, behind a test of the number of planes, were a trip to memory each: 64 rows of an 8B layer 8.4 us,
-// now 5.6). PLANES: 1, 2, 4 or 8, at least as many as there are up to eight; one beyond the last is the last again and
+// now 6.0). PLANES: 1, 2, 4 or 8, at least as many as there are up to eight; one beyond the last is the last again and
 // not added. Planes are added in order.
 template <int N, int PLANES, typename TX>
 struct PlanedElements {

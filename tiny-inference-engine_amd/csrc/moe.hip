@@ -73,7 +73,7 @@ __device__ __forceinline__ void wave_order() {
 // GROUPED (up to 64 experts, an expert a lane; a group's score the sum of its one or two best): a lane finds its group's
 // score among its group's lanes and counts the groups before its own; the experts of other than the `keep` best groups
 // stand behind all others. 8 rows of 36 experts in 4 groups, with the sort behind it: 10.7 us one choice after the other
-// through LDS, 6.6 so. Everything that is read is asked for first.
+// through LDS, 7.6 so. Everything that is read is asked for first.
 template <int PER, bool GROUPED = false>
 __device__ void route_row_ranked(const RouteParams& p, size_t t, int lane, int* ids_lds) {
   const float* z = p.logits + t * p.row;
