@@ -188,6 +188,75 @@ def test_a_launch_list_as_words(monkeypatch):
         kernels.LaunchList([second]).run([[0, 0]])
 
 
+@pytest.mark.parametrize("layers,at_once", [(4, None), (6, None), (7, [2, 2]), (9, [2, 4]), (18, [2, 4, 8, 1])])
+def test_a_launch_list_is_made_for_layers_enough_and_run_a_few_layers_first(monkeypatch, layers, at_once):
+    """Three layers run their own code and show what the others launch. Making a list costs the host more than calls for a
+    few layers do; and a long list is not written down whole before the GPU gets its first layers."""
+    import torch
+
+    from tie_amd import kernels
+
+    model = Model(qwen3_spec(layers))
+    made, ran, called = [], [], []
+
+    class Listed:
+        MIN_LAYERS = kernels.LaunchList.MIN_LAYERS
+
+        @staticmethod
+        def of(launches):
+            made.append(launches)
+            return Listed
+
+        @staticmethod
+        def run(addresses):
+            ran.append([row[0] for row in addresses])
+
+    class Step:
+        device, pending_linear = "cuda", None
+        cache_of = cache_places = staticmethod(lambda index: [])
+
+    class Block:
+        @staticmethod
+        def forward(ctx, x, layer, cache):
+            pass
+
+    class Layer:
+        block = Block
+
+    monkeypatch.setattr(kernels, "LaunchList", Listed)
+    monkeypatch.setattr(kernels, "replay_call", lambda fn, what, args: called.append(args[0]))
+    monkeypatch.setattr(kernels, "start_recording", list)
+    noted = kernels.rms_norm
+    monkeypatch.setattr(Model, "_launch_list", staticmethod(lambda *a: [_launch(noted)]))
+    model.layers = [Layer] * layers
+    model._layer_tensors = {i: [(1000 + i, 1)] for i in range(layers)}
+    model._layer_projections = {i: [] for i in range(layers)}
+    model._run_alike(Step(), torch.zeros(1), 0, layers)
+    rest = [1000 + i for i in range(3, layers)]
+    if at_once is None:
+        assert not made and not ran and called == rest
+    else:
+        assert len(made) == 1 and not called
+        assert [len(part) for part in ran] == at_once and [a for part in ran for a in part] == rest
+
+
+def _launch(fn):
+    from tie_amd.models.builder import _Launch
+
+    return _Launch(fn, "rms_norm", (0,), ((0, 0, 0),))
+
+
+def test_arguments_that_fit_no_word_make_no_launch_list():
+    from tie_amd import kernels
+
+    norm = kernels._lib("elementwise").tie_rms_norm
+    args = (1000, 0, 2000, 1e-6, 3000, 1, None, 4, 256, 7)
+    assert kernels.LaunchList.of([(norm, "rms_norm", args, ())]) is not None
+    for wrong in (args[:7] + (4.0,) + args[8:], args[:3] + ("eps",) + args[4:], args[:3] + (1e39,) + args[4:], args[:-1],
+                  args[:7] + (2 ** 63,) + args[8:]):
+        assert kernels.LaunchList.of([(norm, "rms_norm", wrong, ())]) is None
+
+
 def test_lists_go_to_the_device_together():
     import torch
 

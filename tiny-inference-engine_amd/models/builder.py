@@ -350,12 +350,17 @@ class Model:
             tensors.append(self._entry_tensors(ctx, index, cache, place if carried else None))
             carried = carried and self._pending_place(ctx, index) == place
         launches = self._launch_list(noted[0], noted[1], tensors[0], tensors[1]) if carried else None
-        if launches is not None and torch.device(ctx.device).type == "cuda":
-            listed = [(launch.fn, launch.what, launch.args, launch.patches) for launch in launches]
-            if kernels.LaunchList.takes(listed):
-                kernels.LaunchList(listed).run(
-                    [[address for address, _ in self._entry_tensors(ctx, index, ctx.cache_places(index), place)]
-                     for index in range(start + 3, end)])
+        if launches is not None and end - start - 3 >= kernels.LaunchList.MIN_LAYERS and \
+                torch.device(ctx.device).type == "cuda":
+            listed = kernels.LaunchList.of([(launch.fn, launch.what, launch.args, launch.patches) for launch in launches])
+            if listed is not None:
+                # A few layers first, then more at a time: the GPU works on these while the host writes down the next.
+                first, count = start + 3, 2
+                while first < end:
+                    behind = min(end, first + count)
+                    listed.run([[address for address, _ in self._entry_tensors(ctx, index, ctx.cache_places(index), place)]
+                                for index in range(first, behind)])
+                    first, count = behind, 2 * count
                 self.layers_replayed += end - start - 3
                 if place is not None:
                     ctx.pending_linear = self._layer_projections[end - 1][place]
