@@ -349,6 +349,34 @@ def test_the_decode_products_plan_for_17_to_64_rows():
     assert kernels.gemm_tile(64, 51200, 5120, True, 1) == 8 and kernels.gemm_tile(64, 151936, 4096, True, 1) == 8
 
 
+def test_sequences_of_different_lengths_stay_whole_where_no_compute_unit_waits_for_another():
+    """Waves of whole sequences against shares of one length: by the tiles of the busiest compute unit, for head sizes that
+    were measured, and only where every sequence is one wave's."""
+    import random
+
+    from tie_amd import kernels
+
+    def spread(n, longest):
+        return [max(1, longest // 16 + (longest - longest // 16) * i // (n - 1)) for i in range(n)]
+
+    rng = random.Random(3)
+    at_random = [max(1, int(2500 * rng.random() ** 2)) for _ in range(80)]
+    assert kernels.decode_share_plan(spread(64, 1500), 8, 2048, head_dim=128) == (1, 0)
+    assert kernels.decode_share_plan(spread(32, 500), 16, 1024, head_dim=64) == (1, 0)
+    assert kernels.decode_share_plan([1500] * 20 + [500] * 44, 8, 2048, head_dim=128) == (1, 0)
+    # long sequences that meet on one unit; heads whose waves walk a tile more slowly or were not better; nothing known
+    assert kernels.decode_share_plan(at_random, 8, 4096, head_dim=128)[1] > 0
+    assert kernels.decode_share_plan([2000] * 8 + ([100] * 24 + [2000] * 8) + [100] * 24, 8, 2048, head_dim=128)[1] > 0
+    for head_dim in (0, 16, 32, 256):
+        assert kernels.decode_share_plan(spread(64, 1500), 8, 2048, head_dim=head_dim) == (8, 17)
+    # one wave a unit (256 pairs), and sequences cut into shares of their own: the same plan for every head size
+    for lens, heads in ((spread(32, 3000), 8), (at_random[:56], 8), ([4000] * 14 + [800] * 42, 8), (at_random, 4), (at_random + at_random[:20], 6)):
+        plans = {kernels.decode_share_plan(lens, heads, 4096, head_dim=d) for d in (0, 64, 96, 128, 256)}
+        assert len(plans) == 1 and plans.pop()[1] > 0, (len(lens), heads)
+    # in a window a sequence has no more tiles than the window shows
+    assert kernels.decode_share_plan([100] * 8 + [30000] * 56, 8, 32768, window=1024, head_dim=128) == (1, 0)
+
+
 def test_shares_of_one_length_are_planned_for_sequences_of_very_different_lengths():
     import random
 

@@ -1591,11 +1591,35 @@ BALANCED_SHARES_GRID = 8
 # shorter pays (16 sequences of 8 KV heads, 100 to 4000 keys, 4 shares each: 37.7 us a layer, shares of one
 # length 36.8 to 44.8; one sequence of 32 k keys beside 23 of 1 k: 176 -> 74).
 BALANCED_SHARES_MAX_EQUAL = 3
-TILES_A_WALK = 174       # tiles of 32 keys that a step's waves bring at 4.75 TB/s while one of them walks a tile in 0.6 us
+# Sequences stay whole, lengths however different, where no compute unit has more than this many times the mean number of
+# tiles to bring (``whole_sequences_fill``), for head sizes within these bounds.
+WHOLE_SEQUENCES_BUSIEST = 1.7
+WHOLE_SEQUENCES_HEAD_DIMS = (64, 128)
+COMPUTE_UNITS = 256
+
+
+def whole_sequences_fill(tiles, num_kv_heads: int, head_dim: int) -> bool:
+    """Whether waves that each walk a whole sequence (``tiles`` tiles of 32 keys) of a KV head keep the GPU as busy as
+    shares of one length would.
+
+    From 512 (sequence, KV head) pairs on every compute unit has two waves or more from the start, numbers n, n + 256, ...,
+    and it is what the busiest of them brings that the step waits for, not the longest sequence. Against shares of one
+    length, 97 steps of 512 to 900 pairs, 4, 8 and 16 heads of 64, 96 and 128: with the busiest unit at 1.0 to 1.72 times
+    the mean 0 to 30 % less (64 sequences of 94 to 1500 keys, 1.42: 46.6 and 50.5 us a layer, of 31 to 500 18.0 and 24.0), at
+    1.77 to 1.86 1 % more to 18 % less, from 1.87 on 9 % less to 2.2 times as long (80 of 0 to 2500 at random, 3.19: 90.7 and
+    62.5). Not for heads of 256, whose waves walk a tile four times as slowly (64 of 94 to 1500: 375 and 106), nor of 32 (1.0
+    to 1.42: 14 % more to 20 % less); with 256 pairs there is one wave a unit and nothing to make up for a long one.
+    """
+    low, high = WHOLE_SEQUENCES_HEAD_DIMS
+    if len(tiles) * num_kv_heads < 2 * COMPUTE_UNITS or COMPUTE_UNITS % num_kv_heads or not low <= head_dim <= high:
+        return False
+    apart = COMPUTE_UNITS // num_kv_heads        # sequences that far apart have their waves on the same units
+    busiest = max(sum(tiles[i::apart]) for i in range(apart))
+    return busiest * COMPUTE_UNITS <= WHOLE_SEQUENCES_BUSIEST * num_kv_heads * sum(tiles)
 
 
 def decode_share_plan(context_lens, num_kv_heads: int, plan_context: int, block_size: int = 16,
-                      window: Optional[int] = None) -> "tuple":
+                      window: Optional[int] = None, head_dim: int = 0) -> "tuple":
     """``(shares, share_tiles)`` for a step of single decoded tokens over sequences of these lengths.
 
     ``share_tiles`` = 0: every sequence's keys go into ``shares`` equal parts of its own (``decode_splits``): the
@@ -1610,11 +1634,8 @@ def decode_share_plan(context_lens, num_kv_heads: int, plan_context: int, block_
     grow) is empty (those steps: 68, 62, 43 and 52 us; 64 sequences, 2 of them long: 94 -> 53). Taken only if the
     longest share gets half as long, a quarter where a sequence's own shares are more than three: between that
     and equal the merge and the empty shares cost what the balance gains (56 sequences, a quarter long: 94 -> 109
-    us at two thirds; two of 16 k beside six of 2 k: 56 -> 57 at a third). And only where the longest share is what the
-    step waits for: a wave walks a tile in 0.6 us, in which all together bring ``TILES_A_WALK`` tiles from memory, so a
-    longest share below that part of all tiles ends with the others, and empty shares and the merge are for nothing (64
-    sequences of 94 to 1500 keys 44.2 us as they are and 46 in shares of 17 tiles, of 31 to 500 18.1 and 22; 56, a quarter
-    4000 and the others 800, 69.5 and 71; but 32 of 62 to 1000 21.3 and 20.9, 32, a quarter 4096 beside 1400, 82 and 57).
+    us at two thirds; two of 16 k beside six of 2 k: 56 -> 57 at a third). Where every sequence is one wave's, only if such
+    waves leave the GPU idle (``whole_sequences_fill``; ``head_dim`` 0: not known, the shares of one length are taken).
     """
     S = len(context_lens)
     equal = decode_splits(S, num_kv_heads, plan_context, block_size)
@@ -1628,6 +1649,8 @@ def decode_share_plan(context_lens, num_kv_heads: int, plan_context: int, block_
     longest = max(tiles)
     if longest * S < 1.25 * sum(tiles):
         return equal, 0
+    if equal == 1 and whole_sequences_fill(tiles, num_kv_heads, head_dim):
+        return equal, 0
     pairs = S * num_kv_heads
     target = (512 if pairs <= 128 else 768 if pairs <= 256 else 1024) // num_kv_heads      # waves with keys, a KV head
     if target <= S:
@@ -1640,8 +1663,6 @@ def decode_share_plan(context_lens, num_kv_heads: int, plan_context: int, block_
         else:
             lo = mid + 1
     before = -(-longest // equal)
-    if before * TILES_A_WALK <= num_kv_heads * sum(tiles):
-        return equal, 0
     if (2 * lo > before) if equal <= BALANCED_SHARES_MAX_EQUAL else (4 * lo >= before):
         return equal, 0
     grid = BALANCED_SHARES_GRID
@@ -2031,7 +2052,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             planned = batch.memo.get(shares_key)
             if planned is None:                # this step runs eagerly: the shares' length goes to the device by itself
                 lens = [c for c, n in zip(batch.host_context_lens, batch.host_new_tokens) if n == 1]
-                nsplit, length = decode_share_plan(lens, KVH, batch.plan_context, bs, reach)
+                nsplit, length = decode_share_plan(lens, KVH, batch.plan_context, bs, reach, Dh)
                 if together and not length:
                     keys = min(batch.plan_context, reach or batch.plan_context)
                     nsplit = max(nsplit, min(-(-MIXED_WAVES // (num_single * KVH)), keys // 128, MAX_KEY_SPLITS))
