@@ -349,6 +349,18 @@ def test_the_decode_products_plan_for_17_to_64_rows():
     assert kernels.gemm_tile(64, 51200, 5120, True, 1) == 8 and kernels.gemm_tile(64, 151936, 4096, True, 1) == 8
 
 
+def test_portions_give_way_to_single_rows_that_bring_more():
+    from tie_amd import kernels
+
+    spread = [1900 // 16 + (1900 - 1900 // 16) * i // 30 for i in range(31)]
+    assert kernels.portions_give_way(spread, 8, 1181)
+    assert kernels.portions_give_way(spread, 8, 2048) and not kernels.portions_give_way(spread, 8, 2049)   # late portions
+    assert not kernels.portions_give_way([350] * 28, 8, 1181)          # little to bring
+    assert kernels.portions_give_way([32 * 16] * 32, 8, 700) and not kernels.portions_give_way([32 * 16] * 32, 4, 700)
+    assert not kernels.portions_give_way([32 * 16] * 31 + [32 * 15], 8, 700)
+    assert not kernels.portions_give_way([20000] * 32, 8, 700, reach=480)      # as much as the window shows
+
+
 def test_sequences_of_different_lengths_stay_whole_where_no_compute_unit_waits_for_another():
     """Waves of whole sequences against shares of one length: by the tiles of the busiest compute unit, for head sizes that
     were measured, and only where every sequence is one wave's."""

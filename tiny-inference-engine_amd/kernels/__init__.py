@@ -1963,6 +1963,26 @@ def attention_mixed_bf16(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
           _stream())
 
 
+# Portions beside single rows are cut into fewer shares where the single rows bring at least this many tiles of 32 keys a
+# compute unit and the portions reach no further than so many keys (``portions_give_way``).
+GIVE_WAY_TILES = 16
+GIVE_WAY_CONTEXT = 2048
+
+
+def portions_give_way(single_lens, num_kv_heads: int, items_context: int, reach: Optional[int] = None) -> bool:
+    """Whether it is the single rows of a launch (of these lengths) that set its time, so that the portions beside them
+    (the longest context ``items_context``) are better cut into fewer shares.
+
+    Steps of 8 layers, portions of 260 to 1000 rows behind 200 to 12000, 17 to 60 single rows, 16 and 32 heads of 128 over 8
+    or 4, 32 of 64 over 8. Where both hold, fewer shares are 4.4 % less to 1.4 % more (24 rows of up to 1900 keys beside 481
+    behind 700: 1221 and 1178 us). With less to bring for the single rows up to 4 % more (28 rows of up to 700 keys beside
+    481 behind 700: 1137 and 1165), behind more keys up to 20 % (32 of up to 1900 beside 1000 behind 5000, 32 heads of 64:
+    2152 and 2586; beside 481 behind 12000 1547 and 1821)."""
+    seen = (min(n, reach) if reach else n for n in single_lens)
+    return items_context <= GIVE_WAY_CONTEXT and \
+        num_kv_heads * sum((n - 1) // 32 + 1 for n in seen) >= GIVE_WAY_TILES * COMPUTE_UNITS
+
+
 def prefill_splits(num_items: int, num_kv_heads: int, group_size: int, max_context: int, num_rows: int,
                    reach: Optional[int] = None, beside_waves: bool = False) -> int:
     """Shares the keys of every prefill item are cut into: more than one only where the items alone leave CUs idle.
@@ -1974,11 +1994,12 @@ def prefill_splits(num_items: int, num_kv_heads: int, group_size: int, max_conte
     shares take 180 us for 223 behind 6000 earlier positions and 64 for 59 in a prompt, with 384 up to four shares gain
     6 % or lose 6 %, with 504 two lose 9 to 28 %.
 
-    ``beside_waves``: the launch carries waves of single rows too, which hold a part of the chip and set the launch's time;
-    64 workgroups and more are then cut for 256 places, in shares of about eight tiles (two at least), which is less to
-    write and to merge (31 sequences of up to 1900 keys beside 481 rows behind 700, 16 heads over 8: 4 shares 49 us a layer
-    with the merge, 2 shares 40; beside 1000 rows 4 shares 3 to 7 us more than 2; beside 500 behind 1500 8 shares 2 to 6 us
-    more than 4). With fewer workgroups the portion's chain of tiles is the longer one and is cut as if it were alone.
+    ``beside_waves``: the launch carries waves of single rows too, which hold a part of the chip and set the launch's time
+    (``portions_give_way``); 64 workgroups and more are then cut for 256 places, in shares of about eight tiles (two at
+    least), which is less to write and to merge (31 sequences of up to 1900 keys beside 481 rows behind 700, 16 heads over 8:
+    4 shares 49 us a layer with the merge, 2 shares 40; beside 1000 rows 4 shares 3 to 7 us more than 2; beside 500 behind
+    1500 8 shares 2 to 6 us more than 4). With fewer workgroups the portion's chain of tiles is the longer one and is cut as
+    if it were alone.
     """
     passes = -(-group_size // min(group_size, 4))
     workgroups = num_items * num_kv_heads * passes
@@ -2079,7 +2100,14 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             rows = q.shape[0]
             # by the longest context among the portions themselves: a single row of 32 k keys beside them says nothing
             # about how many tiles a portion's share would hold
-            nsplit = prefill_splits(num_items, KVH, G, items_context, rows, reach, together)
+            give_way = False
+            if together:
+                way_key = ("portions_give_way", KVH, reach, items_context)
+                give_way = batch.memo.get(way_key)
+                if give_way is None:
+                    lens = [c for c, n in zip(batch.host_context_lens, batch.host_new_tokens) if n == 1]
+                    give_way = batch.memo[way_key] = portions_give_way(lens, KVH, items_context, reach)
+            nsplit = prefill_splits(num_items, KVH, G, items_context, rows, reach, give_way)
             part_o = part_ml = None
             if nsplit > 1:
                 part_o = scratch("attention.prefill_split_o", (rows * num_heads * nsplit * Dh,), torch.float32)
