@@ -801,6 +801,47 @@ def test_attention_decode_with_the_newest_token_as_a_share_of_its_own(nsplit, sh
     close(fused, apart, 1e-2, f"{nsplit} shares, {planes} planes")     # probabilities in bfloat16, summed in other orders
 
 
+@pytest.mark.parametrize("S", [32767, 32768, 65535])
+@pytest.mark.parametrize("nsplit,write_kv", [(2, True), (4, True), (2, False), (1, True)])
+def test_attention_decode_prepares_for_as_many_sequences_as_any(S, nsplit, write_kv):
+    """The C interface's limit of 65535 sequences, beyond what the grid holds beside newest tokens that are shares of their
+    own. One cached key and the newest a sequence, one key where the number divides by seven: the softmax by hand."""
+    from tie_amd import kernels
+
+    Dh, bs = 32, 16
+    g = torch.Generator(device="cuda").manual_seed(S)
+    qkv = torch.randn(S, 3 * Dh, generator=g, device="cuda")
+    kc = torch.zeros(S, 1, bs, Dh, dtype=torch.bfloat16, device="cuda")
+    vc = torch.zeros(S, 1, Dh, bs, dtype=torch.bfloat16, device="cuda")
+    kc[:, 0, 0], vc[:, 0, :, 0] = torch.randn(S, Dh, generator=g, device="cuda"), torch.randn(S, Dh, generator=g, device="cuda")
+    at = torch.arange(S, device="cuda")
+    alone = at % 7 == 0
+    context = torch.where(alone, 1, 2).int()
+    tables = torch.randperm(S, generator=g, device="cuda").int()
+    angles = torch.cat([torch.ones(S, Dh // 2), torch.zeros(S, Dh // 2)], 1).cuda()          # no rotation
+    q, k, v = (qkv[:, i * Dh:(i + 1) * Dh].bfloat16().float() for i in range(3))
+    page, newest = tables.long(), (context - 1).long()
+    if not write_kv:
+        kc[page, 0, newest], vc[page, 0, :, newest] = k.bfloat16(), v.bfloat16()
+    old_k, old_v = kc[page, 0, 0].float(), vc[page, 0, :, 0].float()
+    out = torch.full((S, Dh), float("nan"), dtype=torch.bfloat16, device="cuda")
+    part_o = torch.full((S * nsplit * Dh,), float("nan"), device="cuda")
+    part_ml = torch.full((S * nsplit * 2,), float("nan"), device="cuda")
+    start = torch.arange(S + 1, dtype=torch.int32, device="cuda")
+    status = kernels._lib("attention_decode_bf16", Dh).tie_attention_decode_prepared_bf16(
+        qkv.data_ptr(), S * 3 * Dh, 1, 3 * Dh, None, None, 1e-6, angles.data_ptr(), int(write_kv), kc.data_ptr(), vc.data_ptr(),
+        out.data_ptr(), part_o.data_ptr(), part_ml.data_ptr(), start.data_ptr(), context.data_ptr(), tables.data_ptr(), None,
+        S, 1, 1, bs, 1, Dh ** -0.5, 0, nsplit, None, 0, kernels._stream())
+    assert status == 0
+    assert torch.equal(kc[page, 0, newest].float(), k) and torch.equal(vc[page, 0, :, newest].float(), v)
+    weight = torch.softmax(torch.stack([(q * old_k).sum(1), (q * k).sum(1)], 1) * Dh ** -0.5, 1)
+    want = torch.where(alone[:, None], v, weight[:, :1] * old_v + weight[:, 1:] * v)
+    # a probability and the result are rounded to bfloat16's eight bits: 2^-8 each, of the largest value a row is made of
+    # at most (and float32's exponentials and sums, 1e-5)
+    bound = (2 ** -7 + 1e-5) * torch.maximum(old_v.abs(), v.abs()).amax(1, keepdim=True)
+    assert bool(((out.float() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("H,KVH,Dh,bs", [(6, 2, 32, 16), (5, 5, 80, 16), (8, 2, 128, 16), (2, 1, 256, 32), (4, 4, 112, 64)])
 @pytest.mark.parametrize("nsplit,window", [(1, None), (2, None), (5, None), (1, 100), (3, 77)])
 def test_attention_decode_bf16_with_tiles_in_flight(H, KVH, Dh, bs, nsplit, window):

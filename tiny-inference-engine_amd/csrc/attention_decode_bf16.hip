@@ -240,7 +240,7 @@ static int launch_decode(const bf16_t* q, const QkSource* src, bf16_t* k_cache, 
   // kept first positions go beside a window, with uncapped scores and queries that come ready
   if (keep < 0 || (keep > 0 && (window <= 0 || softcap > 0.f || src != nullptr))) return TIE_BAD_ARGUMENT;
   const int column_groups = KVH > 0 ? (H / KVH + 15) / 16 : 1;    // waves of up to 16 query heads a KV head
-  if (num_seqs <= 0 || num_seqs > 65535 || (src != nullptr && num_seqs > 32767) || H <= 0 || KVH <= 0 || KVH * column_groups > 65535 || H % KVH != 0 ||
+  if (num_seqs <= 0 || num_seqs > 65535 || H <= 0 || KVH <= 0 || KVH * column_groups > 65535 || H % KVH != 0 ||
       (src != nullptr && H / KVH > 16) ||
       block_size < 4 || (block_size & (block_size - 1)) != 0 || max_blocks <= 0 || nsplit <= 0 ||
       nsplit > MERGE_MAX_SPLITS || depth < 0 || depth > 4 || (depth > 1 && block_size < 16) ||
@@ -253,10 +253,11 @@ static int launch_decode(const bf16_t* q, const QkSource* src, bf16_t* k_cache, 
   if (src != nullptr && (depth < 2 || !PREPARE_HEAD_DIM)) return TIE_BAD_ARGUMENT;
   if (share_tiles != nullptr && (depth < 2 || nsplit == 1)) return TIE_BAD_ARGUMENT;   // the ring kernel's, with a merge
   const dim3 grid(nsplit, KVH * column_groups, num_seqs);
-  // A prepared step whose newest tokens are shares of their own: the grid holds the other shares, then those.
+  // A prepared step whose newest tokens are shares of their own: the grid holds the other shares, then those, of as many
+  // sequences as fit its third dimension (two places a sequence at most).
   const bool newest_alone = src != nullptr && src->write_kv && nsplit > 1;
   const int tile_shares = newest_alone ? nsplit - 1 : nsplit;      // the ring kernel's `shares`
-  const dim3 prepared_grid(tile_shares, KVH * column_groups, num_seqs + (newest_alone ? (num_seqs + tile_shares - 1) / tile_shares : 0));
+  constexpr int SEQS_AT_ONCE = 32767;
   const int block_shift = __builtin_ctz(block_size);
   const float scale_log2e = scale * 1.44269504088896340736f;
   const float cap = softcap > 0.f ? softcap / scale : 0.f;   // softcap * tanh(scale s / softcap) = scale * cap tanh(s / cap)
@@ -273,7 +274,16 @@ static int launch_decode(const bf16_t* q, const QkSource* src, bf16_t* k_cache, 
       attention_decode_ring_kernel<DEPTH, PREPARE_NOTHING, false><<<grid, TIE_WAVE, 0, stream>>>(RING_ARGS, QkSource{}, 0); \
     } else if constexpr (PREPARE_HEAD_DIM) {                                                                             \
       if (nsplit > 1)                                                                                                    \
-        attention_decode_ring_kernel<DEPTH, PREPARE_SHARES, false><<<prepared_grid, TIE_WAVE, 0, stream>>>(RING_ARGS, *src, 0); \
+        for (int first = 0; first < num_seqs; first += SEQS_AT_ONCE) {                                                   \
+          const int count = num_seqs - first < SEQS_AT_ONCE ? num_seqs - first : SEQS_AT_ONCE, at = seq_ids ? 0 : first; \
+          const size_t slot = static_cast<size_t>(first) * H * nsplit;                                                   \
+          attention_decode_ring_kernel<DEPTH, PREPARE_SHARES, false>                                                     \
+              <<<dim3(tile_shares, KVH, count + (newest_alone ? (count + tile_shares - 1) / tile_shares : 0)), TIE_WAVE, 0, stream>>>( \
+                  query_start + at, context_lens + at, block_tables + static_cast<size_t>(at) * max_blocks,              \
+                  seq_ids ? seq_ids + first : nullptr, max_blocks, count, window, nsplit, H, KVH, q, k_cache, v_cache,   \
+                  out, part_o + slot * DH, part_ml + slot * 2, block_size, block_shift, scale_log2e, cap, sinks,         \
+                  share_tiles, *src, 0);                                                                                 \
+        }                                                                                                                \
       else                                                                                                               \
         attention_decode_ring_kernel<DEPTH, PREPARE_WHOLE, false><<<grid, TIE_WAVE, 0, stream>>>(RING_ARGS, *src, 0);    \
     }                                                                                                                    \
