@@ -761,15 +761,27 @@ def test_attention_decode_with_the_newest_token_as_a_share_of_its_own(nsplit, sh
     """A prepared step cut into shares gives the newest token one of its own; alone (one share) a wave takes it behind its
     tiles. Any number of planes, page tables longer than the 256 entries a wave keeps of them (8300 and 4200 keys in pages
     of 16), shares without keys, and a cache that holds the token already, against the q/k kernel and the decode
-    attention that looks its pages up per lane."""
+    attention that looks its pages up per lane, and against the formula in 64 bits.
+
+    Of the long sequences the first query head of a KV head finds a number of keys that outweigh all others together, the
+    same for each: the newest token, the first and last key of every share, those on either side of entry 256 of the page
+    table, of the window's start (outside it: not seen) and of the sequence. Each has a dimension of the values to itself, so
+    that any of them left out, counted twice or taken from another page shows as a whole, not as one of thousands."""
     from tie_amd import kernels
 
     H, KVH, Dh = 8, 2, 128
+    group = H // KVH
     lens = [1, 33, 4096, 4200, 8300]
     case, S = attention_case(H, KVH, Dh, bs, lens_new=[1] * len(lens), lens_ctx=lens, seed=47, dtype=torch.bfloat16,
                              window=window)
     width = (H + 2 * KVH) * Dh
+    long = [s for s, c in enumerate(lens) if c > 1000]
     qkv = (rnd(planes, S, width, seed=48) / planes).cuda()
+    heads = qkv.view(planes, S, H + 2 * KVH, Dh)
+    for s in long:                      # the newest key is what that head looks for, its value has the last dimension
+        heads[:, s, H:H + KVH] = heads[:, s, 0:H:group]
+        heads[:, s, H + KVH:] = 0
+        heads[0, s, H + KVH:, Dh - 1] = 20.0
     weight = (1 + 0.1 * rnd(Dh, seed=49)).cuda()
     inv_freq = torch.from_numpy(plain.rope_inv_freq(1e4, Dh)).float().cuda()
     positions = i32([c - 1 for c in lens])
@@ -786,10 +798,30 @@ def test_attention_decode_with_the_newest_token_as_a_share_of_its_own(nsplit, sh
         block_tables = tables
         key_shares = (nsplit, i32([share_tiles]) if share_tiles else None)
 
+    def prepare(kc, vc):
+        q = torch.empty(S, H * Dh, dtype=torch.bfloat16, device="cuda")
+        kernels.qk_norm_rope_kv_write(qkv[0], q, weight, weight, 1e-5, inv_freq, positions, slots, kc, vc, H, KVH, Dh, bs,
+                                      planes=planes, plane_stride=S * width, angles=angles)
+        return q
+
+    sought = prepare(case["kc"].clone(), case["vc"].clone()).view(S, H, Dh)[:, ::group]
+    for s in long:
+        c = lens[s]
+        first, tiles = (max(0, c - window) // 32 if window else 0), (c - 1) // 32 + 1
+        length = max(-(-(tiles - first) // nsplit), share_tiles)
+        begins = [32 * t for t in range(first, tiles, length)]
+        places = begins + [256 * bs - 1, 256 * bs, 0, c - 2] + ([c - window - 1, c - window] if window else []) + \
+            [b - 1 for b in begins[1:50]]
+        places = [p for p in dict.fromkeys(places) if 0 <= p < c - 1]
+        assert len(places) < Dh
+        for dim, p in enumerate(places):
+            page = int(tables[s, p // bs])
+            case["kc"][page, :, p % bs] = sought[s]
+            case["vc"][page, :, :, p % bs] = 0
+            case["vc"][page, :, dim, p % bs] = 20.0
+
     kc1, vc1 = case["kc"].clone(), case["vc"].clone()
-    q = torch.empty(S, H * Dh, dtype=torch.bfloat16, device="cuda")
-    kernels.qk_norm_rope_kv_write(qkv[0], q, weight, weight, 1e-5, inv_freq, positions, slots, kc1, vc1, H, KVH, Dh, bs,
-                                  planes=planes, plane_stride=S * width, angles=angles)
+    q = prepare(kc1, vc1)
     apart = torch.full_like(q, float("nan"))
     kernels.attention_decode_bf16(q, kc1, vc1, apart, case["query_start"], case["context_lens"], tables, S, H, Dh ** -0.5,
                                   window, 1, depth=1)
@@ -799,6 +831,15 @@ def test_attention_decode_with_the_newest_token_as_a_share_of_its_own(nsplit, sh
                                      window, lambda name, shape, dtype: torch.full(shape, float("nan"), dtype=dtype, device="cuda"))
     assert torch.equal(kc2, kc1) and torch.equal(vc2, vc1), "the newest keys or values differ"
     close(fused, apart, 1e-2, f"{nsplit} shares, {planes} planes")     # probabilities in bfloat16, summed in other orders
+    for s, c in enumerate(lens):
+        lo = max(0, c - window) if window else 0
+        at = torch.arange(lo, c, device="cuda")
+        pages = tables[s, at // bs].long()
+        keys, values = (x.to(F64).repeat_interleave(group, 1) for x in (kc1[pages, :, at % bs], vc1[pages, :, :, at % bs]))
+        scores = (keys * q[s].view(1, H, Dh).to(F64)).sum(2) * Dh ** -0.5
+        want = (torch.softmax(scores, 0)[..., None] * values).sum(0)
+        for h in range(H):       # each by its own largest value: probabilities and results in bfloat16, 2^-8 each
+            close(fused.view(S, H, Dh)[s, h], want[h], 1e-2, f"{nsplit} shares, {c} keys, head {h}")
 
 
 @pytest.mark.parametrize("S", [32767, 32768, 65535])
