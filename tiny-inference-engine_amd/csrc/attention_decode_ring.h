@@ -335,6 +335,12 @@ __device__ __forceinline__ void attention_decode_newest(
     store_share(acc, m, l, nullptr, part_o, part_ml, t, place, head0 + col, H, quad, nsplit, nsplit - 1, scale_log2e, nullptr);
 }
 
+// What the wave's lanes have read from and written to LDS so far comes before what follows, for the compiler as well.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // One wave: share `share` of `shares` of the keys, (KV head, group of 16 heads) `unit`, sequence `place` of the launch.
 // nsplit: the shares the merge takes, one more than `shares` where the newest token is one of its own. table_lds:
 // TABLE_AHEAD ints of LDS, the wave's own; q_lds (16 DH) and newest_lds (2 DH) only where it prepares.
@@ -365,9 +371,12 @@ __device__ __forceinline__ void attention_decode_ring_wave(
   const int* table = block_tables + static_cast<size_t>(s) * max_blocks;
   // The wave's copy of the page table: entries table_first .. + TABLE_AHEAD - 1, moved on where a share goes further.
   int table_first = 0, table_ahead[TABLE_AHEAD / TIE_WAVE];
+  // (lanes read what other lanes wrote: the hardware keeps the order of a wave's LDS accesses, the fences have the compiler
+  // keep it too, here and where the copy moves on; they wait for nothing)
   auto keep_table = [&] {
 #pragma unroll
     for (int j = 0; j < TABLE_AHEAD / TIE_WAVE; ++j) table_lds[j * TIE_WAVE + lane] = table_ahead[j];
+    wave_lds_order();
   };
 #pragma unroll
   for (int j = 0; j < TABLE_AHEAD / TIE_WAVE; ++j) table_ahead[j] = table[min(j * TIE_WAVE + lane, max_blocks - 1)];
@@ -423,6 +432,7 @@ __device__ __forceinline__ void attention_decode_ring_wave(
 #pragma unroll
     for (int j = 0; j < TABLE_AHEAD / TIE_WAVE; ++j)
       table_ahead[j] = table[min(table_first + j * TIE_WAVE + lane, max_blocks - 1)];
+    wave_lds_order();
     keep_table();
   };
   auto page_of = [&](int entry) { return __builtin_amdgcn_readfirstlane(table_lds[entry - table_first]); };
