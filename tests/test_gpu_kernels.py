@@ -233,6 +233,36 @@ def test_the_end_of_a_sub_layer_in_workgroups_of_half_a_tile(M, N, K):
         close(out, plain.rms_norm(want, norm_w, 1e-6) @ after.to(F64).T, 5e-3, "the product behind the norm")
 
 
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("K", [2048, 8064, 8192, 8448])
+@pytest.mark.parametrize("tiles", [1, 2, 3, 4])
+def test_products_of_few_rows_in_either_loop(tiles, K, packed):
+    """Two register sets that take turns, or one batch copied over the other: by the rows (16, 24), the weight's tiles a
+    workgroup and the length of a wave's walk (64 blocks of 32 k: K of 8192). A row's sums are formed in the same order in
+    either, so they are the same bits whatever rows are beside it; against 64 bits too."""
+    from tie_amd import kernels
+
+    N = 208                                        # 13 tiles: the last workgroup has fewer
+    x, w = rnd(33, K, seed=81).bfloat16().cuda(), (rnd(N, K, seed=82) * K ** -0.5).bfloat16().cuda()
+    x[7] = float("nan")                            # stays in its row
+    weight = kernels.pack_weight(w).blocks if packed else w
+    launch = kernels._lib("skinny_gemm_bf16").tie_skinny_gemm_bf16_with
+    base = rnd(33, N, seed=83).cuda()
+    got = {}
+    for M in (1, 8, 15, 16, 17, 24, 25, 32, 33):
+        out = base[:M].clone()
+        assert launch(x.data_ptr(), weight.data_ptr(), out.data_ptr(), kernels.F32, 1, 0, M, N, K, 1, int(packed), tiles, -1,
+                      kernels._stream()) == 0
+        got[M] = out
+    whole = got[33]
+    for M, out in got.items():
+        rows = [m for m in range(M) if m != 7]
+        assert torch.equal(out[rows], whole[rows]), f"{M} rows beside each other"
+        assert M <= 7 or bool(out[7].isnan().all())
+    rows = [m for m in range(33) if m != 7]
+    close(whole[rows], (base.to(F64) + x.to(F64) @ w.to(F64).T)[rows], 2e-6, "sums")       # float32 sums of bfloat16 products
+
+
 @pytest.mark.parametrize("planes", [2, 3, 4, 5, 8, 9])
 @pytest.mark.parametrize("T,mix,biased,cache", [(5, None, False, torch.bfloat16), (5, "blend", True, torch.bfloat16),
                                                 (35, "keep", True, torch.bfloat16), (35, "blend", False, torch.bfloat16),

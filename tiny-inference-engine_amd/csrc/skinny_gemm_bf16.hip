@@ -109,8 +109,9 @@ __device__ __forceinline__ float sum_of_16_lanes(float v) {
 // launches whose sums are to be scaled (SkNorm::scale_squares).
 extern __shared__ float sk_scale_parts[];
 
-// MT: 16-row tiles of x; RT: 16-row tiles of w per workgroup; U: k-blocks of 32 in one batch of loads.
-template <int MT, int RT, int U, typename TO, bool PACKED, int WAVES = SK_WAVES>
+// MT: 16-row tiles of x; RT: 16-row tiles of w per workgroup; U: k-blocks of 32 in one batch of loads; TURNS: two batches
+// take turns in register sets of their own (four waves).
+template <int MT, int RT, int U, typename TO, bool PACKED, bool TURNS, int WAVES = SK_WAVES>
 __global__ __launch_bounds__(WAVES* TIE_WAVE) void skinny_gemm_kernel(const bf16_t* __restrict__ x,
                                                                          const bf16_t* __restrict__ w,
                                                                          TO* __restrict__ out, int M, int N, int K,
@@ -193,43 +194,44 @@ __global__ __launch_bounds__(WAVES* TIE_WAVE) void skinny_gemm_kernel(const bf16
   // Main loop: batches of U blocks. The loads of the next batch are issued before the matrix instructions
   // of the current one, so 2 U blocks of every tile are in flight per wave: a workgroup's share of a narrow
   // weight is a few dozen KB, and it is the bytes in flight, not the instruction rate, that its time hangs on.
-  // Two register sets take turns (a copy from one to the other would wait for its loads), and lanes beyond the
-  // rows read row 0 (loads under a lane's condition would make the compiler wait for all that are in flight; a
-  // row of x reaches its own row of the sums only, and theirs are dropped at the store). 16 rows over 12288 x 2048
-  // gated 12.2 -> 11.4 us, over 4096 x 4096 9.2 -> 8.8, 24 rows 11.3 -> 10.9; others 0 to 3 %. Not in wide workgroups,
-  // which read as much of x as of w: what those lanes bring costs more than the waiting there (12 rows over
-  // 4096 x 12288 22.3 us, and 23.2 with either or both).
+  // In workgroups of four waves, lanes beyond the rows read row 0 (loads under a lane's condition would make the compiler
+  // wait for all that are in flight; a row of x reaches its own row of the sums only, and theirs are dropped at the
+  // store). TURNS: two register sets take turns; else the next batch is copied over the current one, which waits for its
+  // loads (skinny_takes_turns says where that is the better one). Not so in wide workgroups, which read as much of x as
+  // of w: what those lanes bring costs more than the waiting there (12 rows over 4096 x 12288 22.3 us, and 23.2 with
+  // either or both).
   const int batches = (min(kb_end, K / 32) - kb_begin) / U;
   if (batches > 0) {
-    bf16x8_t b[2][RT][U], a[2][MT][U];
-    auto load_batch = [&](auto set, int at) {
-      constexpr int S = decltype(set)::value;
+    // (The two ways are written out apart: with one pair of functions over arrays given by reference the compiler's order of
+    // the turns was 0.5 to 0.9 % slower at up to 8 rows.)
+    if constexpr (TURNS) {
+      bf16x8_t b[2][RT][U], a[2][MT][U];
+      auto load_batch = [&](auto set, int at) {
+        constexpr int S = decltype(set)::value;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int k = (at + u) * 32 + g * 8;
+        for (int u = 0; u < U; ++u) {
+          const int k = (at + u) * 32 + g * 8;
 #pragma unroll
-        for (int t = 0; t < RT; ++t) b[S][t][u] = load_weight_frag<PACKED>(wp[t] + static_cast<size_t>(at + u) * KB_STRIDE);
+          for (int t = 0; t < RT; ++t) b[S][t][u] = load_weight_frag<PACKED>(wp[t] + static_cast<size_t>(at + u) * KB_STRIDE);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          a[S][mt][u] = WAVES == SK_WAVES || xvalid[mt] ? load_frag(xp[mt] + k) : zero_frag();
-      }
-      if constexpr (WAVES == SK_WAVES) __builtin_amdgcn_sched_barrier(0);      // asked for here, not where they are used
-    };
-    auto multiply = [&](auto set) {
-      constexpr int S = decltype(set)::value;
+          for (int mt = 0; mt < MT; ++mt) a[S][mt][u] = load_frag(xp[mt] + k);
+        }
+        __builtin_amdgcn_sched_barrier(0);      // asked for here, not where they are used
+      };
+      auto multiply = [&](auto set) {
+        constexpr int S = decltype(set)::value;
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+          for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-          for (int t = 0; t < RT; ++t)
-            acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[S][mt][u], b[S][t][u], acc[mt][t], 0, 0, 0);
-    };
-    constexpr std::integral_constant<int, 0> first{};
-    constexpr std::integral_constant<int, 1> second{};
-    load_batch(first, kb);
-    int i = 1;
-    if constexpr (WAVES == SK_WAVES) {
+            for (int t = 0; t < RT; ++t)
+              acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[S][mt][u], b[S][t][u], acc[mt][t], 0, 0, 0);
+      };
+      constexpr std::integral_constant<int, 0> first{};
+      constexpr std::integral_constant<int, 1> second{};
+      load_batch(first, kb);
+      int i = 1;
       for (; i + 1 < batches; i += 2) {
         load_batch(second, kb + U);
         multiply(first);
@@ -246,19 +248,42 @@ __global__ __launch_bounds__(WAVES* TIE_WAVE) void skinny_gemm_kernel(const bf16
         multiply(first);
       }
     } else {
-      for (; i < batches; ++i) {
-        load_batch(second, kb + U);
-        multiply(first);
+      bf16x8_t b[RT][U], a[MT][U];
+      auto load_batch = [&](bf16x8_t (&bb)[RT][U], bf16x8_t (&aa)[MT][U], int at) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int k = (at + u) * 32 + g * 8;
+#pragma unroll
+          for (int t = 0; t < RT; ++t) bb[t][u] = load_weight_frag<PACKED>(wp[t] + static_cast<size_t>(at + u) * KB_STRIDE);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) aa[mt][u] = WAVES == SK_WAVES || xvalid[mt] ? load_frag(xp[mt] + k) : zero_frag();
+        }
+        if constexpr (WAVES == SK_WAVES) __builtin_amdgcn_sched_barrier(0);
+      };
+      auto multiply = [&](const bf16x8_t (&bb)[RT][U], const bf16x8_t (&aa)[MT][U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+              acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aa[mt][u], bb[t][u], acc[mt][t], 0, 0, 0);
+      };
+      load_batch(b, a, kb);
+      for (int i = 1; i < batches; ++i) {
+        bf16x8_t nb[RT][U], na[MT][U];
+        load_batch(nb, na, kb + U);
+        multiply(b, a);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
-          for (int t = 0; t < RT; ++t) b[0][t][u] = b[1][t][u];
+          for (int t = 0; t < RT; ++t) b[t][u] = nb[t][u];
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) a[0][mt][u] = a[1][mt][u];
+          for (int mt = 0; mt < MT; ++mt) a[mt][u] = na[mt][u];
         }
         kb += U;
       }
-      multiply(first);
+      multiply(b, a);
     }
     kb += U;
   }
@@ -684,6 +709,22 @@ static int choose_rt(int M, int N, int splits) {
   return best;
 }
 
+// Whether the kernel that reads x from memory (four waves) keeps two batches of loads in register sets that take turns,
+// or copies the next batch over the current one, which waits for it. The sums are the same. Against copies with loads
+// under a lane's condition, which stood here before, over 17 shapes of 1024 to 51200 rows of w (w cold, whole K or planes):
+//   up to 16 rows, one weight tile a workgroup 0 to 39 % less with turns (2560 x 9728 whole, one row: 39; but 3 to 4 % more
+//     for one row over 5120 x 17408 and 25600 whole), three or four 2 to 12 % less (10240 x 5120, 8 rows: 11.5, with
+//     copies 4);
+//   up to 16 rows, two weight tiles: with turns up to 9 % more where a wave walks far (5120 x 25600 whole, 16 rows 59.3 ->
+//     64.4 us), with copies 2 to 7 % less;
+//   17 to 24 rows (the second tile of rows mostly empty): with turns 4 to 12 % less (2048 x 6144 whole, 20 rows: 10), but
+//     6 % more from walks of 64 k-blocks a wave on (5120 x 25600 whole 66.0 -> 69.8), where copies take 6 % less;
+//   25 to 64 rows: with turns up to 10 % more (5120 x 25600 whole, 32 rows 80.0 -> 87.9), with copies 0 to 10 % less.
+static bool skinny_takes_turns(int M, int rt, int per_wave) {
+  if (M <= 16) return rt != 2;
+  return M <= 24 && per_wave < 64;
+}
+
 // Which kernel, how many weight tiles a workgroup and how many ranges of K a product of 17 to 64 rows takes
 // (up to 16 rows: the kernel that reads x from memory, choose_rt and tie_skinny_gemm_splits). One score for
 // every candidate, the smallest wins:
@@ -874,7 +915,7 @@ static int launch_skinny(const void* x, const void* w, void* out, int out_dtype,
     const dim3 wgrid(((N + 15) / 16 + rt - 1) / rt, 1);
     if (u == 0) u = waves == 8 ? 8 / rt : 4;
 #define LAUNCH_W(RT, U, W)                                                                                      \
-  skinny_gemm_kernel<1, RT, U, float, true, W><<<wgrid, W * TIE_WAVE, scale_lds, stream>>>(                     \
+  skinny_gemm_kernel<1, RT, U, float, true, false, W><<<wgrid, W * TIE_WAVE, scale_lds, stream>>>(                     \
       static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), static_cast<float*>(out), M, N, K, accumulate, \
       gated, per_wave, norm)
     if (rt == 1 && waves == 8 && u == 8) LAUNCH_W(1, 8, 8);
@@ -904,14 +945,21 @@ static int launch_skinny(const void* x, const void* w, void* out, int out_dtype,
       for (u = most; u > 2 && 2 * u > per_wave; u /= 2) {}
   }
   if (u != 2 && u != 4 && u != 8) return TIE_BAD_ARGUMENT;
-#define LAUNCH_P(MT, RT, U, TO, P)                                                                           \
-  skinny_gemm_kernel<MT, RT, U, TO, P><<<grid, SK_WAVES * TIE_WAVE, scale_lds, stream>>>(                     \
+  // (with one or four tiles of rows the rule asks for the weight's tiles alone, so only two tiles have both kernels)
+  const bool turns = skinny_takes_turns(M, rt, per_wave);
+#define LAUNCH_T(MT, RT, U, TO, P, TURNS)                                                                     \
+  skinny_gemm_kernel<MT, RT, U, TO, P, TURNS><<<grid, SK_WAVES * TIE_WAVE, scale_lds, stream>>>(              \
       static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), static_cast<TO*>(out), M, N, K, accumulate, \
       gated, per_wave, norm)
+#define LAUNCH_P(MT, RT, U, TO, P)                                                     \
+  {                                                                                    \
+    if (MT == 2 && turns) LAUNCH_T(MT, RT, U, TO, P, MT == 2 || (MT == 1 && RT != 2)); \
+    else LAUNCH_T(MT, RT, U, TO, P, MT == 1 && RT != 2);                               \
+  }
 #define LAUNCH(MT, RT, U, TO)                  \
   {                                            \
-    if (packed) LAUNCH_P(MT, RT, U, TO, true); \
-    else LAUNCH_P(MT, RT, U, TO, false);       \
+    if (packed) LAUNCH_P(MT, RT, U, TO, true)  \
+    else LAUNCH_P(MT, RT, U, TO, false)        \
   }
 #define LAUNCH_U(MT, RT, TO)                               \
   if (u == 2) LAUNCH(MT, RT, 2, TO)                        \
@@ -934,6 +982,7 @@ static int launch_skinny(const void* x, const void* w, void* out, int out_dtype,
 #undef LAUNCH_U
 #undef LAUNCH
 #undef LAUNCH_P
+#undef LAUNCH_T
   return tie_launch_status();
 }
 
