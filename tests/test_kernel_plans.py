@@ -376,7 +376,7 @@ def test_sequences_of_different_lengths_stay_whole_where_no_compute_unit_waits_f
     assert kernels.decode_share_plan(spread(64, 1500), 8, 2048, head_dim=128) == (1, 0)
     assert kernels.decode_share_plan(spread(32, 500), 16, 1024, head_dim=64) == (1, 0)
     assert kernels.decode_share_plan([1500] * 20 + [500] * 44, 8, 2048, head_dim=128) == (1, 0)
-    # long sequences that meet on one unit; heads whose waves walk a tile more slowly or were not better; nothing known
+    # long sequences that meet on one unit; heads that were not better or not searched; nothing known
     assert kernels.decode_share_plan(at_random, 8, 4096, head_dim=128)[1] > 0
     assert kernels.decode_share_plan([2000] * 8 + ([100] * 24 + [2000] * 8) + [100] * 24, 8, 2048, head_dim=128)[1] > 0
     for head_dim in (0, 16, 32, 256):

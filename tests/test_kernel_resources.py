@@ -15,9 +15,9 @@ if not READELF.exists():
     READELF = pathlib.Path("/opt/rocm/llvm/bin/llvm-readelf")
 
 
-def scratch_bytes(tmp_path, name, source):
+def scratch_bytes(tmp_path, name, source, defines=None):
     """Bytes of scratch a lane of every kernel of that library, by its mangled name."""
-    data = build.compile_library(name, source).read_bytes()
+    data = build.compile_library(name, source, defines).read_bytes()
     found, at = {}, 1
     while (at := data.find(b"\x7fELF", at)) > 0:
         if data[at + 18:at + 20] != b"\xe0\x00":          # not a GPU's code object
@@ -47,3 +47,13 @@ def test_kernels_without_scratch(tmp_path, name, source, kernels, count):
     scratch = {k: v for k, v in scratch_bytes(tmp_path, name, source).items() if re.search(kernels, k)}
     assert len(scratch) == count
     assert not [k for k, v in scratch.items() if v]
+
+
+@pytest.mark.skipif(not READELF.exists(), reason="no llvm-readelf here")
+@pytest.mark.parametrize("head_dim", [16, 64, 128, 256])
+def test_the_ring_of_tiles_fits_the_registers(tmp_path, head_dim):
+    """Decode attention holds tiles of keys in register sets that are loaded far ahead: as many as there is room for."""
+    scratch = scratch_bytes(tmp_path, f"tie_attention_decode_bf16_hd{head_dim}", "attention_decode_bf16.hip",
+                            {"HEAD_DIM": head_dim})
+    ring = {k: v for k, v in scratch.items() if "attention_decode_ring_kernel" in k}
+    assert len(ring) >= 3 and not [k for k, v in ring.items() if v]

@@ -190,6 +190,13 @@ __global__ __launch_bounds__(TIE_WAVE) void attention_decode_kernel(
               sinks);
 }
 
+// The most register sets of the ring: a set holds a tile's 32 keys and values, DH / 2 registers, and beside them stand the
+// accumulators (DH / 4), the queries (DH / 8) and some 60 more, 512 in all. Sets that do not fit go through scratch memory
+// on every tile (heads of 256, 64 sequences of 94 to 1500 keys: whole sequences in four sets 375 us a layer and in two 87,
+// shares of 17 tiles in three sets 106 and in two 92), and the compiler has been seen to lose the fourth register of a
+// piece of 16 bytes that it had put away in two parts: wrong results.
+constexpr int RING_DEPTH = DH <= 160 ? 4 : (DH <= 224 ? 3 : 2);
+
 // One wave a workgroup; shares are the fastest part of its number. Newest tokens that are shares of their own come
 // behind all others (places from num_seqs on), as they are short: between the others they would shift which compute
 // units carry one wave more (8 sequences of 8 KV heads and 4090 keys, 512 long waves and 64 short ones: 4 % of a step).
@@ -250,6 +257,7 @@ static int launch_decode(const bf16_t* q, const QkSource* src, bf16_t* k_cache, 
   // Measured: the ring of three register sets where the keys are cut into shares, of four where a wave walks
   // a whole sequence.
   if (depth == 0) depth = block_size < 16 ? 1 : (nsplit == 1 ? 4 : 3);
+  if (depth > RING_DEPTH) depth = RING_DEPTH;
   if (src != nullptr && (depth < 2 || !PREPARE_HEAD_DIM)) return TIE_BAD_ARGUMENT;
   if (share_tiles != nullptr && (depth < 2 || nsplit == 1)) return TIE_BAD_ARGUMENT;   // the ring kernel's, with a merge
   const dim3 grid(nsplit, KVH * column_groups, num_seqs);
@@ -298,8 +306,8 @@ static int launch_decode(const bf16_t* q, const QkSource* src, bf16_t* k_cache, 
     else attention_decode_kernel<WIDE, false><<<grid, TIE_WAVE, 0, stream>>>(q, k_cache, v_cache, ARGS, 0);  \
   }
   if (src != nullptr && cap > 0.f) return TIE_BAD_ARGUMENT;   // the kernel that makes its own queries caps nothing
-  if (depth == 4) LAUNCH_RING(4)
-  else if (depth == 3) LAUNCH_RING(3)
+  if (depth == 4) LAUNCH_RING((RING_DEPTH < 4 ? RING_DEPTH : 4))
+  else if (depth == 3) LAUNCH_RING((RING_DEPTH < 3 ? RING_DEPTH : 3))
   else if (depth == 2) LAUNCH_RING(2)
   else if (block_size % 8 == 0) LAUNCH_PLAIN(true)
   else LAUNCH_PLAIN(false)
@@ -314,7 +322,7 @@ static int launch_decode(const bf16_t* q, const QkSource* src, bf16_t* k_cache, 
 }
 
 // depth: 0 = by the rule, 1 = the kernel that looks its pages up per lane (any page size), 2 to 4 = the ring
-// kernel with that many register sets (pages of 16 positions or more); for tests and sweeps.
+// kernel with that many register sets, or as many as fit (RING_DEPTH; pages of 16 positions or more); for tests and sweeps.
 // share_tiles (or null): one int on the device, the tiles of 32 keys of a share where the sequences' lengths differ
 // much (the ring kernel and more than one share only; 0 there means shares by each sequence's own length).
 // chunk > 0 (then window must be 0): a query reads the keys of its own chunk of that many positions, counted from

@@ -1607,8 +1607,8 @@ def whole_sequences_fill(tiles, num_kv_heads: int, head_dim: int) -> bool:
     length, 97 steps of 512 to 900 pairs, 4, 8 and 16 heads of 64, 96 and 128: with the busiest unit at 1.0 to 1.72 times
     the mean 0 to 30 % less (64 sequences of 94 to 1500 keys, 1.42: 46.6 and 50.5 us a layer, of 31 to 500 18.0 and 24.0), at
     1.77 to 1.86 1 % more to 18 % less, from 1.87 on 9 % less to 2.2 times as long (80 of 0 to 2500 at random, 3.19: 90.7 and
-    62.5). Not for heads of 256, whose waves walk a tile four times as slowly (64 of 94 to 1500: 375 and 106), nor of 32 (1.0
-    to 1.42: 14 % more to 20 % less); with 256 pairs there is one wave a unit and nothing to make up for a long one.
+    62.5). Heads of 32 are left out (1.0 to 1.42: 14 % more to 20 % less) and those above 128, which were not searched (256, 64
+    of 94 to 1500 keys: 87 and 92); with 256 pairs there is one wave a unit and nothing to make up for a long one.
     """
     low, high = WHOLE_SEQUENCES_HEAD_DIMS
     if len(tiles) * num_kv_heads < 2 * COMPUTE_UNITS or COMPUTE_UNITS % num_kv_heads or not low <= head_dim <= high:
