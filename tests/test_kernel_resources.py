@@ -42,6 +42,8 @@ def scratch_bytes(tmp_path, name, source, defines=None):
     ("tie_skinny_gemm_bf16", "skinny_gemm_bf16.hip", r"skinny_gemm_kernelILi1E.*Li(8|16)EEv", 8),
     ("tie_skinny_gemm_bf16", "skinny_gemm_bf16.hip", r"skinny_gemm_kernelILi[12]E.*Li4EEv", 96 + 48),
     ("tie_skinny_gemm_bf16", "skinny_gemm_bf16.hip", r"skinny_(half_tile|rows)_kernel", 4 + 12),
+    # the norm of a sub-layer's result: up to eight values of a row a thread of 1024
+    ("tie_elementwise", "elementwise.hip", r"norm_add_norm_row_kernel", 2 * (3 * 3 + 2)),
 ])
 def test_kernels_without_scratch(tmp_path, name, source, kernels, count):
     scratch = {k: v for k, v in scratch_bytes(tmp_path, name, source).items() if re.search(kernels, k)}

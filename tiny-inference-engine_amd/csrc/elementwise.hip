@@ -1010,29 +1010,31 @@ __global__ void norm_add_norm_kernel(const float* __restrict__ y, size_t plane_s
 }
 
 // The same with a thread's V values of the row in registers from the first load to the last store (n <= V x
-// threads): the stream, both norm weights and up to G of the result's planes or parts are asked for before the first
+// threads): the stream, both norm weights and G of the result's planes or parts are asked for before the first
 // sum, so the kernel waits for memory once, and once more for where the parts are. Steps of a few rows are bound by
 // exactly that. No load is behind a condition that lanes or the number of planes decide (one beyond the row's end or the
 // last plane is the last again): the compiler waited for each of those before it asked for the next.
-template <typename TO, int V>
+template <typename TO, int V, int G>
 __global__ void norm_add_norm_row_kernel(const float* __restrict__ y, size_t plane_stride, int count, RoutedParts rp,
                                          const float* __restrict__ w_post, float eps_post, float* __restrict__ x,
                                          const float* __restrict__ w_next, float eps_next, TO* __restrict__ out,
                                          int n) {
-  constexpr int G = V == 8 ? 4 : 8;
   __shared__ float scratch[16];
   const size_t r = blockIdx.x;
   const size_t row = r * n;
   float yv[V], xv[V], wp[V], wn[V], part[G][V];
-  int at[V];
+  // In bytes of float32: a load takes a scalar address and this one, no 64-bit sum of its own (with those, V = 8 and G = 4
+  // did not fit the 128 registers a thread of 1024 has).
+  unsigned at[V];
 #pragma unroll
-  for (int j = 0; j < V; ++j) at[j] = min(static_cast<int>(threadIdx.x + j * blockDim.x), n - 1);
+  for (int j = 0; j < V; ++j) at[j] = 4u * min(static_cast<int>(threadIdx.x + j * blockDim.x), n - 1);
+  auto of = [](const float* p, unsigned bytes) { return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + bytes); };
   const float* next = w_next != nullptr ? w_next : w_post;
 #pragma unroll
   for (int j = 0; j < V; ++j) {
-    xv[j] = x[row + at[j]];
-    wp[j] = w_post[at[j]];
-    wn[j] = next[at[j]];
+    xv[j] = of(x + row, at[j]);
+    wp[j] = of(w_post, at[j]);
+    wn[j] = of(next, at[j]);
     yv[j] = 0.f;
   }
   if (rp.parts != nullptr) {
@@ -1050,14 +1052,14 @@ __global__ void norm_add_norm_row_kernel(const float* __restrict__ y, size_t pla
 #pragma unroll
       for (int g = 0; g < G; ++g)
 #pragma unroll
-        for (int j = 0; j < V; ++j) part[g][j] = rp.parts[static_cast<size_t>(max(where[g], 0)) * n + at[j]];
+        for (int j = 0; j < V; ++j) part[g][j] = of(rp.parts + static_cast<size_t>(max(where[g], 0)) * n, at[j]);
       uint32_t self[V];                      // as stored
       if (self_f32) {
 #pragma unroll
-        for (int j = 0; j < V; ++j) self[j] = static_cast<const uint32_t*>(rp.self)[row + at[j]];
+        for (int j = 0; j < V; ++j) self[j] = __float_as_uint(of(static_cast<const float*>(rp.self) + row, at[j]));
       } else {
 #pragma unroll
-        for (int j = 0; j < V; ++j) self[j] = static_cast<const bf16_t*>(rp.self)[row + at[j]];
+        for (int j = 0; j < V; ++j) self[j] = static_cast<const bf16_t*>(rp.self)[row + at[j] / 4];
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1076,7 +1078,7 @@ __global__ void norm_add_norm_row_kernel(const float* __restrict__ y, size_t pla
       for (int g = 0; g < G; ++g)
 #pragma unroll
         for (int j = 0; j < V; ++j)
-          part[g][j] = y[static_cast<size_t>(min(s0 + g, count - 1)) * plane_stride + row + at[j]];
+          part[g][j] = of(y + static_cast<size_t>(min(s0 + g, count - 1)) * plane_stride + row, at[j]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int g = 0; g < G; ++g)
@@ -1130,21 +1132,32 @@ extern "C" int tie_norm_add_norm(const float* y, long plane_stride, int count, c
     // up to 1024 threads with 1, 2, 4 or 8 values each
     const int per = n <= 1024 ? 1 : (n <= 2048 ? 2 : (n <= 4096 ? 4 : 8));
     const int row_threads = ((n + per - 1) / per + TIE_WAVE - 1) / TIE_WAVE * TIE_WAVE;
-#define ROW(TO, V)                                                                                               \
-  norm_add_norm_row_kernel<TO, V><<<R, row_threads, 0, stream>>>(y, static_cast<size_t>(plane_stride), count, rp,  \
-                                                                 w_post, eps_post, x, w_next, eps_next,          \
-                                                                 static_cast<TO*>(out), n)
-#define ROWS(TO)                \
-  {                             \
-    if (per == 1) ROW(TO, 1);   \
-    else if (per == 2) ROW(TO, 2); \
-    else if (per == 4) ROW(TO, 4); \
-    else ROW(TO, 8);            \
+    // Terms at once: as many as there are up to four and up to eight, beyond that four (what is asked for again behind the
+    // last term costs too). Against a term after the other, one row of 1024 values: 2 planes 3.14 us and 3.14, 4 parts 3.83
+    // and 3.78, 9 parts 5.1 and 4.55; of 4096: 2 planes 3.98 and 4.24, 4 parts 4.78 and 6.56; of 8192 7.1 and 14.0 (8 planes).
+    const int terms = parts != nullptr ? top : count;
+#define ROW_G(TO, V, G)                                                                                             \
+  norm_add_norm_row_kernel<TO, V, G><<<R, row_threads, 0, stream>>>(y, static_cast<size_t>(plane_stride), count, rp, \
+                                                                    w_post, eps_post, x, w_next, eps_next,          \
+                                                                    static_cast<TO*>(out), n)
+#define ROW(TO, V)                                                        \
+  {                                                                       \
+    if (terms <= 2) ROW_G(TO, V, 2);                                      \
+    else if (terms <= 4 || terms > 8 || V == 8) ROW_G(TO, V, 4);          \
+    else ROW_G(TO, V, V < 8 ? 8 : 4);                                     \
+  }
+#define ROWS(TO)                  \
+  {                               \
+    if (per == 1) ROW(TO, 1)      \
+    else if (per == 2) ROW(TO, 2) \
+    else if (per == 4) ROW(TO, 4) \
+    else ROW(TO, 8)               \
   }
     if (w_next == nullptr || out_dtype == TIE_F32) ROWS(float)
     else ROWS(bf16_t)
 #undef ROWS
 #undef ROW
+#undef ROW_G
     return tie_launch_status();
   }
   const int threads = n >= 4096 ? 1024 : (n >= 1024 ? 512 : (n >= 256 ? 256 : 64));
