@@ -481,7 +481,7 @@ def test_products_of_33_to_64_rows_around_the_width_of_a_vocabulary(M, N, K):
     close(out, plain.linear(x.cpu(), w.cpu()), 1e-5, f"vocabulary product {M}x{N}x{K}")
 
 
-@pytest.mark.parametrize("R,n", [(1, 24), (5, 200), (8, 4096), (64, 1024), (3, 20000)])
+@pytest.mark.parametrize("R,n", [(1, 24), (5, 200), (8, 4096), (64, 1024), (3, 20000), (2, 4100), (2, 5120), (3, 8192), (2, 12284)])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_add_partials_alone_and_with_rms_norm(R, n, out_dtype):
     from tie_amd import kernels

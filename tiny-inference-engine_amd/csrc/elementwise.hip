@@ -71,9 +71,11 @@ __global__ void rms_norm_kernel(const TX* __restrict__ x, const float* __restric
 // Float32 rows of up to four float4 a thread (n % 4 == 0) stay in registers between the sum of
 // squares and the scaling. With COUNT > 0 the row first receives COUNT planes of partial sums
 // (x[r] += p_0[r] + p_1[r] + ..., written back): see the section on partial sums below. All loads
-// of a thread are issued before the first use; the kernel is bound by latency, not by bytes. A lane behind the row's end
-// asks for its last float4 again and counts nothing: with the loads behind that condition the compiler waited for all
-// that was asked for in their middle.
+// of a thread are issued before the first use; the kernel is bound by latency, not by bytes. Where a thread has one float4
+// of the row, a lane behind its end asks for the last one again and counts nothing: with the loads behind that condition
+// the compiler waited for all that was asked for in their middle (4 planes of 1024 to 4096 values 4 to 9 % longer). Longer
+// rows keep the condition: what those lanes bring costs more there (5120, two float4 a thread of 1024: 4 planes of one
+// row 3.30 us, and 3.83 without it; of 8192 4.01 and 4.19).
 template <typename TO, int COUNT, int V>
 __global__ void rms_norm_row_kernel(float* __restrict__ x, const float* __restrict__ partials, size_t plane_stride,
                                     const float* __restrict__ w, float eps, TO* __restrict__ out,
@@ -84,14 +86,17 @@ __global__ void rms_norm_row_kernel(float* __restrict__ x, const float* __restri
   float4 v[V], p[COUNT > 0 ? COUNT : 1][V], wv[V];
 #pragma unroll
   for (int j = 0; j < V; ++j) {
-    const int i = min(static_cast<int>(threadIdx.x + j * blockDim.x) * 4, n - 4);
-    v[j] = *reinterpret_cast<const float4*>(x + row + i);
-    wv[j] = *reinterpret_cast<const float4*>(w + i);
+    const int own = (threadIdx.x + j * blockDim.x) * 4;
+    const bool in = V == 1 || own < n;
+    const int i = V == 1 ? min(own, n - 4) : own;
+    v[j] = in ? *reinterpret_cast<const float4*>(x + row + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    wv[j] = in ? *reinterpret_cast<const float4*>(w + i) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int s = 0; s < COUNT; ++s)
-      p[s][j] = *reinterpret_cast<const float4*>(partials + static_cast<size_t>(s) * plane_stride + row + i);
+      p[s][j] = in ? *reinterpret_cast<const float4*>(partials + static_cast<size_t>(s) * plane_stride + row + i)
+                   : make_float4(0.f, 0.f, 0.f, 0.f);
   }
-  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (V == 1) __builtin_amdgcn_sched_barrier(0);
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < V; ++j) {
@@ -104,8 +109,10 @@ __global__ void rms_norm_row_kernel(float* __restrict__ x, const float* __restri
     }
     const int i = (threadIdx.x + j * blockDim.x) * 4;
     if (COUNT > 0 && i < n) *reinterpret_cast<float4*>(x + row + i) = v[j];
-    if (i >= n) v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-    ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+    if (V == 1 && i >= n) v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    // Which square is rounded by itself is said here: left to the compiler, it changed with the form of the loads.
+    const float pair = V == 1 ? fmaf(v[j].y, v[j].y, v[j].x * v[j].x) : fmaf(v[j].x, v[j].x, v[j].y * v[j].y);
+    ss += fmaf(v[j].w, v[j].w, fmaf(v[j].z, v[j].z, pair));
   }
   ss = block_sum(ss, scratch);
   const float inv = 1.0f / sqrtf(ss / static_cast<float>(n) + eps);
