@@ -127,7 +127,11 @@ __device__ __forceinline__ void store_share(const floatx4 (&acc)[DTILES], float 
 // than the others). PREPARE_WHOLE: a wave walks a whole sequence and takes the newest token behind its tiles.
 enum DecodePrepare { PREPARE_NOTHING, PREPARE_SHARES, PREPARE_WHOLE };
 
-constexpr int TABLE_AHEAD = 256;   // entries of a page table that a wave keeps: 4096 keys in pages of 16
+// Entries of a page table that a wave keeps: 4096 keys in pages of 16. A share that begins behind them asks again, a trip
+// more than the others, and still no step over 8 k to 32 k keys is slower than with a scalar load a tile (1.7B, one sequence
+// 1395 -> 1259 us over 8 k and 1722 -> 1608 over 32 k, four 1751 -> 1658 and 3251 -> 3181; 12 layers of the 8B shape, one
+// 1396 -> 1350 over 32 k, eight 1693 -> 1678 over 8 k and 2998 -> 2985 over 32 k).
+constexpr int TABLE_AHEAD = 256;
 
 struct QkSource {
   const float* qkv;        // [planes][rows][in_row] float32: q heads, k heads, v heads of a row

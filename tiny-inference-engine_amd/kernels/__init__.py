@@ -961,7 +961,7 @@ NORMS_IN_PRODUCTS = True
 
 class RowScale:
     """Rows that are a norm's input times its weight, the ``1 / rms`` still to come: ``squares[m]`` holds, per
-    16-column tile of the row the norm saw, the sum of its squares; the factor is
+    16 (or 8: ``norm_square_columns``) columns of the row the norm saw, the sum of its squares; the factor is
     ``1 / sqrt(squares[m].sum() / n + eps)`` and belongs on whatever product is formed from the rows."""
 
     __slots__ = ("squares", "n", "eps")

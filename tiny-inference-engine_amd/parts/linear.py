@@ -139,7 +139,9 @@ class Linear:
     def add_to_and_prepare_norm(self, x: torch.Tensor, out: torch.Tensor, norm_weight: torch.Tensor,
                                 next_rows: torch.Tensor, squares: torch.Tensor) -> None:
         """out += x @ W^T in one plane, and in the same epilogue ``next_rows = bfloat16(out * norm_weight)`` and the
-        sums of ``out ** 2`` per 16-column tile (``prepares_norms`` says whether this product can)."""
+        sums of ``out ** 2`` (``prepares_norms`` says whether this product can). ``squares`` is
+        ``[rows, out columns / kernels.norm_square_columns(rows, self.weight)]``, a sum to 8 or 16 columns, and its width
+        chooses the kernel: sums of 16 columns where 8 are asked for are right too, from the slower one."""
         kernels.skinny_gemm_bf16(x, self.weight, out, accumulate=True, next_norm=(norm_weight, next_rows, squares))
 
     @staticmethod
