@@ -160,6 +160,23 @@ def test_the_tiled_product_plans_by_rounds_of_workgroups():
     assert kernels.gemm_splits(128, 4096, 4096) == 8 and kernels.gemm_splits(128, 4096, 256) == 1
 
 
+@pytest.mark.parametrize("M,N,K,want", [(2048, 4096, 12288, (1, 5)), (2048, 4096, 4096, (1, 5)), (2048, 2048, 6144, (2, 5)),
+                                        (512, 4096, 12288, (4, 5)), (512, 2048, 2048, (4, 7))])
+def test_products_that_add_to_the_stream_have_a_plan_of_their_own(M, N, K, want):
+    """The best of all forced (ranges, tile), each timed with the norm behind it, or within 2 % of it; every plan is one the
+    kernel takes: no range shorter than 512 of K, and up to 128 rows the same as of products that store."""
+    from tie_amd import kernels
+
+    assert kernels.gemm_adding_plan(M, N, K) == want
+    for rows in list(range(129, 2300, 61)) + [65, 100, 128, 48]:
+        ranges, tile = kernels.gemm_adding_plan(rows, N, K)
+        assert ranges in (1, 2, 4, 8) and (ranges == 1 or K // ranges >= 512), (rows, N, K, ranges)
+        if rows > 128:
+            assert tile in TILE_ROWS_COLS
+        else:
+            assert (ranges, tile) == (kernels.gemm_splits(rows, N, K, True), kernels.gemm_tile(rows, N, K, True))
+
+
 def test_the_tiled_product_plans_for_a_last_row_tile_that_is_nearly_empty():
     """A nearly empty last row tile makes the others faster, tiles that are no multiple of eight slower: the best of all
     forced (tile, ranges) at 576, 320 and 144 rows, by 3 to 20 % (4096 x 12288 at 576 rows: 128 x 192 tiles in two

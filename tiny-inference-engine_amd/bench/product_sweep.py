@@ -90,15 +90,20 @@ def main(argv=None) -> int:
                     kernels.linear_swiglu(x, weights[i], act)
             else:
                 decode = kernels.decode_product_rows(M, weights[0])
+                own_tile = 0
                 if decode:
                     own_splits = kernels.skinny_splits(N, K) if M <= 16 else kernels.few_rows_plan(M, N, K)[2]
-                else:
+                elif proj == "qkv":
                     own_splits = kernels.gemm_splits(M, N, K, True)
+                else:                                        # added to the stream
+                    own_splits, own_tile = kernels.gemm_adding_plan(M, N, K)
 
                 def own(i):
                     if own_splits > 1:
-                        (kernels.skinny_gemm_bf16 if decode else kernels.gemm_bf16)(x, weights[i], planes[own_splits],
-                                                                                    splits=own_splits)
+                        if decode:
+                            kernels.skinny_gemm_bf16(x, weights[i], planes[own_splits], splits=own_splits)
+                        else:
+                            kernels.gemm_bf16(x, weights[i], planes[own_splits], splits=own_splits, tile=own_tile)
                     else:
                         kernels.linear(x, weights[i], stream, True)
                     consume(own_splits)

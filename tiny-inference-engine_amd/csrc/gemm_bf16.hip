@@ -302,7 +302,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
   constexpr int PA = BM / 64;                   // wave instructions that stage x's rows (16 rows each, 4 waves)
   constexpr int PB = BN / 64;                   // wave instructions that stage w's rows likewise
   static_assert(BM == 256 || BM == 128 || BM == 64, "rows of a tile");
-  constexpr int G = GdShape<BM, BN>::GROUP;     // slices that x's rows are staged by
+  constexpr int G = GdShape<BM, BN>::X_GROUP;   // slices that x's rows are staged by
   extern __shared__ bf16_t lds[];
 
   const int total = tiles_m * tiles_n;
@@ -457,15 +457,14 @@ static bool gemm_dma_takes(const void* x, const void* w, const void* out, int N,
 //   * a round is a few microseconds of start and end plus its slices of 32 along K at the tile's own pace, both more where
 //     it fills every compute unit;
 //   * every plane is written once here and read once by its consumer.
-// start, full, slice and press are a least-squares fit, tile by tile, to sweeps over eight packed projections (2048 x 2048
-// to 24576 x 4096, every tile, 1 to 8 ranges) at 200 to 2048 rows, and to those at 96 and 128 rows, where the weights come
-// from memory by few workgroups; lead and scatter were then chosen, above 128 rows, on the projections of eight layer
-// shapes 1024 to 8192 wide at ten row counts, full tiles and not, and 22 weights of random sizes (768 to 40000 rows, K 768
-// to 20000) at random row counts, every candidate timed with its consumer and the weights from memory. The choice lies
-// 0.9 % above the best forced (tile, ranges) there, 1.1 % over 22 random weights held out, 10 % at worst but for K above
-// 8000 over fewer than 2000 rows of w (35 %); without the two it lay 1.9 and 1.3 % above and took 98 us where 81 do
-// (576 rows over 4096 x 12288). 65 to 128 rows: 0.4 % above the best over the eight shapes, 0.9 % over the random weights,
-// 15 % at worst. Rows of fewer than 65 over row-major weights and odd K or N stay with the older tiles and their rule.
+// The constants are fitted tile by tile to sweeps of every (tile, ranges) over the packed projections of fifteen layer
+// shapes, 768 to 8192 wide with inner sizes of 3072 to 28672, at six to fifteen row counts from 140 to 2048, each candidate
+// timed with its consumer and the weights from memory. The choice lies 1.4 % (products that store) and 2.1 % (products that
+// add to the stream) above the best forced one there, 1.5 and 2.3 % over seven shapes held out; 0.4 % over the shapes of
+// 1024 to 4096 that models have; a third at worst, where K below 1024 is not cut. 65 to 128 rows: 0.4 % above the best. Rows
+// of fewer than 65 over row-major weights and odd K or N stay with the older tiles and their rule.
+// A product that adds to the stream has a table of its own: in place it reads what it adds to, and its planes are read by the
+// norm. 2048 rows over 4096 x 12288 with the norm behind it: two planes of 256 x 256 tiles 203 us, 256 x 128 in place 182.
 struct GemmPlan { int tile, splits; };
 
 static int legacy_splits(int M, int N, int K) {
@@ -489,12 +488,19 @@ static int legacy_splits(int M, int N, int K) {
 // are no multiple of eight, so that the row tiles of one piece of w do not follow each other on one die.
 // per_cu workgroups on one compute unit each take `shared` times as long.
 struct DmaTile { int id, bm, bn; float start_us, full_us, slice_us, press, lead, scatter; int per_cu; float shared; };
-static const DmaTile kDmaTiles[] = {{4, 256, 256, 8.57f, 7.37f, 0.629f, 0.17f, 0.17f, 0.18f, 1, 1.f},
-                                    {10, 256, 192, 6.14f, 2.53f, 0.580f, 0.15f, 0.18f, 0.f, 1, 1.f},
-                                    {5, 256, 128, 6.91f, 0.f, 0.367f, 0.32f, 0.11f, 0.11f, 1, 1.f},
-                                    {6, 128, 256, 6.20f, 0.91f, 0.400f, 0.18f, 0.10f, 0.16f, 1, 1.f},
-                                    {11, 128, 192, 5.10f, 0.f, 0.327f, 0.12f, 0.f, 0.12f, 1, 1.f},
-                                    {7, 128, 128, 3.48f, 0.91f, 0.250f, 0.14f, 0.12f, 0.19f, 1, 1.f}};
+static const DmaTile kDmaTiles[] = {{4, 256, 256, 7.02f, 4.26f, 0.622f, 0.135f, 0.121f, 0.114f, 1, 1.f},
+                                    {10, 256, 192, 6.07f, 3.00f, 0.522f, 0.070f, 0.163f, 0.051f, 1, 1.f},
+                                    {5, 256, 128, 8.10f, 0.00f, 0.365f, 0.300f, 0.208f, 0.101f, 1, 1.f},
+                                    {6, 128, 256, 5.80f, 1.45f, 0.401f, 0.160f, 0.102f, 0.162f, 1, 1.f},
+                                    {11, 128, 192, 4.42f, 0.00f, 0.284f, 0.175f, 0.020f, 0.247f, 1, 1.f},
+                                    {7, 128, 128, 3.36f, 0.12f, 0.247f, 0.085f, 0.196f, 0.289f, 1, 1.f}};
+// Products that add to the stream (O and down): the same, fitted to those alone, each timed with the norm behind it.
+static const DmaTile kAddingTiles[] = {{4, 256, 256, 5.96f, 3.70f, 0.623f, 0.224f, 0.168f, 0.109f, 1, 1.f},
+                                       {10, 256, 192, 5.81f, 4.57f, 0.526f, 0.112f, 0.159f, 0.000f, 1, 1.f},
+                                       {5, 256, 128, 5.86f, 0.52f, 0.363f, 0.211f, 0.175f, 0.055f, 1, 1.f},
+                                       {6, 128, 256, 5.14f, 0.00f, 0.371f, 0.371f, 0.081f, 0.156f, 1, 1.f},
+                                       {11, 128, 192, 4.81f, 0.41f, 0.317f, 0.227f, 0.113f, 0.094f, 1, 1.f},
+                                       {7, 128, 128, 4.09f, 0.29f, 0.250f, 0.278f, 0.215f, 0.094f, 1, 1.f}};
 static const DmaTile kFewRowsTiles[] = {{6, 128, 256, 6.11f, 3.12f, 0.440f, 0.20f, 0.f, 0.f, 1, 1.f},
                                         {7, 128, 128, 3.91f, 0.68f, 0.276f, 0.43f, 0.f, 0.f, 1, 1.f},
                                         {8, 64, 256, 3.62f, 0.87f, 0.373f, 0.27f, 0.f, 0.f, 1, 1.f},
@@ -520,7 +526,8 @@ static float estimated_us(const DmaTile& t, int M, int N, int K, int ranges, flo
 }
 
 // splits: 0 = free to choose (the caller adds planes), else the number of ranges the caller has fixed (1: none).
-static GemmPlan gemm_plan(int M, int N, int K, bool straight_to_lds, int splits, bool packed) {
+// adds: the product's sums go into the float32 stream that the next norm reads.
+static GemmPlan gemm_plan(int M, int N, int K, bool straight_to_lds, int splits, bool packed, bool adds = false) {
   const bool may_split = splits == 0;
   if (straight_to_lds && packed && M <= 64) {
     // Up to 64 rows over packed weights: tiles of 64 rows, one workgroup a compute unit, the weights read once. The
@@ -555,7 +562,7 @@ static GemmPlan gemm_plan(int M, int N, int K, bool straight_to_lds, int splits,
     float best_us = 0.f;
     const int k_slices = K / GD_BK;
     auto offer = [&](const DmaTile& t, int r) {
-      const float us = estimated_us(t, M, N, K, r, M <= 128 ? 0.24f : 0.32f);
+      const float us = estimated_us(t, M, N, K, r, M <= 128 ? 0.24f : 0.26f);
       if (best_us == 0.f || us < best_us * 0.98f) {         // ties go to fewer planes, then to the larger tile
         best = {t.id, r};
         best_us = us;
@@ -567,7 +574,7 @@ static GemmPlan gemm_plan(int M, int N, int K, bool straight_to_lds, int splits,
       if (M <= 128)
         for (const DmaTile& t : kFewRowsTiles) offer(t, r);
       else
-        for (const DmaTile& t : kDmaTiles) offer(t, r);
+        for (const DmaTile& t : adds ? kAddingTiles : kDmaTiles) offer(t, r);
     }
     return best;
   }
@@ -595,6 +602,15 @@ extern "C" int tie_gemm_bf16_wins_few_rows(int M, int N, int K, int packed, int 
 extern "C" int tie_gemm_bf16_splits(int M, int N, int K, int packed) {
   if (packed && !straight_to_lds_shape(N, K)) return 1;
   return gemm_plan(M, N, K, straight_to_lds_shape(N, K), 0, packed != 0).splits;
+}
+
+// The same for a product over a packed weight that is added to the float32 stream, in place (1) or as planes that the next norm adds: the tile
+// it then runs on in *tile.
+extern "C" int tie_gemm_bf16_adding_plan(int M, int N, int K, int* tile) {
+  const bool straight = straight_to_lds_shape(N, K);
+  const GemmPlan plan = gemm_plan(M, N, K, straight, straight ? 0 : 1, true, true);
+  *tile = plan.tile;
+  return plan.splits;
 }
 
 // The tile a product left to choose runs on (the numbers of tie_gemm_bf16's `tile`), with `splits` ranges of K
@@ -626,7 +642,7 @@ extern "C" int tie_gemm_bf16(const void* x, const void* w, void* out, int out_dt
   const bool straight = gemm_dma_takes(x, w, out, N, K, splits);
   if (packed && (N % 16 != 0 || !straight || (tile != 0 && (tile < 4 || tile > 11)))) return TIE_BAD_ARGUMENT;
   if (tile == 0) {
-    tile = gemm_plan(M, N, K, straight, splits, packed != 0).tile;
+    tile = gemm_plan(M, N, K, straight, splits, packed != 0, accumulate != 0).tile;
   } else if (tile < 4 && splits > 1) {
     tile = 1;
   }

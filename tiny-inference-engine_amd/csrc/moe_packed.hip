@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void moe_packed_many_rows_kernel(const bf16_t*
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr bool GATED = MODE == 1 || MODE == 3 || MODE == 4;
   constexpr bool GATHER = MODE != 0;
-  constexpr int TN = BN / 64, TM = BM / 64, G = GdShape<BM, BN>::GROUP;
+  constexpr int TN = BN / 64, TM = BM / 64, G = GdShape<BM, BN>::X_GROUP;
   extern __shared__ bf16_t lds[];
   const int total = *rw.num_tiles * tiles_n;
   const int per_xcd = (total + 7) / 8;

@@ -246,6 +246,7 @@ _SIGNATURES = {
     },
     "gemm_bf16": {
         "tie_gemm_bf16_splits": [_c_int, _c_int, _c_int, _c_int],
+        "tie_gemm_bf16_adding_plan": [_c_int, _c_int, _c_int, ctypes.POINTER(_c_int)],
         "tie_gemm_bf16_tile": [_c_int, _c_int, _c_int, _c_int, _c_int],
         "tie_gemm_bf16_wins_few_rows": [_c_int, _c_int, _c_int, _c_int, _c_int],
         "tie_gemm_bf16": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
@@ -1037,6 +1038,14 @@ def skinny_gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumu
 def gemm_splits(M: int, N: int, K: int, packed: bool = False) -> int:
     """Ranges of K a product of M > 64 rows over a ``[N, K]`` weight is best cut into when its caller adds partial sums."""
     return int(_lib("gemm_bf16").tie_gemm_bf16_splits(M, N, K, int(packed)))
+
+
+def gemm_adding_plan(M: int, N: int, K: int) -> tuple:
+    """``(ranges, tile)`` of a product of M > 64 rows over a packed ``[N, K]`` weight that is added to the float32 stream: in place with one range, else
+    as planes that the next norm adds."""
+    tile = _c_int(0)
+    ranges = int(_lib("gemm_bf16").tie_gemm_bf16_adding_plan(M, N, K, ctypes.byref(tile)))
+    return ranges, int(tile.value)
 
 
 def gemm_tile(M: int, N: int, K: int, packed: bool = False, splits: int = 0) -> int:

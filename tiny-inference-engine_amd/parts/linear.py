@@ -37,7 +37,7 @@ class Linear:
         self.init_std = init_std
         self.weight: torch.Tensor = None
         self._splits = None
-        self._tiled_splits = {}
+        self._tiled_plans = {}
 
     @property
     def total_out(self) -> int:
@@ -129,7 +129,7 @@ class Linear:
         # An earlier product's planes may still be owed and live in the buffer the new planes take:
         # add them before they are overwritten (after a norm that took the debt this does nothing).
         ctx.settle()
-        planes = self.partial_planes(ctx, x, "linear.partials", bias_added=True)
+        planes = self.partial_planes(ctx, x, "linear.partials", adds=True)
         if planes is not None:
             ctx.defer_add(out, planes)
             return out
@@ -155,16 +155,17 @@ class Linear:
             return None
         return scale
 
-    def partial_planes(self, ctx, x: torch.Tensor, name: str, bias_added: bool = False):
+    def partial_planes(self, ctx, x: torch.Tensor, name: str, adds: bool = False):
         """Runs the product as ``[S, M, N]`` float32 planes of partial sums if that is the faster way; else None.
 
         The decode product decides by the weight's shape alone up to 16 rows and by its plan for the number of rows
         above (up to 32 rows, or 64 where the tiled product is not the faster); the tiled product is cut along K
-        when its tiles alone would leave most of the GPU idle, and so is the float32 product.
+        when its tiles alone would leave most of the GPU idle, and so is the float32 product. ``adds``: the sums go into the
+        stream, where a bias has gone already; adding there in place is then the other way, not storing.
         """
         M, K = x.shape
         w = self.weight
-        if x.dtype == torch.float32 and w.dtype == torch.float32 and K % 4 == 0 and (self.bias is None or bias_added):
+        if x.dtype == torch.float32 and w.dtype == torch.float32 and K % 4 == 0 and (self.bias is None or adds):
             splits = kernels.gemm_f32_splits(M, w.shape[0], K)
             if splits > 1:
                 planes = ctx.scratch(name, (splits, M, w.shape[0]), torch.float32)
@@ -172,9 +173,10 @@ class Linear:
                     kernels.gemm_f32(x, w, planes, splits=splits)
                     return planes
             return None
-        if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or K % 8 or (self.bias is not None and not bias_added):
+        if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or K % 8 or (self.bias is not None and not adds):
             return None      # planes hold the product alone: a bias must have gone to the target already
         decode_product = kernels.decode_product_rows(M, w)
+        tile = 0
         if decode_product:
             if M <= 16 or not isinstance(w, kernels.PackedWeight):
                 if self._splits is None:
@@ -183,9 +185,13 @@ class Linear:
             else:
                 splits = kernels.few_rows_plan(M, w.shape[0], K)[2]
         else:
-            splits = self._tiled_splits.get(M)
-            if splits is None:
-                splits = self._tiled_splits[M] = kernels.gemm_splits(M, w.shape[0], K, isinstance(w, kernels.PackedWeight))
+            plan = self._tiled_plans.get((M, adds))
+            if plan is None:
+                packed = isinstance(w, kernels.PackedWeight)
+                plan = kernels.gemm_adding_plan(M, w.shape[0], K) if adds and packed else \
+                    (kernels.gemm_splits(M, w.shape[0], K, packed), 0)
+                self._tiled_plans[(M, adds)] = plan
+            splits, tile = plan
         if splits <= 1:
             return None
         planes = ctx.scratch(name, (splits, M, w.shape[0]), torch.float32)
@@ -193,5 +199,5 @@ class Linear:
         if decode_product:
             kernels.skinny_gemm_bf16(x, w, planes, splits=splits, row_scale=scale)
         else:
-            kernels.gemm_bf16(x, w, planes, splits=splits)      # above the rows a scale travels with: none here
+            kernels.gemm_bf16(x, w, planes, splits=splits, tile=tile)      # above the rows a scale travels with: none here
         return planes
