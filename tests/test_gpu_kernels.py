@@ -97,6 +97,32 @@ def test_gemm_generic(T, N, K, dtypes):
     assert torch.equal(one[0], out[T - 1])
 
 
+@pytest.mark.parametrize("H,KVH,Dh,bs,window", [(8, 4, 64, 16, None), (4, 4, 128, 16, 100), (24, 4, 96, 32, None)])
+def test_whole_sequences_in_the_planned_order_have_the_same_bits(H, KVH, Dh, bs, window):
+    """A decode step of more than 512 (sequence, KV head) pairs with the order that its builder plans, and without one."""
+    from tie_amd import kernels
+
+    lens = [1 + (i * 37) % 400 for i in range(129)]
+    case, S = attention_case(H, KVH, Dh, bs, lens_new=[1] * len(lens), lens_ctx=lens, seed=29, dtype=torch.bfloat16, window=window)
+
+    class Batch:
+        all_decode, num_seqs, plan_context, memo = True, S, 1024, {}
+        query_start, context_lens = case["query_start"], case["context_lens"]
+
+    shares, length, order = kernels.decode_wave_plan(lens, KVH, 1024, bs, window, Dh)
+    assert (shares, length) == (1, 0) and order is not None
+    outs = []
+    for ids in (None, torch.from_numpy(order).cuda()):
+        class Step:
+            block_tables, key_shares, wave_order = case["tables"], (1, None), ids
+
+        outs.append(torch.full_like(case["q"], float("nan")))
+        kernels.paged_attention(case["q"], case["kc"], case["vc"], outs[-1], Step, Batch, H, Dh ** -0.5, window,
+                                lambda name, shape, dtype: torch.empty(shape, dtype=dtype, device="cuda"))
+    assert torch.equal(outs[0], outs[1])
+    close(outs[1], case["want"], 1e-2, f"whole sequences in order, H={H} KVH={KVH} Dh={Dh} bs={bs} window={window}")
+
+
 @pytest.mark.parametrize("H,KVH,Dh,bs", [(4, 2, 16, 4), (6, 2, 32, 16), (3, 1, 48, 8), (5, 5, 80, 16), (8, 2, 128, 16),
                                          (2, 1, 256, 4), (2, 2, 512, 2)])
 def test_qk_norm_rope_kv_write(H, KVH, Dh, bs):

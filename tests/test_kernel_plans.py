@@ -406,6 +406,42 @@ def test_sequences_of_different_lengths_stay_whole_where_no_compute_unit_waits_f
     assert kernels.decode_share_plan([100] * 8 + [30000] * 56, 8, 32768, window=1024, head_dim=128) == (1, 0)
 
 
+@pytest.mark.parametrize("S,heads", [(64, 8), (90, 8), (129, 4), (64, 16), (86, 6), (512, 1), (2, 300)])
+def test_whole_sequences_are_launched_so_that_long_ones_meet_short_ones(S, heads):
+    """A permutation; with sequences of lengths at random the busiest compute unit brings little more than the mean where
+    every unit has the same number of waves. Without whole sequences, and below two waves a unit, there is no order; the plan
+    for sequences of any length keeps the shares that the rule for them gives unless whole ones in order fill the units."""
+    import random
+
+    from tie_amd import kernels
+
+    rng = random.Random(S)
+    lens = [rng.randint(50, 2000) for _ in range(S)]
+    tiles = kernels.key_tiles(lens)
+    order = kernels.whole_sequences_order(tiles, heads)
+    assert sorted(order.tolist()) == list(range(S)) and order.dtype.name == "int32"
+    apart = max(1, 256 // heads)
+    if S % apart == 0 and S > apart:
+        assert kernels.whole_sequences_fill([tiles[i] for i in order], heads, 128, 1.2) or 256 % heads
+    shares, length, planned = kernels.decode_wave_plan(lens, heads, 2048, 16, None, 128)
+    assert planned is None or (shares, length) == (1, 0) and planned.tolist() == order.tolist()
+    assert (shares, length) in ((1, 0), kernels.decode_share_plan(lens, heads, 2048, 16, None, 128))
+    assert kernels.decode_wave_plan(lens[:511 // heads or 1], heads, 2048, 16, None, 128)[2] is None
+
+
+def test_whole_sequences_in_order_where_shares_were_planned():
+    """64 sequences of which the long ones come 32 apart: 1.9 times the mean as they come, 1.0 in order."""
+    from tie_amd import kernels
+
+    lens = [2000] * 8 + ([100] * 24 + [2000] * 8) + [100] * 24
+    assert kernels.decode_share_plan(lens, 8, 2048, head_dim=128)[1] > 0
+    assert kernels.decode_wave_plan(lens, 8, 2048, head_dim=128)[:2] == kernels.decode_share_plan(lens, 8, 2048, head_dim=128)
+    lens = [2000] * 16 + [200] * 16 + [2000] * 16 + [200] * 16
+    assert kernels.decode_share_plan(lens, 8, 2048, head_dim=128)[1] > 0
+    shares, length, order = kernels.decode_wave_plan(lens, 8, 2048, head_dim=128)
+    assert (shares, length) == (1, 0) and all(lens[a] + lens[b] == 2200 for a, b in zip(order[:32], order[32:]))
+
+
 def test_shares_of_one_length_are_planned_for_sequences_of_very_different_lengths():
     import random
 

@@ -49,6 +49,8 @@ class GroupStep:
         # a step of single tokens over sequences of very different lengths: (shares, their length in tiles of 32
         # keys as one int32 on the device) for the decode attention kernel; None: the rule by the step's size
         self.key_shares = None
+        # a step of single tokens whose waves each walk a whole sequence: int32 [S], the order they are launched in
+        self.wave_order = None
 
 
 class StepBatch:
@@ -253,6 +255,9 @@ class BatchBuilder:
             offset += _align(S * MB)
             layout[("share_tiles", g)] = (offset, 1)
             offset += _align(1)
+            if all_single:
+                layout[("wave_order", g)] = (offset, S)
+                offset += _align(S)
         host_t, dev_t = self._buffers(offset)
         host = host_t.numpy()
 
@@ -273,9 +278,11 @@ class BatchBuilder:
         shares = {}
         for g in groups:
             need = self.cache.plan.groups[g].need
-            shares[g] = (kernels.decode_share_plan(batch.host_context_lens, need.num_kv_heads, batch.plan_context,
-                                                   self.cache.block_size, need.reach, need.head_dim) if all_single else (0, 0))
+            shares[g] = (kernels.decode_wave_plan(batch.host_context_lens, need.num_kv_heads, batch.plan_context,
+                                                  self.cache.block_size, need.reach, need.head_dim) if all_single else (0, 0, None))
             view(("share_tiles", g))[0] = shares[g][1]
+            if shares[g][2] is not None:
+                view(("wave_order", g))[:] = shares[g][2]
 
         dev_t[:offset].copy_(host_t[:offset], non_blocking=True)
         if self.device.type == "cuda":
@@ -297,6 +304,8 @@ class BatchBuilder:
             batch.groups[g] = GroupStep(dev(("slots", g)), dev(("tables", g), (S, MB)))
             if shares[g][1] > 0:
                 batch.groups[g].key_shares = (shares[g][0], dev(("share_tiles", g)))
+            if shares[g][2] is not None:
+                batch.groups[g].wave_order = dev(("wave_order", g))
         batch.share_key = tuple(shares[g][0] if shares[g][1] > 0 else 0 for g in groups)
         batch.max_new_tokens = max(batch.host_new_tokens)
         batch.all_decode = batch.max_new_tokens == 1
