@@ -62,6 +62,23 @@ def test_key_shares_never_exceed_what_the_merge_takes():
         == [2, 4, 2, 2]
 
 
+def test_float32_attention_cuts_keys_while_all_workgroups_run_at_once():
+    """At most 256 workgroups where there is more than one share, no share empty, none of fewer than four tiles of 16 keys
+    but by what rounding leaves, at most 24 shares; the measured choices."""
+    from tie_amd import kernels
+
+    for tiles in (1, 2, 4, 5, 8, 16, 31, 32, 33, 301):
+        for kv_heads, group in ((8, 2), (4, 8), (1, 40), (2, 16)):
+            workgroups = tiles * kv_heads * -(-group // 16)
+            for context in (1, 16, 17, 64, 65, 129, 300, 601, 1000, 4096, 33000):
+                n, key_tiles = kernels.attention_f32_splits(tiles, kv_heads, group, context), -(-context // 16)
+                share = -(-key_tiles // n)
+                assert 1 <= n <= 24 and (n == 1 or workgroups * n <= 256), (tiles, kv_heads, group, context, n)
+                assert share * (n - 1) < key_tiles and (n == 1 or share >= 3), (tiles, kv_heads, group, context, n)
+    assert [kernels.attention_f32_splits(1, 8, 2, c) for c in (64, 65, 300, 1000, 4000)] == [1, 2, 5, 16, 23]
+    assert [kernels.attention_f32_splits(t, 8, 2, 601) for t in (4, 8, 16, 32, 38)] == [8, 4, 2, 1, 1]
+
+
 def test_sizes_no_kernel_takes_are_refused_when_the_model_is_built():
     from tie_amd.config.qwen3 import Qwen3Config
     from tie_amd.errors import InvalidArgument

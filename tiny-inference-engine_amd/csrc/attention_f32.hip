@@ -11,8 +11,9 @@
 //   O^T = V^T P^T the weights are those sums in place: instruction i takes keys 4 c + i, for which a page, whose values
 //                 lie transposed, holds 16 consecutive bytes a dimension
 // so a tile of 16 keys and a head size of 128 is 16 loads and 64 instructions of 32 cycles, without LDS or barriers.
-// Bound by latency at the sizes the 32-bit path sees: four sequences of 600 keys, 16 heads over 8, take 12.0 us and 3.9 to
-// merge (one workgroup a row and head, key by key, took 150), a prompt of 301 tokens 23.9 us (463).
+// Bound by latency at the sizes the 32-bit path sees: four sequences of 600 keys, 16 heads over 8, take 11.1 us with the
+// merge (in two shares of the keys 16.5; one workgroup a row and head, key by key, took 150), a prompt of 301 tokens 17.7
+// (463). A workgroup of eight waves of 211 registers fills a compute unit.
 // Keys are cut into shares over workgroups where the columns alone leave the chip idle; a second kernel merges them.
 // Key tiles are cut at multiples of 16 positions: what is computed for a position does not depend on pages, on other
 // sequences or on the cutting into steps, beyond rounding (shares and waves follow from the step's sizes).
@@ -62,8 +63,11 @@ __global__ __launch_bounds__(W* TIE_WAVE) void attention_f32_kernel(
   const int heads = min(16, group - 16 * head_tile);         // query heads of a row in this tile
   const int rows = group <= 16 ? 16 / group : 1;             // query rows of a tile
 
-  // The sequence of this column tile: tiles are counted sequence by sequence.
-  int s = blockIdx.y, first_row = 0;
+  // The sequence of this column tile: tiles are counted sequence by sequence. The last ones start first: a portion's late
+  // rows see the most keys, and what a second round of workgroups gets should be short (a prompt of 301 tokens, 304
+  // workgroups of which 256 run at once, 23.3 -> 17.7 us; 400 tokens 29.9 -> 24.4).
+  const int column_tile = static_cast<int>(gridDim.y - 1 - blockIdx.y);
+  int s = column_tile, first_row = 0;
   if (T != S) {
     int before = 0;
     s = -1;
@@ -75,11 +79,11 @@ __global__ __launch_bounds__(W* TIE_WAVE) void attention_f32_kernel(
         const int v = __shfl_up(upto, off, TIE_WAVE);
         if (lane >= off) upto += v;
       }
-      const unsigned long long past = __ballot(before + upto > static_cast<int>(blockIdx.y));
+      const unsigned long long past = __ballot(before + upto > column_tile);
       if (past != 0) {
         const int at = __ffsll(static_cast<long long>(past)) - 1;
         s = base + at;
-        first_row = (static_cast<int>(blockIdx.y) - before - (__shfl(upto, at, TIE_WAVE) - __shfl(mine, at, TIE_WAVE))) * rows;
+        first_row = (column_tile - before - (__shfl(upto, at, TIE_WAVE) - __shfl(mine, at, TIE_WAVE))) * rows;
       }
       before += __shfl(upto, TIE_WAVE - 1, TIE_WAVE);
     }

@@ -1351,11 +1351,19 @@ def attention_f32_tiles(new_tokens, group_size: int) -> int:
 
 
 def attention_f32_splits(tiles: int, num_kv_heads: int, group_size: int, max_context: int) -> int:
-    """Shares the keys of every column tile are cut into: more than one only where the tiles alone leave CUs idle."""
+    """Shares the keys of every column tile are cut into: more than one only where the tiles alone leave CUs idle.
+
+    One workgroup fills a CU, so all of them run at once up to 256: beyond that a second round costs more than shorter
+    shares give (16 sequences of 1000 keys, 8 KV heads: two shares 30.3 us, three 39.4). Up to there a share is down to four
+    tiles of 16 keys, half a tile for each of its waves: what a workgroup starts and ends with and the merge weigh more
+    then (one sequence of 300 keys: 1, 2, 4, 5, 8 shares 15.2, 12.6, 10.8, 9.9, 9.7 us; 24 shares of 4000 keys 16.2,
+    32 of them 17.6). Same in the other head sizes: 256 dimensions, 4 KV heads, 300 keys 22.7 us in one share, 11.3 in ten.
+    """
     workgroups = tiles * num_kv_heads * -(-group_size // 16)
-    by_fill = 512 // max(1, workgroups)
-    by_length = -(-max_context // 16) // 16                 # at least sixteen tiles of 16 keys a share
-    return max(1, min(16, by_fill, by_length))
+    by_fill = 256 // max(1, workgroups)
+    key_tiles = max(1, -(-max_context // 16))
+    shares = max(1, min(24, by_fill, -(-key_tiles // 4)))
+    return -(-key_tiles // -(-key_tiles // shares))         # none of them empty
 
 
 def attention_f32(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, out: torch.Tensor,
