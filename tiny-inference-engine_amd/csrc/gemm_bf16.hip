@@ -290,7 +290,8 @@ static int launch_gemm(const void* x, const void* w, void* out, int epi, int M, 
 // The same product with operand slices going global memory -> LDS directly (gemm_dma.h), for K % 32 == 0 and
 // N % 4 == 0; reads weights row-major or (PW) in packed blocks.
 // BM: 256, 128 or 64 rows of x a workgroup; the waves are 2 x 2 in every case, a wave covering BM / 2 rows.
-template <int BM, int BN, int EPI, bool PW>
+// W_ONCE: w is asked for past the caches, which keep x and the planes then.
+template <int BM, int BN, int EPI, bool PW, bool W_ONCE>
 __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __restrict__ x_all,
                                                             const bf16_t* __restrict__ w_all,
                                                             void* __restrict__ out_all, int M, int N, int K,
@@ -364,7 +365,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
   }
 
   floatx16 acc[TM][TN];
-  gemm_dma_tile<BM, BN, PW>(lds, a_rsrc, a_off, b_rsrc, b_off, b_tile_off, k_tiles, acc);
+  gemm_dma_tile<BM, BN, PW, W_ONCE>(lds, a_rsrc, a_off, b_rsrc, b_off, b_tile_off, k_tiles, acc);
 
   const bool gated_n = EPI == 3 || EPI == 4;
 #pragma unroll
@@ -416,8 +417,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
 #endif
 }
 
-template <int BM, int BN, bool PW>
-static int launch_gemm_dma(const void* x, const void* w, void* out, int epi, int M, int N, int K, int splits,
+template <int BM, int BN, bool PW, bool W_ONCE>
+static int launch_gemm_dma_as(const void* x, const void* w, void* out, int epi, int M, int N, int K, int splits,
                            hipStream_t stream) {
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const int k_slices = K / GD_BK;
@@ -432,17 +433,34 @@ static int launch_gemm_dma(const void* x, const void* w, void* out, int epi, int
   {                                                                                                          \
     static bool raised = false;                                                                              \
     if (!raised) {                                                                                           \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_bf16_dma_kernel<BM, BN, EPI, PW>),  \
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_bf16_dma_kernel<BM, BN, EPI, PW, W_ONCE>),  \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(shared)); \
       if (e != hipSuccess) return static_cast<int>(e);                                                       \
       raised = true;                                                                                         \
     }                                                                                                        \
-    gemm_bf16_dma_kernel<BM, BN, EPI, PW><<<grid, 256, shared, stream>>>(                                    \
+    gemm_bf16_dma_kernel<BM, BN, EPI, PW, W_ONCE><<<grid, 256, shared, stream>>>(                                    \
         static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), out, M, N, K, tiles_m, tiles_n, per_split); \
   }
   if (epi == 0) LAUNCH(0) else if (epi == 1) LAUNCH(1) else if (epi == 2) LAUNCH(2) else if (epi == 3) LAUNCH(3) else LAUNCH(4)
 #undef LAUNCH
   return tie_launch_status();
+}
+
+// Weights of a product that reads them once, or nearly so, go past the caches: one row tile of 64 or 128 rows, two of 64, and
+// tiles of 128 x 192, whose row tiles run beside each other. Cold weights, kept and not kept: 64 rows over 6144 x 4096
+// 14.4 and 13.8 us, over 4096 x 12288 22.3 and 21.1, 128 rows over 24576 x 4096 54.4 and 51.8, over 6144 x 4096 16.9 and
+// 16.0, 512 rows over a gated 12288 x 2048 on 128 x 192 31.3 and 29.8. More row tiles want them back from the L2 (512 rows
+// over 2048 x 2048 in four ranges on 128 x 128 10.6 and 11.5), tiles of 256 rows are the same either way. Rows of
+// row-major weights come as half lines, two loads a line, and stay cached.
+template <int BM, int BN, bool PW>
+static int launch_gemm_dma(const void* x, const void* w, void* out, int epi, int M, int N, int K, int splits,
+                           hipStream_t stream) {
+  if constexpr (PW && (BM == 64 || (BM == 128 && BN == 192))) {
+    return launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream);
+  } else if constexpr (PW && BM == 128) {
+    if (M <= BM) return launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream);
+  }
+  return launch_gemm_dma_as<BM, BN, PW, false>(x, w, out, epi, M, N, K, splits, stream);
 }
 
 // Whether the direct-to-LDS kernel takes this product: whole slices of 32, at least three per range of K,

@@ -61,6 +61,8 @@ struct GdShape {
 // Fourth word of a raw buffer descriptor on gfx9-family GPUs: 32-bit float data format, destination
 // selects x, y, z, w; no swizzle, no stride (the compiler's own default for raw buffers on this target).
 #define GD_RSRC_FLAGS 0x27000
+// The non-temporal bit of a buffer load's cache policy on gfx942 and gfx950.
+#define GD_NT 2
 
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -227,7 +229,7 @@ __device__ __forceinline__ void gemm_dma_tile_x_pairs(bf16_t* lds, const __amdgp
 // PW, lane * 16 with `b_tile_off` the byte offset of block row 4 p + wave. A lane ends with, in acc[i][j], row
 // wm BM / 2 + 32 i + lane % 32 and in word 4 g + v column wn BN / 2 + 32 j + 8 g + 4 (lane / 32) + v, wm = wave / 2 and
 // wn = wave % 2.
-template <int BM, int BN, bool PW>
+template <int BM, int BN, bool PW, bool W_ONCE>
 __device__ __forceinline__ void gemm_dma_tile_groups(bf16_t* lds, const __amdgpu_buffer_rsrc_t a_rsrc,
                                                      const unsigned (&a_off)[BM * GdShape<BM, BN>::X_GROUP / 64],
                                                      const __amdgpu_buffer_rsrc_t b_rsrc, const unsigned (&b_off)[BN / 64],
@@ -267,7 +269,7 @@ __device__ __forceinline__ void gemm_dma_tile_groups(bf16_t* lds, const __amdgpu
 #pragma unroll
       for (int p = 0; p < PB; ++p)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, (lds_void_t*)(buf + (p * 64 + wave * 16) * BK), 16,
-                                                 b_off[p], PW ? b_tile_off[p] + kt * 1024 : kt * BK * 2, 0, 0);
+                                                 b_off[p], PW ? b_tile_off[p] + kt * 1024 : kt * BK * 2, 0, W_ONCE ? GD_NT : 0);
     }
   };
 
@@ -411,7 +413,7 @@ __device__ __forceinline__ void gemm_dma_tile_groups(bf16_t* lds, const __amdgpu
   }
 }
 
-template <int BM, int BN, bool PW>
+template <int BM, int BN, bool PW, bool W_ONCE = false>
 __device__ __forceinline__ void gemm_dma_tile(bf16_t* lds, const __amdgpu_buffer_rsrc_t a_rsrc,
                                               const unsigned (&a_off)[BM * GdShape<BM, BN>::X_GROUP / 64],
                                               const __amdgpu_buffer_rsrc_t b_rsrc, const unsigned (&b_off)[BN / 64],
@@ -420,6 +422,6 @@ __device__ __forceinline__ void gemm_dma_tile(bf16_t* lds, const __amdgpu_buffer
   if constexpr (GdShape<BM, BN>::X_PAIRS)
     gemm_dma_tile_x_pairs<BM, BN, PW>(lds, a_rsrc, a_off, b_rsrc, b_off, b_tile_off, k_tiles, acc);
   else
-    gemm_dma_tile_groups<BM, BN, PW>(lds, a_rsrc, a_off, b_rsrc, b_off, b_tile_off, k_tiles, acc);
+    gemm_dma_tile_groups<BM, BN, PW, W_ONCE>(lds, a_rsrc, a_off, b_rsrc, b_off, b_tile_off, k_tiles, acc);
 }
 #endif
