@@ -21,6 +21,8 @@
 #include "expert_activation.h"
 #include "gemm_dma.h"
 
+typedef uint32_t moe_u32x4_t __attribute__((ext_vector_type(4)));
+
 struct MoeRows {
   const int* offsets;      // [real + 1]: places of each expert's slots
   const int* slot_at;      // [slots]
@@ -68,11 +70,13 @@ __global__ __launch_bounds__(256) void moe_packed_few_rows_kernel(const bf16_t* 
   int kb = wave;
   auto blocks = [&](auto depth, auto first) {                // DEPTH of this wave's k-blocks, every load before the first use
     constexpr int DEPTH = decltype(depth)::value;
-    uint4 xf[DEPTH], wf[NT][DEPTH];
+    uint4 xf[DEPTH];
+    moe_u32x4_t wf[NT][DEPTH];
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) wf[nt][i] = *reinterpret_cast<const uint4*>(wr[nt] + static_cast<size_t>(kb + 4 * i) * 512);
+      for (int nt = 0; nt < NT; ++nt)
+        wf[nt][i] = __builtin_nontemporal_load(reinterpret_cast<const moe_u32x4_t*>(wr[nt] + static_cast<size_t>(kb + 4 * i) * 512));
     __builtin_amdgcn_sched_barrier(0);                       // the weights are on their way before the slot is waited for
     if constexpr (decltype(first)::value) look_up();
 #pragma unroll
