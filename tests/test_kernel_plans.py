@@ -271,6 +271,18 @@ def test_float32_products_of_many_rows_take_pieces():
     assert kernels.gemm_f32_shape(301, 12288, 2048) == 10 and kernels.gemm_f32_shape(48, 12288, 2048) <= 8
 
 
+@pytest.mark.parametrize("M,N,K", [(301, 4096, 2048), (301, 4096, 4096), (160, 6144, 4096), (400, 6144, 4096), (220, 5120, 5120)])
+def test_float32_products_in_three_ranges(M, N, K):
+    """Where three ranges of K fill a round of workgroups better than powers of two: tiles of 256 columns on pieces, ranges of
+    at least 384 of K, and a caller that fixes another number gets that number's shape."""
+    from tie_amd import kernels
+
+    assert kernels.gemm_f32_splits(M, N, K) == 3 and K // 3 >= 384
+    assert kernels.gemm_f32_shape(M, N, K, 3) in (9, 10)
+    for splits in (1, 2, 4):
+        assert 1 <= kernels.gemm_f32_shape(M, N, K, splits) <= 12
+
+
 def test_float32_products_run_on_what_was_fastest():
     """Up to 32 rows no weight takes pieces, in however many ranges of K. (rows, w): the choices within a tenth of the fastest
     one that was timed."""
