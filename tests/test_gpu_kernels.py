@@ -61,6 +61,24 @@ def test_rms_norm(n, out_dtype):
     assert torch.equal(picked, out[rows.long()])
 
 
+@pytest.mark.parametrize("n", [2044, 2048, 2560, 3072, 4096, 5120, 5632, 8192, 16384])
+@pytest.mark.parametrize("R", [511, 512, 1030])
+def test_rms_norm_of_many_rows(R, n):
+    """From 512 rows on a thread has two or four float4 of a row: a row's sum of squares is added in another order there,
+    which the rounding of n terms bounds, n * 6e-8 / 2 of the result at the worst and about its root as a rule."""
+    from tie_amd import kernels
+
+    x = rnd(R, n, seed=2, scale=3.0).cuda()
+    w = (1 + 0.1 * rnd(n, seed=3)).cuda()
+    out = torch.full((R, n), float("nan"), device="cuda")
+    kernels.rms_norm(x, w, 1e-5, out)
+    close(out, plain.rms_norm(x.cpu(), w.cpu(), 1e-5), 1e-6, f"{R} rows of {n}")
+    rows = torch.randperm(R, generator=torch.Generator().manual_seed(5)).to(torch.int32).cuda()
+    picked = torch.full((R, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    kernels.rms_norm(x, w, 1e-5, picked, rows)
+    assert torch.equal(picked, out[rows.long()].bfloat16())
+
+
 def test_swiglu():
     from tie_amd import kernels
 
