@@ -31,6 +31,7 @@
 
 #define DC_ROWS 64                 // tokens of a chunk at most
 #define DC_THREADS 256
+#define DC_PREPARE_THREADS 512
 #define DC_AR (DC_ROWS + 4)        // words from one row of A in LDS to the next
 #define DC_TR 20                   // ... of an inverted diagonal block
 
@@ -80,7 +81,7 @@ struct DeltaChunks {
 
 // WIDE: q and k of every head start on 16-byte addresses and d is a multiple of 4.
 template <bool WIDE>
-__global__ __launch_bounds__(DC_THREADS) void delta_chunk_prepare_kernel(DeltaChunks g) {
+__global__ __launch_bounds__(DC_PREPARE_THREADS) void delta_chunk_prepare_kernel(DeltaChunks g) {
   extern __shared__ __attribute__((aligned(16))) float keys[];             // [64][D + 4]: the chunk's keys
   __shared__ __attribute__((aligned(16))) float A[DC_ROWS * DC_AR];
   __shared__ __attribute__((aligned(16))) float inv[4][16 * DC_TR];        // (I + A_rr)^-1 of the diagonal blocks
@@ -117,50 +118,62 @@ __global__ __launch_bounds__(DC_THREADS) void delta_chunk_prepare_kernel(DeltaCh
     if (lane == TIE_WAVE - 1) g.decay[entry] = e_b;
   }
   const int kr = g.D + 4, quads = g.D / 4, blocks = g.D / 16;
-  for (int i = threadIdx.x; i < DC_ROWS * quads; i += DC_THREADS) {      // rows behind the chunk's end: the last one's
+  for (int i = threadIdx.x; i < DC_ROWS * quads; i += DC_PREPARE_THREADS) {      // rows behind the chunk's end: the last one's
     const int t = i / quads, c = (i % quads) * 4;
     *reinterpret_cast<float4*>(keys + t * kr + c) =
         dc_load4<WIDE>(rows + static_cast<size_t>(min(t, n - 1)) * g.row + k_at, c, g.d);
   }
   __syncthreads();
-  // rows 16 tile .. of K K^T and Q K^T; which wave has the longest rows turns with the workgroup
+  // rows 16 tile .. of K K^T (the first four waves) and of Q K^T (the others); which wave has the longest rows turns with the
+  // workgroup
   const int tile = (wave + blockIdx.x) & 3;
-  dc_floatx4 kk[4], qk[4];
+  dc_floatx4 acc[4];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) kk[nt] = qk[nt] = dc_floatx4{0.f, 0.f, 0.f, 0.f};
-  const float* own = rows + static_cast<size_t>(min(tile * 16 + r16, n - 1)) * g.row + q_at;
-  const float own_eb = eb[tile * 16 + r16];
-  float* qe = g.q + (entry * 4 + tile) * blocks * 256 + lane * 4;
-#pragma unroll 2
-  for (int kb = 0; kb < blocks; ++kb) {
-    const int i0 = kb * 16 + quad * 4;
-    const float4 qa = dc_load4<WIDE>(own, i0, g.d);
-    const float4 ka = *reinterpret_cast<const float4*>(keys + (tile * 16 + r16) * kr + i0);
-    *reinterpret_cast<float4*>(qe + kb * 256) = make_float4(qa.x * own_eb, qa.y * own_eb, qa.z * own_eb, qa.w * own_eb);
+  for (int nt = 0; nt < 4; ++nt) acc[nt] = dc_floatx4{0.f, 0.f, 0.f, 0.f};
+  auto products = [&](int kb, float4 a) {
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
       if (nt > tile) continue;
-      const float4 v = *reinterpret_cast<const float4*>(keys + (nt * 16 + r16) * kr + i0);
-      const dc_floatx4 kv4 = {v.x, v.y, v.z, v.w};
-      kk[nt] = dc_mfma4(ka, kv4, kk[nt]);
-      qk[nt] = dc_mfma4(qa, kv4, qk[nt]);
+      const float4 v = *reinterpret_cast<const float4*>(keys + (nt * 16 + r16) * kr + kb * 16 + quad * 4);
+      acc[nt] = dc_mfma4(a, dc_floatx4{v.x, v.y, v.z, v.w}, acc[nt]);
     }
-  }
+  };
   float* pe = g.p + entry * DC_ROWS * DC_ROWS;
+  // e^(b_i - b_j) of the lane's elements of block nt, 0 above the diagonal and behind the chunk's end
+  auto decay = [&](int i, int j) { return i < n && j <= i ? expf(static_cast<float>(b[i] - b[j])) : 0.f; };
+  if (wave < 4) {
+#pragma unroll 2
+    for (int kb = 0; kb < blocks; ++kb)
+      products(kb, *reinterpret_cast<const float4*>(keys + (tile * 16 + r16) * kr + kb * 16 + quad * 4));
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const int j = nt * 16 + r16;
+    for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = tile * 16 + quad * 4 + r;
-      const bool in = i < n && j <= i;
-      const float f = in ? expf(static_cast<float>(b[i] - b[j])) : 0.f;
-      A[i * DC_AR + j] = in && j < i ? beta[i] * f * kk[nt][r] : 0.f;
-      pe[(tile * 4 + nt) * 256 + (r16 / 4) * 64 + (quad * 4 + r) * 4 + r16 % 4] = in ? f * qk[nt][r] : 0.f;
+      for (int r = 0; r < 4; ++r) {
+        const int i = tile * 16 + quad * 4 + r, j = nt * 16 + r16;
+        const float f = decay(i, j);
+        A[i * DC_AR + j] = i < n && j < i ? beta[i] * f * acc[nt][r] : 0.f;
+      }
+  } else {
+    const float* own = rows + static_cast<size_t>(min(tile * 16 + r16, n - 1)) * g.row + q_at;
+    const float own_eb = eb[tile * 16 + r16];
+    float* qe = g.q + (entry * 4 + tile) * blocks * 256 + lane * 4;
+#pragma unroll 2
+    for (int kb = 0; kb < blocks; ++kb) {
+      const float4 qa = dc_load4<WIDE>(own, kb * 16 + quad * 4, g.d);
+      *reinterpret_cast<float4*>(qe + kb * 256) = make_float4(qa.x * own_eb, qa.y * own_eb, qa.z * own_eb, qa.w * own_eb);
+      products(kb, qa);
     }
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = tile * 16 + quad * 4 + r, j = nt * 16 + r16;
+        const float f = decay(i, j);
+        pe[(tile * 4 + nt) * 256 + (r16 / 4) * 64 + (quad * 4 + r) * 4 + r16 % 4] = i < n && j <= i ? f * acc[nt][r] : 0.f;
+      }
   }
   __syncthreads();
-  {     // wave r inverts diagonal block r, a lane a column (the four quads the same ones)
+  if (wave < 4) {     // wave r inverts diagonal block r, a lane a column (the four quads the same ones)
     const float* Ar = A + wave * 16 * DC_AR + wave * 16;
     float x[16];
 #pragma unroll
@@ -193,7 +206,7 @@ __global__ __launch_bounds__(DC_THREADS) void delta_chunk_prepare_kernel(DeltaCh
     }
   }
   // 16 columns of [diag(beta) V | diag(beta e^b) K] a wave at a time
-  for (int nt = wave; nt * 16 < g.ep + g.D; nt += 4) {
+  for (int nt = wave; nt * 16 < g.ep + g.D; nt += DC_PREPARE_THREADS / TIE_WAVE) {
     const bool is_k = nt * 16 >= g.ep;
     const int c = nt * 16 - (is_k ? g.ep : 0) + r16;
     const bool live = c < (is_k ? g.d : g.e);
@@ -449,8 +462,8 @@ extern "C" int tie_delta_chunks(const float* tok, int row, float* out, int out_r
     }
     raised = true;
   }
-  if (wide) delta_chunk_prepare_kernel<true><<<static_cast<unsigned>(entries), DC_THREADS, lds, stream>>>(g);
-  else delta_chunk_prepare_kernel<false><<<static_cast<unsigned>(entries), DC_THREADS, lds, stream>>>(g);
+  if (wide) delta_chunk_prepare_kernel<true><<<static_cast<unsigned>(entries), DC_PREPARE_THREADS, lds, stream>>>(g);
+  else delta_chunk_prepare_kernel<false><<<static_cast<unsigned>(entries), DC_PREPARE_THREADS, lds, stream>>>(g);
   int rc = tie_launch_status();
   if (rc != TIE_OK) return rc;
   const int pairs = num_seqs * heads;
