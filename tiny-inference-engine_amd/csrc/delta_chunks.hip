@@ -29,6 +29,8 @@
 // kernel took 101 us of a 2048-token prompt of 16 heads.)
 #include "common.h"
 
+#include <type_traits>
+
 #define DC_ROWS 64                 // tokens of a chunk at most
 #define DC_THREADS 256
 #define DC_PREPARE_THREADS 512
@@ -59,6 +61,25 @@ __device__ __forceinline__ dc_floatx4 dc_mfma4(float4 a, dc_floatx4 b, dc_floatx
   c = dc_mfma(a.y, b[1], c);
   c = dc_mfma(a.z, b[2], c);
   return dc_mfma(a.w, b[3], c);
+}
+
+// Four lanes' four values each, transposed: lane a of them ends with everyone's value a, in the order of the lanes.
+__device__ __forceinline__ float4 dc_transpose4(float v0, float v1, float v2, float v3, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  auto across = [](float v, auto control) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), decltype(control)::value, 0xf, 0xf, true));
+  };
+  constexpr std::integral_constant<int, 0xB1> by_one{};     // lanes 1 0 3 2 of every four
+  constexpr std::integral_constant<int, 0x4E> by_two{};     // lanes 2 3 0 1
+  const bool odd = lane & 1, upper = lane & 2;
+  const float a = across(odd ? v0 : v1, by_one), b = across(odd ? v2 : v3, by_one);
+  v0 = odd ? a : v0, v1 = odd ? v1 : a, v2 = odd ? b : v2, v3 = odd ? v3 : b;
+  const float c = across(upper ? v0 : v2, by_two), d = across(upper ? v1 : v3, by_two);
+  v0 = upper ? c : v0, v2 = upper ? v2 : c, v1 = upper ? d : v1, v3 = upper ? v3 : d;
+  return make_float4(v0, v1, v2, v3);
+#else
+  return make_float4(v0, v1, v2, v3);
+#endif
 }
 
 // A launch's geometry and the chunks' memory; entry (chunk * heads + head - head0) of each array.
@@ -164,13 +185,17 @@ __global__ __launch_bounds__(DC_PREPARE_THREADS) void delta_chunk_prepare_kernel
       products(kb, qa);
     }
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < 4; ++nt) {
+      float p[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int i = tile * 16 + quad * 4 + r, j = nt * 16 + r16;
         const float f = decay(i, j);
-        pe[(tile * 4 + nt) * 256 + (r16 / 4) * 64 + (quad * 4 + r) * 4 + r16 % 4] = i < n && j <= i ? f * acc[nt][r] : 0.f;
+        p[r] = i < n && j <= i ? f * acc[nt][r] : 0.f;
       }
+      *reinterpret_cast<float4*>(pe + (tile * 4 + nt) * 256 + (r16 / 4) * 64 + (quad * 4 + r16 % 4) * 4) =
+          dc_transpose4(p[0], p[1], p[2], p[3], lane);
+    }
   }
   __syncthreads();
   if (wave < 4) {     // wave r inverts diagonal block r, a lane a column (the four quads the same ones)
@@ -240,9 +265,9 @@ __global__ __launch_bounds__(DC_PREPARE_THREADS) void delta_chunk_prepare_kernel
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       if (is_k) {
-        float* dst = g.w + ((entry * 4 + r) * blocks + c / 16) * 256 + (r16 / 4) * 64 + r16 % 4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dst[(quad * 4 + i) * 4] = x[r][i];
+        // an A operand's block: row 4 quad + r16 % 4, its columns 4 (r16 / 4) .. + 3
+        *reinterpret_cast<float4*>(g.w + ((entry * 4 + r) * blocks + c / 16) * 256 + (r16 / 4) * 64 + (quad * 4 + r16 % 4) * 4) =
+            dc_transpose4(x[r][0], x[r][1], x[r][2], x[r][3], lane);
       } else {
         *reinterpret_cast<float4*>(g.u + ((entry * (g.ep / 16) + nt) * 4 + r) * 256 + lane * 4) =
             make_float4(x[r][0], x[r][1], x[r][2], x[r][3]);
