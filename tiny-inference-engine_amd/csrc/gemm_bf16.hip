@@ -455,12 +455,13 @@ static int launch_gemm_dma_as(const void* x, const void* w, void* out, int epi, 
 template <int BM, int BN, bool PW>
 static int launch_gemm_dma(const void* x, const void* w, void* out, int epi, int M, int N, int K, int splits,
                            hipStream_t stream) {
-  if constexpr (PW && (BM == 64 || (BM == 128 && BN == 192))) {
+  if constexpr (PW && (BM == 64 || (BM == 128 && BN == 192)))
     return launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream);
-  } else if constexpr (PW && BM == 128) {
-    if (M <= BM) return launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream);
-  }
-  return launch_gemm_dma_as<BM, BN, PW, false>(x, w, out, epi, M, N, K, splits, stream);
+  else if constexpr (PW && BM == 128)
+    return M <= BM ? launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream)
+                   : launch_gemm_dma_as<BM, BN, PW, false>(x, w, out, epi, M, N, K, splits, stream);
+  else
+    return launch_gemm_dma_as<BM, BN, PW, false>(x, w, out, epi, M, N, K, splits, stream);
 }
 
 // Whether the direct-to-LDS kernel takes this product: whole slices of 32, at least three per range of K,
