@@ -451,15 +451,15 @@ static int launch_gemm_dma_as(const void* x, const void* w, void* out, int epi, 
 // 14.4 and 13.8 us, over 4096 x 12288 22.3 and 21.1, 128 rows over 24576 x 4096 54.4 and 51.8, over 6144 x 4096 16.9 and
 // 16.0, 512 rows over a gated 12288 x 2048 on 128 x 192 31.3 and 29.8. More row tiles want them back from the L2 (120 rows on
 // the 1.7B shape, two tiles of 64: a step 2025 and 2068 us; 512 rows
-// over 2048 x 2048 in four ranges on 128 x 128 10.6 and 11.5), tiles of 256 rows are the same either way. Rows of
-// row-major weights come as half lines, two loads a line, and stay cached.
+// over 2048 x 2048 in four ranges on 128 x 128 10.6 and 11.5), tiles of 256 rows are the same either way. Weights under 32 MB
+// are the same by themselves and lose in a step (64 sequences on the 1.7B shape 1921 and 1931 us). Rows of row-major weights come as half lines, two loads a line, and stay cached.
 template <int BM, int BN, bool PW>
 static int launch_gemm_dma(const void* x, const void* w, void* out, int epi, int M, int N, int K, int splits,
                            hipStream_t stream) {
   if constexpr (PW && BM == 128 && BN == 192)
     return launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream);
   else if constexpr (PW && BM <= 128)
-    return M <= BM ? launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream)
+    return M <= BM && static_cast<long>(N) * K >= 1L << 24 ? launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream)
                    : launch_gemm_dma_as<BM, BN, PW, false>(x, w, out, epi, M, N, K, splits, stream);
   else
     return launch_gemm_dma_as<BM, BN, PW, false>(x, w, out, epi, M, N, K, splits, stream);
