@@ -89,7 +89,7 @@ def test_gemm_f32_on_pieces(shape, M, N, K):
     acc = base.clone()
     kernels.gemm_f32(x, w, acc, accumulate=True, shape=shape)
     close(acc, want + base.cpu().to(F64), 6e-6, "added to what was there")
-    for splits in (2, 16):
+    for splits in (2, 3, 16):
         planes = torch.full((splits, M, N), float("nan"), device="cuda")
         kernels.gemm_f32(x, w, planes, splits=splits, shape=shape)
         close(planes.sum(0), want, 6e-6, f"{splits} planes")
@@ -104,6 +104,25 @@ def test_gemm_f32_on_pieces(shape, M, N, K):
     kernels.gemm_f32(x, w, out2, shape=shape)
     assert not bool(torch.isfinite(out2[0]).any()) and bool(torch.isnan(out2[:, 0]).all())
     assert torch.equal(out2[1:, 1:], out[1:, 1:])
+
+
+def test_gemm_f32_cut_in_three_by_its_plan():
+    """301 rows over 4096 x 2048: 22, 22 and 20 slices of 32 k. The planes' sum, and what the norm that adds them makes of it;
+    the same bound as above."""
+    from tie_amd import kernels
+
+    M, N, K = 301, 4096, 2048
+    assert kernels.gemm_f32_splits(M, N, K) == 3
+    x, w, base = rnd(M, K, seed=M), rnd(N, K, seed=N, scale=0.1), rnd(M, N, seed=7)
+    want = plain.linear(x, w)
+    planes = torch.full((3, M, N), float("nan"), device="cuda")
+    kernels.gemm_f32(x.cuda(), w.cuda(), planes, splits=3)
+    close(planes.sum(0), want, 6e-6, "three planes")
+    weight, stream, normed = (1 + 0.1 * rnd(N, seed=3)).cuda(), base.cuda(), torch.full((M, N), float("nan"), device="cuda")
+    kernels.add_partials(stream, planes, weight, 1e-6, normed)
+    total = want.double() + base.double()
+    close(stream, total, 6e-6, "the stream with three planes")
+    close(normed, plain.rms_norm(total.float(), weight.cpu(), 1e-6), 6e-6, "its norm")
 
 
 @pytest.mark.parametrize("shape", [9, 10, 11, 12])

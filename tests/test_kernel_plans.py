@@ -271,16 +271,31 @@ def test_float32_products_of_many_rows_take_pieces():
     assert kernels.gemm_f32_shape(301, 12288, 2048) == 10 and kernels.gemm_f32_shape(48, 12288, 2048) <= 8
 
 
-@pytest.mark.parametrize("M,N,K", [(301, 4096, 2048), (301, 4096, 4096), (160, 6144, 4096), (400, 6144, 4096), (220, 5120, 5120)])
-def test_float32_products_in_three_ranges(M, N, K):
+@pytest.mark.parametrize("M,N,K,powers", [(301, 4096, 2048, (12, 10, 10)), (180, 6144, 4096, (5, 10, 10)), (350, 3072, 3072, (5, 10, 10)),
+                                          (530, 4096, 2048, (10, 10, 10))])
+def test_float32_products_in_three_ranges(M, N, K, powers):
     """Where three ranges of K fill a round of workgroups better than powers of two: tiles of 256 columns on pieces, ranges of
-    at least 384 of K, and a caller that fixes another number gets that number's shape."""
+    at least 384 of K, and a caller that fixes 1, 2 or 4 ranges gets that number's shape."""
     from tie_amd import kernels
 
     assert kernels.gemm_f32_splits(M, N, K) == 3 and K // 3 >= 384
     assert kernels.gemm_f32_shape(M, N, K, 3) in (9, 10)
-    for splits in (1, 2, 4):
-        assert 1 <= kernels.gemm_f32_shape(M, N, K, splits) <= 12
+    assert tuple(kernels.gemm_f32_shape(M, N, K, splits) for splits in (1, 2, 4)) == powers
+
+
+@pytest.mark.parametrize("N,K,rows", [(4096, 4096, {301: 8, 513: 8, 600: 8}), (6144, 4096, {140: 8, 321: 8, 384: 8, 400: 4, 700: 4}),
+                                      (4096, 12288, {300: 8, 529: 8, 600: 8, 900: 8}), (4096, 2048, {301: 4, 513: 4, 587: 4, 640: 4}),
+                                      (2048, 6144, {600: 8}), (5120, 5120, {220: 8, 400: 8, 500: 8, 800: 4}),
+                                      (3072, 3072, {641: 8, 700: 4}), (7168, 5120, {160: 8, 270: 8, 350: 4, 600: 4})])
+def test_float32_products_in_three_ranges_sum_in_no_fewer_chains(N, K, rows):
+    """Beside the chains of sums (groups of waves along K, times ranges of K) of the best choice among powers of two: three
+    ranges, where they are taken, have as many at least. The error of a sum grows with the length of its chains."""
+    from tie_amd import kernels
+
+    for M, chains in rows.items():
+        splits = kernels.gemm_f32_splits(M, N, K)
+        shape = kernels.gemm_f32_shape(M, N, K, splits)
+        assert shape > 8 and (1, 2, 1, 2)[shape - 9] * splits >= chains, (M, N, K, splits, shape, chains)
 
 
 def test_float32_products_run_on_what_was_fastest():
