@@ -275,12 +275,24 @@ def test_float32_products_of_many_rows_take_pieces():
                                           (530, 4096, 2048, (10, 10, 10))])
 def test_float32_products_in_three_ranges(M, N, K, powers):
     """Where three ranges of K fill a round of workgroups better than powers of two: tiles of 256 columns on pieces, ranges of
-    at least 384 of K, and a caller that fixes 1, 2 or 4 ranges gets that number's shape."""
+    at least 384 of K, all workgroups at once on the fullest die too, and a caller that fixes 1, 2 or 4 ranges gets that
+    number's shape."""
     from tie_amd import kernels
 
     assert kernels.gemm_f32_splits(M, N, K) == 3 and K // 3 >= 384
-    assert kernels.gemm_f32_shape(M, N, K, 3) in (9, 10)
+    shape = kernels.gemm_f32_shape(M, N, K, 3)
+    assert shape in (9, 10) and -(-M // 64) * -(-3 * N // (8 * 256)) <= 32 * (2, 1)[shape - 9]
     assert tuple(kernels.gemm_f32_shape(M, N, K, splits) for splits in (1, 2, 4)) == powers
+
+
+@pytest.mark.parametrize("M,N,K", [(400, 3072, 2048), (440, 3072, 2048), (420, 3072, 3072), (380, 6144, 2560), (600, 4096, 2048),
+                                   (350, 7168, 5120), (720, 7168, 5120), (850, 3072, 8192), (470, 5120, 3072)])
+def test_float32_products_are_not_cut_in_three_for_a_second_round(M, N, K):
+    """A die takes whole pieces of w: three ranges that leave one of them with more workgroups than run at once took up to
+    1.4 times as long (400 rows over 3072 x 2048, 35 on a die of 32 compute units: 68.6 us, in two ranges 50.1)."""
+    from tie_amd import kernels
+
+    assert kernels.gemm_f32_splits(M, N, K) in (1, 2, 4, 8)
 
 
 @pytest.mark.parametrize("N,K,rows", [(4096, 4096, {301: 8, 513: 8, 600: 8}), (6144, 4096, {140: 8, 321: 8, 384: 8, 400: 4, 700: 4}),
