@@ -684,6 +684,36 @@ def test_tiles_that_stage_two_slices_at_a_time(M, N, slices):
                 assert torch.equal(torch.nan_to_num(out, nan=1e30), torch.nan_to_num(want, nan=1e30)), (tile, splits)
 
 
+@pytest.mark.parametrize("tile,splits,N,K,rows", [
+    (6, 1, 4096, 4096, (1, 65, 128, 129)), (6, 4, 4096, 4096, (65, 128)), (7, 1, 4096, 4096, (1, 65, 128, 129)), (7, 4, 4080, 4096, (128,)),
+    (7, 4, 4096, 4096, (65, 128)), (8, 1, 4096, 4096, (1, 64, 65)), (8, 4, 4096, 4096, (64,)), (9, 1, 4096, 4096, (1, 64, 65)),
+    (9, 8, 4096, 4096, (64,)), (9, 8, 4080, 4096, (64,)), (11, 1, 1536, 1536, (128, 200, 256, 384, 900, 1100)), (11, 2, 1536, 1024, (256, 300, 1100)),
+    (11, 1, 1552, 1536, (256,))])
+def test_weights_past_the_caches_change_no_bit(tile, splits, N, K, rows):
+    """Packed weights on both sides of the rule that sends their loads past the caches, in every epilogue, against the
+    row-major ones, whose loads are never sent there."""
+    from tie_amd import kernels
+
+    w = rnd(N, K, seed=71, scale=0.1, dtype=torch.bfloat16).cuda()
+    packed, seen = kernels.pack_weight(w), set()
+    for M in rows:
+        seen.add(kernels.gemm_weights_past_caches(M, N, K, tile, splits))
+        x = rnd(M, K, seed=72 + M, dtype=torch.bfloat16).cuda()
+        ways = [dict(splits=splits)] if splits > 1 else [{}, dict(accumulate=True), dict(gated=1), dict(gated=2), dict(half=True)]
+        for way in ways:
+            gated, half = way.get("gated", 0), way.pop("half", False)
+            shape = (splits, M, N) if splits > 1 else (M, N // 2 if gated else N)
+            outs = []
+            for weight in (w, packed):
+                out = torch.ones(shape, dtype=torch.bfloat16 if gated or half else torch.float32, device="cuda")
+                kernels.gemm_bf16(x, weight, out, tile=tile, **way)
+                outs.append(out)
+            assert torch.equal(*outs), (tile, splits, M, way, half)
+            if splits == 1 and not way and not half:
+                close(outs[1], plain.linear(x.cpu(), w.cpu()), 1e-5, f"tile {tile}, {M} rows")
+    assert seen == ({False} if N in (4080, 1552) else {True} if splits > 1 and tile != 11 else {True, False})
+
+
 @pytest.mark.parametrize("N,K", [(16, 96), (48, 128), (208, 4096), (1024, 352)])
 def test_packed_weight_feeds_both_products_the_same_numbers(N, K):
     """The blocked weight layout changes where bytes lie, not one sum: results equal the row-major ones bit for bit."""

@@ -177,6 +177,22 @@ def test_the_tiled_product_plans_by_rounds_of_workgroups():
     assert kernels.gemm_splits(128, 4096, 4096) == 8 and kernels.gemm_splits(128, 4096, 256) == 1
 
 
+@pytest.mark.parametrize("tile,splits,M,N,K,past", [
+    (7, 4, 128, 4096, 4096, True), (7, 4, 128, 4080, 4096, False), (7, 4, 129, 4096, 4096, False), (9, 8, 64, 4096, 4096, True),
+    (9, 8, 65, 4096, 4096, False), (6, 1, 100, 51200, 5120, True), (8, 1, 40, 65520, 3072, True), (10, 1, 256, 24576, 4096, False),
+    (11, 2, 512, 6144, 4096, True), (11, 1, 256, 24576, 4096, True), (11, 1, 512, 12288, 2048, True), (11, 4, 256, 3072, 8192, True),
+    (11, 1, 160, 24576, 4096, True), (11, 1, 450, 10240, 5120, False),
+    (11, 1, 200, 19456, 2560, False), (11, 1, 200, 17920, 1536, False), (11, 1, 400, 10240, 5120, False),
+    (11, 1, 900, 5120, 3072, False), (11, 1, 1107, 4096, 2048, False), (11, 1, 1200, 3584, 3584, False), (11, 1, 3000, 6144, 4096, False)])
+def test_packed_weights_go_past_the_caches_where_they_are_read_once(tile, splits, M, N, K, past):
+    """One row tile of 64 or 128 rows over 32 MB and more; on 128 x 192 row tiles that run beside each other on one die: tiles
+    a multiple of eight, at most eight of them along M, the last one full enough for the length of a range. Those at the end
+    took 3 to 10 us longer past the caches."""
+    from tie_amd import kernels
+
+    assert kernels.gemm_weights_past_caches(M, N, K, tile, splits) == past
+
+
 @pytest.mark.parametrize("M,N,K,want", [(2048, 4096, 12288, (1, 5)), (2048, 4096, 4096, (1, 5)), (2048, 2048, 6144, (2, 5)),
                                         (512, 4096, 12288, (4, 5)), (512, 2048, 2048, (4, 7))])
 def test_products_that_add_to_the_stream_have_a_plan_of_their_own(M, N, K, want):

@@ -290,7 +290,7 @@ static int launch_gemm(const void* x, const void* w, void* out, int epi, int M, 
 // The same product with operand slices going global memory -> LDS directly (gemm_dma.h), for K % 32 == 0 and
 // N % 4 == 0; reads weights row-major or (PW) in packed blocks.
 // BM: 256, 128 or 64 rows of x a workgroup; the waves are 2 x 2 in every case, a wave covering BM / 2 rows.
-// W_ONCE: w is asked for past the caches, which keep x and the planes then.
+// W_ONCE: w is asked for past the caches (w_past_caches).
 template <int BM, int BN, int EPI, bool PW, bool W_ONCE>
 __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __restrict__ x_all,
                                                             const bf16_t* __restrict__ w_all,
@@ -446,23 +446,36 @@ static int launch_gemm_dma_as(const void* x, const void* w, void* out, int epi, 
   return tie_launch_status();
 }
 
-// Weights of a product that reads them once, or nearly so, go past the caches: one row tile of 64 or 128 rows, and tiles of
-// 128 x 192, whose row tiles run beside each other. Cold weights, kept and not kept: 64 rows over 6144 x 4096
-// 14.4 and 13.8 us, over 4096 x 12288 22.3 and 21.1, 128 rows over 24576 x 4096 54.4 and 51.8, over 6144 x 4096 16.9 and
-// 16.0, 512 rows over a gated 12288 x 2048 on 128 x 192 31.3 and 29.8. More row tiles want them back from the L2 (120 rows on
-// the 1.7B shape, two tiles of 64: a step 2025 and 2068 us; 512 rows
-// over 2048 x 2048 in four ranges on 128 x 128 10.6 and 11.5), tiles of 256 rows are the same either way. Weights under 32 MB
-// are the same by themselves and lose in a step (64 sequences on the 1.7B shape 1921 and 1931 us). Rows of row-major weights come as half lines, two loads a line, and stay cached.
+// Whether a product over packed weights asks for them past the caches, which keep x and the planes then. Whole steps, all
+// weights cold, one product's loads changed at a time:
+//   * one row tile of 64 or 128 rows reads a weight once. 65 to 128 rows 4.6 to 5.5 % less a step on the 8B shape, 6.2 to 8.5
+//     on the 14B, 11.5 to 12.1 on the 32B (51200 x 5120 17 to 20 us a product, 6144 x 4096 0.7 to 1.2); weights under 32 MB
+//     lose (64 sequences on the 1.7B shape 1921 us kept and 1931).
+//   * tiles of 128 x 192 only where a die has all row tiles of a piece of w (tiles a multiple of eight), up to eight of them,
+//     and they stay together: from four on a last one with few rows runs ahead, by the more the longer the range, and the
+//     others find nothing in the L2 of what it read. Inside the rule 512 rows over 6144 x 4096 2.6 us less, 256 over 24576 x 4096 2.1, 400
+//     over 12288 x 2048 0.5; 75 products 55 us less and 5.0 more, 1.2 the worst. Outside it 200 rows over 19456 x 2560 5.3 us
+//     more, 200 over 17920 x 1536 2.8, 400 over 10240 x 5120 10.3, 1107 over 4096 x 2048 7.8 (a step 3.7 %).
+// More row tiles of the others want w back from the L2 (512 rows over 2048 x 2048 in four ranges on 128 x 128 10.6 us kept and
+// 11.5); tiles of 256 rows are the same either way. Rows of row-major weights come as half lines, two loads a line, and stay
+// cached.
+static bool w_past_caches(int bm, int bn, int M, int N, int K, int splits) {
+  const long tiles_m = (M + bm - 1) / bm, tiles = tiles_m * ((N + bn - 1) / bn);
+  if (bm == 128 && bn == 192) {
+    const int per_split = (K / GD_BK + splits - 1) / splits;
+    return tiles % GB_XCDS == 0 && tiles_m <= 8 && (tiles_m <= 3 || (tiles_m * bm - M) * per_split <= 44L * bm);
+  }
+  return bm <= 128 && tiles_m == 1 && static_cast<long>(N) * K >= 1L << 24;
+}
+
 template <int BM, int BN, bool PW>
 static int launch_gemm_dma(const void* x, const void* w, void* out, int epi, int M, int N, int K, int splits,
                            hipStream_t stream) {
-  if constexpr (PW && BM == 128 && BN == 192)
-    return launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream);
-  else if constexpr (PW && BM <= 128)
-    return M <= BM && static_cast<long>(N) * K >= 1L << 24 ? launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream)
-                   : launch_gemm_dma_as<BM, BN, PW, false>(x, w, out, epi, M, N, K, splits, stream);
-  else
-    return launch_gemm_dma_as<BM, BN, PW, false>(x, w, out, epi, M, N, K, splits, stream);
+  if constexpr (PW && BM <= 128) {
+    if (w_past_caches(BM, BN, M, N, K, splits))
+      return launch_gemm_dma_as<BM, BN, PW, true>(x, w, out, epi, M, N, K, splits, stream);
+  }
+  return launch_gemm_dma_as<BM, BN, PW, false>(x, w, out, epi, M, N, K, splits, stream);
 }
 
 // Whether the direct-to-LDS kernel takes this product: whole slices of 32, at least three per range of K,
@@ -648,6 +661,13 @@ extern "C" int tie_gemm_bf16_adding_plan(int M, int N, int K, int* tile) {
 // fixed by the caller (1: none) or 0 for the plan's own number; for tests and sweeps.
 extern "C" int tie_gemm_bf16_tile(int M, int N, int K, int packed, int splits) {
   return gemm_plan(M, N, K, straight_to_lds_shape(N, K), splits, packed != 0).tile;
+}
+
+// Whether that product over packed weights, on tile 4 to 11, asks for them past the caches; for tests and sweeps.
+extern "C" int tie_gemm_bf16_w_past_caches(int M, int N, int K, int tile, int splits) {
+  static const int rows[] = {256, 256, 128, 128, 64, 64, 256, 128}, columns[] = {256, 128, 256, 128, 256, 128, 192, 192};
+  if (tile < 4 || tile > 11 || M <= 0 || splits < 1) return 0;
+  return w_past_caches(rows[tile - 4], columns[tile - 4], M, N, K, splits);
 }
 
 // out_dtype: TIE_F32 or TIE_BF16; accumulate adds into a float32 output; gated (bfloat16 output of N / 2

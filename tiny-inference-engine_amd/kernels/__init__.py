@@ -248,6 +248,7 @@ _SIGNATURES = {
         "tie_gemm_bf16_splits": [_c_int, _c_int, _c_int, _c_int],
         "tie_gemm_bf16_adding_plan": [_c_int, _c_int, _c_int, ctypes.POINTER(_c_int)],
         "tie_gemm_bf16_tile": [_c_int, _c_int, _c_int, _c_int, _c_int],
+        "tie_gemm_bf16_w_past_caches": [_c_int, _c_int, _c_int, _c_int, _c_int],
         "tie_gemm_bf16_wins_few_rows": [_c_int, _c_int, _c_int, _c_int, _c_int],
         "tie_gemm_bf16": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                           _c_int, _c_void],
@@ -1051,6 +1052,11 @@ def gemm_adding_plan(M: int, N: int, K: int) -> tuple:
 def gemm_tile(M: int, N: int, K: int, packed: bool = False, splits: int = 0) -> int:
     """The tile (``gemm_bf16``'s numbering) a product left to choose runs on, with ``splits`` ranges of K fixed (0: the plan's own)."""
     return int(_lib("gemm_bf16").tie_gemm_bf16_tile(M, N, K, int(packed), splits))
+
+
+def gemm_weights_past_caches(M: int, N: int, K: int, tile: int, splits: int = 1) -> bool:
+    """Whether ``gemm_bf16`` on ``tile`` (4 to 11) asks for a packed ``[N, K]`` weight past the caches."""
+    return bool(_lib("gemm_bf16").tie_gemm_bf16_w_past_caches(M, N, K, tile, splits))
 
 
 def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool = False, tile: int = 0,
