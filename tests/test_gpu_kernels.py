@@ -685,10 +685,10 @@ def test_tiles_that_stage_two_slices_at_a_time(M, N, slices):
 
 
 @pytest.mark.parametrize("tile,splits,N,K,rows", [
-    (6, 1, 4096, 4096, (1, 65, 128, 129)), (6, 4, 4096, 4096, (65, 128)), (7, 1, 4096, 4096, (1, 65, 128, 129)), (7, 4, 4080, 4096, (128,)),
-    (7, 4, 4096, 4096, (65, 128)), (8, 1, 4096, 4096, (1, 64, 65)), (8, 4, 4096, 4096, (64,)), (9, 1, 4096, 4096, (1, 64, 65)),
-    (9, 8, 4096, 4096, (64,)), (9, 8, 4080, 4096, (64,)), (11, 1, 1536, 1536, (128, 200, 256, 384, 900, 1100)), (11, 2, 1536, 1024, (256, 300, 1100)),
-    (11, 1, 1552, 1536, (256,))])
+    (6, 1, 4096, 4096, (1, 65, 128, 129)), (6, 4, 4096, 4096, (65, 128)), (7, 1, 4096, 4096, (1, 65, 128, 129)),
+    (7, 4, 4080, 4096, (128,)), (7, 4, 4096, 4096, (65, 128)), (8, 1, 4096, 4096, (1, 64, 65)), (8, 4, 4096, 4096, (64,)),
+    (9, 1, 4096, 4096, (1, 64, 65)), (9, 8, 4096, 4096, (64,)), (9, 8, 4080, 4096, (64,)),
+    (11, 1, 1536, 1536, (128, 200, 256, 384, 900, 1100)), (11, 2, 1536, 1024, (256, 300, 1100)), (11, 1, 1552, 1536, (256,))])
 def test_weights_past_the_caches_change_no_bit(tile, splits, N, K, rows):
     """Packed weights on both sides of the rule that sends their loads past the caches, in every epilogue, against the
     row-major ones, whose loads are never sent there."""
@@ -709,9 +709,30 @@ def test_weights_past_the_caches_change_no_bit(tile, splits, N, K, rows):
                 kernels.gemm_bf16(x, weight, out, tile=tile, **way)
                 outs.append(out)
             assert torch.equal(*outs), (tile, splits, M, way, half)
-            if splits == 1 and not way and not half:
-                close(outs[1], plain.linear(x.cpu(), w.cpu()), 1e-5, f"tile {tile}, {M} rows")
+            if not (gated or half or way.get("accumulate")):
+                close(outs[1].view(splits, M, N).sum(0), plain.linear(x.cpu(), w.cpu()), 1e-5, f"tile {tile}, {M} rows")
     assert seen == ({False} if N in (4080, 1552) else {True} if splits > 1 and tile != 11 else {True, False})
+
+
+@pytest.mark.parametrize("tile,splits,M,N,K", [
+    (7, 2, 256, 1024, 512), (7, 2, 257, 1024, 512), (7, 4, 512, 256, 480), (7, 2, 130, 208, 256), (7, 8, 400, 512, 992),
+    (7, 8, 160, 2048, 6144), (5, 4, 300, 384, 2048), (5, 2, 1100, 128, 224), (9, 3, 120, 512, 352), (9, 3, 120, 528, 352),
+    (11, 4, 300, 1536, 512), (4, 4, 600, 1024, 1312), (10, 2, 300, 208, 192)])
+def test_every_unit_of_a_product_in_ranges_is_done_once(tile, splits, M, N, K):
+    """Workgroups numbered by tiles in every range, and with the ranges last, over tiles that are a multiple of eight and
+    over others: each plane is the product over its own range of K, bit for bit."""
+    from tie_amd import kernels
+
+    x = rnd(M, K, seed=73, dtype=torch.bfloat16).cuda()
+    w = rnd(N, K, seed=74, scale=0.1, dtype=torch.bfloat16).cuda()
+    out = torch.full((splits, M, N), float("nan"), device="cuda")
+    kernels.gemm_bf16(x, kernels.pack_weight(w), out, tile=tile, splits=splits)
+    each = -(-(K // 32) // splits) * 32
+    for s in range(splits):
+        part = slice(s * each, min(K, (s + 1) * each))
+        want = torch.full((M, N), float("nan"), device="cuda")
+        kernels.gemm_bf16(x[:, part].contiguous(), w[:, part].contiguous(), want, tile=tile)
+        assert torch.equal(out[s], want), (tile, splits, s, kernels.gemm_ranges_last(M, N, K, tile, splits))
 
 
 @pytest.mark.parametrize("N,K", [(16, 96), (48, 128), (208, 4096), (1024, 352)])

@@ -193,6 +193,19 @@ def test_packed_weights_go_past_the_caches_where_they_are_read_once(tile, splits
     assert kernels.gemm_weights_past_caches(M, N, K, tile, splits) == past
 
 
+@pytest.mark.parametrize("tile,splits,M,N,K,last", [
+    (7, 1, 512, 2048, 2048, False), (7, 4, 128, 2048, 2048, False), (7, 4, 512, 2048, 2048, True), (7, 2, 400, 4096, 2048, True),
+    (9, 4, 120, 2048, 2048, False), (9, 8, 120, 2048, 6144, False), (9, 4, 120, 2000, 2048, False), (9, 4, 120, 2064, 2048, True),
+    (7, 4, 256, 1024, 3072, False), (7, 4, 200, 3584, 3584, False), (7, 4, 160, 4096, 4096, False), (7, 2, 300, 4096, 2048, False),
+    (7, 8, 160, 2048, 6144, True), (4, 4, 600, 4096, 12288, True), (11, 2, 300, 2560, 4096, True), (10, 2, 700, 3584, 18944, True)])
+def test_ranges_of_k_come_last_where_a_die_then_reads_less(tile, splits, M, N, K, last):
+    """Tiles that are no multiple of eight, four row tiles and more, or ranges that spare a die 1.5 MB of x. Elsewhere the
+    order by tiles is the faster one, by up to 1.6 us a product (256 rows over 1024 x 3072, 200 over 3584 x 3584)."""
+    from tie_amd import kernels
+
+    assert kernels.gemm_ranges_last(M, N, K, tile, splits) == last
+
+
 @pytest.mark.parametrize("M,N,K,want", [(2048, 4096, 12288, (1, 5)), (2048, 4096, 4096, (1, 5)), (2048, 2048, 6144, (2, 5)),
                                         (512, 4096, 12288, (4, 5)), (512, 2048, 2048, (4, 7))])
 def test_products_that_add_to_the_stream_have_a_plan_of_their_own(M, N, K, want):

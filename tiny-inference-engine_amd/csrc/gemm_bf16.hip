@@ -307,10 +307,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
   extern __shared__ bf16_t lds[];
 
   // Workgroups go to the eight dies in turn; a die takes a run of consecutive tiles, in which the row tiles of one piece of w
-  // follow each other. Ranges of K (a grid of one dimension): a run of consecutive units, the ranges last, so that a die
-  // reads its ranges' part of x alone, where it read x whole with its columns of every range: 512 rows over 2048 x 2048 in
-  // four ranges 11.9 -> 10.8 us, over 4096 x 12288 54.4 -> 51.9, over 2048 x 6144 21.7 -> 21.1. One row tile is too little to
-  // read for that (64 rows over 6144 x 4096 in four 15.9 us, 16.2 that way).
+  // follow each other. In a grid of one dimension (dma_ranges_last) a run of consecutive units, the ranges of K last.
   const int total = tiles_m * tiles_n;
   int id = blockIdx.x, split = blockIdx.y;
   if (EPI == 0 && static_cast<int>(gridDim.x) != total) {
@@ -417,6 +414,24 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
 #endif
 }
 
+// Whether a product in ranges of K counts its workgroups through with the ranges last (a grid of one dimension), so that a die
+// takes its ranges whole and reads their part of x alone; else a die takes its tiles in every range. Steps of 65 to 4096 rows
+// over nine layer shapes, the products' order changed one by one:
+//   * tiles that are no multiple of eight: without it their row tiles are on different dies. 0.5 to 15 us a product less.
+//   * four row tiles and more: 0.9 us less in the mean (512 rows over 4096 x 2048 in two ranges the same, over 2048 x 2048 in
+//     four 0.9, 400 over 2048 x 6144 0.8, 1024 over 6144 x 2560 13).
+//   * two and three: in four ranges and more where what is not read again, the other ranges' part of x, is 1.5 MB and more
+//     (160 rows over 2048 x 6144 in eight 0.6 less, 300 over 4096 x 12288 2.4). Below that it is the longer way, by the
+//     division and by ranges that all dies would write: 256 rows over 1024 x 3072 1.0 us more, 200 over 3584 x 3584 1.6, 160
+//     over 4096 x 4096 0.9; 65 to 128 rows on tiles of 64 x 128 the same either way.
+// Taken everywhere 474 products gain 564 us and lose 89, by this rule 535 and 28; a step of 230 tokens on the 0.6B shape 2.1 %
+// less than with it everywhere, 576 on 1536 x 8960 10 % less than without.
+static bool dma_ranges_last(int bm, int bn, int M, int N, int K, int splits) {
+  const long tiles_m = (M + bm - 1) / bm, tiles = tiles_m * ((N + bn - 1) / bn);
+  if (splits == 1 || tiles_m == 1) return false;
+  return tiles % GB_XCDS != 0 || tiles_m >= 4 || (splits >= 4 && 2L * M * K / splits * (splits - 1) >= 3L << 19);
+}
+
 template <int BM, int BN, bool PW, bool W_ONCE>
 static int launch_gemm_dma_as(const void* x, const void* w, void* out, int epi, int M, int N, int K, int splits,
                            hipStream_t stream) {
@@ -427,7 +442,7 @@ static int launch_gemm_dma_as(const void* x, const void* w, void* out, int epi, 
   const size_t shared = GdShape<BM, BN>::LDS_BYTES;
   const long tiles = static_cast<long>(tiles_m) * tiles_n;
   if (tiles * splits > 0x7fffffffL) return TIE_BAD_ARGUMENT;
-  const bool ranges_last = splits > 1 && tiles_m > 1;              // splits > 1: epi 0 (planes)
+  const bool ranges_last = dma_ranges_last(BM, BN, M, N, K, splits);       // splits > 1: epi 0 (planes)
   const dim3 grid(static_cast<unsigned>(ranges_last ? tiles * splits : tiles), ranges_last ? 1 : splits);
 #define LAUNCH(EPI)                                                                                          \
   {                                                                                                          \
@@ -453,9 +468,10 @@ static int launch_gemm_dma_as(const void* x, const void* w, void* out, int epi, 
 //     lose (64 sequences on the 1.7B shape 1921 us kept and 1931).
 //   * tiles of 128 x 192 only where a die has all row tiles of a piece of w (tiles a multiple of eight), up to eight of them,
 //     and they stay together: from four on a last one with few rows runs ahead, by the more the longer the range, and the
-//     others find nothing in the L2 of what it read. Inside the rule 512 rows over 6144 x 4096 2.6 us less, 256 over 24576 x 4096 2.1, 400
-//     over 12288 x 2048 0.5; 75 products 55 us less and 5.0 more, 1.2 the worst. Outside it 200 rows over 19456 x 2560 5.3 us
-//     more, 200 over 17920 x 1536 2.8, 400 over 10240 x 5120 10.3, 1107 over 4096 x 2048 7.8 (a step 3.7 %).
+//     others find nothing in the L2 of what it read. Inside the rule 512 rows over 6144 x 4096 2.6 us less, 256 over
+//     24576 x 4096 2.1, 400 over 12288 x 2048 0.5; 75 products 55 us less and 5.0 more, 1.2 the worst. Outside it 200 rows
+//     over 19456 x 2560 5.3 us more, 200 over 17920 x 1536 2.8, 400 over 10240 x 5120 10.3, 1107 over 4096 x 2048 7.8 (a step
+//     3.7 %).
 // More row tiles of the others want w back from the L2 (512 rows over 2048 x 2048 in four ranges on 128 x 128 10.6 us kept and
 // 11.5); tiles of 256 rows are the same either way. Rows of row-major weights come as half lines, two loads a line, and stay
 // cached.
@@ -663,11 +679,19 @@ extern "C" int tie_gemm_bf16_tile(int M, int N, int K, int packed, int splits) {
   return gemm_plan(M, N, K, straight_to_lds_shape(N, K), splits, packed != 0).tile;
 }
 
+// Rows and columns of tiles 4 to 11.
+static const int kTileRows[] = {256, 256, 128, 128, 64, 64, 256, 128}, kTileColumns[] = {256, 128, 256, 128, 256, 128, 192, 192};
+
 // Whether that product over packed weights, on tile 4 to 11, asks for them past the caches; for tests and sweeps.
 extern "C" int tie_gemm_bf16_w_past_caches(int M, int N, int K, int tile, int splits) {
-  static const int rows[] = {256, 256, 128, 128, 64, 64, 256, 128}, columns[] = {256, 128, 256, 128, 256, 128, 192, 192};
   if (tile < 4 || tile > 11 || M <= 0 || splits < 1) return 0;
-  return w_past_caches(rows[tile - 4], columns[tile - 4], M, N, K, splits);
+  return w_past_caches(kTileRows[tile - 4], kTileColumns[tile - 4], M, N, K, splits);
+}
+
+// Whether its ranges of K come last in the order of the workgroups; for tests and sweeps.
+extern "C" int tie_gemm_bf16_ranges_last(int M, int N, int K, int tile, int splits) {
+  if (tile < 4 || tile > 11 || M <= 0 || splits < 1) return 0;
+  return dma_ranges_last(kTileRows[tile - 4], kTileColumns[tile - 4], M, N, K, splits);
 }
 
 // out_dtype: TIE_F32 or TIE_BF16; accumulate adds into a float32 output; gated (bfloat16 output of N / 2

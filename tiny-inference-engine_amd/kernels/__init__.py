@@ -249,6 +249,7 @@ _SIGNATURES = {
         "tie_gemm_bf16_adding_plan": [_c_int, _c_int, _c_int, ctypes.POINTER(_c_int)],
         "tie_gemm_bf16_tile": [_c_int, _c_int, _c_int, _c_int, _c_int],
         "tie_gemm_bf16_w_past_caches": [_c_int, _c_int, _c_int, _c_int, _c_int],
+        "tie_gemm_bf16_ranges_last": [_c_int, _c_int, _c_int, _c_int, _c_int],
         "tie_gemm_bf16_wins_few_rows": [_c_int, _c_int, _c_int, _c_int, _c_int],
         "tie_gemm_bf16": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                           _c_int, _c_void],
@@ -1057,6 +1058,11 @@ def gemm_tile(M: int, N: int, K: int, packed: bool = False, splits: int = 0) -> 
 def gemm_weights_past_caches(M: int, N: int, K: int, tile: int, splits: int = 1) -> bool:
     """Whether ``gemm_bf16`` on ``tile`` (4 to 11) asks for a packed ``[N, K]`` weight past the caches."""
     return bool(_lib("gemm_bf16").tie_gemm_bf16_w_past_caches(M, N, K, tile, splits))
+
+
+def gemm_ranges_last(M: int, N: int, K: int, tile: int, splits: int) -> bool:
+    """Whether ``gemm_bf16`` on ``tile`` (4 to 11) numbers its workgroups with the ranges of K last."""
+    return bool(_lib("gemm_bf16").tie_gemm_bf16_ranges_last(M, N, K, tile, splits))
 
 
 def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool = False, tile: int = 0,
