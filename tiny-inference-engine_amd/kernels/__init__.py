@@ -1366,15 +1366,20 @@ def attention_f32_splits(tiles: int, num_kv_heads: int, group_size: int, max_con
     """Shares the keys of every column tile are cut into: more than one only where the tiles alone leave CUs idle.
 
     One workgroup fills a CU, so all of them run at once up to 256: beyond that a second round costs more than shorter
-    shares give (16 sequences of 1000 keys, 8 KV heads: two shares 30.3 us, three 39.4). Up to there a share is down to four
-    tiles of 16 keys, half a tile for each of its waves: what a workgroup starts and ends with and the merge weigh more
-    then (one sequence of 300 keys: 1, 2, 4, 5, 8 shares 15.2, 12.6, 10.8, 9.9, 9.7 us; 24 shares of 4000 keys 16.2,
-    32 of them 17.6). Same in the other head sizes: 256 dimensions, 4 KV heads, 300 keys 22.7 us in one share, 11.3 in ten.
+    shares give (16 sequences of 1000 keys, 8 KV heads: two shares 30.3 us, three 39.4; of 30 to 1900 keys a layer of the step
+    2.4 to 3.8 us less with two than with four; heads of 64, of which two would fit, the same within 0.7).
+    ``max_context`` is the longest context of a bucket (1024, 2048, ...) that a recorded step serves (other steps are planned
+    by it too, so that keys cut the same way give the same bits whichever step reads them), and shares for its end cost a
+    short context more than they hold. One to four sequences, 8 KV heads, 30, 100, 250, 500 and 900 keys, a layer against four
+    shares: eight +0.3, +0.3, -0.1, -1.3, -2.8 us, sixteen +1.2, +1.0, +0.4, -1.1, -4.0; prompts of 2 to 40 tokens eight +0.2
+    to +0.6, behind 500 others -1.9. So a share is eight tiles of 16 keys at the bucket's end, one for each of its waves; 1900
+    keys in sixteen take 1.9 to 2.6 us less than in eight, 3900 in twenty-four 1.3 less than in sixteen (32 shares of 4000 keys
+    17.6 us, 24 of them 16.2).
     """
     workgroups = tiles * num_kv_heads * -(-group_size // 16)
     by_fill = 256 // max(1, workgroups)
     key_tiles = max(1, -(-max_context // 16))
-    shares = max(1, min(24, by_fill, -(-key_tiles // 4)))
+    shares = max(1, min(24, by_fill, -(-key_tiles // 8)))
     return -(-key_tiles // -(-key_tiles // shares))         # none of them empty
 
 
