@@ -253,6 +253,38 @@ def test_packed_experts_of_few_rows_take_every_batch_of_blocks(blocks):
     close(parts.cpu()[place], b, 6e-6, "down")                # exact products, float32 sums of K <= 2240
 
 
+@pytest.mark.parametrize("counts", [(16, 17, 0, 1, 33), (40,), (1, 1, 18, 2), (15, 0, 32, 16, 0)])
+def test_rows_of_an_expert_with_several_tiles_keep_their_bits(counts):
+    """Row tiles of 16: an expert's weights are asked for one way where it has one tile and another where it has more. A row's
+    sums are the same ones, in a step of all rows and in steps of up to 16 rows of one expert."""
+    from tie_amd import kernels
+
+    bf, K, F_, E, T = torch.bfloat16, 352, 96, len(counts), sum(counts)
+    h = rnd(T, K, seed=1).to(bf).cuda()
+    gate, up, down = (rnd(*n, seed=s, scale=0.1).to(bf).cuda() for n, s in (((E, F_, K), 2), ((E, F_, K), 3), ((E, K, F_), 4)))
+    up_packed, down_packed = kernels.pack_experts(gate, up, down)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=torch.Generator().manual_seed(2))]
+    ids = ids.to(torch.int32)
+
+    def results(picked):
+        n, get = len(picked), scratch_memory()
+        rows = kernels.moe_align(ids[picked].view(-1, 1).cuda(), E, 16, get)
+        act, parts = get("act", (n, F_), bf), get("parts", (n, K))
+        kernels.moe_gate_up(h[picked.cuda()], None, up_packed, rows, act)
+        kernels.moe_down(act, down_packed, rows, parts)
+        at = rows.where.view(-1).long()
+        return act[at], parts[at]
+
+    act, parts = results(torch.arange(T))
+    assert bool(torch.isfinite(parts).all())
+    for e in range(E):
+        mine = torch.nonzero(ids == e).view(-1)
+        for first in range(0, len(mine), 16):
+            picked = mine[first:first + 16]
+            alone = results(picked)
+            assert torch.equal(alone[0], act[picked.cuda()]) and torch.equal(alone[1], parts[picked.cuda()]), (e, first)
+
+
 @pytest.mark.parametrize("activation", ["silu", "sigmoid"])
 def test_the_gated_norm_of_the_heads_outputs(activation):
     from tie_amd import kernels

@@ -13,8 +13,10 @@
 // of 32 experts of 768 x 2048, 4 a row: 1 row 7.9 and 4.8 us -> 6.5 and 4.4, 8 rows 26.8 and 13.4 -> 25.7 and 12.2, 32
 // rows 37.4 and 19.5 -> 33.6 and 18.8. Weights before x's rows, all in registers of their own: mixed, the compiler gave
 // them 40 registers in turn and waited in between. Six blocks at once where a wave has six or seven left: an inner size of
-// 768 in one trip (measured at that size alone). The weights go past the caches: a block is read by one workgroup (a decode
-// step of 8 rows over five such layers 484 -> 465 us).
+// 768 in one trip (measured at that size alone). The weights of an expert with one row tile go past the caches: a block is
+// then read by one workgroup (a decode step of 8 rows over five such layers 484 -> 465 us, of 16 rows over four layers of 64
+// experts of 1536 x 4096 855 -> 791). Those of an expert with more rows than a tile holds stay in them for the next tile: past
+// the caches 170 rows, 10.6 an expert in the mean and unevenly routed, took a step 2093 to 2159 us where kept 2047 to 2071.
 // Row tiles of 64, 128 or 256 (many rows an expert): the dense product's tile (gemm_dma.h), x's rows gathered by slot on
 // their way into LDS. Which tiles exist is known on the device only; the grid covers the most there can be, and the
 // workgroups that have one are numbered so that each of the 8 XCDs works on a contiguous run of tiles (an expert's row
@@ -44,7 +46,8 @@ __global__ __launch_bounds__(256) void moe_packed_few_rows_kernel(const bf16_t* 
   // nothing that is used.
   const int tiles = *rw.num_tiles;
   const int e = rw.tiles[2 * tile], place0 = rw.tiles[2 * tile + 1];
-  asm volatile("" ::"s"(e), "s"(place0));                    // else the compiler moves their loads behind the branch
+  const int before = rw.tiles[max(2 * tile - 2, 0)], after = rw.tiles[min(2 * tile + 2, 2 * static_cast<int>(gridDim.x) - 2)];
+  asm volatile("" ::"s"(e), "s"(place0), "s"(before), "s"(after));      // else the compiler moves their loads behind the branch
   if (tile >= tiles) return;                                 // the whole workgroup leaves
   __shared__ floatx4_t sums[NT][4][TIE_WAVE];
   const int lane = threadIdx.x & (TIE_WAVE - 1);
@@ -69,15 +72,17 @@ __global__ __launch_bounds__(256) void moe_packed_few_rows_kernel(const bf16_t* 
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) acc[nt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
   int kb = wave;
-  auto blocks = [&](auto depth, auto first) {                // DEPTH of this wave's k-blocks, every load before the first use
+  auto blocks = [&](auto depth, auto first, auto once) {     // DEPTH of this wave's k-blocks, every load before the first use
     constexpr int DEPTH = decltype(depth)::value;
     uint4 xf[DEPTH];
     moe_u32x4_t wf[NT][DEPTH];
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-        wf[nt][i] = __builtin_nontemporal_load(reinterpret_cast<const moe_u32x4_t*>(wr[nt] + static_cast<size_t>(kb + 4 * i) * 512));
+      for (int nt = 0; nt < NT; ++nt) {
+        const moe_u32x4_t* p = reinterpret_cast<const moe_u32x4_t*>(wr[nt] + static_cast<size_t>(kb + 4 * i) * 512);
+        wf[nt][i] = decltype(once)::value ? __builtin_nontemporal_load(p) : *p;
+      }
     __builtin_amdgcn_sched_barrier(0);                       // the weights are on their way before the slot is waited for
     if constexpr (decltype(first)::value) look_up();
 #pragma unroll
@@ -91,25 +96,30 @@ __global__ __launch_bounds__(256) void moe_packed_few_rows_kernel(const bf16_t* 
                                                           *reinterpret_cast<const bf16x8_t*>(&xf[i]), acc[nt], 0, 0, 0);
     kb += 4 * DEPTH;
   };
-  constexpr std::true_type first{};
-  constexpr std::false_type later{};
-  if (kb + 28 < kblocks) {
-    blocks(std::integral_constant<int, 8>{}, first);
-    while (kb + 28 < kblocks) blocks(std::integral_constant<int, 8>{}, later);
-  } else if (kb + 20 < kblocks) {
-    blocks(std::integral_constant<int, 6>{}, first);
-  } else if (kb + 12 < kblocks) {
-    blocks(std::integral_constant<int, 4>{}, first);
-  } else if (kb + 4 < kblocks) {
-    blocks(std::integral_constant<int, 2>{}, first);
-  } else {
-    if (kb < kblocks) blocks(std::integral_constant<int, 1>{}, first);
-    else look_up();
-  }
-  if (kb + 20 < kblocks) blocks(std::integral_constant<int, 6>{}, later);
-  if (kb + 12 < kblocks) blocks(std::integral_constant<int, 4>{}, later);
-  if (kb + 4 < kblocks) blocks(std::integral_constant<int, 2>{}, later);
-  if (kb < kblocks) blocks(std::integral_constant<int, 1>{}, later);
+  auto walk = [&](auto once) {
+    constexpr std::true_type first{};
+    constexpr std::false_type later{};
+    if (kb + 28 < kblocks) {
+      blocks(std::integral_constant<int, 8>{}, first, once);
+      while (kb + 28 < kblocks) blocks(std::integral_constant<int, 8>{}, later, once);
+    } else if (kb + 20 < kblocks) {
+      blocks(std::integral_constant<int, 6>{}, first, once);
+    } else if (kb + 12 < kblocks) {
+      blocks(std::integral_constant<int, 4>{}, first, once);
+    } else if (kb + 4 < kblocks) {
+      blocks(std::integral_constant<int, 2>{}, first, once);
+    } else {
+      if (kb < kblocks) blocks(std::integral_constant<int, 1>{}, first, once);
+      else look_up();
+    }
+    if (kb + 20 < kblocks) blocks(std::integral_constant<int, 6>{}, later, once);
+    if (kb + 12 < kblocks) blocks(std::integral_constant<int, 4>{}, later, once);
+    if (kb + 4 < kblocks) blocks(std::integral_constant<int, 2>{}, later, once);
+    if (kb < kblocks) blocks(std::integral_constant<int, 1>{}, later, once);
+  };
+  // An expert's tiles are neighbours in the table.
+  if ((tile > 0 && before == e) || (tile + 1 < tiles && after == e)) walk(std::false_type{});
+  else walk(std::true_type{});
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) sums[nt][wave][lane] = acc[nt];
   __syncthreads();
