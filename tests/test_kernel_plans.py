@@ -515,6 +515,17 @@ def test_whole_sequences_are_launched_so_that_long_ones_meet_short_ones(S, heads
     assert kernels.decode_wave_plan(lens[:511 // heads or 1], heads, 2048, 16, None, 128)[2] is None
 
 
+@pytest.mark.parametrize("S,heads,tokens,window", [(64, 8, 500, None), (129, 4, 1000, None), (86, 6, 33, None), (64, 8, 3000, 1024)])
+def test_sequences_of_one_length_are_not_sorted(monkeypatch, S, heads, tokens, window):
+    """They meet their like in any order: the host, which eager and short steps wait for, plans nothing for them. A recorded
+    step reads an order all the same."""
+    from tie_amd import kernels
+
+    monkeypatch.setattr(kernels, "whole_sequences_order", lambda *args: pytest.fail("sorted"))
+    shares, length, order = kernels.decode_wave_plan([tokens] * S, heads, 4096, 16, window, 128)
+    assert (shares, length) == (1, 0) and order.dtype.name == "int32" and order.tolist() == list(range(S))
+
+
 def test_whole_sequences_in_order_where_shares_were_planned():
     """64 sequences of which the long ones come 32 apart: 1.9 times the mean as they come, 1.0 in order."""
     from tie_amd import kernels

@@ -1673,8 +1673,9 @@ def whole_sequences_fill(tiles, num_kv_heads: int, head_dim: int, limit: Optiona
 
 
 def decode_share_plan(context_lens, num_kv_heads: int, plan_context: int, block_size: int = 16,
-                      window: Optional[int] = None, head_dim: int = 0) -> "tuple":
-    """``(shares, share_tiles)`` for a step of single decoded tokens over sequences of these lengths.
+                      window: Optional[int] = None, head_dim: int = 0, tiles: "Optional[list]" = None) -> "tuple":
+    """``(shares, share_tiles)`` for a step of single decoded tokens over sequences of these lengths (``tiles``: their
+    ``key_tiles``, where the caller has them).
 
     ``share_tiles`` = 0: every sequence's keys go into ``shares`` equal parts of its own (``decode_splits``): the
     rule for sequences of about one length. A wave walks its share tile after tile, so the longest share sets
@@ -1695,7 +1696,8 @@ def decode_share_plan(context_lens, num_kv_heads: int, plan_context: int, block_
     equal = decode_splits(S, num_kv_heads, plan_context, block_size)
     if block_size < 16 or S < 2 or BALANCED_SHARES_MAX_EQUAL <= 0:
         return equal, 0
-    tiles = key_tiles(context_lens, window)
+    if tiles is None:
+        tiles = key_tiles(context_lens, window)
     longest = max(tiles)
     if longest * S < 1.25 * sum(tiles):
         return equal, 0
@@ -1730,13 +1732,15 @@ def decode_wave_plan(context_lens, num_kv_heads: int, plan_context: int, block_s
     mean (64 sequences of 20 to 3000 keys at random, 1.54 in order: 63.2 us a layer, in shares of one length 60.5; 90 of up to
     2000, 1.16: 65.6).
     """
-    shares, share_tiles = decode_share_plan(context_lens, num_kv_heads, plan_context, block_size, window, head_dim)
-    if len(context_lens) * num_kv_heads < 2 * COMPUTE_UNITS or shares > 1 and not share_tiles:
-        return shares, share_tiles, None
     tiles = key_tiles(context_lens, window)
+    shares, share_tiles = decode_share_plan(context_lens, num_kv_heads, plan_context, block_size, window, head_dim, tiles)
+    if len(tiles) * num_kv_heads < 2 * COMPUTE_UNITS or shares > 1 and not share_tiles:
+        return shares, share_tiles, None
+    if min(tiles) == max(tiles):         # any order will do; a recorded step reads one
+        return shares, share_tiles, np.arange(len(tiles), dtype=np.int32) if shares == 1 else None
     order = whole_sequences_order(tiles, num_kv_heads)
     if share_tiles and decode_splits(len(tiles), num_kv_heads, plan_context, block_size) == 1 and \
-            whole_sequences_fill([tiles[i] for i in order], num_kv_heads, head_dim, WHOLE_SEQUENCES_ORDERED):
+            whole_sequences_fill([tiles[i] for i in order.tolist()], num_kv_heads, head_dim, WHOLE_SEQUENCES_ORDERED):
         shares, share_tiles = 1, 0
     return shares, share_tiles, order if shares == 1 else None
 
