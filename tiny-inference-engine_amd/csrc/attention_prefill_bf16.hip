@@ -882,8 +882,10 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // run backwards, so that long and short ones meet. Four in a row, the shares and heads of one sequence, made its
     // compute unit the one that the launch waited for (300 rows beside 31 sequences of 50 to 2500 keys at random, a step of
     // 28 layers 4250 -> 3710 us, beside 60 of up to 1500 4430 -> 3980). Where most shares are empty, as in grids
-    // of many shares of one length, they are better off in a row (two of 4000 keys among 29 of 300, 32 shares each: 3790 and
-    // 3890; eight of 3000 among 40, 16 shares: 3875 and 3855).
+    // of many shares of one length, they are better off in a row: beside 300 and 1000 rows and 512 behind 1500, 32 shares each
+    // of two sequences of 4000 keys among 29 of 300 take 0.3 to 2.9 % more dealt out, of one among 60 of 100 2.9 to 5.0 %, of
+    // four of 8000 among 28 of 200 0 to 1.4 % (64 shares of one of 16000 among 31 of 500 0.2 to 1.1 % less); 16 shares, eight
+    // of 3000 among 40, 0.5 to 1.0 % less, 8 shares 4.2 % less to 0.6 more, shares of their own up to four 2.5 to 8.1 % less.
     const int in_run = static_cast<int>(blockIdx.x);
     const int at = single.share_tiles != nullptr && single.nsplit > 16 ? in_run * single.waves + wave
                                                  : wave * decode_groups + (wave & 1 ? decode_groups - 1 - in_run : in_run);

@@ -100,7 +100,7 @@ struct DeltaChunks {
   float* decay;            // [1]: e^(b_end)
 };
 
-// WIDE: q and k of every head start on 16-byte addresses and d is a multiple of 4. Bound by memory: 160 KB in and 144 KB out
+// WIDE: q and k of every head start on 16-byte addresses and d is a multiple of 4. Bound by memory: 96 KB in and 144 KB out
 // a workgroup, of which a compute unit holds two. 2048 tokens of 16 heads: 35.5 us with eight waves, 37.5 with four, which
 // did both products one after the other; 34.1 (3.6 TB/s) since W and P leave in whole lines and not word by word.
 template <bool WIDE>

@@ -521,8 +521,10 @@ static bool gemm_dma_takes(const void* x, const void* w, const void* out, int N,
 // shapes, 768 to 8192 wide with inner sizes of 3072 to 28672, at six to fifteen row counts from 140 to 2048, each candidate
 // timed with its consumer and the weights from memory. The choice lies 1.4 % (products that store) and 2.1 % (products that
 // add to the stream) above the best forced one there, 1.5 and 2.3 % over seven shapes held out; 0.4 % over the shapes of
-// 1024 to 4096 that models have; a third at worst, where K below 1024 is not cut. 65 to 128 rows: 0.4 % above the best. Rows
-// of fewer than 65 over row-major weights and odd K or N stay with the older tiles and their rule.
+// 1024 to 4096 that models have; a third at worst, where K below 1024 is not cut. 65 to 128 rows: 0.4 % above the best over
+// eight of those shapes, 0.9 % over random weights, 15 % at worst, fitted before the tiles of 128 x 128 and 128 x 256 read two
+// steps ahead (about 5 % less a slice since; those of 64 rows by 128 have the loop they had). Rows of fewer than 65 over
+// row-major weights and odd K or N stay with the older tiles and their rule.
 // A product that adds to the stream has a table of its own: in place it reads what it adds to, and its planes are read by the
 // norm. 2048 rows over 4096 x 12288 with the norm behind it: two planes of 256 x 256 tiles 203 us, 256 x 128 in place 182.
 struct GemmPlan { int tile, splits; };
@@ -545,7 +547,8 @@ static int legacy_splits(int M, int N, int K) {
 // of workgroups to a full one both grow, by full_us and by the factor 1 + press: the units share the L2 and the clock.
 // lead: what a slice gains as the last row tile empties: its workgroups run ahead and bring w into the L2 for the others
 // (576 rows over 4096 x 12288 in two ranges of 256 x 256 take 117 us, 512 take 146). scatter: what it loses where the tiles
-// are no multiple of eight, so that the row tiles of one piece of w do not follow each other on one die.
+// are no multiple of eight, so that the row tiles of one piece of w do not follow each other on one die; fitted before ranges
+// of such tiles came last (dma_ranges_last), which then lose less than it says.
 // per_cu workgroups on one compute unit each take `shared` times as long.
 struct DmaTile { int id, bm, bn; float start_us, full_us, slice_us, press, lead, scatter; int per_cu; float shared; };
 static const DmaTile kDmaTiles[] = {{4, 256, 256, 7.02f, 4.26f, 0.622f, 0.135f, 0.121f, 0.114f, 1, 1.f},
@@ -664,8 +667,8 @@ extern "C" int tie_gemm_bf16_splits(int M, int N, int K, int packed) {
   return gemm_plan(M, N, K, straight_to_lds_shape(N, K), 0, packed != 0).splits;
 }
 
-// The same for a product over a packed weight that is added to the float32 stream, in place (1) or as planes that the next norm adds: the tile
-// it then runs on in *tile.
+// The same for a product over a packed weight that is added to the float32 stream, in place (1) or as planes that the next
+// norm adds: the tile it then runs on in *tile.
 extern "C" int tie_gemm_bf16_adding_plan(int M, int N, int K, int* tile) {
   const bool straight = straight_to_lds_shape(N, K);
   const GemmPlan plan = gemm_plan(M, N, K, straight, straight ? 0 : 1, true, true);

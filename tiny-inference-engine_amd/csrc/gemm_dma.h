@@ -6,10 +6,9 @@
 // wave tiles above. k advances in groups of G slices of 32 through a ring of LDS stages: while group t is
 // multiplied, the groups behind it are landing or landed and the loads of t + STAGES - 1 (its w rows) and t + STAGES
 // (its x rows) are issued, a few between the matrix instructions so that neither the texture
-// path nor the in-order instruction stream of the one wave backs up. One barrier a group: it sits before the last 16 k's
-// matrix instructions, when their fragments are in
-// registers already, so that the stage is free and the next group's first fragments can be read
-// while they multiply.
+// path nor the in-order instruction stream of the one wave backs up. One barrier a group: it sits before the matrix
+// instructions of the last steps of 16 k (GdShape::AHEAD: two in groups of two slices, else one), when their fragments are
+// in registers already, so that the stage is free and the next group's first fragments can be read while they multiply.
 //
 // A group is two slices wherever three stages of that size fit the LDS: half the barriers, and x's rows come as whole
 // 128-byte lines. With one slice a row is half a line, for which the vector cache takes as long: the product then stood
@@ -310,12 +309,11 @@ __device__ __forceinline__ void gemm_dma_tile_groups(bf16_t* lds, const __amdgpu
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[set][j], fa[set][i], acc[i][j], 0, 0, 0);
   };
 
-  // A stage is free once every wave has passed the barrier of the slice that read it, which stands in the
-  // middle of that slice (its last fragments are in registers by then). Slice j's x rows are asked for right
-  // after the barrier of slice j - STAGES, into the stage that slice has just left, and its w rows before the barrier
-  // of slice j - STAGES + 1: the loads of STAGES - 2 to STAGES - 1 slices are in flight at any time, which is what
-  // the latency of L2 asks for at a slice every 0.4 us. (With four stages of 256 x 256, 64 to 96 KB; one slice less ahead,
-  // the matrix cores waited a third of the time.) The first slices here.
+  // A stage is free once every wave has passed the barrier of the group that read it, which stands in the
+  // middle of that group (its last fragments are in registers by then). Group j's x rows are asked for right
+  // after the barrier of group j - STAGES, into the stage that group has just left, and its w rows before the barrier
+  // of group j - STAGES + 1: the loads of STAGES - 2 to STAGES - 1 groups are in flight at any time, which is what
+  // the latency of L2 asks for. The first groups here.
 #pragma unroll
   for (int t = 0; t < STAGES - 1; ++t) {
     if ((G > 1 || t > 2) && t >= steps) break;          // the host gives every range of K at least three slices

@@ -1043,8 +1043,8 @@ def gemm_splits(M: int, N: int, K: int, packed: bool = False) -> int:
 
 
 def gemm_adding_plan(M: int, N: int, K: int) -> tuple:
-    """``(ranges, tile)`` of a product of M > 64 rows over a packed ``[N, K]`` weight that is added to the float32 stream: in place with one range, else
-    as planes that the next norm adds."""
+    """``(ranges, tile)`` of a product of M > 64 rows over a packed ``[N, K]`` weight that is added to the float32 stream: in
+    place with one range, else as planes that the next norm adds."""
     tile = _c_int(0)
     ranges = int(_lib("gemm_bf16").tie_gemm_bf16_adding_plan(M, N, K, ctypes.byref(tile)))
     return ranges, int(tile.value)
