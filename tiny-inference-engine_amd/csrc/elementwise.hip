@@ -130,17 +130,21 @@ __global__ void rms_norm_row_kernel(float* __restrict__ x, const float* __restri
 template <typename TO, int COUNT>
 static void launch_rms_norm_row(float* x, const float* partials, size_t stride, const float* w, float eps, TO* out,
                                 const int* rows, int R, int n, hipStream_t stream) {
-  // As many threads as the row has float4, up to 1024: measured faster than fewer threads with more loads each. Where many rows
-  // come without planes, fewer threads are: a compute unit holds two workgroups of 1024, which wait for memory and for each
-  // other in turn, and eight of 256. 2048 rows of 4096 12.1 -> 9.2 us, of 5120 13.1 -> 12.0, of 2048 6.2 -> 5.3, 512 rows of
-  // 4096 4.7 -> 4.4; with planes it is the same time either way (2048 rows of 4096, two planes 23.4 and 23.2).
+  // As many threads as the row has float4, up to 1024: measured faster than fewer threads with more loads each. Where more rows
+  // than run at once come without planes, fewer threads are: a compute unit holds two workgroups of 1024, which wait for memory
+  // and for each other in turn, and eight of 256. 2048 rows of 4096 12.1 -> 9.2 us, of 5120 13.1 -> 12.0, of 2048 6.2 -> 5.3;
+  // 576 to 1300 rows of 2560 to 8192 3 to 21 % less. Up to what runs at once (512 rows, 1024 of 2048 numbers) they are the
+  // same or slower (512 rows of 2048 3.47 -> 3.58, of 6144 5.60 -> 5.81); with planes it is the same time either way (2048
+  // rows of 4096, two planes 23.4 and 23.2).
   const int quads = n / 4;
   if constexpr (COUNT == 0) {
-    if (R >= 512 && quads >= 1024 && quads % 256 == 0) {
+    const int per_simd = (min(quads, 1024) + 4 * TIE_WAVE - 1) / (4 * TIE_WAVE);      // waves of a workgroup on a SIMD, of eight
+    const bool in_turns = R > 256 * (8 / per_simd);
+    if (in_turns && quads >= 1024 && quads % 256 == 0) {
       rms_norm_row_kernel<TO, COUNT, 4><<<R, quads / 4, 0, stream>>>(x, partials, stride, w, eps, out, rows, n);
       return;
     }
-    if (R >= 512 && quads >= 512 && quads <= 2048 && quads % 128 == 0) {
+    if (in_turns && quads >= 512 && quads <= 2048 && quads % 128 == 0) {
       rms_norm_row_kernel<TO, COUNT, 2><<<R, quads / 2, 0, stream>>>(x, partials, stride, w, eps, out, rows, n);
       return;
     }

@@ -421,9 +421,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
 //   * four row tiles and more: 0.9 us less in the mean (512 rows over 4096 x 2048 in two ranges the same, over 2048 x 2048 in
 //     four 0.9, 400 over 2048 x 6144 0.8, 1024 over 6144 x 2560 13).
 //   * two and three: in four ranges and more where what is not read again, the other ranges' part of x, is 1.5 MB and more
-//     (160 rows over 2048 x 6144 in eight 0.6 less, 300 over 4096 x 12288 2.4). Below that it is the longer way, by the
-//     division and by ranges that all dies would write: 256 rows over 1024 x 3072 1.0 us more, 200 over 3584 x 3584 1.6, 160
-//     over 4096 x 4096 0.9; 65 to 128 rows on tiles of 64 x 128 the same either way.
+//     (160 rows over 2048 x 6144 in eight 0.6 less, 300 over 4096 x 12288 2.4). Below that it is the longer way, of which
+//     the division is 0.2 to 0.3: 256 rows over 1024 x 3072 1.0 us more, 200 over 3584 x 3584 1.6, 160 over 4096 x 4096 0.9;
+//     65 to 128 rows on tiles of 64 x 128 the same either way.
 // Taken everywhere 474 products gain 564 us and lose 89, by this rule 535 and 28; a step of 230 tokens on the 0.6B shape 2.1 %
 // less than with it everywhere, 576 on 1536 x 8960 10 % less than without.
 static bool dma_ranges_last(int bm, int bn, int M, int N, int K, int splits) {
